@@ -1,8 +1,8 @@
 """Builds ``libsvodk_gfx950.so`` in-tree with hipcc, for gfx950 only.
 
-``python -m svod_amd.build`` compiles every source under ``csrc/`` into the library and
-then into the code objects under ``co/`` (``--code-objects``: only those).  The
-library is never built implicitly at import: loading fails loudly when it is
+``python -m svod_amd.build`` compiles every kernel source under ``csrc/`` into the library, the Python
+side's calls (``host.cpp``) into ``_host.so``, and then the kernels into the code objects under ``co/``
+(``--code-objects``: only those).  The library is never built implicitly at import: loading fails loudly when it is
 missing, so a stale or absent build cannot hide behind another code path.
 """
 from __future__ import annotations
@@ -15,6 +15,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsvodk_gfx950.so")
+HOST = os.path.join(HERE, "_host.so")  # the Python side's calls (csrc/host.cpp), a module of this package
 SOURCES = ["ops.cpp", "heads_kernel.hip", "attention_kernel.hip", "combine_kernel.hip", "rows_kernel.hip",
            "linear_kernel.hip", "decode_kernel.hip"]
 
@@ -65,6 +66,21 @@ def build(verbose: bool = False) -> str:
         list(pool.map(lambda job: _run(job[1], verbose), jobs))
     _run([cc, *DEVICE_FLAGS, "-shared", "-fPIC", "-o", LIB, *[obj for obj, _ in jobs]], verbose)
     return LIB
+
+
+def build_host(verbose: bool = False) -> str:
+    """``_host.so``: host code over torch's C++ interface, so it is compiled with g++ against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [f"-I{p}" for p in (*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"])]
+    libs = [f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM=1",
+          "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes,
+          os.path.join(CSRC, "host.cpp"), "-o", HOST, *libs], verbose)
+    return HOST
 
 
 def build_code_objects(verbose: bool = False) -> str:
@@ -132,4 +148,5 @@ if __name__ == "__main__":
         print(build_code_objects(verbose=True))
     else:
         print(build(verbose=True))
+        print(build_host(verbose=True))
         print(build_code_objects(verbose=True))

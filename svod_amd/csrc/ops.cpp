@@ -22,7 +22,13 @@
 namespace {
 
 // ---- per-thread records: ops::chosen (tk/src/ops/mod.rs:83-118) and the last error.
-thread_local std::string g_chosen;
+// A record is kept as the static strings it is made of: its text is written when it is asked for, not on every call.
+struct Chosen {
+  const char *op = nullptr, *family = nullptr, *cfg = nullptr;  // a kernel's family and config, or no family:
+  int why = 0;                                                  // the graph, and why
+};
+thread_local Chosen g_chosen;
+thread_local std::string g_chosen_text;
 thread_local std::string g_error;
 
 const char *fallback_name(int why) {
@@ -38,13 +44,18 @@ const char *fallback_name(int why) {
 
 // ran_graph (mod.rs:115-118).
 int ran_graph(const char *op, int why) {
-  g_chosen = std::string("Graph { op: \"") + op + "\", why: " + fallback_name(why) + " }";
+  g_chosen = {op, nullptr, nullptr, why};
   return why;
 }
 
 // ran (mod.rs:110-113).
-void ran(const char *op, const char *family, const char *cfg) {
-  g_chosen = std::string("Kernel { op: \"") + op + "\", family: \"" + family + "\", cfg: \"" + cfg + "\" }";
+void ran(const char *op, const char *family, const char *cfg) { g_chosen = {op, family, cfg, 0}; }
+
+std::string chosen_text() {
+  const Chosen &c = g_chosen;
+  if (c.op == nullptr) return "";
+  if (c.family == nullptr) return std::string("Graph { op: \"") + c.op + "\", why: " + fallback_name(c.why) + " }";
+  return std::string("Kernel { op: \"") + c.op + "\", family: \"" + c.family + "\", cfg: \"" + c.cfg + "\" }";
 }
 
 int fail(int status, const char *fmt, ...) {
@@ -256,7 +267,10 @@ extern "C" {
 
 int svodk_abi_version(void) { return SVODK_ABI_VERSION; }
 
-const char *svodk_last_chosen(void) { return g_chosen.c_str(); }
+const char *svodk_last_chosen(void) {
+  g_chosen_text = chosen_text();
+  return g_chosen_text.c_str();
+}
 
 const char *svodk_last_error(void) { return g_error.c_str(); }
 

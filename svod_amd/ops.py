@@ -151,6 +151,25 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     return lib
 
 
+_native = None
+
+
+def _calls():
+    """The native side of the calls below (``csrc/host.cpp``): tensors and option objects in, the library's
+    functions underneath.  Bound to the library ``load_library`` has loaded, once."""
+    global _native
+    if _native is None:
+        lib = load_library()
+        from . import _host
+
+        names = ("attention", "attention_noalloc", "attention_packed", "attention_workspace", "heads", "linear", "layer_norm",
+                 "add_layer_norm", "rms_norm", "add_rms_norm", "order_rows")
+        _host.bind({"svodk_" + n: ctypes.cast(getattr(lib, "svodk_" + n), ctypes.c_void_p).value for n in names}, OpError,
+                   _finish, tuple(_DTYPES))
+        _native = _host
+    return _native
+
+
 class Fallback(enum.IntEnum):
     """``Fallback`` of tk/src/ops/shape.rs:26-39."""
 
@@ -204,10 +223,6 @@ def _ref(keep: list, t: Optional[torch.Tensor]):
     d = _desc(t)
     keep.append(d)
     return ctypes.pointer(d)
-
-
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream if t.is_cuda else 0
 
 
 def _finish(op: str, status: int):
@@ -313,51 +328,19 @@ def _attn_options(opts: Attn, keep: list) -> _Attn:
     return a
 
 
-def _lend_workspace(lib, a: _Attn, qd: _Tensor, kd: _Tensor, device, workspace, keep: list) -> None:
-    """The partial tensors of a split call, which the reference op allocates itself
-    (tk/src/ops/attention.rs:285-293): here the harness does, like the output."""
-    if a.splits == 1:
-        return
-    need = int(lib.svodk_attention_workspace(ctypes.byref(qd), ctypes.byref(kd), ctypes.byref(a)))
-    if workspace is None and need > 0:
-        workspace = _fresh(need, torch.uint8, device)
-    if workspace is not None:
-        keep.append(workspace)
-        a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-
-
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, opts: Optional[Attn] = None,
               out: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``softmax(q·kᵀ·scale)·v`` over ``q [B,T,H,D]`` and ``k``/``v [B,Tk,H_kv,D]``;
     returns ``[B,T,H,D]`` (tk/src/ops/attention.rs:98-103).  Enqueued on the
     current stream of ``q``'s device; returns without synchronising."""
-    opts = opts or Attn()
-    lib = load_library()
-    if out is None:
-        # The op allocates its output at capacity (tk/src/ops/mod.rs:423-429).
-        out = _fresh(q.shape, q.dtype, q.device)
-    keep: list = []
-    a = _attn_options(opts, keep)
-    qd, kd, vd, od = _desc(q), _desc(k), _desc(v), _desc(out)
-    _lend_workspace(lib, a, qd, kd, q.device, workspace, keep)
-    status = lib.svodk_attention(ctypes.byref(qd), ctypes.byref(kd), ctypes.byref(vd), ctypes.byref(a),
-                                 ctypes.byref(od), ctypes.c_void_p(_stream(q)))
-    _finish("attention", status)
-    return out
+    return (_native or _calls()).attention(q, k, v, opts, out, workspace, _fresh if POISON else None)
 
 
 def attention_noalloc(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, opts: Attn, out: torch.Tensor) -> torch.Tensor:
     """``attention`` through ``svodk_attention_noalloc``: the partial states of a split call live in
     the library's static device array (``noalloc_scratch_bytes()`` per GPU), nothing is allocated
     below this call, and the caller brings ``out``.  No counterpart in the reference."""
-    lib = load_library()
-    keep: list = []
-    a = _attn_options(opts, keep)
-    qd, kd, vd, od = _desc(q), _desc(k), _desc(v), _desc(out)
-    status = lib.svodk_attention_noalloc(ctypes.byref(qd), ctypes.byref(kd), ctypes.byref(vd), ctypes.byref(a),
-                                         ctypes.byref(od), ctypes.c_void_p(_stream(q)))
-    _finish("attention", status)
-    return out
+    return (_native or _calls()).attention_noalloc(q, k, v, opts, out)
 
 
 def noalloc_scratch_bytes() -> int:
@@ -391,52 +374,13 @@ def attention_packed(qkv: torch.Tensor, heads: int, kv_heads: int, opts: Optiona
                      out: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``attention`` over a fused projection ``qkv [B,T,(heads+2·kv_heads)·D]`` read in place;
     returns ``[B,T,heads,D]`` (tk/src/ops/attention.rs:104-122)."""
-    opts = opts or Attn()
-    lib = load_library()
-    slots = heads + 2 * kv_heads
-    if out is None and qkv.dim() == 3 and slots > 0 and qkv.shape[2] % slots == 0:
-        out = _fresh((qkv.shape[0], qkv.shape[1], heads, qkv.shape[2] // slots), qkv.dtype, qkv.device)
-    if out is None:
-        out = torch.empty((1, 1, 1, 1), dtype=qkv.dtype, device=qkv.device)  # the op rejects the shape itself
-    keep: list = []
-    a = _attn_options(opts, keep)
-    xd, od = _desc(qkv), _desc(out)
-    if a.splits > 1 and qkv.dim() == 3:
-        kd = _Tensor()  # the keys' view of the fused rows: [B, T, kv_heads, D]
-        kd.data, kd.dtype, kd.rank = xd.data, xd.dtype, 4
-        kd.shape[0], kd.shape[1], kd.shape[2], kd.shape[3] = qkv.shape[0], qkv.shape[1], kv_heads, out.shape[3]
-        _lend_workspace(lib, a, od, kd, qkv.device, workspace, keep)
-    status = lib.svodk_attention_packed(ctypes.byref(xd), heads, kv_heads, ctypes.byref(a), ctypes.byref(od),
-                                        ctypes.c_void_p(_stream(qkv)))
-    _finish("attention", status)
-    return out
+    return (_native or _calls()).attention_packed(qkv, heads, kv_heads, opts, out, workspace, _fresh if POISON else None)
 
 
 def heads(qkv: torch.Tensor, opts: Qkv, out: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None):
     """``qkv [B,T,(heads+2·kv_heads)·head_dim]`` → ``(q [B,T,heads,D], k, v [B,T,kv_heads,D])``
     (tk/src/ops/heads.rs:35-37)."""
-    lib = load_library()
-    if qkv.dim() == 3 and out is None:
-        b, t = qkv.shape[0], qkv.shape[1]
-        mk = lambda n: _fresh((b, t, n, opts.head_dim), qkv.dtype, qkv.device)
-        out = (mk(opts.heads), mk(opts.kv_heads), mk(opts.kv_heads))
-    elif out is None:
-        # Let the library word the shape error; the outputs are never touched.
-        e = torch.empty((0, 0, 0, 0), dtype=qkv.dtype, device=qkv.device)
-        out = (e, e, e)
-    keep: list = []
-    o = _Qkv()
-    o.heads, o.kv_heads, o.head_dim = opts.heads, opts.kv_heads, opts.head_dim
-    o.q_norm, o.k_norm = _ref(keep, opts.q_norm), _ref(keep, opts.k_norm)
-    o.eps = float(opts.eps)
-    cos, sin = opts.rope if opts.rope is not None else (None, None)
-    o.cos, o.sin = _ref(keep, cos), _ref(keep, sin)
-    o.batch_live = opts.batch_live or 0
-    xd, qd, kd, vd = _desc(qkv), _desc(out[0]), _desc(out[1]), _desc(out[2])
-    status = lib.svodk_heads(ctypes.byref(xd), ctypes.byref(o), ctypes.byref(qd), ctypes.byref(kd), ctypes.byref(vd),
-                             ctypes.c_void_p(_stream(qkv)))
-    _finish("heads", status)
-    return out
+    return (_native or _calls()).heads(qkv, opts, out, _fresh if POISON else None)
 
 
 class Act(enum.IntEnum):
@@ -475,31 +419,7 @@ class Linear:
 def linear(x: torch.Tensor, w: torch.Tensor, opts: Optional[Linear] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x [lead..., K] · w [N, K]ᵀ (+ bias)`` → ``[lead..., N]``, a fused projection's first heads rotated in the
     GEMM's store (tk/src/ops/linear.rs:60-63)."""
-    opts = opts or Linear()
-    lib = load_library()
-    keep: list = []
-    o = _Linear()
-    if opts.into is not None:
-        out, at = opts.into
-        o.has_into, o.into_at = 1, int(at)
-    if out is None:
-        n = w.shape[0] // 2 if opts.gated else w.shape[0]
-        out = _fresh((*x.shape[:-1], n), x.dtype, x.device)
-    o.bias, o.residual = _ref(keep, opts.bias), _ref(keep, opts.residual)
-    o.act, o.gated = int(opts.act), int(opts.gated)
-    if opts.scale is not None:
-        o.has_scale, o.scale = 1, float(opts.scale)
-    if opts.rope is not None:
-        r = _Rotary()
-        r.cos, r.sin = _ref(keep, opts.rope.cos), _ref(keep, opts.rope.sin)
-        r.heads, r.head_dim = int(opts.rope.heads), int(opts.rope.head_dim)
-        keep.append(r)
-        o.rope = ctypes.pointer(r)
-    o.batch_live = opts.batch_live or 0
-    xd, wd, od = _desc(x), _desc(w), _desc(out)
-    status = lib.svodk_linear(ctypes.byref(xd), ctypes.byref(wd), ctypes.byref(o), ctypes.byref(od), ctypes.c_void_p(_stream(x)))
-    _finish("linear", status)
-    return out
+    return (_native or _calls()).linear(x, w, opts, out, _fresh if POISON else None)
 
 
 def plan_linear(has_target: bool, dtypes, x_dims, n: int) -> Optional[Fallback]:
@@ -510,31 +430,10 @@ def plan_linear(has_target: bool, dtypes, x_dims, n: int) -> Optional[Fallback]:
     return _plan(lib.svodk_plan_linear(int(has_target), dt, len(dtypes), xd, 0 if x_dims is None else len(x_dims), n))
 
 
-def _norm(name: str, x, residual, w, b, eps, batch_live, out):
-    lib = load_library()
-    keep: list = []
-    fused = residual is not None
-    if out is None:
-        out = ((_fresh(x.shape, x.dtype, x.device), _fresh(x.shape, x.dtype, x.device)) if fused
-               else _fresh(x.shape, x.dtype, x.device))
-    none = ctypes.POINTER(_Tensor)()
-    args = [_ref(keep, x)]
-    if fused:
-        args.append(_ref(keep, residual))
-    args.append(_ref(keep, w))
-    if "layer" in name:
-        args.append(_ref(keep, b) if b is not None else none)
-    args += [ctypes.c_double(float(eps)), ctypes.c_int32(batch_live or 0)]
-    args += [_ref(keep, out[0]), _ref(keep, out[1])] if fused else [_ref(keep, out)]
-    status = getattr(lib, "svodk_" + name)(*args, ctypes.c_void_p(_stream(x)))
-    _finish("layer_norm" if "layer" in name else "rms_norm", status)
-    return out
-
-
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, eps: float = 1e-5,
                out: Optional[torch.Tensor] = None, batch_live: Optional[int] = None) -> torch.Tensor:
     """``(x - mean)·rsqrt(var + eps)·w + b`` over the last dim of ``x`` (tk/src/ops/norm.rs:16-19)."""
-    return _norm("layer_norm", x, None, w, b, eps, batch_live, out)
+    return (_native or _calls()).layer_norm(x, None, w, b, eps, batch_live, out, _fresh if POISON else None)
 
 
 def add_layer_norm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None,
@@ -542,20 +441,20 @@ def add_layer_norm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, b: 
                    batch_live: Optional[int] = None):
     """``(x + residual, layer_norm(x + residual))``, the sum rounded to the input type first
     (tk/src/ops/norm.rs:21-31); ``out`` is ``(sum, y)``."""
-    return _norm("add_layer_norm", x, residual, w, b, eps, batch_live, out)
+    return (_native or _calls()).layer_norm(x, residual, w, b, eps, batch_live, out, _fresh if POISON else None)
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5, out: Optional[torch.Tensor] = None,
              batch_live: Optional[int] = None) -> torch.Tensor:
     """``x·rsqrt(mean(x²) + eps)·w`` over the last dim of ``x`` (tk/src/ops/norm.rs:33-36)."""
-    return _norm("rms_norm", x, None, w, None, eps, batch_live, out)
+    return (_native or _calls()).rms_norm(x, None, w, None, eps, batch_live, out, _fresh if POISON else None)
 
 
 def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, eps: float = 1e-5,
                  out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, batch_live: Optional[int] = None):
     """``(x + residual, rms_norm(x + residual))``, the sum rounded to the input type first
     (tk/src/ops/norm.rs:38-42); ``out`` is ``(sum, y)``."""
-    return _norm("add_rms_norm", x, residual, w, None, eps, batch_live, out)
+    return (_native or _calls()).rms_norm(x, residual, w, None, eps, batch_live, out, _fresh if POISON else None)
 
 
 def plan_norm(has_target: bool, dtypes, x_dims) -> Optional[Fallback]:
@@ -570,13 +469,7 @@ def order_rows(keys: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.
     """The batch rows in descending order of their key counts (ties by row) as int32 ``[B]``, for
     ``Attn.row_order``; ``keys`` is ``[B]`` lengths or a ``[B, Tk]`` key mask.  A variable-length batch whose
     rows run grouped by length ends on its short tiles."""
-    lib = load_library()
-    if out is None:
-        out = _fresh(keys.shape[:1], torch.int32, keys.device)
-    keep: list = []
-    status = lib.svodk_order_rows(_ref(keep, keys), _ref(keep, out), ctypes.c_void_p(_stream(keys)))
-    _finish("order_rows", status)
-    return out
+    return (_native or _calls()).order_rows(keys, out, _fresh if POISON else None)
 
 
 def chosen() -> str:
