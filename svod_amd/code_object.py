@@ -133,10 +133,9 @@ def entries() -> Dict[str, dict]:
         for turn in (0, 64, 128):  # the projection GEMM, plain or with the first `heads` heads of `turn` columns turned
             out[f"svodk_linear_{'rope%d_' % turn if turn else ''}{dtype}"] = {
                 "file": "svodk_linear.co", "source": "linear_kernel.hip", "params": _LINEAR, "local": [512, 1, 1],
-                "workgroups": "(((rows + 255) // 256 + 7) // 8 * ((n + 255) // 256) if (rows + 255) // 256 >= 16 "
-                              "else ((rows + 255) // 256 * ((n + 255) // 256) + 7) // 8) * 8",
+                "workgroups": "((rows + 255) // 256 * ((n + 255) // 256) + 7) // 8 * 8",
                 "op": "linear", "dtype": dtype, "rope_head_dim": turn,
-                "cfg": f"GemmCfg {{ bm: 256, bn: 256, bk: 64, stages: 2, waves: 8, core: mfma_f32_32x32x16_{dtype}"
+                "cfg": f"GemmCfg {{ bm: 256, bn: 256, bk: 64, stages: 2, waves: 8, core: mfma_f32_16x16x32_{dtype}"
                        + (", epilogue: rope }" if turn else " }")}
         for kind, params in _ROWS.items():
             for dmax in (1024, 2048, 4096):

@@ -7,21 +7,21 @@
 // come out rotated and its values plain, so a model without QK norms needs no prologue pass at all
 // (tk/src/ops/linear.rs:47-58).
 //
-// The mapping onto CDNA4 is this file's own.  A workgroup of 8 waves owns a 256 x 256 output tile; a wave
-// owns 64 rows x 128 columns as 2 x 4 accumulators of v_mfma_f32_32x32x16.  The product runs transposed,
-// C^T = W . X^T, so that a lane owns one output ROW and, per accumulator register quad, four CONSECUTIVE
-// columns: the rotation's partner column (32 or 64 columns along) is the same lane's register of another
-// accumulator, and the tables (staged through LDS once the ring is done with) are read as 8-byte runs of the
-// lane's row.  The finished tile goes through LDS once more, a wave's rows in a stretch of its own, and
-// leaves as whole 256-byte row segments, 16 bytes a lane.
-// X and W tiles of 64 k-columns stream through a two-stage LDS ring (64 KiB a stage), filled global -> LDS
-// by buffer_load_dwordx4 ... lds a stage ahead.  What bounds this kernel is the way from L2 into LDS: the
-// part moves about 18 TB/s along it when every fill takes whole 128-byte lines and about 12 TB/s when it
-// takes half lines (measured: the fills of this kernel alone, without its products).  Hence tiles this
-// large (1 GiB of fills at the projection shape where 256 x 128 tiles move 1.5 GiB) and rows of 128 bytes,
-// a whole line each; their eight 16-byte chunks are XOR-swizzled by (row / 2) % 8 through the lanes' source
-// addresses so that a ds_read_b128 of 16 rows at one logical chunk touches every bank once.  Rows past the
-// operands' ends read as zeros through the buffer descriptors' bounds.  One barrier a stage (32 MFMAs a wave).
+// The mapping onto CDNA4 is this file's own.  A workgroup of 4 x WN waves owns a tile of the output, at its largest
+// 256 x 256 by 8 waves of 64 rows x 128 columns.  The product runs transposed, C^T = W . X^T, on
+// v_mfma_f32_16x16x32: a lane owns one output ROW of a 16 x 16 block and four CONSECUTIVE columns of it, and the
+// rotation's partner column (32 or 64 columns along) is the same lane's register of another block.  The 16 x 16 atom
+// and not the 32 x 32 x 16 one because the part holds a higher clock under it: 2.12 PFLOP/s against 1.90 for nothing
+// but matrix instructions on live data (it moves half the accumulator registers a flop).
+// X and W tiles of 64 k-columns stream through an LDS ring, filled global -> LDS by buffer_load_dwordx4 ... lds.
+// What bounds this kernel is the way from L2 into LDS beside the matrix pipe: a compute unit takes in some 80 bytes a
+// nanosecond when every fill takes whole 128-byte lines (half lines: two thirds of that), so a 256 x 256 x 64 stage's
+// 64 KiB are 0.8 us beside 0.85 us of matrix instructions.  Hence rows of 128 bytes, a whole line each, tiles as large
+// as LDS holds where there are enough of them, and fills one at a time between the products: issued together behind
+// the barrier they fill the address path's queue and the waves stand there instead of issuing products (130 -> 124 us
+// at [16384, 1024] x [4096, 1024]).  A row's eight 16-byte chunks are XOR-swizzled by (row / 2) % 8 through the lanes'
+// source addresses so that a ds_read_b128 of 16 rows at one logical chunk touches every bank once.  Rows past the
+// operands' ends read as zeros through the buffer descriptors' bounds.  One barrier a stage.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -40,7 +40,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
@@ -48,24 +48,50 @@ typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 constexpr int kXcds = 8;
 constexpr int kBk = 64;                 // k-columns a stage: a row of a tile is one 128-byte line
-constexpr int kSteps = kBk / 16;        // k-steps of the matrix instruction a stage
-constexpr int kStages = 2;
 constexpr int kGroup = 8;               // column tiles an XCD's resident workgroups spread over
 constexpr int kRowBytes = kBk * 2;      // a tile row in LDS
-constexpr int kOutPitch = 128 * 2 + 16;               // a wave's row of the finished tile in LDS
-// The workgroup's output tile in two sizes.  S = 2: 256 x 256 by 8 waves (4 along the rows x 2 along the columns,
-// 64 rows x 128 columns a wave), the size for a product with tiles enough to fill the part.  S = 1: 128 x 128 by
-// 4 waves (32 rows x 128 columns a wave), two workgroups a compute unit: a product of few rows gets four times the
-// workgroups, at twice the fills a flop.  A wave's 128 columns hold whole heads of 64 or 128 either way.
-template <int S>
+constexpr int kAhead = 4;               // column blocks between a W fragment's request and its products
+
+// The workgroup's output tile: 4 waves along the rows, 16 RB rows each, x WN waves along the columns, 16 CB columns
+// each.  The W tiles of SW stages and the X tiles of SX stages lie in LDS.
+template <int RB_, int CB_, int WN_, int SW_, int SX_>
 struct Tile {
-  static constexpr int kWaves = 4 * S;
-  static constexpr int kBm = 128 * S, kBn = 128 * S;
-  static constexpr int kTileBytes = kBm * kRowBytes;           // one operand's tile: 32 (16) KiB
-  static constexpr int kStageBytes = 2 * kTileBytes;           // W tile, then X tile
-  static constexpr int kLds = kStages * kStageBytes;           // 128 (64) KiB
-  static constexpr int kFills = kStageBytes / 1024 / kWaves;   // wave instructions of 1 KiB per wave and stage: 8
+  static constexpr int RB = RB_, CB = CB_, WN = WN_, SW = SW_, SX = SX_;
+  static constexpr int kWaves = 4 * WN;
+  static constexpr int kBm = 64 * RB, kBn = 16 * CB * WN;
+  static constexpr int kWBytes = kBn * kRowBytes, kXBytes = kBm * kRowBytes;
+  static constexpr int kLds = SW * kWBytes + SX * kXBytes;     // the W ring, then the X ring
+  static constexpr int kWFills = kWBytes / 1024 / kWaves;      // wave instructions of 1 KiB per wave and stage
+  static constexpr int kXFills = kXBytes / 1024 / kWaves;
+  static constexpr int kOutPitch = CB * 32 + 16;               // a wave's row of the finished tile in LDS
+  static_assert(kWBytes % (1024 * kWaves) == 0 && kXBytes % (1024 * kWaves) == 0, "a tile fills in whole instructions a wave");
   static_assert(kWaves * 32 * kOutPitch <= kLds, "32 rows a wave of the finished tile fit where the ring was");
+  static_assert(CB >= kAhead && (2 * CB) % kAhead == 0 && RB % 2 == 0 && RB <= 2 * (kAhead - 1), "the k loop's schedule");
+  static_assert(SX >= 2 && (SW == SX || SW == SX + 1), "the k loop's waits");
+};
+// 256 x 256 by 8 waves (64 rows x 128 columns each), 128 KiB: the tile for a product with tiles enough to fill the part.
+// (A third W tile in the ring gives 1 % at k = 4096 and nothing at 1024.)
+typedef Tile<4, 8, 2, 2, 2> Large;
+// 256 x 192 by 8 waves (64 x 96 each), 136 KiB: where it leaves fewer compute units idle in the last round.
+typedef Tile<4, 6, 2, 3, 2> Wide;
+// 128 x 128 by 8 waves (32 x 64 each), 80 KiB, two workgroups a compute unit: four times the workgroups, at twice the
+// fills a flop.  Its products leave a fill less time to arrive, so the third W tile pays: 139 -> 132 us at [16384, 1024]
+// x [4096, 1024].
+typedef Tile<2, 4, 2, 3, 2> Mid;
+// 128 x 64 by 4 waves (32 x 64 each), 72 KiB: where Mid would leave compute units without any tile.
+typedef Tile<2, 4, 1, 3, 3> Narrow;
+
+// Where a wave's column blocks lie in the tile.  A turned head's halves have to meet in one wave: two waves of 64
+// columns take 32 columns of each half of a head of 128 instead of a half each.
+template <int HD, typename T>
+struct Columns {
+  static constexpr bool kSplit = HD == 128 && T::CB == 4 && T::WN == 2;
+  static_assert(HD == 0 || kSplit || (T::CB * 16) % (HD > 0 ? HD : 1) == 0, "a wave holds whole turned heads");
+  static constexpr int kWaveStep = kSplit ? 32 : 16 * T::CB;  // from a wave's columns to the next's
+  // Block cb's first column in a wave whose columns start at 0.
+  __host__ __device__ static constexpr int at(int cb) { return kSplit ? 64 * (cb >> 1) + 16 * (cb & 1) : 16 * cb; }
+  static constexpr int kHalfBlocks = kSplit ? 2 : HD / 32;  // from a block to its partner
+  __host__ __device__ static constexpr bool first_half(int cb) { return HD > 0 && at(cb) % (HD > 0 ? HD : 1) < HD / 2; }
 };
 
 template <bool F16>
@@ -85,11 +111,11 @@ __device__ __forceinline__ float widen(uint32_t bits16) {
 }
 
 template <bool F16>
-__device__ __forceinline__ f32x16 mma(const u32x4 &a, const u32x4 &b, const f32x16 &c) {
+__device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
   if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // A raw buffer descriptor over `bytes` bytes at `base`: loads past the end return zero.
@@ -116,134 +142,108 @@ __device__ __forceinline__ void load4(const uint16_t *p, float (&out)[4]) {
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // HD: the head size a turning kernel is built for (64 or 128), 0: no turn.
-template <bool F16, int HD, int S = 2>
+template <bool F16, int HD, typename T>
 __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
                                             const uint16_t *__restrict__ bias, const uint16_t *__restrict__ cos_t,
                                             const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y, int64_t y_ld,
                                             int64_t rows, int32_t n, int32_t k, int32_t seq, int32_t heads,
-                                            uint32_t tiles_n, uint32_t tiles, uint32_t per_xcd, uint32_t band) {
-  constexpr int kWaves = Tile<S>::kWaves, kBm = Tile<S>::kBm, kBn = Tile<S>::kBn, kTileBytes = Tile<S>::kTileBytes;
-  constexpr int kStageBytes = Tile<S>::kStageBytes, kLds = Tile<S>::kLds, kFills = Tile<S>::kFills;
+                                            uint32_t tiles_n, uint32_t tiles, uint32_t per_xcd) {
+  constexpr int kWaves = T::kWaves, kBm = T::kBm, kBn = T::kBn, kWBytes = T::kWBytes, kXBytes = T::kXBytes;
+  constexpr int kLds = T::kLds, kWFills = T::kWFills, kXFills = T::kXFills, kFills = kWFills + kXFills;
+  constexpr int SW = T::SW, SX = T::SX, RB = T::RB, CB = T::CB, kXRing = SW * kWBytes;
+  typedef Columns<HD, T> Cols;
   const int tid = __builtin_amdgcn_workitem_id_x();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 5, ln = lane & 31;
-  // Workgroups are dealt to the 8 XCDs in turn, each XCD with an L2 of its own.  With rows enough
-  // (`band` > 0) XCD x owns a band of `band` row tiles and walks it in groups of up to kGroup column
-  // tiles, row tile by row tile within a group: the workgroups resident together then share few w tiles
-  // (read once per XCD) and few x tiles (read once per group), instead of streaming all of w past every
-  // row tile.  With few rows XCD x takes a run of consecutive tiles, column tile fastest.
+  const int g = lane >> 4, ln = lane & 15;
+  // Workgroups are dealt to the 8 XCDs in turn, each XCD with an L2 of its own.  The tiles stand in one row: groups
+  // of up to kGroup column tiles, row tile after row tile within a group; XCD x takes the x-th eighth of that row.
+  // The workgroups resident together on an XCD then share few w tiles and few x tiles, and no XCD has more than one
+  // tile more than another: whole bands of row tiles an XCD, the order before, gave XCDs 0..5 36 tiles for their 32
+  // compute units and XCD 7 none at [6216, 768] x [2304, 768] (225 tiles: 46 us, two rounds; 26 us in one).
   const uint32_t wg = __builtin_amdgcn_workgroup_id_x();
-  const uint32_t xcd = wg % kXcds, local = wg / kXcds;
-  uint32_t tm, tn;
-  if (band > 0) {
-    const uint32_t full = band * kGroup;            // workgroups of a full-width group
-    const uint32_t ng = local / full;               // the group
-    const uint32_t first = ng * kGroup;             // its first column tile
-    if (first >= tiles_n) return;
-    const uint32_t width = min((uint32_t)kGroup, tiles_n - first);
-    const uint32_t r = local - ng * full;
-    const uint32_t tm_local = r / width;
-    if (tm_local >= band) return;
-    tm = xcd * band + tm_local;
-    tn = first + (r - tm_local * width);
-    if ((uint64_t)tm * tiles_n + tn >= tiles) return;  // past the last row tile
-  } else {
-    const uint32_t tile = xcd * per_xcd + local;
-    if (local >= per_xcd || tile >= tiles) return;
-    tm = tile / tiles_n;
-    tn = tile - tm * tiles_n;
-  }
+  const uint32_t turn = wg % kXcds * per_xcd + wg / kXcds;
+  if (turn >= tiles) return;
+  const uint32_t tiles_m = tiles / tiles_n, full = tiles_m * kGroup;  // workgroups of a full-width group
+  const uint32_t ng = turn / full;
+  const uint32_t first_tn = ng * kGroup;  // the group's first column tile
+  const uint32_t width = min((uint32_t)kGroup, tiles_n - first_tn);
+  const uint32_t in_group = turn - ng * full;
+  const uint32_t tm = in_group / width, tn = first_tn + (in_group - tm * width);
   const int64_t m0 = (int64_t)tm * kBm;
   const int32_t n0 = (int32_t)tn * kBn;
   const int64_t row_bytes = (int64_t)k * 2;
 
-  // ---- this wave's fills of a stage: 8 rows x 8 chunk places an instruction; a stage is 64 of them, the
-  // W tile's 32 and then the X tile's 32, and wave v takes instructions v, v + 8, ...  Those are 64 rows
-  // apart, a multiple of the swizzle's period of 16, so one lane offset serves all eight; the descriptors'
-  // bases differ.
+  // ---- this wave's fills of a stage: 8 rows x 8 chunk places an instruction; a stage is the W tile's and then
+  // the X tile's, and wave v takes instructions v, v + waves, ...  Those are a multiple of 32 rows apart and the
+  // swizzle's period is 16, so one lane offset serves them all; the descriptors' bases differ.
   const int frow = lane >> 3, place = lane & 7;
   const int src = frow * (int)row_bytes + ((place ^ ((4 * (wave & 1) + (frow >> 1)) & 7)) << 4);
-  i32x4 rsrc[kFills];
-  int lds_at[kFills];
+  const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)(smem) + wave * 1024;
+  i32x4 rsrc[kFills];  // the W tile's instructions, then the X tile's
 #pragma unroll
   for (int f = 0; f < kFills; f++) {
-    const int j = wave + kWaves * f;  // the instruction of the stage
-    const bool is_x = f >= kFills / 2;
-    const int block_row = 8 * (is_x ? j - kTileBytes / 1024 : j);
-    const int64_t first = (is_x ? m0 : (int64_t)n0) + block_row;
+    const bool is_x = f >= kWFills;
+    const int64_t first = (is_x ? m0 : (int64_t)n0) + 8 * (wave + kWaves * (is_x ? f - kWFills : f));
     const int64_t limit = is_x ? rows : (int64_t)n;
-    const uint16_t *base = is_x ? x : w;
-    rsrc[f] = make_rsrc((const uint8_t *)base + first * row_bytes, (limit - first) * row_bytes);
-    lds_at[f] = (int)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)(smem) + j * 1024;
+    rsrc[f] = make_rsrc((const uint8_t *)(is_x ? x : w) + first * row_bytes, (limit - first) * row_bytes);
   }
-  // k is a multiple of 32: a last stage may hold two k-steps only.  The lanes that would fetch the second
+  // k is a multiple of 32: a last stage may hold one k-step only.  The lanes that would fetch the second
   // half of its rows (the next rows' data) then address past every descriptor's bound and land zeros.
   const int nk = (k + kBk - 1) / kBk;
   const bool short_tail = (k % kBk) != 0;
   const bool second_half = ((place ^ ((4 * (wave & 1) + (frow >> 1)) & 7)) & 4) != 0;
-  // Stage `s` of the k loop into its ring slot; past the last stage an empty descriptor (zeros land in a
-  // slot nothing reads any more) keeps the count of fills in flight the same in every iteration.
-  auto fill = [&](int s) {
-    const int slot = (s % kStages) * kStageBytes;
+  // Fill `f` of stage `s` of the k loop into slot `slot` of its ring; past the last stage an empty descriptor (zeros
+  // land in a slot nothing reads any more) keeps the count of fills in flight the same in every iteration.
+  auto fill = [&](int s, int slot, int f) {
     const int voff = (short_tail && s == nk - 1 && second_half) ? (int)0xfffffff0u : src + s * kRowBytes;
-#pragma unroll
-    for (int f = 0; f < kFills; f++) {
-      i32x4 r = rsrc[f];
-      if (s >= nk) r[2] = 0;
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                   :
-                   : "s"(lds_at[f] + slot), "v"(voff), "s"(r)
-                   : "memory");
-    }
+    const int at = f < kWFills ? slot * kWBytes + f * kWaves * 1024 : kXRing + slot * kXBytes + (f - kWFills) * kWaves * 1024;
+    i32x4 r = rsrc[f];
+    if (s >= nk) r[2] = 0;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds0 + at), "v"(voff), "s"(r)
+                 : "memory");
   };
-  fill(0);
-  fill(1);
 
-  // ---- operand reads: A = W rows (the output's columns), B = X rows (the output's rows); fragment
-  // (block of 32 rows, k-step ks): row ln of the block, logical chunk 2 * ks + g.
-  const int wave_m = wave & 3, wave_n = wave >> 2;  // 32 S-row and 128-column shares of the tile
-  int a_read[4], b_read[S];
+  // ---- the schedule of a stage: two k-steps of 32, each CB column blocks of RB products (W fragment cb against the
+  // RB fragments of X).  A W fragment is asked for kAhead blocks before its products, a k-step's X fragments in the
+  // last blocks of the k-step before.  Ahead of the last kAhead - 1 blocks of a stage therefore stands its barrier:
+  // every wave's fills of the next stage have landed and its reads of this one are back (the last of them asked for
+  // two blocks earlier), so the next stage is whole and this stage's slots are free.  The fills follow one by one: X of
+  // the stage SX further on beside those last blocks, W of the stage SX + 1 further on (with SW = SX + 1; else SX)
+  // beside the next stage's first blocks, from where it has more than a stage to arrive.
+  constexpr int kBlocks = 2 * CB, kBarrier = kBlocks - kAhead + 1;
+  constexpr int kXPer = (kXFills + kAhead - 2) / (kAhead - 1), kWPer = (kWFills + 3) / 4;  // fills a block
+  static_assert((kWFills + kWPer - 1) / kWPer <= kBarrier, "a stage's fills are out before its barrier");
+  constexpr int kWLead = SW - 1;  // a stage's first blocks ask for W of the stage this much further on
 #pragma unroll
-  for (int cb = 0; cb < 4; cb++) a_read[cb] = (wave_n * 128 + cb * 32 + ln) * kRowBytes;
+  for (int s = 0; s < SX; s++)
 #pragma unroll
-  for (int rb = 0; rb < S; rb++) b_read[rb] = kTileBytes + (wave_m * 32 * S + rb * 32 + ln) * kRowBytes;
+    for (int f = s < kWLead ? 0 : kWFills; f < kFills; f++) fill(s, s, f);
+
+  // ---- operand reads: A = W rows (the output's columns), B = X rows (the output's rows); a fragment is 16 rows, its
+  // lane (ln, g) reads logical chunk 4 ks + g of row ln.
+  const int wave_m = wave & 3, wave_n = wave >> 2;
   const int swz = (ln >> 1) & 7;  // every block starts on a multiple of 16 rows
-  int chunk_at[kSteps];
+  int w_read[2], x_read[2];
 #pragma unroll
-  for (int ks = 0; ks < kSteps; ks++) chunk_at[ks] = ((2 * ks + g) ^ swz) << 4;
-
-  f32x16 acc[S][4];
-  const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  for (int ks = 0; ks < 2; ks++) {
+    const int chunk = ((4 * ks + g) ^ swz) << 4;
+    w_read[ks] = (wave_n * Cols::kWaveStep + ln) * kRowBytes + chunk;
+    x_read[ks] = kXRing + (wave_m * 16 * RB + ln) * kRowBytes + chunk;
+  }
+  f32x4 acc[RB][CB];
 #pragma unroll
-  for (int rb = 0; rb < S; rb++)
+  for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-    for (int cb = 0; cb < 4; cb++) acc[rb][cb] = zero;
-
-  // One k-step: the 4 S products of the fragment set `set` (four fragments of W: this wave's column blocks; S of
-  // X: its row blocks), and beside them the 4 + S fragment reads of k-step `nks` of stage slot `nslot` into the
-  // other set (one beside each of the first six of eight products; with four products, two beside the first), so
-  // that a product's operands were asked for a k-step earlier.  The fences keep the order: left to itself the
-  // scheduler gathers the reads in front of the products that want them.
-  constexpr int kReads = 4 + S, kProducts = 4 * S;
-  u32x4 af[2][4], bf[2][S];
-  auto read_fragment = [&](int slot, int ks, int i, int set) {
-    const uint8_t *st = smem + slot * kStageBytes;
-    if (i < S)
-      bf[set][i] = *reinterpret_cast<const u32x4 *>(st + b_read[i] + chunk_at[ks]);
-    else
-      af[set][i - S] = *reinterpret_cast<const u32x4 *>(st + a_read[i - S] + chunk_at[ks]);
+    for (int cb = 0; cb < CB; cb++) acc[rb][cb] = f32x4{0, 0, 0, 0};
+  u32x4 wf[kAhead], xf[2][RB];
+  auto read_w = [&](int slot, int block) {  // block 0 .. kBlocks - 1 of a stage
+    wf[block % kAhead] = *reinterpret_cast<const u32x4 *>(smem + slot * kWBytes + w_read[block / CB] + Cols::at(block % CB) * kRowBytes);
   };
-  auto step = [&](int set, int nslot, int nks, bool reads) {
-#pragma unroll
-    for (int i = 0; i < kProducts; i++) {
-      acc[i % S][i / S] = mma<F16>(af[set][i / S], bf[set][i % S], acc[i % S][i / S]);
-      if (reads) {
-        if (i < kReads) read_fragment(nslot, nks, i, set ^ 1);
-        if (i == 0 && kReads > kProducts) read_fragment(nslot, nks, kProducts, set ^ 1);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  auto read_x = [&](int slot, int ks, int rb) {
+    xf[ks][rb] = *reinterpret_cast<const u32x4 *>(smem + slot * kXBytes + x_read[ks] + rb * 16 * kRowBytes);
   };
   // The rotary tables' rows of this tile (16 bytes a lane along the rows, kTables loads a table and lane)
   // are asked for behind the barrier of the last stage but one: they arrive under the last stage's products
@@ -251,79 +251,92 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
   constexpr int kHalf = (HD > 0 ? HD : 64) / 2, kTChunks = kHalf * 2 / 16, kTables = kBm * kTChunks / (kWaves * 64);
   const bool turning = HD > 0 && n0 < heads * HD;  // the same for the whole workgroup
   u32x4 tc[kTables], ts[kTables];
-  bool tables_in = false;
+  const int tables_at = nk > 1 ? nk - 2 : 0;
   auto load_tables = [&]() {
-    const uint32_t pos0 = (uint32_t)(m0 % seq);
+    // gemm.rs:685: the table row of the token's position.  A lane's rows are kWaves * 64 / kTChunks apart.
+    const uint32_t useq = (uint32_t)seq, step = (uint32_t)(kWaves * 64 / kTChunks) % useq;
+    uint32_t pos = ((uint32_t)(m0 % seq) + (uint32_t)(tid / kTChunks)) % useq;
 #pragma unroll
     for (int i = 0; i < kTables; i++) {
-      const int c = tid + i * kWaves * 64, r = c / kTChunks, ch = c % kTChunks;
-      const uint32_t pos = (pos0 + (uint32_t)r) % (uint32_t)seq;  // gemm.rs:685: the table row of the token's position
-      tc[i] = *reinterpret_cast<const u32x4 *>(cos_t + (int64_t)pos * kHalf + ch * 8);
-      ts[i] = *reinterpret_cast<const u32x4 *>(sin_t + (int64_t)pos * kHalf + ch * 8);
+      const int64_t at = (int64_t)pos * (kHalf * 2) + tid % kTChunks * 16;
+      tc[i] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(cos_t) + at);
+      ts[i] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(sin_t) + at);
+      pos += step;
+      pos = pos >= useq ? pos - useq : pos;
     }
-    tables_in = true;
   };
 
-  // A stage is four k-steps.  Before its last one every wave makes sure its own fills of the next stage
-  // have landed and its reads of this stage are back, and meets the others: behind that barrier the next
-  // stage is whole and this stage's slot is free, so the fills of the stage after next go out and the next
-  // stage's first fragments are asked for under this stage's last products.
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFills) : "memory");  // stage 0 is in
+  // In flight behind stage 0 there: X of stages 1 .. SX - 1 and W of stages 1 .. min(SX, kWLead) - 1.
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SX - 1) * kXFills + ((SX < kWLead ? SX : kWLead) - 1) * kWFills) : "memory");
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kReads; i++) read_fragment(0, 0, i, 0);
+  for (int rb = 0; rb < RB; rb++) read_x(0, 0, rb);
+#pragma unroll
+  for (int b = 0; b < kAhead; b++) read_w(0, b);
+  int ws = 0, xs = 0, wfill = kWLead;  // the slots of this stage, and of the W tile that its first blocks ask for
   for (int s = 0; s < nk; s++) {
-    const int slot = s & 1;
-    step(0, slot, 1, true);
-    step(1, slot, 2, true);
-    step(0, slot, 3, true);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // stage s + 1 is in, stage s is read
-    __syncthreads();
-    fill(s + 2);
-    if (HD > 0 && turning && s == nk - 2) load_tables();
-    step(1, slot ^ 1, 0, true);
+    const int ws_next = ws + 1 == SW ? 0 : ws + 1, xs_next = xs + 1 == SX ? 0 : xs + 1;
+#pragma unroll
+    for (int b = 0; b < kBlocks; b++) {
+      const int ks = b / CB, cb = b % CB;
+      if (b == kBarrier) {
+        // Stage s + 1 is in: behind it in flight are X of the SX - 2 and W of the kWLead - 1 stages after it.
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SX - 2) * kXFills + (kWLead - 1) * kWFills) : "memory");
+        __syncthreads();
+        if (HD > 0 && turning && s == tables_at) load_tables();
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; rb++) acc[rb][cb] = mma<F16>(wf[b % kAhead], xf[ks][rb], acc[rb][cb]);
+      if (b == kBarrier) read_w(ws_next, 0);
+      if (b < kBlocks - kAhead)
+        read_w(ws, b + kAhead);
+      else if (b >= kBarrier)
+        read_w(ws_next, b + kAhead - kBlocks);
+#pragma unroll
+      for (int i = 0; i < 2; i++) {  // two fragments of the next k-step's X a block
+        const int xr = 2 * (cb - (CB - kAhead + 1)) + i;
+        if (xr >= 0 && xr < RB) read_x(ks == 0 ? xs : xs_next, ks ^ 1, xr);
+      }
+#pragma unroll
+      for (int i = 0; i < kXPer; i++)
+        if (b >= kBarrier && (b - kBarrier) * kXPer + i < kXFills) fill(s + SX, xs, kWFills + (b - kBarrier) * kXPer + i);
+#pragma unroll
+      for (int i = 0; i < kWPer; i++)
+        if (b * kWPer + i < kWFills) fill(s + kWLead, wfill, b * kWPer + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wfill = ws;
+    ws = ws_next;
+    xs = xs_next;
   }
-  if (HD > 0 && turning && !tables_in) load_tables();  // a k loop of one stage
   // The empty fills still in flight write LDS: they land before the workgroup's LDS is given away.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  // ---- epilogue.  Accumulator (rb, cb) register i: row m0 + 64 wave_m + 32 rb + ln, column
-  // n0 + 128 wave_n + 32 cb + 8 (i / 4) + 4 g + i % 4.
-  const int col_base = n0 + wave_n * 128 + 4 * g;
-  if (bias != nullptr) {
+  // ---- epilogue.  Accumulator (rb, cb) element e: row m0 + 16 RB wave_m + 16 rb + ln, column
+  // wave_n0 + Cols::at(cb) + 4 g + e.
+  const int wave_n0 = n0 + wave_n * Cols::kWaveStep;
+  // The bias, or -0 without one (x + -0 is x): a branch around the whole addition would have the compiler keep a second
+  // set of accumulators for where its two ways meet.
 #pragma unroll
-    for (int cb = 0; cb < 4; cb++) {
+  for (int cb = 0; cb < CB; cb++) {
+    float b4[4] = {-0.0f, -0.0f, -0.0f, -0.0f};
+    if (bias != nullptr) load4<F16>(bias + min(wave_n0 + Cols::at(cb) + 4 * g, n - 4), b4);  // columns past the end are not stored
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int col = col_base + 32 * cb + 8 * q;
-        if (col >= n) continue;
-        float b4[4];
-        load4<F16>(bias + col, b4);
+    for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-        for (int rb = 0; rb < S; rb++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) acc[rb][cb][4 * q + e] += b4[e];
-      }
-    }
+      for (int e = 0; e < 4; e++) acc[rb][cb][e] += b4[e];
   }
-  const int turned = HD > 0 ? heads * HD : 0;
   if (HD > 0 && turning) {
-    // The head size is 64 or 128: a head's halves are whole 32-column blocks of a wave's 128 columns, the
-    // partner of block cb is block cb +- nb, and a head never straddles two waves.
-    constexpr int head_dim = HD > 0 ? HD : 64;
-    constexpr int half = head_dim >> 1, nb = half >> 5;
-    // The tile's 256 rows of the tables go through LDS (the ring is done with): loaded 16 bytes a lane
-    // along the rows, read back 8 bytes a lane down them.  A lane owns a ROW of the output, so reading
-    // the tables straight from memory would touch 32 lines an instruction.  Rows of 2 * half + 8 bytes
-    // keep the reads off each other's banks.
-    constexpr int kPitch = half * 2 + 8, kChunks = half * 2 / 16;
+    // The tile's rows of the tables go through LDS (the ring is done with): loaded 16 bytes a lane along the rows,
+    // read back 8 bytes a lane down them.  A lane owns a ROW of the output, so reading the tables straight from
+    // memory would touch 16 lines an instruction.  Rows of 2 * kHalf + 8 bytes keep the reads off each other's banks.
+    constexpr int kPitch = kHalf * 2 + 8;
     uint8_t *cos_lds = smem, *sin_lds = smem + kBm * kPitch;
     __syncthreads();  // every wave's last fragments are read and its last fills have landed
     static_assert(2 * kBm * kPitch <= kLds, "the tables fit where the ring was");
-    static_assert(kChunks == kTChunks && half == kHalf, "the prefetch's chunks are the tables'");
 #pragma unroll
     for (int i = 0; i < kTables; i++) {
-      const int c = tid + i * kWaves * 64, r = c / kChunks, ch = c % kChunks;
+      const int c = tid + i * kWaves * 64, r = c / kTChunks, ch = c % kTChunks;
       const u32x4 vc = tc[i], vs = ts[i];
       u32x2 *cd = reinterpret_cast<u32x2 *>(cos_lds + r * kPitch + ch * 16);
       u32x2 *sd = reinterpret_cast<u32x2 *>(sin_lds + r * kPitch + ch * 16);
@@ -333,114 +346,109 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
       sd[1] = u32x2{vs[2], vs[3]};
     }
     __syncthreads();
-    if (n0 + wave_n * 128 < turned) {
+    const int turned = heads * HD;
 #pragma unroll
-      for (int rb = 0; rb < S; rb++) {
-        const int r = wave_m * 32 * S + rb * 32 + ln;
-        const uint16_t *cos_row = reinterpret_cast<const uint16_t *>(cos_lds + r * kPitch);
-        const uint16_t *sin_row = reinterpret_cast<const uint16_t *>(sin_lds + r * kPitch);
+    for (int cb = 0; cb < CB; cb++) {
+      if (!Cols::first_half(cb)) continue;  // second halves are turned with their first
+      constexpr int hd = HD > 0 ? HD : 64;
+      const int pb = cb + Cols::kHalfBlocks < CB ? cb + Cols::kHalfBlocks : cb;  // the partner block (always the first)
+      const int col = wave_n0 + Cols::at(cb);
+      if (col >= turned) continue;
+      const int at = (col & (hd - 1)) + 4 * g;  // index into the table row, < kHalf
 #pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-          constexpr int kBlocks = 4;
-          const int in_head = (cb * 32) & (head_dim - 1);  // the block's first column within its head
-          if (in_head >= half) continue;                   // second halves are turned with their first
-          if (n0 + wave_n * 128 + cb * 32 >= turned) continue;
-          const int pb = (cb + nb) % kBlocks;  // the partner block (a head's halves lie in one wave)
+      for (int rb = 0; rb < RB; rb++) {
+        const int r = wave_m * 16 * RB + rb * 16 + ln;
+        float c4[4], s4[4];
+        load4<F16>(reinterpret_cast<const uint16_t *>(cos_lds + r * kPitch) + at, c4);
+        load4<F16>(reinterpret_cast<const uint16_t *>(sin_lds + r * kPitch) + at, s4);
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const int at = in_head + 8 * q + 4 * g;  // index into the table row, < half
-            float c4[4], s4[4];
-            load4<F16>(cos_row + at, c4);
-            load4<F16>(sin_row + at, s4);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              const float y1 = acc[rb][cb][4 * q + e], y2 = acc[rb][pb][4 * q + e];
-              // gemm.rs:702-705: x cos, then the partner's product joined by one fused multiply-add.
-              const float y1c = y1 * c4[e], y2c = y2 * c4[e];
-              acc[rb][cb][4 * q + e] = __builtin_fmaf(y2, -s4[e], y1c);
-              acc[rb][pb][4 * q + e] = __builtin_fmaf(y1, s4[e], y2c);
-            }
-          }
+        for (int e = 0; e < 4; e++) {
+          const float y1 = acc[rb][cb][e], y2 = acc[rb][pb][e];
+          // gemm.rs:702-705: x cos, then the partner's product joined by one fused multiply-add.
+          const float y1c = y1 * c4[e], y2c = y2 * c4[e];
+          acc[rb][cb][e] = __builtin_fmaf(y2, -s4[e], y1c);
+          acc[rb][pb][e] = __builtin_fmaf(y1, s4[e], y2c);
         }
       }
     }
   }
   // ---- the store.  A lane owns rows, not runs of columns: written from the registers an instruction would
-  // touch 32 rows with 16 bytes each.  The rounded tile goes through LDS instead (every wave is done with the
+  // touch 16 rows with 32 bytes each.  The rounded tile goes through LDS instead (every wave is done with the
   // ring, and with the tables), 32 rows of a wave at a time in a stretch of its own, and leaves as whole row
-  // segments: an instruction stores 4 rows of 256 bytes, 16 bytes a lane.
+  // segments, 16 bytes a lane.
   __syncthreads();
+  constexpr int kOutPitch = T::kOutPitch, kRowChunks = CB * 2, kRowsPer = 64 / kRowChunks;
   uint8_t *stage = smem + wave * 32 * kOutPitch;
-  const int orow = lane >> 4, ochunk = lane & 15;
-  const int col = n0 + wave_n * 128 + ochunk * 8;  // n is a multiple of 8: a run of eight lies inside or outside
+  const int orow = lane / kRowChunks, ochunk = lane % kRowChunks;
+  const int col = wave_n0 + Cols::at(ochunk >> 1) + 8 * (ochunk & 1);  // n is a multiple of 8: a run of eight lies inside or outside
 #pragma unroll
-  for (int rb = 0; rb < S; rb++) {
-    uint8_t *srow = stage + ln * kOutPitch + 8 * g;
+  for (int half = 0; half < RB / 2; half++) {
 #pragma unroll
-    for (int cb = 0; cb < 4; cb++) {
+    for (int i = 0; i < 2; i++) {
+      const int rb = 2 * half + i;
+      uint8_t *srow = stage + (16 * i + ln) * kOutPitch + 8 * g;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
+      for (int cb = 0; cb < CB; cb++) {
         u32x2 out;
-        out[0] = pack2<F16>(acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1]);
-        out[1] = pack2<F16>(acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]);
-        *reinterpret_cast<u32x2 *>(srow + (32 * cb + 8 * q) * 2) = out;
+        out[0] = pack2<F16>(acc[rb][cb][0], acc[rb][cb][1]);
+        out[1] = pack2<F16>(acc[rb][cb][2], acc[rb][cb][3]);
+        *reinterpret_cast<u32x2 *>(srow + 32 * cb) = out;
       }
     }
 #pragma unroll
-    for (int it = 0; it < 8; it++) {
-      const int r = it * 4 + orow;
-      const u32x4 out = *reinterpret_cast<const u32x4 *>(stage + r * kOutPitch + ochunk * 16);
-      const int64_t row = m0 + wave_m * 32 * S + rb * 32 + r;
+    for (int it = 0; it < (32 + kRowsPer - 1) / kRowsPer; it++) {
+      const int r = it * kRowsPer + orow;
+      const bool mine = (kRowsPer * kRowChunks == 64 && 32 % kRowsPer == 0) || (orow < kRowsPer && r < 32);
+      const int64_t row = m0 + wave_m * 16 * RB + half * 32 + r;
       // Streaming stores: the output is not read again here, and left out of L2 it does not push the operands out.
-      if (row < rows && col < n) __builtin_nontemporal_store(out, reinterpret_cast<u32x4 *>(y + row * y_ld + col));
+      if (mine && row < rows && col < n)
+        __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(stage + r * kOutPitch + ochunk * 16),
+                                    reinterpret_cast<u32x4 *>(y + row * y_ld + col));
     }
   }
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
-template <bool F16, int HD, int S>
-__global__ __launch_bounds__(Tile<S>::kWaves * 64, 3 - S) void linear_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                                const uint16_t *__restrict__ bias,
-                                                                const uint16_t *__restrict__ cos_t,
-                                                                const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y,
-                                                                int64_t y_ld, int64_t rows, int32_t n, int32_t k, int32_t seq,
-                                                                int32_t heads,
-                                                                uint32_t tiles_n, uint32_t tiles, uint32_t per_xcd,
-                                                                uint32_t band) {
+template <bool F16, int HD, typename T>
+__global__ __launch_bounds__(T::kWaves * 64, T::kLds > 80 * 1024 ? T::kWaves / 4 : T::kWaves / 2) void linear_kernel(
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const uint16_t *__restrict__ bias,
+    const uint16_t *__restrict__ cos_t, const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y, int64_t y_ld,
+    int64_t rows, int32_t n, int32_t k, int32_t seq, int32_t heads, uint32_t tiles_n, uint32_t tiles, uint32_t per_xcd) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  linear_body<F16, HD, S>(smem, x, w, bias, cos_t, sin_t, y, y_ld, rows, n, k, seq, heads, tiles_n, tiles, per_xcd, band);
+  linear_body<F16, HD, T>(smem, x, w, bias, cos_t, sin_t, y, y_ld, rows, n, k, seq, heads, tiles_n, tiles, per_xcd);
 #endif
 }
 
-template <bool F16, int HD, int S>
+template <bool F16, int HD, typename T>
 hipError_t launch(const LinearArgs &a, hipStream_t stream) {
-  constexpr int kBm = Tile<S>::kBm, kBn = Tile<S>::kBn, kLds = Tile<S>::kLds, kWaves = Tile<S>::kWaves;
-  const int64_t tiles_m = (a.rows + kBm - 1) / kBm, tiles_n = (a.n + kBn - 1) / kBn;
+  const int64_t tiles_m = (a.rows + T::kBm - 1) / T::kBm, tiles_n = (a.n + T::kBn - 1) / T::kBn;
   const int64_t tiles = tiles_m * tiles_n;
   if (tiles == 0) return hipSuccess;
-  // Bands of row tiles per XCD where every XCD gets at least two row tiles; else runs of tiles.
-  const int64_t band = tiles_m >= 2 * kXcds ? (tiles_m + kXcds - 1) / kXcds : 0;
-  const int64_t per_xcd = band > 0 ? band * tiles_n : (tiles + kXcds - 1) / kXcds;
-  if (per_xcd * kXcds > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  auto kernel = linear_kernel<F16, HD, S>;
+  const int64_t per_xcd = (tiles + kXcds - 1) / kXcds;
+  if (tiles_m * kGroup > 0x7fffffffLL || per_xcd * kXcds > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  auto kernel = linear_kernel<F16, HD, T>;
   static std::atomic<uint64_t> configured{0};  // a bit per device ordinal, devices past 63 always ask
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
   const uint64_t bit = device < 64 ? 1ull << device : 0;
   if ((configured.load(std::memory_order_acquire) & bit) == 0) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds);
     if (e != hipSuccess) return e;
     configured.fetch_or(bit, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)(per_xcd * kXcds)), dim3(kWaves * 64), kLds, stream, (const uint16_t *)a.x,
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)(per_xcd * kXcds)), dim3(T::kWaves * 64), T::kLds, stream, (const uint16_t *)a.x,
                      (const uint16_t *)a.w, (const uint16_t *)a.bias, (const uint16_t *)a.cos, (const uint16_t *)a.sin,
                      (uint16_t *)a.y, a.y_ld > 0 ? a.y_ld : (int64_t)a.n, a.rows, a.n, a.k, a.seq, a.heads, (uint32_t)tiles_n,
-                     (uint32_t)tiles,
-                     (uint32_t)per_xcd, (uint32_t)band);
+                     (uint32_t)tiles, (uint32_t)per_xcd);
   return hipGetLastError();
+}
+
+template <int HD, typename T>
+hipError_t launch_hd(const LinearArgs &a, hipStream_t stream) {
+  return a.f16 ? launch<true, HD, T>(a, stream) : launch<false, HD, T>(a, stream);
 }
 
 }  // namespace
@@ -458,23 +466,19 @@ __device__ __forceinline__ void linear_entry(uint8_t *smem, const uint16_t *x, c
                                              const uint16_t *cos_t, const uint16_t *sin_t, uint16_t *y, int32_t rows,
                                              int32_t n, int32_t k, int32_t seq, int32_t heads) {
   if (rows <= 0 || n <= 0 || k <= 0) return;
-  constexpr int kBm = Tile<2>::kBm, kBn = Tile<2>::kBn;  // the code objects hold the 256 x 256 form
-  const uint32_t tiles_m = ((uint32_t)rows + kBm - 1) / kBm, tiles_n = ((uint32_t)n + kBn - 1) / kBn;
-  const uint32_t tiles = tiles_m * tiles_n;
-  // The library's launch geometry (see launch below in the library build): bands of row tiles per XCD
-  // where every XCD gets at least two, else runs of tiles.
-  const uint32_t band = tiles_m >= 2 * kXcds ? (tiles_m + kXcds - 1) / kXcds : 0;
-  const uint32_t per_xcd = band > 0 ? band * tiles_n : (tiles + kXcds - 1) / kXcds;
-  linear_body<F16, HD>(smem, x, w, bias, cos_t, sin_t, y, (int64_t)n, (int64_t)rows, n, k, seq > 0 ? seq : 1, heads, tiles_n,
-                       tiles, per_xcd, band);
+  // The code objects hold the 256 x 256 form, with the library's launch geometry.
+  const uint32_t tiles_n = ((uint32_t)n + Large::kBn - 1) / Large::kBn;
+  const uint32_t tiles = ((uint32_t)rows + Large::kBm - 1) / Large::kBm * tiles_n;
+  linear_body<F16, HD, Large>(smem, x, w, bias, cos_t, sin_t, y, (int64_t)n, (int64_t)rows, n, k, seq > 0 ? seq : 1, heads,
+                              tiles_n, tiles, (tiles + kXcds - 1) / kXcds);
 }
 
 #define SVODK_LINEAR_ENTRY(NAME, F16, HD)                                                                             \
-  extern "C" __global__ __launch_bounds__(Tile<2>::kWaves * 64, 1) void NAME(                                                  \
+  extern "C" __global__ __launch_bounds__(Large::kWaves * 64, 2) void NAME(                                                    \
       const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const uint16_t *__restrict__ bias,              \
       const uint16_t *__restrict__ cos_t, const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y, int32_t rows, \
       int32_t n, int32_t k, int32_t seq, int32_t heads) {                                                             \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[Tile<2>::kLds];                                                   \
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[Large::kLds];                                                     \
     linear_entry<F16, HD>(smem, x, w, bias, cos_t, sin_t, y, rows, n, k, seq, heads);                                 \
   }
 SVODK_LINEAR_ENTRY(svodk_linear_bf16, false, 0)
@@ -495,8 +499,6 @@ bool linear_supports(int64_t n, int64_t k) { return n > 0 && n % 8 == 0 && k >= 
 
 bool linear_turns(int32_t head_dim) { return head_dim == 64 || head_dim == 128; }
 
-// The tile a call's shape takes: 256 x 256 unless that makes fewer workgroups than half the compute units (256 on
-// this part; read from the device on a launch), where 128 x 128 makes four times as many.
 namespace {
 std::atomic<int> g_linear_tile{0};  // 0: by the shape; 128 or 256: every call
 }
@@ -504,11 +506,35 @@ int linear_tile(int32_t tile) {
   if (tile == 0 || tile == 128 || tile == 256) g_linear_tile.store(tile, std::memory_order_relaxed);
   return g_linear_tile.load(std::memory_order_relaxed);
 }
-int linear_tile_of(int64_t rows, int64_t n, int units) {
+
+LinearTile linear_tile_of(int64_t rows, int64_t n, int64_t k, int head_dim, int units) {
   const int named = g_linear_tile.load(std::memory_order_relaxed);
-  if (named != 0) return named;
-  const int64_t wide = ((rows + 255) / 256) * ((n + 255) / 256);
-  return 2 * wide <= units ? 128 : 256;
+  if (named != 0) return named == 128 ? kTile128x128 : kTile256x256;
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((rows + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  // A head of 128 does not fit the 64 columns' two halves.
+  if (k >= 512 && head_dim != 128 && tiles(128, 64) <= units) return kTile128x64;
+  // What is left is priced by rounds of workgroups over the part.  A round took, at k = 1024 and n = 3072 and 4096: 29 us
+  // of 256 x 256 tiles, 22 of 256 x 192 (whose 96 columns a wave hold no whole heads to turn), 16 of two 128 x 128 tiles
+  // a unit, 10 of one.
+  const int64_t large = tiles(256, 256), wide = tiles(256, 192), mid = tiles(128, 128);
+  auto rounds = [](int64_t t, int64_t each) { return (t + each - 1) / each; };
+  const int64_t cost_large = 58 * rounds(large, units), cost_wide = 44 * rounds(wide, units);
+  const int64_t left = mid % (2 * units);
+  const int64_t cost_mid = 32 * (mid / (2 * units)) + (left == 0 ? 0 : left <= units ? 20 : 32);
+  if (head_dim == 0 && cost_wide < cost_large && cost_wide < cost_mid) return kTile256x192;
+  return cost_mid < cost_large ? kTile128x128 : kTile256x256;
+}
+
+const char *linear_config(const LinearArgs &a) {
+  static const char *const kText[4][2] = {
+#define SVODK_GEMM(BM, BN, STAGES, WARPS)                                                                          \
+  {"GemmCfg { bm: " #BM ", bn: " #BN ", bk: 64, stages: " STAGES ", warps: " WARPS ", epilogue: { bias } }",        \
+   "GemmCfg { bm: " #BM ", bn: " #BN ", bk: 64, stages: " STAGES ", warps: " WARPS ", epilogue: { bias, rope } }"},
+      SVODK_GEMM(128, 64, "3", "[4, 1]")
+      SVODK_GEMM(128, 128, "2", "[4, 2]") SVODK_GEMM(256, 192, "2", "[4, 2]") SVODK_GEMM(256, 256, "2", "[4, 2]")
+#undef SVODK_GEMM
+  };
+  return kText[a.tile][a.cos != nullptr ? 1 : 0];
 }
 
 hipError_t launch_linear(const LinearArgs &a, hipStream_t stream) {
@@ -516,12 +542,18 @@ hipError_t launch_linear(const LinearArgs &a, hipStream_t stream) {
   if (a.cos != nullptr && (!linear_turns(a.head_dim) || a.seq <= 0 || (int64_t)a.heads * a.head_dim > a.n))
     return hipErrorInvalidValue;
   const int hd = a.cos != nullptr ? a.head_dim : 0;
-  if (a.tile == 128) {
-    if (a.f16) return hd == 0 ? launch<true, 0, 1>(a, stream) : hd == 64 ? launch<true, 64, 1>(a, stream) : launch<true, 128, 1>(a, stream);
-    return hd == 0 ? launch<false, 0, 1>(a, stream) : hd == 64 ? launch<false, 64, 1>(a, stream) : launch<false, 128, 1>(a, stream);
+  switch (a.tile) {
+    case kTile128x64:
+      if (hd == 128) return hipErrorInvalidValue;
+      return hd == 0 ? launch_hd<0, Narrow>(a, stream) : launch_hd<64, Narrow>(a, stream);
+    case kTile128x128:
+      return hd == 0 ? launch_hd<0, Mid>(a, stream) : hd == 64 ? launch_hd<64, Mid>(a, stream) : launch_hd<128, Mid>(a, stream);
+    case kTile256x192:
+      return hd == 0 ? launch_hd<0, Wide>(a, stream) : hipErrorInvalidValue;
+    case kTile256x256:
+      return hd == 0 ? launch_hd<0, Large>(a, stream) : hd == 64 ? launch_hd<64, Large>(a, stream) : launch_hd<128, Large>(a, stream);
   }
-  if (a.f16) return hd == 0 ? launch<true, 0, 2>(a, stream) : hd == 64 ? launch<true, 64, 2>(a, stream) : launch<true, 128, 2>(a, stream);
-  return hd == 0 ? launch<false, 0, 2>(a, stream) : hd == 64 ? launch<false, 64, 2>(a, stream) : launch<false, 128, 2>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace svodk

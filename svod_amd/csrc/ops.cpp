@@ -1167,13 +1167,8 @@ int svodk_linear(const svodk_tensor *x, const svodk_tensor *w, const svodk_linea
   a.heads = rope ? rope->heads : 0;
   a.head_dim = rope ? rope->head_dim : 0;
   a.f16 = x->dtype == SVODK_F16;
-  a.tile = svodk::linear_tile_of(rows, n, current_device_units());
-  if (a.tile == 128)
-    ran(op, "gemm", rope ? "GemmCfg { bm: 128, bn: 128, bk: 64, stages: 2, warps: [4, 1], epilogue: { bias, rope } }"
-                         : "GemmCfg { bm: 128, bn: 128, bk: 64, stages: 2, warps: [4, 1], epilogue: { bias } }");
-  else
-    ran(op, "gemm", rope ? "GemmCfg { bm: 256, bn: 256, bk: 64, stages: 2, warps: [4, 2], epilogue: { bias, rope } }"
-                         : "GemmCfg { bm: 256, bn: 256, bk: 64, stages: 2, warps: [4, 2], epilogue: { bias } }");
+  a.tile = svodk::linear_tile_of(rows, n, k, a.head_dim, current_device_units());
+  ran(op, "gemm", svodk::linear_config(a));
   const hipError_t e = svodk::launch_linear(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
   return SVODK_KERNEL;

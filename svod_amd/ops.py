@@ -365,8 +365,8 @@ def tune_decode(rows: int) -> None:
 
 
 def tune_linear(tile: int) -> None:
-    """The output tile of every later ``linear`` call: 256 (8 waves) or 128 (4 waves); 0 = by the shape (128 where
-    256 x 256 tiles would be fewer than half the compute units).  Process-wide; the two give the same bits."""
+    """The output tile of every later ``linear`` call: 256 (256 x 256) or 128 (128 x 128); 0 = by the shape.
+    Process-wide; the two give the same bits."""
     load_library().svodk_tune_linear(int(tile))
 
 
