@@ -341,9 +341,10 @@ void svodk_tune_streaming(int32_t workgroups_per_xcd);
 void svodk_tune_decode(int32_t rows);
 /*
  * No counterpart in the reference, whose tuner picks a GEMM's tile by measurement (tk/src/tune.rs, GemmCfg of
- * tk/src/ops/config/gemm.rs).  svodk_linear's tile follows the shape: 128 x 64 to 256 x 256.  `tile` = 256 or 128 names the (square) tile of every later call, 0 gives the
- * choice back to the shape.  Process-wide.  All of them give the same bits: a
- * column's k-steps are summed in the same order.
+ * tk/src/ops/config/gemm.rs).  svodk_linear's tile follows the shape: 16 x 16 to 64 x 64 where all rows together make
+ * few tiles, 128 x 64 to 256 x 256 above.  `tile` = 256 or 128 names the (square) tile of every later call, 0 gives the
+ * choice back to the shape.  Process-wide.  The two named tiles give the same bits, as do all from 128 x 64 up: a
+ * column's k-steps are summed in the same order.  The smaller ones sum k in eight shares.
  */
 void svodk_tune_linear(int32_t tile);
 /* The set the next streaming launch would take, and takes it (no device work): for tests of the

@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsvodk_gfx950.so")
 HOST = os.path.join(HERE, "_host.so")  # the Python side's calls (csrc/host.cpp), a module of this package
 SOURCES = ["ops.cpp", "heads_kernel.hip", "attention_kernel.hip", "combine_kernel.hip", "rows_kernel.hip",
-           "linear_kernel.hip", "decode_kernel.hip"]
+           "linear_kernel.hip", "linear_few_kernel.hip", "decode_kernel.hip"]
 
 # Packed-FP32 VALU ops are switched off for device code; the host pass of hipcc
 # does not know the feature and says so, which is harmless.

@@ -59,8 +59,9 @@ struct LinearArgs {
   int32_t f16;
   int32_t tile;      // a LinearTile, linear_tile_of's answer
 };
-// The workgroup's output tile, rows x columns.
+// The workgroup's output tile, rows x columns: linear_few_kernel's, smallest first, then linear_kernel's.
 enum LinearTile {
+  kFew16x16, kFew32x16, kFew32x32, kFew64x32, kFew64x64,
   kTile128x64, kTile128x128, kTile256x192, kTile256x256,
 };
 // The tile of a call (head_dim: of the heads it turns, 0: none) on a device of `units` compute units, unless
@@ -70,6 +71,9 @@ int linear_tile(int32_t tile);
 // Text of the tile configuration (for chosen()).
 const char *linear_config(const LinearArgs &a);
 hipError_t launch_linear(const LinearArgs &a, hipStream_t stream);
+// The kernel of the kFew tiles (linear_few_kernel.hip), for k up to kLinearFewMaxK.
+constexpr int64_t kLinearFewMaxK = 1 << 20;
+hipError_t launch_linear_few(const LinearArgs &a, hipStream_t stream);
 // Shapes the GEMM takes (n a multiple of 8, k a multiple of 32), and head sizes it turns.
 bool linear_supports(int64_t n, int64_t k);
 bool linear_turns(int32_t head_dim);

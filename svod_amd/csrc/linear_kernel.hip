@@ -511,6 +511,17 @@ LinearTile linear_tile_of(int64_t rows, int64_t n, int64_t k, int head_dim, int 
   const int named = g_linear_tile.load(std::memory_order_relaxed);
   if (named != 0) return named == 128 ? kTile128x128 : kTile256x256;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((rows + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  // A product with fewer than a compute unit's worth of tiles each wants as many compute units as it can get: the
+  // smallest tile that does not make more workgroups than there are units ([16, 1024] x [4096, 1024] 3.6 us in 16 x 16
+  // tiles, 5.2 in 64 x 64; 256 rows 19.6 and 7.1).  From k = 512 on: eight waves share k out a line at a time, and a
+  // shorter loop is all start and store whatever the tile.
+  if (k >= 512 && k <= kLinearFewMaxK) {
+    if (tiles(16, 16) <= units) return kFew16x16;
+    if (tiles(32, 16) <= units) return kFew32x16;
+    if (tiles(32, 32) <= units) return kFew32x32;
+    if (tiles(64, 32) <= units) return kFew64x32;
+    if (tiles(64, 64) <= units) return kFew64x64;
+  }
   // A head of 128 does not fit the 64 columns' two halves.
   if (k >= 512 && head_dim != 128 && tiles(128, 64) <= units) return kTile128x64;
   // What is left is priced by rounds of workgroups over the part.  A round took, at k = 1024 and n = 3072 and 4096: 29 us
@@ -526,11 +537,12 @@ LinearTile linear_tile_of(int64_t rows, int64_t n, int64_t k, int head_dim, int 
 }
 
 const char *linear_config(const LinearArgs &a) {
-  static const char *const kText[4][2] = {
+  static const char *const kText[9][2] = {
 #define SVODK_GEMM(BM, BN, STAGES, WARPS)                                                                          \
   {"GemmCfg { bm: " #BM ", bn: " #BN ", bk: 64, stages: " STAGES ", warps: " WARPS ", epilogue: { bias } }",        \
    "GemmCfg { bm: " #BM ", bn: " #BN ", bk: 64, stages: " STAGES ", warps: " WARPS ", epilogue: { bias, rope } }"},
-      SVODK_GEMM(128, 64, "3", "[4, 1]")
+      SVODK_GEMM(16, 16, "1", "k8") SVODK_GEMM(32, 16, "1", "k8") SVODK_GEMM(32, 32, "1", "k8")
+      SVODK_GEMM(64, 32, "1", "k8") SVODK_GEMM(64, 64, "1", "k8") SVODK_GEMM(128, 64, "3", "[4, 1]")
       SVODK_GEMM(128, 128, "2", "[4, 2]") SVODK_GEMM(256, 192, "2", "[4, 2]") SVODK_GEMM(256, 256, "2", "[4, 2]")
 #undef SVODK_GEMM
   };
@@ -552,8 +564,8 @@ hipError_t launch_linear(const LinearArgs &a, hipStream_t stream) {
       return hd == 0 ? launch_hd<0, Wide>(a, stream) : hipErrorInvalidValue;
     case kTile256x256:
       return hd == 0 ? launch_hd<0, Large>(a, stream) : hd == 64 ? launch_hd<64, Large>(a, stream) : launch_hd<128, Large>(a, stream);
+    default: return launch_linear_few(a, stream);
   }
-  return hipErrorInvalidValue;
 }
 
 }  // namespace svodk

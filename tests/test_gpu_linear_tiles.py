@@ -1,5 +1,5 @@
 """The projection GEMM's tiles at the sizes where each can go wrong: rows and columns on and off the tile, k in whole
-and half lines, turned heads of both sizes, a bias, both types, a window of a
+and half lines and shared out unevenly over eight waves, turned heads of both sizes, a bias, both types, a window of a
 wider output.  Against the unrounded f64 epilogue at the reference's bar (tk/src/test/unit/ops.rs:312)."""
 import numpy as np
 import pytest
@@ -14,6 +14,18 @@ pytestmark = pytest.mark.gpu
 
 # (rows, n, k, head size turned or 0, heads turned, bias, f16) -> the tile the shape takes
 CASES = [
+    ((1, 8, 512, 0, 0, True, False), (16, 16)),
+    ((16, 4096, 544, 128, 24, False, False), (16, 16)),
+    ((17, 200, 1024, 64, 3, True, True), (16, 16)),
+    ((33, 584, 832, 0, 0, True, False), (16, 16)),
+    ((30, 4096, 512, 64, 40, True, False), (32, 16)),
+    ((32, 2320, 608, 0, 0, False, True), (32, 16)),
+    ((45, 3072, 576, 128, 23, True, False), (32, 32)),
+    ((64, 4096, 512, 64, 1, False, True), (32, 32)),
+    ((100, 2304, 768, 64, 24, True, False), (64, 32)),
+    ((127, 4040, 512, 0, 0, True, False), (64, 32)),
+    ((250, 2304, 544, 128, 17, True, False), (64, 64)),
+    ((193, 4096, 512, 64, 33, False, True), (64, 64)),
     ((257, 4032, 544, 64, 60, True, False), (128, 64)),
     ((512, 4096, 512, 0, 0, False, True), (128, 64)),
     ((300, 4096, 512, 128, 31, True, False), (128, 128)),
