@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "kernels.h"
 
@@ -735,6 +736,15 @@ struct Ranges {
   int32_t app_lens_i64;
 };
 
+// What a kernel that has neither takes in their place: a launch's arguments are copied and written out to the device on
+// every call, and these are two thirds of them (a launch of 232 bytes of arguments 3.6 us of host time, of 72 3.0).
+struct NoSplits {};
+struct NoRanges {};
+template <bool SPLIT>
+using SplitsOf = std::conditional_t<SPLIT, Splits, NoSplits>;
+template <bool RANGED, bool BIASED, bool CACHED>
+using RangesOf = std::conditional_t<RANGED || BIASED || CACHED, Ranges, NoRanges>;
+
 // GROUPED: the query tile's rows are (head of the KV head's group, query) pairs instead of 128
 // queries of one head, for calls whose whole group fits a tile (a decoder step: heads / kv_heads
 // * T <= 128).  The group's heads then share one pass over their K and V instead of one each.
@@ -1280,8 +1290,13 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED && !(RANGED && CACHED)
     uint32_t units, uint32_t heads_group, const void *__restrict__ key_lens, const int32_t *__restrict__ row_order,
     int32_t t, uint32_t tk_lens64, const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
     const uint16_t *__restrict__ v, uint16_t *__restrict__ o, const void *__restrict__ key_mask, int32_t mask_bytes,
-    float scale, Splits sp, int32_t q_row_elems, int32_t kv_row_elems, Ranges rg) {
+    float scale, int32_t q_row_elems, int32_t kv_row_elems, SplitsOf<SPLIT> split_args,
+    RangesOf<RANGED, BIASED, CACHED> range_args) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  Splits sp{};
+  Ranges rg{};
+  if constexpr (SPLIT) sp = split_args;
+  if constexpr (RANGED || BIASED || CACHED) rg = range_args;
   // The first 14 dwords of the arguments (up to tk_lens64) arrive in registers with the wave
   // (kernarg preload, scalars and pointers only): they are what the workgroup's coordinates,
   // its batch row and its length need, so none of those waits for an argument load.
@@ -1716,39 +1731,45 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   }
   const uint32_t heads_group = (uint32_t)a.heads | geo.group << 16;
   const uint32_t tk_lens64 = (uint32_t)a.tk | (a.lens_i64 ? 0x80000000u : 0u);
-  Splits sp;
-  sp.count = (uint32_t)splits;
-  sp.rcp = rcp(sp.count);
-  sp.o_part = a.o_part;
-  sp.m_part = a.m_part;
-  sp.l_part = a.l_part;
-  sp.nbatch = (uint32_t)a.batch;
-  if (splits > 1 && (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr)) return hipErrorInvalidValue;
-  Ranges rg;
-  rg.win_left = a.win_left;
-  rg.win_right = a.win_right;
-  rg.chunk_size = a.chunk_size;
-  rg.chunk_left = a.chunk_left;
-  rg.chunk_right = a.chunk_right;
-  rg.seg_start = a.seg_start;
-  rg.seg_i64 = a.seg_i64;
-  rg.bias = (const uint16_t *)a.bias;
-  rg.bias_per_batch = a.bias_per_batch;
-  rg.bias_cols = a.tk + a.app_rows;
-  rg.kv_head_start = a.kv_head_start;
-  rg.row_map = a.row_map;
-  rg.row_map_i64 = a.row_map_i64;
-  rg.cache_rows = a.cache_rows;
-  rg.k_app = (const uint16_t *)a.k_app;
-  rg.v_app = (const uint16_t *)a.v_app;
-  rg.app_rows = a.app_rows;
-  rg.app_lens = a.app_lens;
-  rg.app_lens_i64 = a.app_lens_i64;
+  SplitsOf<SPLIT> split_args{};
+  RangesOf<RANGED, BIASED, CACHED> range_args{};
+  if constexpr (SPLIT) {
+    Splits &sp = split_args;
+    sp.count = (uint32_t)splits;
+    sp.rcp = rcp(sp.count);
+    sp.o_part = a.o_part;
+    sp.m_part = a.m_part;
+    sp.l_part = a.l_part;
+    sp.nbatch = (uint32_t)a.batch;
+    if (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr) return hipErrorInvalidValue;
+  }
+  if constexpr (RANGED || BIASED || CACHED) {
+    Ranges &rg = range_args;
+    rg.win_left = a.win_left;
+    rg.win_right = a.win_right;
+    rg.chunk_size = a.chunk_size;
+    rg.chunk_left = a.chunk_left;
+    rg.chunk_right = a.chunk_right;
+    rg.seg_start = a.seg_start;
+    rg.seg_i64 = a.seg_i64;
+    rg.bias = (const uint16_t *)a.bias;
+    rg.bias_per_batch = a.bias_per_batch;
+    rg.bias_cols = a.tk + a.app_rows;
+    rg.kv_head_start = a.kv_head_start;
+    rg.row_map = a.row_map;
+    rg.row_map_i64 = a.row_map_i64;
+    rg.cache_rows = a.cache_rows;
+    rg.k_app = (const uint16_t *)a.k_app;
+    rg.v_app = (const uint16_t *)a.v_app;
+    rg.app_rows = a.app_rows;
+    rg.app_lens = a.app_lens;
+    rg.app_lens_i64 = a.app_lens_i64;
+  }
   hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(NW * 64), smem, stream, geo.unit_size, geo.unit_rcp, geo.nqt,
                      geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp, geo.units, heads_group, a.key_lens,
                      (const int32_t *)a.row_order, a.t, tk_lens64, (const uint16_t *)a.q, (const uint16_t *)a.k,
-                     (const uint16_t *)a.v, (uint16_t *)a.o, a.key_mask, a.mask_bytes, a.scale, sp, (int32_t)q_row,
-                     (int32_t)kv_row, rg);
+                     (const uint16_t *)a.v, (uint16_t *)a.o, a.key_mask, a.mask_bytes, a.scale, (int32_t)q_row,
+                     (int32_t)kv_row, split_args, range_args);
   return hipGetLastError();
 }
 
