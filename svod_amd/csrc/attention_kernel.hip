@@ -35,6 +35,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 #if !defined(SVODK_CODE_OBJECT)
@@ -742,8 +743,27 @@ struct NoSplits {};
 struct NoRanges {};
 template <bool SPLIT>
 using SplitsOf = std::conditional_t<SPLIT, Splits, NoSplits>;
-template <bool RANGED, bool BIASED, bool CACHED>
-using RangesOf = std::conditional_t<RANGED || BIASED || CACHED, Ranges, NoRanges>;
+template <bool RANGED, bool BIASED>
+using RangesOf = std::conditional_t<RANGED || BIASED, Ranges, NoRanges>;
+// A word of the arguments as the address of memory that nothing writes while the kernel runs: reads at wave-uniform
+// indexes are scalar loads.
+template <typename T>
+__device__ __forceinline__ const T *constant(uint64_t word) {
+  return (const T *)(__attribute__((address_space(4))) const T *)word;
+}
+__device__ __forceinline__ const void *constant(const void *p) { return constant<void>((uint64_t)(uintptr_t)p); }
+// The rest of an instantiation's arguments.  What it does not have takes no byte: the plain kernel's record is then the
+// 112 bytes up to which a launch is cheap (launch.h; two empty structs as arguments of their own made it 116).
+template <bool SPLIT, bool RANGED, bool BIASED>
+struct TailOf {
+  const uint16_t *q, *k, *v;
+  uint16_t *o;
+  int32_t mask_bytes;
+  float scale;
+  int32_t q_row_elems, kv_row_elems;
+  [[no_unique_address]] SplitsOf<SPLIT> splits;
+  [[no_unique_address]] RangesOf<RANGED, BIASED> ranges;
+};
 
 // GROUPED: the query tile's rows are (head of the KV head's group, query) pairs instead of 128
 // queries of one head, for calls whose whole group fits a tile (a decoder step: heads / kv_heads
@@ -1284,24 +1304,45 @@ __device__ __forceinline__ void flash_fwd_body(
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16>
-__global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED && !(RANGED && CACHED)) ? 3 : (D <= 128 ? 2 : 1)) void flash_fwd_kernel(
+template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED, bool F16>
+__global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 : 1)) void flash_fwd_kernel(
+    uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u, uint32_t kvh_rcp,
+    uint32_t units, uint32_t heads_group, uint64_t key_lens, uint64_t row_order, int32_t t, uint32_t tk_lens64,
+    const void *__restrict__ key_mask, TailOf<SPLIT, RANGED, BIASED> tail) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  Splits sp{};
+  Ranges rg{};
+  if constexpr (SPLIT) sp = tail.splits;
+  if constexpr (RANGED || BIASED) {
+    rg = tail.ranges;
+    rg.seg_start = constant(rg.seg_start);
+  }
+  // The first 14 dwords of the arguments (up to tk_lens64) arrive in registers with the wave
+  // (kernarg preload, scalars only; the two addresses as words, which the launch does not look up):
+  // they are what the workgroup's coordinates, its batch row and its length need, so none of those
+  // waits for an argument load.
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, false, GROUPED, F16>(
+      smem, unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, units, heads_group, constant<void>(key_lens),
+      constant<int32_t>(row_order), t, tk_lens64, tail.q, tail.k, tail.v, tail.o, key_mask,
+      tail.mask_bytes, tail.scale, sp, tail.q_row_elems, tail.kv_row_elems, rg);
+#endif
+}
+
+// Over a cache, with the addresses as arguments of their own: of a struct's the compiler cannot tell that nothing writes
+// what they name, and the appended rows' count, read behind the loop's fills, is then no scalar load.
+template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED, bool F16>
+__global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED && !RANGED) ? 3 : (D <= 128 ? 2 : 1)) void flash_fwd_cached_kernel(
     uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u, uint32_t kvh_rcp,
     uint32_t units, uint32_t heads_group, const void *__restrict__ key_lens, const int32_t *__restrict__ row_order,
     int32_t t, uint32_t tk_lens64, const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
     const uint16_t *__restrict__ v, uint16_t *__restrict__ o, const void *__restrict__ key_mask, int32_t mask_bytes,
-    float scale, int32_t q_row_elems, int32_t kv_row_elems, SplitsOf<SPLIT> split_args,
-    RangesOf<RANGED, BIASED, CACHED> range_args) {
+    float scale, int32_t q_row_elems, int32_t kv_row_elems, SplitsOf<SPLIT> split_args, Ranges rg) {
 #if defined(__HIP_DEVICE_COMPILE__)
   Splits sp{};
-  Ranges rg{};
   if constexpr (SPLIT) sp = split_args;
-  if constexpr (RANGED || BIASED || CACHED) rg = range_args;
-  // The first 14 dwords of the arguments (up to tk_lens64) arrive in registers with the wave
-  // (kernarg preload, scalars and pointers only): they are what the workgroup's coordinates,
-  // its batch row and its length need, so none of those waits for an argument load.
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, CACHED, GROUPED, F16>(
+  flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, true, GROUPED, F16>(
       smem, unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, units, heads_group, key_lens, row_order, t, tk_lens64,
       q, k, v, o, key_mask, mask_bytes, scale, sp, q_row_elems, kv_row_elems, rg);
 #endif
@@ -1644,25 +1685,13 @@ hipError_t launch_stream(const AttnArgs &a, hipStream_t stream, int64_t slots, c
                          int64_t kv_row) {
   using TL = Tile<D>;
   constexpr int smem = TL::kLds + NW * kWaveRows * TL::kRowBytes + 16;  // ring, Q stage, two words
-  auto kernel = flash_stream_kernel<D, NW, CAUSAL, F16>;
-  static std::atomic<uint64_t> configured{0};
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = device < 64 ? 1ull << device : 0;
-  if ((configured.load(std::memory_order_acquire) & bit) == 0) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return e;
-    configured.fetch_or(bit, std::memory_order_release);
-  }
   const uint32_t heads_group = (uint32_t)a.heads | geo.group << 16;
   const uint32_t tk_lens64 = (uint32_t)a.tk | (a.lens_i64 ? 0x80000000u : 0u);
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)(slots * kXcds)), dim3(NW * 64), smem, stream, geo.unit_size, geo.unit_rcp,
-                     geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp, geo.units, heads_group, a.key_lens,
-                     (const uint16_t *)a.q, a.t, tk_lens64, (const uint16_t *)a.k, (const uint16_t *)a.v,
-                     (uint16_t *)a.o, a.scale, (int32_t)q_row, (int32_t)kv_row, (uint32_t)slots,
-                     next_queue_set(), (const int32_t *)a.row_order);
-  return hipGetLastError();
+  return Launch<flash_stream_kernel<D, NW, CAUSAL, F16>>::run(
+      slots * kXcds, NW * 64, smem, smem, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads,
+      geo.kvh_rcp, geo.units, heads_group, a.key_lens, (const uint16_t *)a.q, a.t, tk_lens64, (const uint16_t *)a.k,
+      (const uint16_t *)a.v, (uint16_t *)a.o, a.scale, (int32_t)q_row, (int32_t)kv_row, (uint32_t)slots, next_queue_set(),
+      (const int32_t *)a.row_order);
 }
 
 template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16>
@@ -1682,20 +1711,6 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   const int64_t kv_row = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
   // A fill addresses the rows of one key block with 32-bit byte offsets from the block's 64-bit base.
   if (kv_row * 2 * kBkv > 0x7fffffffLL || q_row > 0x7fffffffLL) return hipErrorInvalidValue;
-  auto kernel = flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, CACHED, GROUPED, F16>;
-  // The LDS ring is above the default limit of a launch: one attribute call per instantiation
-  // and device, from whichever thread gets there first (a second call is harmless).
-  static std::atomic<uint64_t> configured{0};  // a bit per device ordinal, devices past 63 always ask
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = device < 64 ? 1ull << device : 0;
-  if ((configured.load(std::memory_order_acquire) & bit) == 0) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            TL::kLds + kMaskLds);
-    if (e != hipSuccess) return e;
-    configured.fetch_or(bit, std::memory_order_release);
-  }
   // Units of work (batch, KV head) are dealt over the XCDs in whole rounds; the workgroups of
   // a round's missing units exit at once.
   const int64_t unit_size = (int64_t)(GROUPED ? 1 : a.heads / a.kv_heads) * nqt;
@@ -1723,7 +1738,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
       // (two graphs, one graph on two streams) would then share it: a capturing stream gets a
       // workgroup per tile, which needs no counters.
       hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-      e = hipStreamIsCapturing(stream, &capturing);
+      const hipError_t e = hipStreamIsCapturing(stream, &capturing);
       if (e != hipSuccess) return e;
       if (capturing == hipStreamCaptureStatusNone)
         return launch_stream<D, NW, CAUSAL, F16>(a, stream, knob, geo, q_row, kv_row);
@@ -1732,7 +1747,6 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   const uint32_t heads_group = (uint32_t)a.heads | geo.group << 16;
   const uint32_t tk_lens64 = (uint32_t)a.tk | (a.lens_i64 ? 0x80000000u : 0u);
   SplitsOf<SPLIT> split_args{};
-  RangesOf<RANGED, BIASED, CACHED> range_args{};
   if constexpr (SPLIT) {
     Splits &sp = split_args;
     sp.count = (uint32_t)splits;
@@ -1743,6 +1757,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     sp.nbatch = (uint32_t)a.batch;
     if (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr) return hipErrorInvalidValue;
   }
+  std::conditional_t<RANGED || BIASED || CACHED, Ranges, NoRanges> range_args{};
   if constexpr (RANGED || BIASED || CACHED) {
     Ranges &rg = range_args;
     rg.win_left = a.win_left;
@@ -1765,12 +1780,22 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     rg.app_lens = a.app_lens;
     rg.app_lens_i64 = a.app_lens_i64;
   }
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(NW * 64), smem, stream, geo.unit_size, geo.unit_rcp, geo.nqt,
-                     geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp, geo.units, heads_group, a.key_lens,
-                     (const int32_t *)a.row_order, a.t, tk_lens64, (const uint16_t *)a.q, (const uint16_t *)a.k,
-                     (const uint16_t *)a.v, (uint16_t *)a.o, a.key_mask, a.mask_bytes, a.scale, (int32_t)q_row,
-                     (int32_t)kv_row, split_args, range_args);
-  return hipGetLastError();
+  constexpr int kMost = TL::kLds + kMaskLds;
+  if constexpr (CACHED) {
+    return Launch<flash_fwd_cached_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
+        grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
+        geo.units, heads_group, a.key_lens, (const int32_t *)a.row_order, a.t, tk_lens64, (const uint16_t *)a.q,
+        (const uint16_t *)a.k, (const uint16_t *)a.v, (uint16_t *)a.o, a.key_mask, a.mask_bytes, a.scale, (int32_t)q_row,
+        (int32_t)kv_row, split_args, range_args);
+  } else {
+    const TailOf<SPLIT, RANGED, BIASED> tail = {(const uint16_t *)a.q, (const uint16_t *)a.k, (const uint16_t *)a.v,
+                                                (uint16_t *)a.o, a.mask_bytes, a.scale, (int32_t)q_row,
+                                                (int32_t)kv_row, split_args, range_args};
+    return Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
+        grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
+        geo.units, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64,
+        a.key_mask, tail);
+  }
 }
 
 template <int D, bool RANGED, bool BIASED, bool CACHED, bool F16>

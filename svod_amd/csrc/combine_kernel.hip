@@ -11,6 +11,7 @@
 #include <atomic>
 
 #include "kernels.h"
+#include "launch.h"
 
 #if !defined(SVODK_CODE_OBJECT)
 // The partial states of a split call whose caller cannot lend a workspace because it cannot allocate
@@ -105,12 +106,16 @@ __device__ __forceinline__ void combine_body(const float *__restrict__ o_part, c
 }
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
+struct CombineCall {
+  const float *o_part, *m_part, *l_part;
+  uint16_t *o;
+  int64_t rows;
+  int32_t splits;
+};
+
 template <int D, bool F16>
-__global__ __launch_bounds__(kThreads) void combine_kernel(const float *__restrict__ o_part,
-                                                           const float *__restrict__ m_part,
-                                                           const float *__restrict__ l_part, uint16_t *__restrict__ o,
-                                                           int64_t rows, int32_t splits) {
-  combine_body<D, F16>(o_part, m_part, l_part, o, rows, splits);
+__global__ __launch_bounds__(kThreads) void combine_kernel(const CombineCall c) {
+  combine_body<D, F16>(c.o_part, c.m_part, c.l_part, c.o, c.rows, c.splits);
 }
 
 template <int D, bool F16>
@@ -119,9 +124,8 @@ hipError_t launch(const CombineArgs &a, hipStream_t stream) {
   if (threads == 0) return hipSuccess;
   const int64_t blocks = (threads + kThreads - 1) / kThreads;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((combine_kernel<D, F16>), dim3((uint32_t)blocks), dim3(kThreads), 0, stream, a.o_part, a.m_part,
-                     a.l_part, (uint16_t *)a.o, a.rows, a.splits);
-  return hipGetLastError();
+  return Launch<combine_kernel<D, F16>>::run(
+      blocks, kThreads, 0, 0, stream, CombineCall{a.o_part, a.m_part, a.l_part, (uint16_t *)a.o, a.rows, a.splits});
 }
 
 std::atomic<void *> g_scratch_at[64];  // `scratch` by device ordinal; devices past 63 ask every time

@@ -18,6 +18,7 @@
 
 #include "convert.h"
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 namespace {
@@ -158,16 +159,21 @@ __device__ __forceinline__ void heads_body(const uint16_t *__restrict__ qkv, con
 }
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
+template <typename Div>
+struct HeadsCall {
+  const uint16_t *qkv, *q_w, *k_w, *cos, *sin;
+  uint16_t *q, *k, *v;
+  int64_t items;
+  Div by_slots, by_t;
+  int32_t heads, kv_heads;
+  float eps;
+  int32_t rope;
+};
+
 template <int D, typename Div, bool F16>
-__global__ __launch_bounds__(kThreads) void heads_kernel(const uint16_t *__restrict__ qkv,
-                                                         const uint16_t *__restrict__ q_w,
-                                                         const uint16_t *__restrict__ k_w,
-                                                         const uint16_t *__restrict__ cos_t,
-                                                         const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ q,
-                                                         uint16_t *__restrict__ k, uint16_t *__restrict__ v,
-                                                         int64_t items, Div by_slots, Div by_t, int32_t heads,
-                                                         int32_t kv_heads, float eps, int32_t rope) {
-  heads_body<D, Div, F16>(qkv, q_w, k_w, cos_t, sin_t, q, k, v, items, by_slots, by_t, heads, kv_heads, eps, rope);
+__global__ __launch_bounds__(kThreads) void heads_kernel(const HeadsCall<Div> c) {
+  heads_body<D, Div, F16>(c.qkv, c.q_w, c.k_w, c.cos, c.sin, c.q, c.k, c.v, c.items, c.by_slots, c.by_t, c.heads,
+                          c.kv_heads, c.eps, c.rope);
 }
 
 template <int D, bool F16>
@@ -181,21 +187,19 @@ hipError_t launch(const HeadsArgs &a, hipStream_t stream) {
   const int64_t blocks = (threads + per_block - 1) / per_block;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const int64_t t = a.t > 0 ? a.t : 1;
+  auto run = [&](auto by_slots, auto by_t) {
+    typedef decltype(by_t) Div;
+    return Launch<heads_kernel<D, Div, F16>>::run(
+        blocks, kThreads, 0, 0, stream,
+        HeadsCall<Div>{(const uint16_t *)a.qkv, (const uint16_t *)a.q_w, (const uint16_t *)a.k_w, (const uint16_t *)a.cos,
+                       (const uint16_t *)a.sin, (uint16_t *)a.q, (uint16_t *)a.k, (uint16_t *)a.v, items, by_slots, by_t,
+                       a.heads, a.kv_heads, a.eps, a.rope});
+  };
   if (blocks * per_block < 0xffffffffLL) {
     auto rcp = [](uint32_t d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); };
-    const Div32 by_slots = {(uint32_t)slots, rcp((uint32_t)slots)}, by_t = {(uint32_t)t, rcp((uint32_t)t)};
-    hipLaunchKernelGGL((heads_kernel<D, Div32, F16>), dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
-                       (const uint16_t *)a.qkv, (const uint16_t *)a.q_w, (const uint16_t *)a.k_w,
-                       (const uint16_t *)a.cos, (const uint16_t *)a.sin, (uint16_t *)a.q, (uint16_t *)a.k,
-                       (uint16_t *)a.v, items, by_slots, by_t, a.heads, a.kv_heads, a.eps, a.rope);
-  } else {
-    const Div64 by_slots = {slots, 0}, by_t = {t, 0};
-    hipLaunchKernelGGL((heads_kernel<D, Div64, F16>), dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
-                       (const uint16_t *)a.qkv, (const uint16_t *)a.q_w, (const uint16_t *)a.k_w,
-                       (const uint16_t *)a.cos, (const uint16_t *)a.sin, (uint16_t *)a.q, (uint16_t *)a.k,
-                       (uint16_t *)a.v, items, by_slots, by_t, a.heads, a.kv_heads, a.eps, a.rope);
+    return run(Div32{(uint32_t)slots, rcp((uint32_t)slots)}, Div32{(uint32_t)t, rcp((uint32_t)t)});
   }
-  return hipGetLastError();
+  return run(Div64{slots, 0}, Div64{t, 0});
 }
 
 }  // namespace

@@ -19,6 +19,7 @@
 
 #include "convert.h"
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 namespace {
@@ -78,13 +79,19 @@ __device__ __forceinline__ i32x4 make_rsrc(const void *base, int64_t bytes) {
   return i32x4{(int)(uint32_t)addr, (int)(uint32_t)((addr >> 32) & 0xffffu), (int)(uint32_t)clamped, 0x00020000};
 }
 
+struct FewCall {
+  const uint16_t *x, *w, *bias, *cos, *sin;
+  uint16_t *y;
+  int64_t y_ld;
+  int32_t rows, n, k, seq, heads;
+  uint32_t tiles_m;
+};
+
 // HD: the head size a turning kernel is built for (64 or 128), 0: no turn.
 template <bool F16, int HD, typename T>
-__global__ __launch_bounds__(kWaves * 64) void linear_few_kernel(
-    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const uint16_t *__restrict__ bias,
-    const uint16_t *__restrict__ cos_t, const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y, int64_t y_ld,
-    int32_t rows, int32_t n, int32_t k, int32_t seq, int32_t heads, uint32_t tiles_m) {
+__global__ __launch_bounds__(kWaves * 64) void linear_few_kernel(const FewCall call) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  const auto [x, w, bias, cos_t, sin_t, y, y_ld, rows, n, k, seq, heads, tiles_m] = call;
   constexpr int RB = T::RB, CB = T::CB, kBm = T::kBm, kBn = T::kBn, kRun = kBn / 2, kPitch = T::kPitch;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = (int)__builtin_amdgcn_workitem_id_x(), lane = tid & 63;
@@ -213,26 +220,13 @@ __global__ __launch_bounds__(kWaves * 64) void linear_few_kernel(
 
 template <bool F16, int HD, typename T>
 hipError_t launch(const LinearArgs &a, hipStream_t stream) {
-  auto kernel = linear_few_kernel<F16, HD, T>;
-  if (T::kLds > 64 * 1024) {
-    static std::atomic<uint64_t> configured{0};  // a bit per device ordinal, devices past 63 always ask
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    if (e != hipSuccess) return e;
-    const uint64_t bit = device < 64 ? 1ull << device : 0;
-    if ((configured.load(std::memory_order_acquire) & bit) == 0) {
-      e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds);
-      if (e != hipSuccess) return e;
-      configured.fetch_or(bit, std::memory_order_release);
-    }
-  }
   const int64_t tiles_m = (a.rows + T::kBm - 1) / T::kBm, tiles = tiles_m * ((a.n + T::kBn - 1) / T::kBn);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles), dim3(kWaves * 64), T::kLds, stream, (const uint16_t *)a.x,
-                     (const uint16_t *)a.w, (const uint16_t *)a.bias, (const uint16_t *)a.cos, (const uint16_t *)a.sin,
-                     (uint16_t *)a.y, a.y_ld > 0 ? a.y_ld : (int64_t)a.n, (int32_t)a.rows, a.n, a.k, a.seq, a.heads,
-                     (uint32_t)tiles_m);
-  return hipGetLastError();
+  return Launch<linear_few_kernel<F16, HD, T>>::run(
+      tiles, kWaves * 64, T::kLds, T::kLds, stream,
+      FewCall{(const uint16_t *)a.x, (const uint16_t *)a.w, (const uint16_t *)a.bias, (const uint16_t *)a.cos,
+              (const uint16_t *)a.sin, (uint16_t *)a.y, a.y_ld > 0 ? a.y_ld : (int64_t)a.n, (int32_t)a.rows, a.n, a.k, a.seq,
+              a.heads, (uint32_t)tiles_m});
 }
 
 template <typename T>

@@ -27,6 +27,7 @@
 #include <atomic>
 
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 namespace {
@@ -410,14 +411,21 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
 #endif  // __HIP_DEVICE_COMPILE__
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
+struct LinearCall {
+  const uint16_t *x, *w, *bias, *cos, *sin;
+  uint16_t *y;
+  int64_t y_ld, rows;
+  int32_t n, k, seq, heads;
+  uint32_t tiles_n, tiles, per_xcd;
+};
+
 template <bool F16, int HD, typename T>
 __global__ __launch_bounds__(T::kWaves * 64, T::kLds > 80 * 1024 ? T::kWaves / 4 : T::kWaves / 2) void linear_kernel(
-    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const uint16_t *__restrict__ bias,
-    const uint16_t *__restrict__ cos_t, const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ y, int64_t y_ld,
-    int64_t rows, int32_t n, int32_t k, int32_t seq, int32_t heads, uint32_t tiles_n, uint32_t tiles, uint32_t per_xcd) {
+    const LinearCall c) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  linear_body<F16, HD, T>(smem, x, w, bias, cos_t, sin_t, y, y_ld, rows, n, k, seq, heads, tiles_n, tiles, per_xcd);
+  linear_body<F16, HD, T>(smem, c.x, c.w, c.bias, c.cos, c.sin, c.y, c.y_ld, c.rows, c.n, c.k, c.seq, c.heads, c.tiles_n,
+                          c.tiles, c.per_xcd);
 #endif
 }
 
@@ -428,22 +436,11 @@ hipError_t launch(const LinearArgs &a, hipStream_t stream) {
   if (tiles == 0) return hipSuccess;
   const int64_t per_xcd = (tiles + kXcds - 1) / kXcds;
   if (tiles_m * kGroup > 0x7fffffffLL || per_xcd * kXcds > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  auto kernel = linear_kernel<F16, HD, T>;
-  static std::atomic<uint64_t> configured{0};  // a bit per device ordinal, devices past 63 always ask
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = device < 64 ? 1ull << device : 0;
-  if ((configured.load(std::memory_order_acquire) & bit) == 0) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds);
-    if (e != hipSuccess) return e;
-    configured.fetch_or(bit, std::memory_order_release);
-  }
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)(per_xcd * kXcds)), dim3(T::kWaves * 64), T::kLds, stream, (const uint16_t *)a.x,
-                     (const uint16_t *)a.w, (const uint16_t *)a.bias, (const uint16_t *)a.cos, (const uint16_t *)a.sin,
-                     (uint16_t *)a.y, a.y_ld > 0 ? a.y_ld : (int64_t)a.n, a.rows, a.n, a.k, a.seq, a.heads, (uint32_t)tiles_n,
-                     (uint32_t)tiles, (uint32_t)per_xcd);
-  return hipGetLastError();
+  return Launch<linear_kernel<F16, HD, T>>::run(
+      per_xcd * kXcds, T::kWaves * 64, T::kLds, T::kLds, stream,
+      LinearCall{(const uint16_t *)a.x, (const uint16_t *)a.w, (const uint16_t *)a.bias, (const uint16_t *)a.cos,
+                 (const uint16_t *)a.sin, (uint16_t *)a.y, a.y_ld > 0 ? a.y_ld : (int64_t)a.n, a.rows, a.n, a.k, a.seq,
+                 a.heads, (uint32_t)tiles_n, (uint32_t)tiles, (uint32_t)per_xcd});
 }
 
 template <int HD, typename T>

@@ -21,6 +21,7 @@
 
 #include "convert.h"
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 namespace {
@@ -166,16 +167,20 @@ __device__ __forceinline__ void rows_body(const uint16_t *__restrict__ x, const 
 }
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
+struct RowsCall {
+  const uint16_t *x, *residual, *w, *b;
+  uint16_t *out, *sum;
+  int64_t rows;
+  int32_t d;
+  float inv_d, eps;
+  uint32_t blocks;  // of the grid
+};
+
 template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16>
-__global__ __launch_bounds__(kRowsPerBlock * 64) void rows_kernel(const uint16_t *__restrict__ x,
-                                                                   const uint16_t *__restrict__ residual,
-                                                                   const uint16_t *__restrict__ w,
-                                                                   const uint16_t *__restrict__ b,
-                                                                   uint16_t *__restrict__ out, uint16_t *__restrict__ sum,
-                                                                   int64_t rows, int32_t d, float inv_d, float eps) {
-  rows_body<SPANS, LAYER, RESIDUAL, BIAS, F16>(x, residual, w, b, out, sum, rows, d, inv_d, eps,
+__global__ __launch_bounds__(kRowsPerBlock * 64) void rows_kernel(const RowsCall c) {
+  rows_body<SPANS, LAYER, RESIDUAL, BIAS, F16>(c.x, c.residual, c.w, c.b, c.out, c.sum, c.rows, c.d, c.inv_d, c.eps,
                                                (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6),
-                                               (int64_t)gridDim.x * kRowsPerBlock);
+                                               (int64_t)c.blocks * kRowsPerBlock);
 }
 
 template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16>
@@ -215,11 +220,10 @@ hipError_t launch_rows(const NormArgs &a, hipStream_t stream) {
       if (best == 0 || cost < best) best = cost, blocks = units * m;
     }
   }
-  hipLaunchKernelGGL((rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16>), dim3((uint32_t)blocks), dim3(kRowsPerBlock * 64), 0,
-                     stream, (const uint16_t *)a.x, (const uint16_t *)a.residual, (const uint16_t *)a.w,
-                     (const uint16_t *)a.b, (uint16_t *)a.out, (uint16_t *)a.sum, a.rows, a.d,
-                     (float)(1.0 / (double)a.d), (float)a.eps);
-  return hipGetLastError();
+  return Launch<rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16>>::run(
+      blocks, kRowsPerBlock * 64, 0, 0, stream,
+      RowsCall{(const uint16_t *)a.x, (const uint16_t *)a.residual, (const uint16_t *)a.w, (const uint16_t *)a.b,
+               (uint16_t *)a.out, (uint16_t *)a.sum, a.rows, a.d, (float)(1.0 / (double)a.d), (float)a.eps, (uint32_t)blocks});
 }
 
 template <int SPANS, bool F16>
