@@ -21,6 +21,7 @@
 #include <atomic>
 
 #include "kernels.h"
+#include "launch.h"
 
 namespace svodk {
 namespace {
@@ -35,6 +36,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNoKey = -1e30f;   // the running maximum before any key: finite, so that its differences are numbers
 constexpr int kMaxWaves = 8;       // waves a workgroup
 constexpr int kAhead = 2;          // passes a lane works on at a time, with as many more in flight
+constexpr int kArrivalSets = 64, kArrivalUnits = 1024;  // counter sets (a stream each) and (batch, KV head) pairs a set
+
+// Waves a workgroup: few workgroups take eight each, so that the launch still has its bytes in flight.
+__host__ __device__ constexpr int decode_waves(int64_t workgroups) { return workgroups >= 256 ? 4 : kMaxWaves; }
 
 // What the kernel takes: AttnArgs without the fields a decoder step does not have.
 struct DecodeArgs {
@@ -50,6 +55,7 @@ struct DecodeArgs {
   int32_t batch, t, tk, heads, kv_heads, group;
   int32_t splits, cached, kv_head_start, cache_rows, app_rows;
   float scale;
+  uint32_t *arrivals;  // of a launch that merges its splits itself: a counter a (batch, KV head), at zero
 };
 
 template <bool F16>
@@ -108,8 +114,24 @@ __device__ __forceinline__ void merge(State &a, const State &b) {
   for (int j = 0; j < 8; j++) a.acc[j] = a.acc[j] * wa + b.acc[j] * wb;
 }
 
+// Partial states that another workgroup of the launch reads go past the L2s, each of which serves one XCD, and are read
+// the same way: stores and loads that are coherent over the device.
+__device__ __forceinline__ void put(float *p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void put2(float *p, const f32x2 &x) {  // 8-byte aligned
+  __hip_atomic_store(reinterpret_cast<uint64_t *>(p), __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float got(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ f32x2 got2(const float *p) {  // 8-byte aligned
+  return __builtin_bit_cast(f32x2, __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// What a launch does with its splits: it has none; it leaves partial states for combine_kernel; the workgroup of a
+// (batch, KV head) that ends last merges them.
+enum { kWhole, kPartial, kMerged };
+
 // The workgroup's program for `nw` waves, for the kernels below to inline.
-template <int D, int R, bool F16, bool SPLIT>
+template <int D, int R, bool F16, int MODE>
 __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // No contraction beyond the fused multiply-adds written out below: the library's kernel (its wave count a launch
@@ -121,14 +143,15 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
   constexpr int U = kAhead;  // the same for every R: a row's arithmetic does not depend on how many rows share the keys
   __shared__ float merged[kMaxWaves][R][LPK][10];
 
+  constexpr bool SPLIT = MODE != kWhole;
   const int wg = (int)__builtin_amdgcn_workgroup_id_x();
+  const int tid = (int)__builtin_amdgcn_workitem_id_x();
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int split = SPLIT ? wg % p.splits : 0;
   const int unit = SPLIT ? wg / p.splits : wg;
   const int b = unit / p.kv_heads;
   const int kvh = unit - b * p.kv_heads;
-  const int tid = (int)__builtin_amdgcn_workitem_id_x();
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pos = lane % LPK;   // which 16 bytes of a row
   const int slot = lane / LPK;  // which row of a wave instruction
   const bool pos_ok = 8 * pos < D;
@@ -326,10 +349,12 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
     }
   }
   __syncthreads();
-  if (wave != 0 || slot != 0 || !pos_ok) return;
+  if (wave != 0) return;
+  const bool mine = slot == 0 && pos_ok;
+  const int64_t states = (int64_t)p.batch * p.t * p.heads;  // of a split
 #pragma unroll
   for (int r = 0; r < R; r++) {
-    if (r >= rows) break;
+    if (r >= rows || !mine) break;
     State all = st[r];
     for (int w = 1; w < nw; w++) {
       State other;
@@ -340,9 +365,17 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
       for (int j = 0; j < 8; j++) other.acc[j] = at[2 + j];
       merge(all, other);
     }
-    if (SPLIT) {
+    if (MODE == kMerged) {
+      const int64_t at = split * states + out_row[r];
+      if (pos == 0) {
+        put(p.m_part + at, all.m);
+        put(p.l_part + at, all.l);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) put2(p.o_part + at * D + 8 * pos + j, f32x2{all.acc[j], all.acc[j + 1]});
+    } else if (SPLIT) {
       // L899-921: the accumulator as it stands, the maximum in the exponent's units, the sum.
-      const int64_t at = (int64_t)split * p.batch * p.t * p.heads + out_row[r];
+      const int64_t at = split * states + out_row[r];
       if (pos == 0) {
         p.m_part[at] = all.m;
         p.l_part[at] = all.l;
@@ -359,34 +392,160 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
       *reinterpret_cast<u32x4 *>(p.o + out_row[r] * D + 8 * pos) = out;
     }
   }
+  if (MODE != kMerged) return;
+  // ---- the merge.  This wave's states are where every workgroup sees them before it counts itself in; the workgroup
+  // that counts itself in last reads them all.  No one waits for anyone.  The arithmetic is combine_kernel's, operation
+  // for operation: a captured launch, which leaves the merge to that kernel, gives the same bits.  It is a chain of four
+  // trips to memory, some 3 us, where a kernel of its own is a launch (2.6 us of host time) and 3.5 us: one sequence over
+  // 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int splits = p.splits;
+  uint32_t *arrivals = p.arrivals + b * p.kv_heads + kvh;
+  uint32_t before = 0;
+  if (lane == 0) before = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((int)__builtin_amdgcn_readfirstlane((int)before) != splits - 1) return;
+  asm volatile("" ::: "memory");  // the states are read from here on
+  if (lane == 0) __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the stream's next launch
+  constexpr int kLanes = D / 4, kBatch = 8;
+  for (int c = lane; c < rows * kLanes; c += 64) {
+    const int r = c / kLanes, chunk = c - r * kLanes;
+    // out_row[r] without an index into registers: a row is (head of the group, token).
+    const int in_group = r / p.t;
+    const int64_t orow = ((int64_t)b * p.t + (r - in_group * p.t)) * p.heads + kvh * p.group + in_group;
+    struct States {
+      float m[kBatch], l[kBatch];
+      f32x2 lo[kBatch], hi[kBatch];
+    };
+    auto ask = [&](States &x, int from) {
+#pragma unroll
+      for (int i = 0; i < kBatch; i++) {
+        const int64_t at = (int64_t)min(from + i, splits - 1) * states + orow;
+        x.m[i] = got(p.m_part + at);
+        x.l[i] = got(p.l_part + at);
+        x.lo[i] = got2(p.o_part + at * D + 4 * chunk);
+        x.hi[i] = got2(p.o_part + at * D + 4 * chunk + 2);
+      }
+    };
+    States x;
+    ask(x, 0);
+    float m = x.m[0];
+#pragma unroll
+    for (int i = 1; i < kBatch; i++) m = __builtin_fmaxf(m, x.m[i]);
+    for (int from = kBatch; from < splits; from += kBatch) {
+      float y[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; i++) y[i] = got(p.m_part + (int64_t)min(from + i, splits - 1) * states + orow);
+#pragma unroll
+      for (int i = 0; i < kBatch; i++) m = __builtin_fmaxf(m, y[i]);
+    }
+    float l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int from = 0; from < splits; from += kBatch) {
+      if (from > 0) ask(x, from);
+#pragma unroll
+      for (int i = 0; i < kBatch; i++) {
+        if (from + i >= splits) break;
+        const float w = __builtin_amdgcn_exp2f(x.m[i] - m);
+        const float part[4] = {x.lo[i][0] * w, x.lo[i][1] * w, x.hi[i][0] * w, x.hi[i][1] * w};
+        const float lw = x.l[i] * w;
+        const bool none = from + i == 0;
+        l = none ? lw : l + lw;
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[j] = none ? part[j] : acc[j] + part[j];
+      }
+    }
+    const float ll = l == 0.0f ? 1.0f : l;
+    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+    const u32x2 out = {pack2<F16>(acc[0] / ll, acc[1] / ll), pack2<F16>(acc[2] / ll, acc[3] / ll)};
+    *reinterpret_cast<u32x2 *>(p.o + orow * D + 4 * chunk) = out;
+  }
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
-template <int D, int R, bool F16, bool SPLIT>
-__global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const DecodeArgs p) {
+// The counters of the launches that merge their splits themselves, zero between them.  A set a stream: the launches of a
+// stream run one after another, and the last workgroup of each puts its counters back.
+__device__ uint32_t g_arrivals[kArrivalSets][kArrivalUnits];
+
+// DecodeArgs as they travel: in 112 bytes (launch.h).  k and v are at the launch's first head, the states in one piece.
+struct Packed {
+  const uint16_t *q, *k, *v;
+  uint16_t *o;
+  const void *keys;  // key_lens, key_mask or null
+  const void *row_map;
+  const uint16_t *k_app, *v_app;
+  const void *app_lens;
+  float *states;
+  int32_t tk, batch, kv_row_elems;
+  float scale;
+  int32_t cache_rows;
+  int32_t splits;
+  uint32_t set;           // of the counters
+  uint32_t kv_heads : 16, group_less_one : 2, t_less_one : 2, app_rows : 7, mask : 1, wide_keys : 1, row_map_i64 : 1,
+      app_lens_i64 : 1, packed_rows : 1;
+};
+static_assert(sizeof(Packed) <= 112 && kDecodeRows <= 4, "the record's size, the group's and the tokens' two bits");
+
+template <int D, int R, bool F16, int MODE>
+__global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  decode_body<D, R, F16, SPLIT>(p, (int)(__builtin_amdgcn_workgroup_size_x() >> 6));
+  DecodeArgs p;
+  p.q = a.q, p.k = a.k, p.v = a.v, p.o = a.o;
+  p.key_lens = a.mask ? nullptr : a.keys, p.key_mask = a.mask ? a.keys : nullptr;
+  p.lens_i64 = a.wide_keys, p.mask_bytes = a.wide_keys ? 4 : 1;
+  p.row_map = a.row_map, p.row_map_i64 = a.row_map_i64, p.cache_rows = a.cache_rows;
+  p.k_app = a.k_app, p.v_app = a.v_app, p.app_lens = a.app_lens, p.app_lens_i64 = a.app_lens_i64, p.app_rows = a.app_rows;
+  p.batch = a.batch, p.tk = a.tk, p.t = a.t_less_one + 1, p.group = a.group_less_one + 1;
+  p.kv_heads = a.kv_heads, p.heads = p.kv_heads * p.group;
+  p.splits = MODE == kWhole ? 1 : a.splits;
+  p.kv_row_elems = a.kv_row_elems, p.q_row_elems = a.packed_rows ? (int64_t)a.kv_row_elems : (int64_t)p.heads * D;
+  p.cached = 1, p.kv_head_start = 0, p.scale = a.scale;
+  const int64_t states = (int64_t)p.splits * p.batch * p.t * p.heads;
+  p.o_part = a.states, p.m_part = a.states + states * D, p.l_part = p.m_part + states;
+  p.arrivals = g_arrivals[a.set];
+  decode_body<D, R, F16, MODE>(p, decode_waves((int64_t)p.batch * p.kv_heads * p.splits));
 #endif
 }
 
 template <int D, int R, bool F16>
-hipError_t launch_r(const DecodeArgs &p, int waves, hipStream_t stream) {
+hipError_t launch_r(const Packed &p, bool merged, hipStream_t stream) {
   const int64_t grid = (int64_t)p.batch * p.kv_heads * p.splits;
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  if (p.splits > 1)
-    hipLaunchKernelGGL((decode_kernel<D, R, F16, true>), dim3((uint32_t)grid), dim3(waves * 64), 0, stream, p);
-  else
-    hipLaunchKernelGGL((decode_kernel<D, R, F16, false>), dim3((uint32_t)grid), dim3(waves * 64), 0, stream, p);
-  return hipGetLastError();
+  const uint32_t threads = (uint32_t)decode_waves(grid) * 64;
+  if (p.splits == 1) return Launch<decode_kernel<D, R, F16, kWhole>>::run(grid, threads, 0, 0, stream, p);
+  return merged ? Launch<decode_kernel<D, R, F16, kMerged>>::run(grid, threads, 0, 0, stream, p)
+                : Launch<decode_kernel<D, R, F16, kPartial>>::run(grid, threads, 0, 0, stream, p);
 }
 
 template <int D>
-hipError_t launch_d(const DecodeArgs &p, int rows, int waves, bool f16, hipStream_t stream) {
-  if (rows <= 1) return f16 ? launch_r<D, 1, true>(p, waves, stream) : launch_r<D, 1, false>(p, waves, stream);
-  if (rows <= 2) return f16 ? launch_r<D, 2, true>(p, waves, stream) : launch_r<D, 2, false>(p, waves, stream);
-  return f16 ? launch_r<D, 4, true>(p, waves, stream) : launch_r<D, 4, false>(p, waves, stream);
+hipError_t launch_d(const Packed &p, int rows, bool merged, bool f16, hipStream_t stream) {
+  if (rows <= 1) return f16 ? launch_r<D, 1, true>(p, merged, stream) : launch_r<D, 1, false>(p, merged, stream);
+  if (rows <= 2) return f16 ? launch_r<D, 2, true>(p, merged, stream) : launch_r<D, 2, false>(p, merged, stream);
+  return f16 ? launch_r<D, 4, true>(p, merged, stream) : launch_r<D, 4, false>(p, merged, stream);
+}
+
+// The counters' set of a stream, or -1: the stream is being captured (a replay may run beside anything), is not one
+// stream (each thread's default stream has the same handle), or the sets have run out.
+int arrival_set(hipStream_t stream) {
+  constexpr int kDevices = 16;
+  static std::atomic<uintptr_t> owner[kDevices][kArrivalSets];  // the stream's handle + 1; 0: free
+  if (stream == hipStreamPerThread || stream == (hipStream_t)1) return -1;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kDevices) return -1;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (capturing != hipStreamCaptureStatusNone) return -1;
+  const uintptr_t me = (uintptr_t)stream + 1;
+  for (int i = 0; i < kArrivalSets; i++) {
+    uintptr_t there = owner[device][i].load(std::memory_order_acquire);
+    if (there == me) return i;
+    if (there == 0 && owner[device][i].compare_exchange_strong(there, me, std::memory_order_acq_rel)) return i;
+    if (there == me) return i;
+  }
+  return -1;
 }
 
 std::atomic<int> g_decode_rows{kDecodeRowsDefault};
@@ -406,50 +565,54 @@ bool attention_decodes(const AttnArgs &a) {
   return rows >= 1 && rows <= g_decode_rows.load(std::memory_order_relaxed);
 }
 
+int32_t decode_arrivals(const AttnArgs &a, hipStream_t stream) {
+  return (int64_t)a.batch * a.kv_heads <= kArrivalUnits ? arrival_set(stream) : -1;
+}
+
 hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
-  DecodeArgs p;
+  const int splits = a.splits > 1 ? a.splits : 1;
+  if (splits > 1 && (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr)) return hipErrorInvalidValue;
+  const int64_t q_row = a.q_row_elems > 0 ? a.q_row_elems : (int64_t)a.heads * a.d;
+  const int64_t kv_row = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
+  const bool packed_rows = q_row != (int64_t)a.heads * a.d;
+  if (kv_row > 0x7fffffffLL || (packed_rows && q_row != kv_row) || a.kv_heads > 0xffff || a.app_rows > 127) return hipErrorInvalidValue;
+  Packed p{};
   p.q = (const uint16_t *)a.q;
-  p.k = (const uint16_t *)a.k;
-  p.v = (const uint16_t *)a.v;
+  p.k = (const uint16_t *)a.k + (a.cached ? (int64_t)a.kv_head_start * a.d : 0);
+  p.v = (const uint16_t *)a.v + (a.cached ? (int64_t)a.kv_head_start * a.d : 0);
   p.o = (uint16_t *)a.o;
-  p.key_lens = a.key_lens;
-  p.key_mask = a.key_mask;
-  p.row_map = a.row_map;
-  p.k_app = (const uint16_t *)a.k_app;
-  p.v_app = (const uint16_t *)a.v_app;
-  p.app_lens = a.app_lens;
-  p.o_part = a.o_part;
-  p.m_part = a.m_part;
-  p.l_part = a.l_part;
-  p.q_row_elems = a.q_row_elems > 0 ? a.q_row_elems : (int64_t)a.heads * a.d;
-  p.kv_row_elems = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
-  p.lens_i64 = a.lens_i64;
-  p.mask_bytes = a.mask_bytes;
-  p.row_map_i64 = a.row_map_i64;
-  p.app_lens_i64 = a.app_lens_i64;
-  p.batch = a.batch;
-  p.t = a.t;
+  p.keys = a.key_mask != nullptr ? a.key_mask : a.key_lens;
+  p.mask = a.key_mask != nullptr;
+  p.wide_keys = a.key_mask != nullptr ? a.mask_bytes == 4 : a.lens_i64 != 0;
+  if (a.cached) {
+    p.row_map = a.row_map;
+    p.row_map_i64 = a.row_map_i64 != 0;
+    p.cache_rows = a.cache_rows;
+    p.k_app = (const uint16_t *)a.k_app;
+    p.v_app = (const uint16_t *)a.v_app;
+    p.app_rows = (uint32_t)a.app_rows;
+    p.app_lens = a.app_lens;
+    p.app_lens_i64 = a.app_lens_i64 != 0;
+  }
+  p.states = a.o_part;
   p.tk = a.tk;
-  p.heads = a.heads;
-  p.kv_heads = a.kv_heads;
-  p.group = a.heads / a.kv_heads;
-  p.splits = a.splits > 1 ? a.splits : 1;
-  p.cached = a.cached;
-  p.kv_head_start = a.kv_head_start;
-  p.cache_rows = a.cache_rows;
-  p.app_rows = a.app_rows;
+  p.batch = a.batch;
+  p.kv_row_elems = (int32_t)kv_row;
   p.scale = a.scale;
-  if (p.splits > 1 && (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr)) return hipErrorInvalidValue;
-  const int rows = p.group * p.t;
-  // Few workgroups take eight waves each, so that the launch still has its bytes in flight.
-  const int64_t grid = (int64_t)p.batch * p.kv_heads * p.splits;
-  const int waves = grid >= 256 ? 4 : kMaxWaves;
+  p.splits = splits;
+  p.kv_heads = (uint32_t)a.kv_heads;
+  p.group_less_one = (uint32_t)(a.heads / a.kv_heads - 1);
+  p.t_less_one = (uint32_t)(a.t - 1);
+  p.packed_rows = packed_rows;
+  p.set = splits > 1 && a.arrivals >= 0 ? (uint32_t)a.arrivals : 0u;
+  const int rows = a.heads / a.kv_heads * a.t;
+  const bool merged = splits > 1 && a.arrivals >= 0;
   switch (a.d) {
-    case 32: return launch_d<32>(p, rows, waves, a.f16 != 0, stream);
-    case 48: return launch_d<48>(p, rows, waves, a.f16 != 0, stream);
-    case 64: return launch_d<64>(p, rows, waves, a.f16 != 0, stream);
-    case 128: return launch_d<128>(p, rows, waves, a.f16 != 0, stream);
-    case 256: return launch_d<256>(p, rows, waves, a.f16 != 0, stream);
+    case 32: return launch_d<32>(p, rows, merged, a.f16 != 0, stream);
+    case 48: return launch_d<48>(p, rows, merged, a.f16 != 0, stream);
+    case 64: return launch_d<64>(p, rows, merged, a.f16 != 0, stream);
+    case 128: return launch_d<128>(p, rows, merged, a.f16 != 0, stream);
+    case 256: return launch_d<256>(p, rows, merged, a.f16 != 0, stream);
   }
   return hipErrorInvalidValue;
 }
@@ -489,7 +652,8 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.batch = batch, p.t = t, p.tk = tk, p.heads = heads, p.kv_heads = kv_heads, p.group = heads / kv_heads;          \
     p.splits = (S) && splits > 1 ? splits : 1, p.cached = cached, p.kv_head_start = kv_head_start;                    \
     p.cache_rows = cache_rows, p.app_rows = app_rows, p.scale = __builtin_bit_cast(float, scale_bits);                \
-    svodk::decode_body<D, R, F16, (S) != 0>(p, 4);                                                                    \
+    p.arrivals = nullptr;                                                                                             \
+    svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole>(p, 4);                                  \
   }
 #define SVODK_DECODE_ROWS_OF(D, T, F16, S) \
   SVODK_DECODE_ENTRY(D, 1, T, F16, S) SVODK_DECODE_ENTRY(D, 2, T, F16, S) SVODK_DECODE_ENTRY(D, 4, T, F16, S)

@@ -101,6 +101,7 @@ struct AttnArgs {
   // m_part and l_part [splits, batch, t, heads], all f32; launch_combine merges them.
   int32_t splits;
   float *o_part, *m_part, *l_part;
+  int32_t arrivals;  // a decoder step merges its splits itself, with this set of counters (decode_arrivals); -1: it does not
   // Elements from a token's row to the next in q and in k/v; 0 = dense (heads * d, kv_heads * d).
   // A fused projection read in place (tk/src/ops/attention.rs:104-122) has its own row for both.
   int64_t q_row_elems, kv_row_elems;
@@ -164,6 +165,9 @@ bool attention_decodes(const AttnArgs &a);
 void attention_decode_rows(int32_t rows);
 int32_t attention_decode_limit();
 hipError_t launch_decode(const AttnArgs &a, hipStream_t stream);
+// The counters with which a split decoder step on `stream` merges its own splits, for AttnArgs::arrivals; -1: it leaves
+// them to launch_combine (a stream under capture, more (batch, KV head) pairs than a set has counters).
+int32_t decode_arrivals(const AttnArgs &a, hipStream_t stream);
 // One head size's kernels each (launch_attention picks by AttnArgs::d).
 hipError_t launch_attention_d32(const AttnArgs &a, hipStream_t stream);
 hipError_t launch_attention_d48(const AttnArgs &a, hipStream_t stream);

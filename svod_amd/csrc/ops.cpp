@@ -679,10 +679,13 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.m_part = a.o_part + (int64_t)a.splits * rows * d;
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
+  // A split decoder step merges its splits itself where it can.
+  a.arrivals = a.splits > 1 && svodk::attention_decodes(a) ? svodk::decode_arrivals(a, (hipStream_t)hip_stream) : -1;
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
-  if (a.splits > 1) {
+  if (a.splits > 1) ran(op, "combine_splits", "NormCfg { br: 4 }");
+  if (a.splits > 1 && a.arrivals < 0) {
     svodk::CombineArgs c{};
     c.o_part = a.o_part;
     c.m_part = a.m_part;
@@ -692,7 +695,6 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     c.d = a.d;
     c.splits = a.splits;
     c.f16 = a.f16;
-    ran(op, "combine_splits", "NormCfg { br: 4 }");
     e = svodk::launch_combine(c, (hipStream_t)hip_stream);
     if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
   }
