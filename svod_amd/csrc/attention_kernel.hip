@@ -781,8 +781,9 @@ __device__ __forceinline__ void flash_fwd_body(
     const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, uint16_t *__restrict__ o,
     const void *__restrict__ key_mask, int32_t mask_bytes, float scale, const Splits &sp, int32_t q_row_elems,
     int32_t kv_row_elems, const Ranges &rg) {
-  // Two of the arguments are packed: heads | group << 16, and tk | (key_lens is 64-bit) << 31.
-  const Geometry geo = {unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, heads_group >> 16, units};
+  // Three of the arguments are packed: heads | group << 16, tk | (key_lens is 64-bit) << 31, and
+  // units | (the rows go longest first) << 31.
+  const Geometry geo = {unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, heads_group >> 16, units & 0x7fffffffu};
   const int heads = (int)(heads_group & 0xffffu);
   const int tk = (int)(tk_lens64 & 0x7fffffffu);
   const bool lens_i64 = (tk_lens64 >> 31) != 0;
@@ -826,6 +827,21 @@ __device__ __forceinline__ void flash_fwd_body(
   // that rows with more keys can go first and the launch ends on its short tiles.
   int b = b_place;
   if (row_order != nullptr) b = row_order[b_place];
+  // Without one, place p of a call with key lengths takes the row with the p-th most keys, which every wave finds from
+  // the lengths (a lane a row: launch() says when): the launch then starts its long tiles first, on compute units of
+  // their own, and ends on its short ones.  [9, 333] x 12 heads of 100 to 333 keys 11.1 -> 9.9 us.  The search is three
+  // instructions a row, in front of a workgroup's first loads.  (For a key mask, whose rows' keys a few probed elements
+  // would have to tell, it takes back more than it gives: 39.3 -> 41.8 us for 32 rows of 512.)
+  constexpr bool kOrders = !SPLIT && !RANGED && !BIASED && !CACHED && !GROUPED;
+  const bool longest_first = kOrders && (units >> 31) != 0;
+  const int lane_row = (int)__builtin_amdgcn_workitem_id_x() & 63;
+  int lane_len = -1;
+  if (longest_first) {
+    if (lane_row < (int)div_by(geo.units, geo.kv_heads, geo.kvh_rcp)) {
+      const long long n = lens_i64 ? ((const long long *)key_lens)[lane_row] : (long long)((const int *)key_lens)[lane_row];
+      lane_len = n < 0 ? 0 : (n < (long long)tk ? (int)n : tk);
+    }
+  }
   // Everything the first loads and fills take from the argument record (past the words that arrive in
   // registers with the wave) is asked for HERE, while the row's number is on its way: left to the
   // compiler those loads sit behind the wait for it, and a workgroup's start is three scalar memory
@@ -835,6 +851,16 @@ __device__ __forceinline__ void flash_fwd_body(
   if (row_order != nullptr) {
     const int nbatch = (int)div_by(geo.units, geo.kv_heads, geo.kvh_rcp);
     b = min(max(b, 0), nbatch - 1);
+  }
+  int len = tk;
+  if (longest_first) {
+    const int nbatch = (int)div_by(geo.units, geo.kv_heads, geo.kvh_rcp);
+    // Keys that differ: the length, then the row's number, the smaller first.
+    const int key = lane_len < 0 ? -1 : (lane_len << 6) + 63 - lane_row;
+    int rank = 0;
+    for (int j = 0; j < nbatch; j++) rank += __builtin_amdgcn_readlane(key, j) > key ? 1 : 0;
+    b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane_len >= 0 && rank == b_place));
+    len = __builtin_amdgcn_readlane(lane_len, b);
   }
   // Grid x of the reference is order * splits + split (L523); geo.nqt counts those.
   int split = 0, tile = order, nqt = (int)geo.nqt;
@@ -855,8 +881,7 @@ __device__ __forceinline__ void flash_fwd_body(
   const int ln = w.lane & 31;  // the query column this lane owns
 
   // L533-536: len = min(key_lens[b], tk).
-  int len = tk;
-  if (key_lens != nullptr) {
+  if (key_lens != nullptr && !longest_first) {
     long long n = lens_i64 ? ((const long long *)key_lens)[b] : (long long)((const int *)key_lens)[b];
     n = n < 0 ? 0 : n;
     len = n < (long long)tk ? (int)n : tk;
@@ -1746,6 +1771,11 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   }
   const uint32_t heads_group = (uint32_t)a.heads | geo.group << 16;
   const uint32_t tk_lens64 = (uint32_t)a.tk | (a.lens_i64 ? 0x80000000u : 0u);
+  // The rows' order is worth finding where tiles are long enough for the rows to differ by and the rows few: 16 rows of
+  // 64 to 512 keys 23.3 -> 22.0 us, of 125 to 1000 65 -> 61; 32 rows of up to 512 38.1 -> 39.9, 60 of up to 140 19.5 -> 24.6.
+  const bool longest_first = !SPLIT && !RANGED && !BIASED && !CACHED && !GROUPED && a.key_lens != nullptr &&
+                             a.row_order == nullptr && a.batch > 2 && a.batch <= 16 && a.tk > 256 && a.tk < (1 << 24);
+  const uint32_t units_order = geo.units | (longest_first ? 0x80000000u : 0u);
   SplitsOf<SPLIT> split_args{};
   if constexpr (SPLIT) {
     Splits &sp = split_args;
@@ -1793,7 +1823,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
                                                 (int32_t)kv_row, split_args, range_args};
     return Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
         grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
-        geo.units, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64,
+        units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64,
         a.key_mask, tail);
   }
 }
