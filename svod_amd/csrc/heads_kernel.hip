@@ -16,6 +16,8 @@
 // needs no lane exchange, and the sum of squares needs log2(d/16) exchanges.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "convert.h"
 #include "kernels.h"
 #include "launch.h"
@@ -46,12 +48,31 @@ struct Div64 {
 // A block owns kItems * kThreads consecutive lanes of the flat (row, slot, part) space, slots
 // fastest: thread i takes lanes i, i + kThreads, ...  All loads of a thread are issued before
 // any arithmetic.  One item per thread measured fastest on an MI355X (2 and 4 were 5 % and
-// 20 % slower: the many small waves keep more of HBM's channels busy than fewer long ones),
-// and every byte is touched once, so loads and stores are marked non-temporal.
+// 20 % slower: the many small waves keep more of HBM's channels busy than fewer long ones).
 constexpr int kItems = 1;
 
+// Every byte is touched once, but the input was written by the call before and the outputs are read by the one after.
+// What a launch of so many bytes of outputs (as many of input) marks non-temporal:
+//   kStream   loads and stores, below 16 MiB: 1400 Qwen3 rows 5.8 us, 6.7 with either kept
+//   kKeep     neither, to 96 MiB: 2800 rows 10.2 -> 9.6, 8000 rows 23.7 -> 22.0
+//   kKeepOut  loads only: at 16384 rows (134 MB) 45.0 -> 44.4 by itself, and the layer's prefill 321.5 -> 315.7, whose
+//             attention then finds the last of the outputs on the chip
+enum { kStream, kKeep, kKeepOut };
+template <int CACHE>
+__device__ __forceinline__ u32x4 take(const uint16_t *p) {
+  if constexpr (CACHE == kKeep) return *reinterpret_cast<const u32x4 *>(p);
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+}
+template <int CACHE>
+__device__ __forceinline__ void leave(uint16_t *p, const u32x4 &x) {
+  if constexpr (CACHE == kStream)
+    __builtin_nontemporal_store(x, reinterpret_cast<u32x4 *>(p));
+  else
+    *reinterpret_cast<u32x4 *>(p) = x;
+}
+
 // The workgroup's program, for the kernels below to inline.
-template <int D, typename Div, bool F16>
+template <int D, typename Div, bool F16, int CACHE>
 __device__ __forceinline__ void heads_body(const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ q_w,
                                            const uint16_t *__restrict__ k_w, const uint16_t *__restrict__ cos_t,
                                            const uint16_t *__restrict__ sin_t, uint16_t *__restrict__ q,
@@ -81,8 +102,8 @@ __device__ __forceinline__ void heads_body(const uint16_t *__restrict__ qkv, con
     const uint16_t *src = qkv + ((int64_t)row[u] * slots + slot[u]) * D + part * 8;
     w1[u] = w2[u] = u32x4{0, 0, 0, 0};
     if (live[u]) {
-      w1[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src));
-      w2[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + kHalf));
+      w1[u] = take<CACHE>(src);
+      w2[u] = take<CACHE>(src + kHalf);
     }
   }
 
@@ -153,8 +174,8 @@ __device__ __forceinline__ void heads_body(const uint16_t *__restrict__ qkv, con
       o1 = w1[u];  // untouched slots (v, or q/k with neither norm nor rope) keep their bits
       o2 = w2[u];
     }
-    __builtin_nontemporal_store(o1, reinterpret_cast<u32x4 *>(dst));
-    __builtin_nontemporal_store(o2, reinterpret_cast<u32x4 *>(dst + kHalf));
+    leave<CACHE>(dst, o1);
+    leave<CACHE>(dst + kHalf, o2);
   }
 }
 
@@ -170,10 +191,10 @@ struct HeadsCall {
   int32_t rope;
 };
 
-template <int D, typename Div, bool F16>
+template <int D, typename Div, bool F16, int CACHE>
 __global__ __launch_bounds__(kThreads) void heads_kernel(const HeadsCall<Div> c) {
-  heads_body<D, Div, F16>(c.qkv, c.q_w, c.k_w, c.cos, c.sin, c.q, c.k, c.v, c.items, c.by_slots, c.by_t, c.heads,
-                          c.kv_heads, c.eps, c.rope);
+  heads_body<D, Div, F16, CACHE>(c.qkv, c.q_w, c.k_w, c.cos, c.sin, c.q, c.k, c.v, c.items, c.by_slots, c.by_t, c.heads,
+                                 c.kv_heads, c.eps, c.rope);
 }
 
 template <int D, bool F16>
@@ -187,9 +208,9 @@ hipError_t launch(const HeadsArgs &a, hipStream_t stream) {
   const int64_t blocks = (threads + per_block - 1) / per_block;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const int64_t t = a.t > 0 ? a.t : 1;
-  auto run = [&](auto by_slots, auto by_t) {
+  auto run = [&](auto by_slots, auto by_t, auto cache) {
     typedef decltype(by_t) Div;
-    return Launch<heads_kernel<D, Div, F16>>::run(
+    return Launch<heads_kernel<D, Div, F16, decltype(cache)::value>>::run(
         blocks, kThreads, 0, 0, stream,
         HeadsCall<Div>{(const uint16_t *)a.qkv, (const uint16_t *)a.q_w, (const uint16_t *)a.k_w, (const uint16_t *)a.cos,
                        (const uint16_t *)a.sin, (uint16_t *)a.q, (uint16_t *)a.k, (uint16_t *)a.v, items, by_slots, by_t,
@@ -197,9 +218,13 @@ hipError_t launch(const HeadsArgs &a, hipStream_t stream) {
   };
   if (blocks * per_block < 0xffffffffLL) {
     auto rcp = [](uint32_t d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); };
-    return run(Div32{(uint32_t)slots, rcp((uint32_t)slots)}, Div32{(uint32_t)t, rcp((uint32_t)t)});
+    const Div32 by_slots = {(uint32_t)slots, rcp((uint32_t)slots)}, by_t = {(uint32_t)t, rcp((uint32_t)t)};
+    const int64_t bytes = items * D * 2;
+    if (bytes < (16 << 20)) return run(by_slots, by_t, std::integral_constant<int, kStream>());
+    if (bytes <= (96 << 20)) return run(by_slots, by_t, std::integral_constant<int, kKeep>());
+    return run(by_slots, by_t, std::integral_constant<int, kKeepOut>());
   }
-  return run(Div64{slots, 0}, Div64{t, 0});
+  return run(Div64{slots, 0}, Div64{t, 0}, std::integral_constant<int, kKeepOut>());
 }
 
 }  // namespace
@@ -241,7 +266,7 @@ __device__ __forceinline__ void heads_entry(const uint16_t *qkv, const uint16_t 
   auto rcp = [](uint32_t d) { return d <= 1 ? 0xffffffffu : 0xffffffffu / d; };  // within one of floor(2^32 / d)
   const uint32_t slots = (uint32_t)(heads + 2 * kv_heads), tt = (uint32_t)(t > 0 ? t : 1);
   const Div32 by_slots = {slots, rcp(slots)}, by_t = {tt, rcp(tt)};
-  heads_body<D, Div32, F16>(qkv, q_w, k_w, cos_t, sin_t, q, k, v, (int64_t)rows * slots, by_slots, by_t, heads, kv_heads,
+  heads_body<D, Div32, F16, kStream>(qkv, q_w, k_w, cos_t, sin_t, q, k, v, (int64_t)rows * slots, by_slots, by_t, heads, kv_heads,
                             __builtin_bit_cast(float, eps_bits), rope);
 }
 
