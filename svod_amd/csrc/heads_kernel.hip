@@ -54,7 +54,7 @@ constexpr int kItems = 1;
 // Every byte is touched once, but the input was written by the call before and the outputs are read by the one after.
 // What a launch of so many bytes of outputs (as many of input) marks non-temporal:
 //   kStream   loads and stores, below 16 MiB: 1400 Qwen3 rows 5.8 us, 6.7 with either kept
-//   kKeep     neither, to 96 MiB: 2800 rows 10.2 -> 9.6, 8000 rows 23.7 -> 22.0
+//   kKeep     neither, to 70 MiB: 2800 rows 10.2 -> 9.6, 8000 rows 23.7 -> 22.0
 //   kKeepOut  loads only: at 16384 rows (134 MB) 45.0 -> 44.4 by itself, and the layer's prefill 321.5 -> 315.7, whose
 //             attention then finds the last of the outputs on the chip
 enum { kStream, kKeep, kKeepOut };
@@ -221,7 +221,7 @@ hipError_t launch(const HeadsArgs &a, hipStream_t stream) {
     const Div32 by_slots = {(uint32_t)slots, rcp((uint32_t)slots)}, by_t = {(uint32_t)t, rcp((uint32_t)t)};
     const int64_t bytes = items * D * 2;
     if (bytes < (16 << 20)) return run(by_slots, by_t, std::integral_constant<int, kStream>());
-    if (bytes <= (96 << 20)) return run(by_slots, by_t, std::integral_constant<int, kKeep>());
+    if (bytes <= (70 << 20)) return run(by_slots, by_t, std::integral_constant<int, kKeep>());
     return run(by_slots, by_t, std::integral_constant<int, kKeepOut>());
   }
   return run(Div64{slots, 0}, Div64{t, 0}, std::integral_constant<int, kKeepOut>());

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "convert.h"
 #include "kernels.h"
@@ -50,9 +51,16 @@ __device__ __forceinline__ float wave_sum(float x) {
   return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
-// The sum is read again only a layer's work later: its stores leave the chip.  The operands are what the call before
-// wrote, and are read as they lie: asked for with a non-temporal mark, they took a tenth longer ([4500, 2048] add+RMSNorm
-// 14.2 -> 12.4 us, [16384, 768] LayerNorm 10.8 -> 9.7).
+// What a launch marks non-temporal, by its size (launch_rows).  The sum, read again only a layer's work later, always is.
+//   kLoadsKept  the normalised rows, not the operands, which the call before wrote: marked, they took a tenth longer
+//   kKept       nothing: the rows are there for the projection that reads them
+//   kOutKept    the operands: more of them than the chip's last cache holds
+enum { kLoadsKept, kKept, kOutKept };
+template <int CACHE>
+__device__ __forceinline__ u32x4 take(const uint16_t *p) {
+  if constexpr (CACHE == kOutKept) return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+  return *reinterpret_cast<const u32x4 *>(p);
+}
 __device__ __forceinline__ void store_once(u32x4 *p, const u32x4 &v) { __builtin_nontemporal_store(v, p); }
 
 // SPANS = ceil(d / 512): the 128-bit accesses a lane makes per row and tensor.
@@ -60,8 +68,7 @@ __device__ __forceinline__ void store_once(u32x4 *p, const u32x4 &v) { __builtin
 // loads are in flight while the row before it is normalised and stored, and the weight (and bias) are read once a
 // wave, not once a row.  (A wave a row, the reference's form, leaves a wave's start and end, and the weight's 2 d
 // bytes from L2, on every row's bill: 25.5 us against 23.3 for a [16384, 2048] RMSNorm.)
-// KEEP: the normalised rows stay on the chip, for the call that reads them next.
-template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16, bool KEEP>
+template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16, int CACHE>
 __device__ __forceinline__ void rows_body(const uint16_t *__restrict__ x, const uint16_t *__restrict__ residual,
                                           const uint16_t *__restrict__ w, const uint16_t *__restrict__ b,
                                           uint16_t *__restrict__ out, uint16_t *__restrict__ sum, int64_t rows, int32_t d,
@@ -91,8 +98,8 @@ __device__ __forceinline__ void rows_body(const uint16_t *__restrict__ x, const 
       const int at = s * kSpan + lane * 8;
       raw.x[s] = raw.r[s] = u32x4{0, 0, 0, 0};
       if (live[s] && row < rows) {
-        raw.x[s] = *reinterpret_cast<const u32x4 *>(x + base + at);
-        if (RESIDUAL) raw.r[s] = *reinterpret_cast<const u32x4 *>(residual + base + at);
+        raw.x[s] = take<CACHE>(x + base + at);
+        if (RESIDUAL) raw.r[s] = take<CACHE>(residual + base + at);
       }
     }
   };
@@ -154,7 +161,7 @@ __device__ __forceinline__ void rows_body(const uint16_t *__restrict__ x, const 
         }
         packed[i] = narrow<F16>(y0, y1);
       }
-      if constexpr (KEEP)
+      if constexpr (CACHE != kLoadsKept)
         *reinterpret_cast<u32x4 *>(out + base + at) = packed;
       else
         store_once(reinterpret_cast<u32x4 *>(out + base + at), packed);
@@ -182,9 +189,9 @@ struct RowsCall {
   uint32_t blocks;  // of the grid
 };
 
-template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16, bool KEEP>
+template <int SPANS, bool LAYER, bool RESIDUAL, bool BIAS, bool F16, int CACHE>
 __global__ __launch_bounds__(kRowsPerBlock * 64) void rows_kernel(const RowsCall c) {
-  rows_body<SPANS, LAYER, RESIDUAL, BIAS, F16, KEEP>(c.x, c.residual, c.w, c.b, c.out, c.sum, c.rows, c.d, c.inv_d, c.eps,
+  rows_body<SPANS, LAYER, RESIDUAL, BIAS, F16, CACHE>(c.x, c.residual, c.w, c.b, c.out, c.sum, c.rows, c.d, c.inv_d, c.eps,
                                                (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6),
                                                (int64_t)c.blocks * kRowsPerBlock);
 }
@@ -203,7 +210,7 @@ hipError_t launch_rows(const NormArgs &a, hipStream_t stream) {
   int known = device >= 0 && device < 64 ? geometry[device].load(std::memory_order_acquire) : 0;
   if (known == 0) {
     int per_unit = 0, units = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, true>,
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, kKept>,
                                                      kRowsPerBlock * 64, 0);
     if (e != hipSuccess) return e;
     e = hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device);
@@ -228,13 +235,19 @@ hipError_t launch_rows(const NormArgs &a, hipStream_t stream) {
   }
   const RowsCall c = {(const uint16_t *)a.x, (const uint16_t *)a.residual, (const uint16_t *)a.w, (const uint16_t *)a.b,
                       (uint16_t *)a.out, (uint16_t *)a.sum, a.rows, a.d, (float)(1.0 / (double)a.d), (float)a.eps, (uint32_t)blocks};
-  // Kept, the rows are there for the projection that reads them (a Qwen3 layer's prefill of 700 tokens 31.8 -> 29.2 us, of
-  // 16384 426 -> 422); from a quarter of what the L2s hold on the launch's end waits for them to be written back
-  // ([6000, 1024] RMSNorm 5.1 -> 6.0), until the launch is long enough for that to go on beside it.
+  // Kept, the rows are there for the projection (a Qwen3 layer's prefill of 700 tokens 32.0 -> 28.8 us); from a quarter of
+  // what the L2s hold on the launch's end waits for them to be written back ([6000, 1024] RMSNorm 5.1 -> 6.0), until the
+  // launch is long enough for that to go on beside it.  Up to some 170 MB of all tensors the operands are found on the chip
+  // ([8000, 2048] add+RMSNorm, 131 MB: 20.4 us, marked 23.2); past that they push the outputs out ([16384, 2048], 268 MB:
+  // 49.8, marked 43.2, marked with the outputs 45.5).
   const int64_t bytes = a.rows * a.d * 2;
-  if (bytes < (6 << 20) || bytes >= (20 << 20))
-    return Launch<rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, true>>::run(blocks, kRowsPerBlock * 64, 0, 0, stream, c);
-  return Launch<rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, false>>::run(blocks, kRowsPerBlock * 64, 0, 0, stream, c);
+  auto run = [&](auto cache) {
+    return Launch<rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, decltype(cache)::value>>::run(blocks, kRowsPerBlock * 64, 0, 0,
+                                                                                               stream, c);
+  };
+  if (bytes * (RESIDUAL ? 4 : 2) > (170 << 20)) return run(std::integral_constant<int, kOutKept>());
+  if (bytes < (6 << 20) || bytes >= (20 << 20)) return run(std::integral_constant<int, kKept>());
+  return run(std::integral_constant<int, kLoadsKept>());
 }
 
 template <int SPANS, bool F16>
@@ -292,21 +305,21 @@ hipError_t launch_norm(const NormArgs &a, hipStream_t stream) {
       const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, uint16_t *__restrict__ out, int32_t rows,         \
       int32_t d, int32_t eps_bits) {                                                                                   \
     if (d <= 0 || d > DMAX) return;                                                                                    \
-    rows_body<DMAX / kSpan, false, false, false, F16, true>(x, nullptr, w, nullptr, out, nullptr, rows, d, 1.0f / (float)d,  \
+    rows_body<DMAX / kSpan, false, false, false, F16, kKept>(x, nullptr, w, nullptr, out, nullptr, rows, d, 1.0f / (float)d,  \
                                                       __builtin_bit_cast(float, eps_bits), SVODK_ROW_OF_WAVE);                            \
   }                                                                                                                    \
   extern "C" __global__ __launch_bounds__(kRowsPerBlock * 64) void svodk_add_rms_norm_d##DMAX##_##TYPE(                \
       const uint16_t *__restrict__ x, const uint16_t *__restrict__ residual, const uint16_t *__restrict__ w,           \
       uint16_t *__restrict__ out, uint16_t *__restrict__ sum, int32_t rows, int32_t d, int32_t eps_bits) {             \
     if (d <= 0 || d > DMAX) return;                                                                                    \
-    rows_body<DMAX / kSpan, false, true, false, F16, true>(x, residual, w, nullptr, out, sum, rows, d, 1.0f / (float)d,      \
+    rows_body<DMAX / kSpan, false, true, false, F16, kKept>(x, residual, w, nullptr, out, sum, rows, d, 1.0f / (float)d,      \
                                                      __builtin_bit_cast(float, eps_bits), SVODK_ROW_OF_WAVE);                             \
   }                                                                                                                    \
   extern "C" __global__ __launch_bounds__(kRowsPerBlock * 64) void svodk_layer_norm_d##DMAX##_##TYPE(                  \
       const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const uint16_t *__restrict__ b,                  \
       uint16_t *__restrict__ out, int32_t rows, int32_t d, int32_t eps_bits) {                                         \
     if (d <= 0 || d > DMAX) return;                                                                                    \
-    rows_body<DMAX / kSpan, true, false, true, F16, true>(x, nullptr, w, b, out, nullptr, rows, d, 1.0f / (float)d,          \
+    rows_body<DMAX / kSpan, true, false, true, F16, kKept>(x, nullptr, w, b, out, nullptr, rows, d, 1.0f / (float)d,          \
                                                     __builtin_bit_cast(float, eps_bits), SVODK_ROW_OF_WAVE);                              \
   }                                                                                                                    \
   extern "C" __global__ __launch_bounds__(kRowsPerBlock * 64) void svodk_add_layer_norm_d##DMAX##_##TYPE(              \
@@ -314,7 +327,7 @@ hipError_t launch_norm(const NormArgs &a, hipStream_t stream) {
       const uint16_t *__restrict__ b, uint16_t *__restrict__ out, uint16_t *__restrict__ sum, int32_t rows, int32_t d, \
       int32_t eps_bits) {                                                                                              \
     if (d <= 0 || d > DMAX) return;                                                                                    \
-    rows_body<DMAX / kSpan, true, true, true, F16, true>(x, residual, w, b, out, sum, rows, d, 1.0f / (float)d,              \
+    rows_body<DMAX / kSpan, true, true, true, F16, kKept>(x, residual, w, b, out, sum, rows, d, 1.0f / (float)d,              \
                                                    __builtin_bit_cast(float, eps_bits), SVODK_ROW_OF_WAVE);                               \
   }
 
