@@ -1946,7 +1946,7 @@ bool attention_groups(const AttnArgs &a) {
 void attention_stream_slots(int32_t slots) { g_stream_slots.store(slots, std::memory_order_relaxed); }
 
 const char *attention_config(const AttnArgs &a) {
-  if (attention_decodes(a))
+  if (a.decodes)
     return a.splits > 1 ? "FaCfg { rows: 4, lanes_per_key: d / 8, splits: n, core: v_dot2_f32, keys streamed through registers }"
                         : "FaCfg { rows: 4, lanes_per_key: d / 8, splits: 1, core: v_dot2_f32, keys streamed through registers }";
   static const char *const kCfg[2][2] = {
@@ -1962,7 +1962,7 @@ const char *attention_config(const AttnArgs &a) {
 }
 
 hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
-  if (attention_decodes(a)) return launch_decode(a, stream);  // a decoder step: no key tiles, a stream of K and V
+  if (a.decodes) return launch_decode(a, stream);  // a decoder step: no key tiles, a stream of K and V
   switch (a.d) {
     case 32: return launch_attention_d32(a, stream);
     case 48: return launch_attention_d48(a, stream);

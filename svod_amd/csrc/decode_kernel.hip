@@ -576,11 +576,11 @@ void attention_decode_rows(int32_t rows) {
 
 int32_t attention_decode_limit() { return g_decode_rows.load(std::memory_order_relaxed); }
 
-bool attention_decodes(const AttnArgs &a) {
+bool attention_decodes(const AttnArgs &a, int32_t limit) {
   const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
   if (a.causal || ranged || a.bias != nullptr || a.kv_heads <= 0 || a.heads % a.kv_heads != 0) return false;
   const int64_t rows = (int64_t)(a.heads / a.kv_heads) * a.t;
-  return rows >= 1 && rows <= g_decode_rows.load(std::memory_order_relaxed);
+  return rows >= 1 && rows <= limit;
 }
 
 int32_t decode_arrivals(const AttnArgs &a, hipStream_t stream) {

@@ -101,6 +101,7 @@ struct AttnArgs {
   // m_part and l_part [splits, batch, t, heads], all f32; launch_combine merges them.
   int32_t splits;
   float *o_part, *m_part, *l_part;
+  int32_t decodes;   // launch_decode's call (attention_decodes): decided once, launch_attention and attention_config follow it
   int32_t arrivals;  // a decoder step merges its splits itself, with this set of counters (decode_arrivals); -1: it does not
   // Elements from a token's row to the next in q and in k/v; 0 = dense (heads * d, kv_heads * d).
   // A fused projection read in place (tk/src/ops/attention.rs:104-122) has its own row for both.
@@ -156,11 +157,13 @@ bool attention_supports(int32_t d);
 bool attention_groups(const AttnArgs &a);
 // The decoder step's kernel (decode_kernel.hip): a call without causal or per-row masks or a bias whose (batch,
 // KV head) has at most kDecodeRows query rows (group * t) streams K and V past them in registers instead of
-// running key tiles through LDS.  launch_attention takes that path by itself; splits, caches, appended rows, key
-// lengths and key masks mean what they mean to the tile kernel.
+// running key tiles through LDS.  Splits, caches, appended rows, key lengths and key masks mean what they mean to the
+// tile kernel.
 constexpr int kDecodeRows = 4;         // the most the kernel is built for
 constexpr int kDecodeRowsDefault = 2;  // the most it takes unasked: up to there it has beaten the tile kernel where measured
-bool attention_decodes(const AttnArgs &a);
+// `limit`: the most rows that path takes, read once a call (attention_decode_limit): the split count, the workspace's use,
+// the launch and who merges all follow from it, and another thread may turn it at any time.
+bool attention_decodes(const AttnArgs &a, int32_t limit);
 // The most rows that path takes, 0..kDecodeRows (0: every call runs key tiles): see svodk_tune_decode.
 void attention_decode_rows(int32_t rows);
 int32_t attention_decode_limit();

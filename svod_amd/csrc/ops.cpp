@@ -313,7 +313,8 @@ int svodk_plan_heads(int32_t has_target, const int32_t *dtypes, int32_t n_dtypes
 // 151.5 -> 29.8 (16), 64 x 32 28.7 -> 16.8 (4), 64 x 64 82.7 -> 37.6 (8), 256 x 64 86.2 -> 67.4
 // (2), 320 x 24 32.7 -> 28.6 (2); from 640 workgroups on the rule answers one, which is fastest.
 // A window, a chunk mask or segment starts leave a tile few of the keys: the rule keeps those whole.
-static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t heads, int64_t kv_heads, int64_t tk) {
+static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t heads, int64_t kv_heads, int64_t tk,
+                       int32_t decode_limit) {
   const int32_t asked = opts->splits;
   const int64_t most = tk > 0 ? (tk + 63) / 64 : 1;
   if (asked == 1) return 1;
@@ -324,7 +325,7 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
   // head, split), splits of at least four key blocks, as many as bring the launch to about a thousand workgroups
   // (one row) or five hundred (more): enough of them resident for the bytes in flight, few enough that their
   // streams do not thrash the memory's open pages.
-  if (!opts->causal && opts->bias == nullptr && group * t >= 1 && group * t <= svodk::attention_decode_limit()) {
+  if (!opts->causal && opts->bias == nullptr && group * t >= 1 && group * t <= decode_limit) {
     const int64_t units = kv_heads * batch;
     if (units <= 0) return 1;
     const int64_t target = group * t == 1 ? 1024 : 512;
@@ -641,7 +642,9 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     }
   }
   // L280-302: key splits.  The partial tensors live in the caller's workspace.
-  a.splits = split_count(opts, a.batch, t, heads, kv_heads, tk);
+  const int32_t decode_limit = svodk::attention_decode_limit();
+  a.decodes = svodk::attention_decodes(a, decode_limit);
+  a.splits = split_count(opts, a.batch, t, heads, kv_heads, tk, decode_limit);
   void *workspace = opts->workspace;
   if (a.splits > 1 && own_scratch) {
     // The library's own array holds the partial states.  A split count the rule chose is lowered to
@@ -680,7 +683,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
   // A split decoder step merges its splits itself where it can.
-  a.arrivals = a.splits > 1 && svodk::attention_decodes(a) ? svodk::decode_arrivals(a, (hipStream_t)hip_stream) : -1;
+  a.arrivals = a.splits > 1 && a.decodes ? svodk::decode_arrivals(a, (hipStream_t)hip_stream) : -1;
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
@@ -780,7 +783,8 @@ int64_t svodk_attention_workspace(const svodk_tensor *q, const svodk_tensor *k, 
   if (!well_formed(q) || !well_formed(k) || opts == nullptr || q->rank != 4 || k->rank != 4) return 0;
   const int64_t batch = opts->batch_live > 0 ? opts->batch_live : q->shape[0];
   const int64_t kv_heads = opts->cache != nullptr ? opts->cache->kv_heads : k->shape[2];
-  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, k->shape[1]);
+  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, k->shape[1],
+                                 svodk::attention_decode_limit());
   if (splits <= 1) return 0;
   return (int64_t)splits * batch * q->shape[1] * q->shape[2] * (q->shape[3] + 2) * 4;
 }

@@ -77,6 +77,32 @@ def test_a_captured_layer_replays_to_the_eager_result(device):
             assert np.array_equal(bits(got), bits(ref)), (seed, name)
 
 
+def test_split_steps_are_written_while_the_decode_knob_turns(device):
+    """A call decides once which kernel runs and who merges its splits: with the process-wide knob turned by another
+    thread between any two of its steps, every output is written, by either path."""
+    b, tk, h, d = 2, 1024, 4, 64
+    g = Lcg(77)
+    q, k, v = (bf16_tensor(g.bf16(s), device) for s in ((b, 1, h, d), (b, tk, h, d), (b, tk, h, d)))
+    want = torch.nn.functional.scaled_dot_product_attention(*(x.cpu().float().transpose(1, 2) for x in (q, k, v))).transpose(1, 2)
+    stop = threading.Event()
+
+    def turn():
+        while not stop.is_set():
+            svod_amd.tune_decode(0)
+            svod_amd.tune_decode(svod_amd.DECODE_ROWS_DEFAULT)
+
+    turner = threading.Thread(target=turn)
+    turner.start()
+    try:
+        got = [svod_amd.attention(q, k, v, Attn(splits=splits)) for _ in range(4000) for splits in (None, 4)]
+    finally:
+        stop.set()
+        turner.join(timeout=60)
+        svod_amd.tune_decode(svod_amd.DECODE_ROWS_DEFAULT)
+    worst = (torch.stack(got).float().cpu() - want).abs().amax(dim=(1, 2, 3, 4))
+    assert bool((worst < 2e-2).all()), (int((~(worst < 2e-2)).sum()), worst.max())  # a NaN, unwritten, compares false
+
+
 def test_threads_launch_side_by_side(device):
     """Four host threads, a stream each, different shapes and options: the same bits as one thread, and
     each thread's `chosen()` is its own (tk/src/ops/mod.rs:83-118: thread-local)."""
