@@ -112,6 +112,10 @@ typedef struct svodk_cache {
  * lets the library choose, as the reference's tuner would: it splits calls with
  * few query tiles and many keys (a decoder step) when the workspace
  * svodk_attention_workspace asks for is lent, and keeps the keys whole without it.
+ * A decoder step (svodk_tune_decode) of up to 64 splits merges them itself, in the one launch, where
+ * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  What the workspace
+ * holds at first does not matter, nor does the stream, nor whether the call is captured; as with the
+ * partial states, no two launches in flight may have the same workspace.
  */
 typedef struct svodk_attn {
   int32_t causal;

@@ -17,8 +17,10 @@
 //   splits do (L948-1014), and the workgroup writes the output rows, or with key splits its partial state for
 //   combine_kernel (L899-921).
 #include <hip/hip_runtime.h>
+#include <sys/random.h>
 
 #include <atomic>
+#include <chrono>
 #include <type_traits>
 
 #include "kernels.h"
@@ -37,7 +39,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNoKey = -1e30f;   // the running maximum before any key: finite, so that its differences are numbers
 constexpr int kMaxWaves = 8;       // waves a workgroup
 constexpr int kAhead = 2;          // passes a lane works on at a time, with as many more in flight
-constexpr int kArrivalSets = 64, kArrivalUnits = 1024;  // counter sets (a stream each) and (batch, KV head) pairs a set
+constexpr int kWordStride = kArrivalBytes / 8;  // of 64-bit words
+constexpr int kCountBits = 7;      // of a word of arrivals: its low bits count, the others are the launch's tag
+static_assert(kMostMergedSplits < 1 << kCountBits, "the count stands at the splits when a launch ends");
 
 // Waves a workgroup: few workgroups take eight each, so that the launch still has its bytes in flight.
 __host__ __device__ constexpr int decode_waves(int64_t workgroups) { return workgroups >= 256 ? 4 : kMaxWaves; }
@@ -56,7 +60,7 @@ struct DecodeArgs {
   int32_t batch, t, tk, heads, kv_heads, group;
   int32_t splits, cached, kv_head_start, cache_rows, app_rows;
   float scale;
-  uint32_t *arrivals;  // of a launch that merges its splits itself: a counter a (batch, KV head), at zero
+  uint64_t *arrivals, tag;  // of a launch that merges its splits itself: a word a (batch, KV head), of any content
 };
 
 template <bool F16>
@@ -315,6 +319,17 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
     }
   };
 
+  // A word of arrivals is the workspace's and holds anything at first.  Every workgroup makes sure, before it counts
+  // itself in, that the word carries this launch's tag: it becomes (tag, 0) by one compare-and-swap out of whatever was
+  // there, and no other write of the launch leaves that tag again, so a late swap out of the old content fails.  Nothing
+  // else ever carries the tag (57 bits, another one a launch) but the word as an earlier replay of the same captured
+  // launch left it, and that one counts `splits`, which no word of a launch under way does while a workgroup of its
+  // (batch, KV head) has yet to come.  The content is asked for ahead of the keys and the swap goes out behind them, so
+  // that neither is waited for: with the swap ahead of the keys a launch takes 1.4 us more.
+  uint64_t *arrivals = p.arrivals + (int64_t)unit * kWordStride;
+  const bool counts = MODE == kMerged && tid == 0;
+  uint64_t found = 0;
+  if (counts) found = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   {
     const int64_t at = (kv_row * tk) * p.kv_row_elems + (int64_t)kv_col * D + 8 * pos;
     const void *mask = nullptr;
@@ -324,6 +339,9 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
     // their pieces of a key row lie side by side.
     stream(p.k + at, p.v + at, p.kv_row_elems, k0, k1, mask, p.mask_bytes, (uint32_t)kv_row * 7u + (uint32_t)split * 3u);
   }
+  if (counts && (found >> kCountBits != p.tag || (int)(found & ((1u << kCountBits) - 1)) >= p.splits))
+    __hip_atomic_compare_exchange_strong(arrivals, &found, p.tag << kCountBits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
   // The appended rows (L739-755, L827-846): scored by the last split after the cached keys, the first
   // app_lens[b] of them visible, from tensors of their own.
   if (p.cached && p.k_app != nullptr && (!SPLIT || split == p.splits - 1)) {
@@ -401,19 +419,20 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
     }
   }
   if (MODE != kMerged) return;
-  // ---- the merge.  This wave's states are where every workgroup sees them before it counts itself in; the workgroup
-  // that counts itself in last reads them all.  No one waits for anyone.  The arithmetic is combine_kernel's, operation
-  // for operation: a captured launch, which leaves the merge to that kernel, gives the same bits.  It is a chain of four
+  // ---- the merge.  This wave's states are where every workgroup sees them before it counts itself in: they were stored
+  // past the L2s, and vmcnt is at zero when the memory behind those has taken them all.  The workgroup that counts itself
+  // in last reads them, from there as well.  No one waits for anyone.  The arithmetic is combine_kernel's, operation
+  // for operation: a launch that leaves the merge to that kernel gives the same bits.  It is a chain of four
   // trips to memory, some 3 us, where a kernel of its own is a launch (2.6 us of host time) and 3.5 us: one sequence over
   // 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   const int splits = p.splits;
-  uint32_t *arrivals = p.arrivals + b * p.kv_heads + kvh;
   uint32_t before = 0;
-  if (lane == 0) before = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if ((int)__builtin_amdgcn_readfirstlane((int)before) != splits - 1) return;
+  if (lane == 0)
+    before = (uint32_t)__hip_atomic_fetch_add(arrivals, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before) & ((1u << kCountBits) - 1);
+  if ((int)before != splits - 1) return;
   asm volatile("" ::: "memory");  // the states are read from here on
-  if (lane == 0) __hip_atomic_store(arrivals, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the stream's next launch
   constexpr int kLanes = D / 4, kBatch = 8;
   for (int c = lane; c < rows * kLanes; c += 64) {
     const int r = c / kLanes, chunk = c - r * kLanes;
@@ -470,11 +489,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
 }
 
 #if !defined(SVODK_CODE_OBJECT)  // the library's kernel and its launch: not part of a code object build
-// The counters of the launches that merge their splits themselves, zero between them.  A set a stream: the launches of a
-// stream run one after another, and the last workgroup of each puts its counters back.
-__device__ uint32_t g_arrivals[kArrivalSets][kArrivalUnits];
-
-// DecodeArgs as they travel: in 112 bytes (launch.h).  k and v are at the launch's first head, the states in one piece.
+// DecodeArgs as they travel: in 112 bytes (launch.h).  k and v are at the launch's first head, the states and the words of
+// arrivals behind them are one piece, a row of keys is counted in heads.
 struct Packed {
   const uint16_t *q, *k, *v;
   uint16_t *o;
@@ -483,13 +499,11 @@ struct Packed {
   const uint16_t *k_app, *v_app;
   const void *app_lens;
   float *states;
-  int32_t tk, batch, kv_row_elems;
+  uint64_t tag : 64 - kCountBits, app_rows : 7;
+  uint64_t splits : 26, kv_row_heads : 19, kv_heads : 16, mask : 1, wide_keys : 1, packed_rows : 1;
+  uint32_t batch : 26, group_less_one : 2, t_less_one : 2, row_map_i64 : 1, app_lens_i64 : 1;
+  int32_t tk, cache_rows;
   float scale;
-  int32_t cache_rows;
-  int32_t splits;
-  uint32_t set;           // of the counters
-  uint32_t kv_heads : 16, group_less_one : 2, t_less_one : 2, app_rows : 7, mask : 1, wide_keys : 1, row_map_i64 : 1,
-      app_lens_i64 : 1, packed_rows : 1;
 };
 static_assert(sizeof(Packed) <= 112 && kDecodeRows <= 4, "the record's size, the group's and the tokens' two bits");
 
@@ -504,12 +518,12 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) 
   p.k_app = a.k_app, p.v_app = a.v_app, p.app_lens = a.app_lens, p.app_lens_i64 = a.app_lens_i64, p.app_rows = a.app_rows;
   p.batch = a.batch, p.tk = a.tk, p.t = a.t_less_one + 1, p.group = a.group_less_one + 1;
   p.kv_heads = a.kv_heads, p.heads = p.kv_heads * p.group;
-  p.splits = MODE == kWhole ? 1 : a.splits;
-  p.kv_row_elems = a.kv_row_elems, p.q_row_elems = a.packed_rows ? (int64_t)a.kv_row_elems : (int64_t)p.heads * D;
+  p.splits = MODE == kWhole ? 1 : (int32_t)a.splits;
+  p.kv_row_elems = (int64_t)a.kv_row_heads * D, p.q_row_elems = a.packed_rows ? p.kv_row_elems : (int64_t)p.heads * D;
   p.cached = 1, p.kv_head_start = 0, p.scale = a.scale;
   const int64_t states = (int64_t)p.splits * p.batch * p.t * p.heads;
   p.o_part = a.states, p.m_part = a.states + states * D, p.l_part = p.m_part + states;
-  p.arrivals = g_arrivals[a.set];
+  p.arrivals = reinterpret_cast<uint64_t *>(p.l_part + states), p.tag = a.tag;
   decode_body<D, R, F16, MODE, KEEP>(p, decode_waves((int64_t)p.batch * p.kv_heads * p.splits));
 #endif
 }
@@ -542,28 +556,15 @@ hipError_t launch_d(const Packed &p, int rows, bool merged, bool f16, hipStream_
   return f16 ? launch_r<D, 4, true>(p, merged, stream) : launch_r<D, 4, false>(p, merged, stream);
 }
 
-// The counters' set of a stream, or -1: the stream is being captured (a replay may run beside anything), is not one
-// stream (each thread's default stream has the same handle), or the sets have run out.
-int arrival_set(hipStream_t stream) {
-  constexpr int kDevices = 16;
-  static std::atomic<uintptr_t> owner[kDevices][kArrivalSets];  // the stream's handle + 1; 0: free
-  if (stream == hipStreamPerThread || stream == (hipStream_t)1) return -1;
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kDevices) return -1;
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
-    (void)hipGetLastError();
-    return -1;
-  }
-  if (capturing != hipStreamCaptureStatusNone) return -1;
-  const uintptr_t me = (uintptr_t)stream + 1;
-  for (int i = 0; i < kArrivalSets; i++) {
-    uintptr_t there = owner[device][i].load(std::memory_order_acquire);
-    if (there == me) return i;
-    if (there == 0 && owner[device][i].compare_exchange_strong(there, me, std::memory_order_acq_rel)) return i;
-    if (there == me) return i;
-  }
-  return -1;
+// A launch's tag: no two of a process have the same, and where they start differs from process to process.
+uint64_t next_tag() {
+  static std::atomic<uint64_t> next{[] {
+    uint64_t seed = 0;
+    if (getrandom(&seed, sizeof seed, GRND_NONBLOCK) != (ssize_t)sizeof seed)
+      seed = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9e3779b97f4a7c15u;
+    return seed;
+  }()};
+  return next.fetch_add(1, std::memory_order_relaxed) & ((uint64_t)-1 >> kCountBits);
 }
 
 std::atomic<int> g_decode_rows{kDecodeRowsDefault};
@@ -583,17 +584,17 @@ bool attention_decodes(const AttnArgs &a, int32_t limit) {
   return rows >= 1 && rows <= limit;
 }
 
-int32_t decode_arrivals(const AttnArgs &a, hipStream_t stream) {
-  return (int64_t)a.batch * a.kv_heads <= kArrivalUnits ? arrival_set(stream) : -1;
-}
-
 hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
   const int splits = a.splits > 1 ? a.splits : 1;
   if (splits > 1 && (a.o_part == nullptr || a.m_part == nullptr || a.l_part == nullptr)) return hipErrorInvalidValue;
   const int64_t q_row = a.q_row_elems > 0 ? a.q_row_elems : (int64_t)a.heads * a.d;
   const int64_t kv_row = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
   const bool packed_rows = q_row != (int64_t)a.heads * a.d;
-  if (kv_row > 0x7fffffffLL || (packed_rows && q_row != kv_row) || a.kv_heads > 0xffff || a.app_rows > 127) return hipErrorInvalidValue;
+  // The fields' widths; the op layer's own limits (64 rows of keys in 2^31 bytes, 64 tiles a row and head in 31 bits, 64
+  // appended rows) are within them.
+  if (kv_row % a.d != 0 || kv_row / a.d >= 1 << 19 || (packed_rows && q_row != kv_row) || a.kv_heads > 0xffff ||
+      a.app_rows > 127 || a.batch >= 1 << 26 || splits >= 1 << 26)
+    return hipErrorInvalidValue;
   Packed p{};
   p.q = (const uint16_t *)a.q;
   p.k = (const uint16_t *)a.k + (a.cached ? (int64_t)a.kv_head_start * a.d : 0);
@@ -608,23 +609,24 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.cache_rows = a.cache_rows;
     p.k_app = (const uint16_t *)a.k_app;
     p.v_app = (const uint16_t *)a.v_app;
-    p.app_rows = (uint32_t)a.app_rows;
+    p.app_rows = (uint64_t)a.app_rows;
     p.app_lens = a.app_lens;
     p.app_lens_i64 = a.app_lens_i64 != 0;
   }
   p.states = a.o_part;
   p.tk = a.tk;
-  p.batch = a.batch;
-  p.kv_row_elems = (int32_t)kv_row;
+  p.batch = (uint32_t)a.batch;
+  p.kv_row_heads = (uint64_t)(kv_row / a.d);
   p.scale = a.scale;
-  p.splits = splits;
-  p.kv_heads = (uint32_t)a.kv_heads;
+  p.splits = (uint64_t)splits;
+  p.kv_heads = (uint64_t)a.kv_heads;
   p.group_less_one = (uint32_t)(a.heads / a.kv_heads - 1);
   p.t_less_one = (uint32_t)(a.t - 1);
   p.packed_rows = packed_rows;
-  p.set = splits > 1 && a.arrivals >= 0 ? (uint32_t)a.arrivals : 0u;
   const int rows = a.heads / a.kv_heads * a.t;
-  const bool merged = splits > 1 && a.arrivals >= 0;
+  const bool merged = splits > 1 && a.merges;
+  if (merged && splits > kMostMergedSplits) return hipErrorInvalidValue;
+  if (merged) p.tag = next_tag();
   switch (a.d) {
     case 32: return launch_d<32>(p, rows, merged, a.f16 != 0, stream);
     case 48: return launch_d<48>(p, rows, merged, a.f16 != 0, stream);
@@ -670,7 +672,7 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.batch = batch, p.t = t, p.tk = tk, p.heads = heads, p.kv_heads = kv_heads, p.group = heads / kv_heads;          \
     p.splits = (S) && splits > 1 ? splits : 1, p.cached = cached, p.kv_head_start = kv_head_start;                    \
     p.cache_rows = cache_rows, p.app_rows = app_rows, p.scale = __builtin_bit_cast(float, scale_bits);                \
-    p.arrivals = nullptr;                                                                                             \
+    p.arrivals = nullptr, p.tag = 0;                                                                                  \
     svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole, false>(p, 4);                           \
   }
 #define SVODK_DECODE_ROWS_OF(D, T, F16, S) \

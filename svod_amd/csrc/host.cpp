@@ -291,8 +291,10 @@ struct Workspace {
   void lend(svodk_attn &a, const svodk_tensor &q, const svodk_tensor &k, PyObject *like, PyObject *lent, PyObject *fresh) {
     if (a.splits == 1) return;
     if (lent == Py_None) {
-      const int64_t need = abi.attention_workspace(&q, &k, &a);
+      int64_t need = abi.attention_workspace(&q, &k, &a);
       if (need <= 0) return;
+      // The words with which a decoder step merges its own splits (svodk.h).
+      need += 128 * (a.batch_live > 0 ? a.batch_live : q.shape[0]) * (a.cache != nullptr ? a.cache->kv_heads : k.shape[2]);
       own = allocate(fresh, {need}, at::kByte, like);
       if (own == nullptr) throw Raised();
       lent = own;

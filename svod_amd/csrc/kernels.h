@@ -102,7 +102,8 @@ struct AttnArgs {
   int32_t splits;
   float *o_part, *m_part, *l_part;
   int32_t decodes;   // launch_decode's call (attention_decodes): decided once, launch_attention and attention_config follow it
-  int32_t arrivals;  // a decoder step merges its splits itself, with this set of counters (decode_arrivals); -1: it does not
+  // A decoder step merges its splits itself: behind l_part the workspace has decode_arrival_bytes(a) more, of any content.
+  int32_t merges;
   // Elements from a token's row to the next in q and in k/v; 0 = dense (heads * d, kv_heads * d).
   // A fused projection read in place (tk/src/ops/attention.rs:104-122) has its own row for both.
   int64_t q_row_elems, kv_row_elems;
@@ -168,9 +169,11 @@ bool attention_decodes(const AttnArgs &a, int32_t limit);
 void attention_decode_rows(int32_t rows);
 int32_t attention_decode_limit();
 hipError_t launch_decode(const AttnArgs &a, hipStream_t stream);
-// The counters with which a split decoder step on `stream` merges its own splits, for AttnArgs::arrivals; -1: it leaves
-// them to launch_combine (a stream under capture, more (batch, KV head) pairs than a set has counters).
-int32_t decode_arrivals(const AttnArgs &a, hipStream_t stream);
+// What a decoder step that merges its own splits, kMostMergedSplits at most, needs behind the partial states: a word a
+// (batch, KV head), on a line of its own (16 sequences of 8 KV heads in 4 splits: 28.9 us, 29.5 with 16 words a line).
+constexpr int kMostMergedSplits = 64;
+constexpr int kArrivalBytes = 128;
+inline int64_t decode_arrival_bytes(const AttnArgs &a) { return (int64_t)a.batch * a.kv_heads * kArrivalBytes; }
 // One head size's kernels each (launch_attention picks by AttnArgs::d).
 hipError_t launch_attention_d32(const AttnArgs &a, hipStream_t stream);
 hipError_t launch_attention_d48(const AttnArgs &a, hipStream_t stream);

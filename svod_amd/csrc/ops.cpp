@@ -646,6 +646,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
   a.decodes = svodk::attention_decodes(a, decode_limit);
   a.splits = split_count(opts, a.batch, t, heads, kv_heads, tk, decode_limit);
   void *workspace = opts->workspace;
+  int64_t workspace_bytes = opts->workspace_bytes;
   if (a.splits > 1 && own_scratch) {
     // The library's own array holds the partial states.  A split count the rule chose is lowered to
     // what the array holds (down to one, as svodk_attention does without a workspace); a count the
@@ -653,6 +654,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     const int64_t per_split = (int64_t)a.batch * t * heads * (d + 2) * 4;
     int64_t have = 0;
     const hipError_t e = svodk::split_scratch(&workspace, &have);
+    workspace_bytes = have;
     if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: the static scratch: %s", op, hipGetErrorString(e));
     if (opts->splits <= 0 && (int64_t)a.splits * per_split > have)
       a.splits = (int32_t)std::max<int64_t>(1, per_split > 0 ? have / per_split : 1);
@@ -671,7 +673,10 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
   }
   if (a.splits > 1) {
     const int64_t rows = (int64_t)a.batch * t * heads;
-    const int64_t need = (int64_t)a.splits * rows * (d + 2) * 4;
+    int64_t need = (int64_t)a.splits * rows * (d + 2) * 4;
+    // A split decoder step merges its splits itself where the workspace has room for its words.
+    a.merges = a.decodes && a.splits <= svodk::kMostMergedSplits && workspace_bytes - need >= svodk::decode_arrival_bytes(a);
+    if (a.merges) need += svodk::decode_arrival_bytes(a);
     Span ws[2] = {{"workspace", workspace, (size_t)need, true}, {"o", out->data, (size_t)numel(out) * 2, true}};
     if (int rc = check_aliasing(op, ws, 2)) return rc;
     for (int i = 0; i < 3; i++) {
@@ -682,13 +687,11 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.m_part = a.o_part + (int64_t)a.splits * rows * d;
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
-  // A split decoder step merges its splits itself where it can.
-  a.arrivals = a.splits > 1 && a.decodes ? svodk::decode_arrivals(a, (hipStream_t)hip_stream) : -1;
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
   if (a.splits > 1) ran(op, "combine_splits", "NormCfg { br: 4 }");
-  if (a.splits > 1 && a.arrivals < 0) {
+  if (a.splits > 1 && !a.merges) {
     svodk::CombineArgs c{};
     c.o_part = a.o_part;
     c.m_part = a.m_part;

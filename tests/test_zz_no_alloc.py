@@ -118,3 +118,18 @@ def test_a_captured_split_call_replays(device):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(bits(out), bits(eager))
+
+
+@pytest.mark.parametrize("b", [1158, 1271])
+def test_a_step_whose_states_fill_the_scratch_leaves_its_merge_to_the_launch(device, b):
+    # Five splits of 1271 x 5 rows are 8 bytes short of the array: no room for the words with which a step merges its own.
+    h, d, splits = 5, 64, 5
+    room = svod_amd.noalloc_scratch_bytes() - splits * b * h * (d + 2) * 4
+    assert 0 <= room and (room >= 128 * b * h) == (b == 1158)
+    g = Lcg(41)
+    q = bf16_tensor(g.bf16((b, 1, h, d)), device)
+    k, v = (bf16_tensor(g.bf16((2, 300, h, d)), device) for _ in range(2))
+    lens = torch.tensor([300 - i % 70 for i in range(b)], dtype=torch.int32, device=device)
+    rows = torch.arange(b, dtype=torch.int32, device=device) % 2
+    got, want = both(device, (q, k, v), Attn(keys=KeyMask.lens(lens), cache=Cache(0, h, rows), splits=splits))
+    assert np.array_equal(bits(got), bits(want))
