@@ -209,9 +209,29 @@ PyObject *held(PyObject *o) {
   return o;
 }
 
+// A tensor's device, the current one while this lives: torch's default stream has the same handle on every device.
+class OnDeviceOf {
+ public:
+  explicit OnDeviceOf(const at::Tensor &t) {
+    if (!t.is_cuda()) return;
+    const c10::DeviceIndex now = c10::hip::current_device();
+    if (t.device().index() == now) return;
+    c10::hip::set_device(t.device().index());
+    back_ = now;
+  }
+  OnDeviceOf(const OnDeviceOf &) = delete;
+  ~OnDeviceOf() {
+    if (back_ >= 0) (void)c10::hip::SetDevice(back_);
+  }
+
+ private:
+  c10::DeviceIndex back_ = -1;
+};
+
 // The launch itself runs without the interpreter lock, as a ctypes call does: it waits when the device's queue is full.
 template <typename F>
-int unlocked(F f) {
+int unlocked(const at::Tensor &on, F f) {
+  const OnDeviceOf device(on);
   int status;
   Py_BEGIN_ALLOW_THREADS status = f();
   Py_END_ALLOW_THREADS return status;
@@ -334,7 +354,7 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   Workspace ws;
   ws.lend(call.a, qd, kd, q, args[5], fresh);
   void *stream = stream_of(tensor(q));
-  const int status = unlocked([&] { return abi.attention(&qd, &kd, &vd, &call.a, &od, stream); });
+  const int status = unlocked(tensor(q), [&] { return abi.attention(&qd, &kd, &vd, &call.a, &od, stream); });
   return answer("attention", status, out);
   SVODK_END
 }
@@ -347,7 +367,7 @@ PyObject *py_attention_noalloc(PyObject *, PyObject *const *args, Py_ssize_t nar
   svodk_tensor qd, kd, vd, od;
   describe(args[0], qd), describe(args[1], kd), describe(args[2], vd), describe(args[4], od);
   void *stream = stream_of(tensor(args[0]));
-  const int status = unlocked([&] { return abi.attention_noalloc(&qd, &kd, &vd, &call.a, &od, stream); });
+  const int status = unlocked(tensor(args[0]), [&] { return abi.attention_noalloc(&qd, &kd, &vd, &call.a, &od, stream); });
   Ref out(held(args[4]));
   return answer("attention", status, out);
   SVODK_END
@@ -379,7 +399,7 @@ PyObject *py_attention_packed(PyObject *, PyObject *const *args, Py_ssize_t narg
   }
   void *stream = stream_of(qkv);
   const int status =
-      unlocked([&] { return abi.attention_packed(&xd, (int32_t)heads, (int32_t)kv_heads, &call.a, &od, stream); });
+      unlocked(qkv, [&] { return abi.attention_packed(&xd, (int32_t)heads, (int32_t)kv_heads, &call.a, &od, stream); });
   return answer("attention", status, out);
   SVODK_END
 }
@@ -425,7 +445,7 @@ PyObject *py_heads(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     describe(args[0], xd), describe(q, qd), describe(k, kd), describe(v, vd);
   }
   void *stream = stream_of(qkv);
-  const int status = unlocked([&] { return abi.heads(&xd, &o, &qd, &kd, &vd, stream); });
+  const int status = unlocked(qkv, [&] { return abi.heads(&xd, &o, &qd, &kd, &vd, stream); });
   return answer("heads", status, out);
   SVODK_END
 }
@@ -474,7 +494,7 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   }
   describe(args[0], xd), describe(args[1], wd), describe(out, od);
   void *stream = stream_of(x);
-  const int status = unlocked([&] { return abi.linear(&xd, &wd, &o, &od, stream); });
+  const int status = unlocked(x, [&] { return abi.linear(&xd, &wd, &o, &od, stream); });
   return answer("linear", status, out);
   SVODK_END
 }
@@ -511,7 +531,7 @@ PyObject *py_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     describe(out, yd);
   }
   void *stream = stream_of(tensor(x));
-  const int status = unlocked([&] {
+  const int status = unlocked(tensor(x), [&] {
     if (LAYER)
       return fused ? abi.add_layer_norm(&xd, &rd, &wd, b, eps, live, &sd, &yd, stream)
                    : abi.layer_norm(&xd, &wd, b, eps, live, &yd, stream);
@@ -530,7 +550,7 @@ PyObject *py_order_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   svodk_tensor kd, od;
   describe(args[0], kd), describe(out, od);
   void *stream = stream_of(keys);
-  const int status = unlocked([&] { return abi.order_rows(&kd, &od, stream); });
+  const int status = unlocked(keys, [&] { return abi.order_rows(&kd, &od, stream); });
   return answer("order_rows", status, out);
   SVODK_END
 }

@@ -23,6 +23,7 @@ struct Launch;
 template <typename... P, void (*Kernel)(P...)>
 struct Launch<Kernel> {
   // `lds`: dynamic LDS of this launch, `most_lds`: the most any launch of the kernel asks for.
+  // The current device is the stream's (the op layer sees to it): the function looked up is that device's.
   static hipError_t run(int64_t grid, uint32_t block, uint32_t lds, uint32_t most_lds, hipStream_t stream, P... args) {
     constexpr int kDevices = 16;  // devices past these look the function up every time
     static std::atomic<hipFunction_t> known[kDevices];

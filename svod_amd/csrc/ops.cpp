@@ -160,6 +160,29 @@ int check_aliasing(const char *op, const Span *spans, int n) {
   return 0;
 }
 
+// The device of the caller's stream is the current one for the length of a call: what is asked of a device (has it kernels,
+// its compute units, its scratch, a kernel's function) is then asked of the one that runs the launch.  The default streams
+// are the current device's own.
+class OnDeviceOf {
+ public:
+  explicit OnDeviceOf(void *hip_stream) {
+    const hipStream_t stream = (hipStream_t)hip_stream;
+    if (stream == nullptr || stream == hipStreamLegacy || stream == hipStreamPerThread) return;
+    int of = -1, now = -1;
+    if (hipStreamGetDevice(stream, &of) != hipSuccess || hipGetDevice(&now) != hipSuccess)
+      (void)hipGetLastError();  // no stream: the launch says so
+    else if (of != now && hipSetDevice(of) == hipSuccess)
+      back_ = now;
+  }
+  OnDeviceOf(const OnDeviceOf &) = delete;
+  ~OnDeviceOf() {
+    if (back_ >= 0) (void)hipSetDevice(back_);
+  }
+
+ private:
+  int back_ = -1;
+};
+
 // ---- the target: ops::supported / planner (mod.rs:161-197), without the cost probes.
 // The library is built for gfx950 alone; any other device has no kernels.
 bool device_is_gfx950(int device) {
@@ -479,6 +502,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     return fail(SVODK_ERR_SHAPE, "%s: live batch %d exceeds the capacity %lld", op, opts->batch_live, (long long)cap);
 
   // L205-208: the plan.  A chunk mask plans as a causal one.
+  const OnDeviceOf on(hip_stream);
   int32_t dtypes[4] = {q->dtype, k->dtype, v->dtype, opts->bias ? opts->bias->dtype : 0};
   const int why = plan_attention(current_device_has_kernels(), dtypes, opts->bias ? 4 : 3, q->shape, k->shape,
                                  opts->causal || opts->has_chunk, opts->bias != nullptr);
@@ -768,6 +792,7 @@ int svodk_order_rows(const svodk_tensor *keys, const svodk_tensor *order, void *
     return fail(SVODK_ERR_DTYPE, "%s: order is %s, the output is Int32", op, dtype_name(order->dtype));
   if (keys->shape[0] > svodk::kMaxOrderedRows || (mask && keys->shape[1] > 0x7fffffff))
     return fail(SVODK_ERR_SHAPE, "%s: %lld rows, at most %d", op, (long long)keys->shape[0], svodk::kMaxOrderedRows);
+  const OnDeviceOf on(hip_stream);
   if (!current_device_has_kernels()) return ran_graph(op, SVODK_GRAPH_TARGET);
   if (keys->data == nullptr || order->data == nullptr) return fail(SVODK_ERR_ARGUMENT, "%s: a null device pointer", op);
   Span spans[2] = {{"keys", keys->data, (size_t)numel(keys) * dtype_bytes(keys->dtype), false},
@@ -867,6 +892,7 @@ int svodk_heads(const svodk_tensor *qkv, const svodk_qkv *opts, const svodk_tens
   if (opts->k_norm) dtypes[n++] = opts->k_norm->dtype;
   if (opts->cos) dtypes[n++] = opts->cos->dtype;
   if (opts->sin) dtypes[n++] = opts->sin->dtype;
+  const OnDeviceOf on(hip_stream);
   const int why = plan_heads(current_device_has_kernels(), dtypes, n, qkv->shape, qkv->rank, (int32_t)d);
   if (why != 0) return ran_graph(op, why);
   const int64_t t = qkv->shape[1];
@@ -963,6 +989,7 @@ static int norm(bool layer, const svodk_tensor *x, const svodk_tensor *residual,
   if (residual) dtypes[n++] = residual->dtype;
   dtypes[n++] = w->dtype;
   if (b) dtypes[n++] = b->dtype;
+  const OnDeviceOf on(hip_stream);
   const int why = plan_norm(current_device_has_kernels(), dtypes, n, x->shape, x->rank);
   if (why != 0) return ran_graph(op, why);
 
@@ -1126,6 +1153,7 @@ int svodk_linear(const svodk_tensor *x, const svodk_tensor *w, const svodk_linea
   dtypes[nd++] = w->dtype;
   if (opts->bias) dtypes[nd++] = opts->bias->dtype;
   if (opts->residual) dtypes[nd++] = opts->residual->dtype;
+  const OnDeviceOf on(hip_stream);
   const int why = plan_linear(current_device_has_kernels(), dtypes, nd, x->shape, x->rank, n);
   if (why != 0) return ran_graph(op, why);
   // The parts of the reference's GEMM family this library has no kernel for keep the graph; so does a
