@@ -61,6 +61,22 @@ struct Ref {
   operator PyObject *() const { return p; }
 };
 
+// The owned references of a call's operands, to its end: an option may be computed when it is asked for, and its tensor's
+// memory is the call's until the launch is in the stream.
+struct Kept {
+  c10::SmallVector<PyObject *, 16> all;
+  Kept() = default;
+  Kept(const Kept &) = delete;
+  ~Kept() {
+    for (PyObject *p : all) Py_DECREF(p);
+  }
+  PyObject *operator()(PyObject *x) {
+    if (x == nullptr) throw Raised();
+    all.push_back(x);
+    return x;
+  }
+};
+
 [[noreturn]] void op_failed(const char *kind, const char *message) {
   if (PyObject *e = PyObject_CallFunction(op_error, "ss", kind, message)) {
     PyErr_SetObject(op_error, e);
@@ -151,9 +167,8 @@ const svodk_tensor *maybe(PyObject *o, svodk_tensor &d) {
   describe(o, d);
   return &d;
 }
-const svodk_tensor *maybe_attr(PyObject *o, PyObject *name, svodk_tensor &d) {
-  Ref x(get(o, name));
-  return maybe(x, d);  // whoever owns the attribute keeps the tensor alive past this reference
+const svodk_tensor *maybe_attr(Kept &kept, PyObject *o, PyObject *name, svodk_tensor &d) {
+  return maybe(kept(get(o, name)), d);
 }
 
 void *stream_of(const at::Tensor &t) {
@@ -242,6 +257,7 @@ struct AttnCall {
   svodk_attn a{};
   svodk_cache c{};
   svodk_tensor keys, seg_start, bias, row_order, row_map, k_app, v_app, app_lens;
+  Kept kept;
 
   explicit AttnCall(PyObject *opts) {
     if (opts == Py_None) return;
@@ -253,7 +269,7 @@ struct AttnCall {
       Ref mask(get(opts, names.keys));
       Ref kind(get(mask, names.kind));
       a.key_kind = (int32_t)as_int(kind);
-      a.keys = maybe_attr(mask, names.tensor, keys);
+      a.keys = maybe_attr(kept, mask, names.tensor, keys);
     }
     {
       Ref w(get(opts, names.window));
@@ -270,23 +286,23 @@ struct AttnCall {
         if (left != Py_None) a.chunk_has_left = 1, a.chunk_left = as_int(left);
       }
     }
-    a.seg_start = maybe_attr(opts, names.seg_start, seg_start);
+    a.seg_start = maybe_attr(kept, opts, names.seg_start, seg_start);
     {
       Ref cache(get(opts, names.cache));
       if (cache != Py_None) {
         Ref head_start(get(cache, names.head_start)), kv_heads(get(cache, names.kv_heads));
         c.head_start = as_int(head_start), c.kv_heads = as_int(kv_heads);
-        c.row_map = maybe_attr(cache, names.row_map, row_map);
+        c.row_map = maybe_attr(kept, cache, names.row_map, row_map);
         Ref app(get(cache, names.appended));
         if (app != Py_None) {
-          Ref k(PySequence_GetItem(app, 0)), v(PySequence_GetItem(app, 1));
-          c.k_app = maybe(k, k_app), c.v_app = maybe(v, v_app);
+          c.k_app = maybe(kept(PySequence_GetItem(app, 0)), k_app);
+          c.v_app = maybe(kept(PySequence_GetItem(app, 1)), v_app);
         }
-        c.app_lens = maybe_attr(cache, names.app_lens, app_lens);
+        c.app_lens = maybe_attr(kept, cache, names.app_lens, app_lens);
         a.cache = &c;
       }
     }
-    a.bias = maybe_attr(opts, names.bias, bias);
+    a.bias = maybe_attr(kept, opts, names.bias, bias);
     {
       Ref x(get(opts, names.splits));
       a.splits = int_or_zero(x);
@@ -299,7 +315,7 @@ struct AttnCall {
       Ref x(get(opts, names.batch_live));
       a.batch_live = int_or_zero(x);
     }
-    a.row_order = maybe_attr(opts, names.row_order, row_order);
+    a.row_order = maybe_attr(kept, opts, names.row_order, row_order);
   }
 };
 
@@ -430,20 +446,19 @@ PyObject *py_heads(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   }
   Ref out(made);
   svodk_tensor q_norm, k_norm, cos, sin, xd, qd, kd, vd;
-  o.q_norm = maybe_attr(opts, names.q_norm, q_norm), o.k_norm = maybe_attr(opts, names.k_norm, k_norm);
+  Kept kept;
+  o.q_norm = maybe_attr(kept, opts, names.q_norm, q_norm), o.k_norm = maybe_attr(kept, opts, names.k_norm, k_norm);
   {
     Ref eps(get(opts, names.eps)), rope(get(opts, names.rope)), live(get(opts, names.batch_live));
     o.eps = as_double(eps);
     if (rope != Py_None) {
-      Ref c(PySequence_GetItem(rope, 0)), s(PySequence_GetItem(rope, 1));
-      o.cos = maybe(c, cos), o.sin = maybe(s, sin);
+      o.cos = maybe(kept(PySequence_GetItem(rope, 0)), cos);
+      o.sin = maybe(kept(PySequence_GetItem(rope, 1)), sin);
     }
     o.batch_live = int_or_zero(live);
   }
-  {
-    Ref q(PySequence_GetItem(out, 0)), k(PySequence_GetItem(out, 1)), v(PySequence_GetItem(out, 2));
-    describe(args[0], xd), describe(q, qd), describe(k, kd), describe(v, vd);
-  }
+  describe(args[0], xd), describe(kept(PySequence_GetItem(out, 0)), qd);
+  describe(kept(PySequence_GetItem(out, 1)), kd), describe(kept(PySequence_GetItem(out, 2)), vd);
   void *stream = stream_of(qkv);
   const int status = unlocked(qkv, [&] { return abi.heads(&xd, &o, &qd, &kd, &vd, stream); });
   return answer("heads", status, out);
@@ -460,6 +475,7 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   svodk_linear_opts o{};
   svodk_rotary r{};
   svodk_tensor bias, residual, cos, sin, xd, wd, od;
+  Kept kept;
   if (opts != Py_None) {
     Ref gated(get(opts, names.gated));
     o.gated = truth(gated);
@@ -480,12 +496,12 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     out.take(allocate(args[4], shape, x.scalar_type(), args[0]));
   }
   if (opts != Py_None) {
-    o.bias = maybe_attr(opts, names.bias, bias), o.residual = maybe_attr(opts, names.residual, residual);
+    o.bias = maybe_attr(kept, opts, names.bias, bias), o.residual = maybe_attr(kept, opts, names.residual, residual);
     Ref act(get(opts, names.act)), scale(get(opts, names.scale)), rope(get(opts, names.rope)), live(get(opts, names.batch_live));
     o.act = (int32_t)as_int(act);
     if (scale != Py_None) o.has_scale = 1, o.scale = (float)as_double(scale);
     if (rope != Py_None) {
-      r.cos = maybe_attr(rope, names.cos, cos), r.sin = maybe_attr(rope, names.sin, sin);
+      r.cos = maybe_attr(kept, rope, names.cos, cos), r.sin = maybe_attr(kept, rope, names.sin, sin);
       Ref heads(get(rope, names.heads)), head_dim(get(rope, names.head_dim));
       r.heads = (int32_t)as_int(heads), r.head_dim = (int32_t)as_int(head_dim);
       o.rope = &r;
@@ -518,6 +534,7 @@ PyObject *py_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   }
   Ref out(made);
   svodk_tensor xd, rd, wd, bd, sd, yd;
+  Kept kept;
   describe(x, xd);
   if (fused) describe(residual, rd);
   describe(args[2], wd);
@@ -525,8 +542,7 @@ PyObject *py_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const double eps = as_double(args[4]);
   const int32_t live = int_or_zero(args[5]);
   if (fused) {
-    Ref sum(PySequence_GetItem(out, 0)), y(PySequence_GetItem(out, 1));
-    describe(sum, sd), describe(y, yd);
+    describe(kept(PySequence_GetItem(out, 0)), sd), describe(kept(PySequence_GetItem(out, 1)), yd);
   } else {
     describe(out, yd);
   }
