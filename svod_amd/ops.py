@@ -160,7 +160,12 @@ def _calls():
     global _native
     if _native is None:
         lib = load_library()
-        from . import _host
+        try:
+            from . import _host
+        except ImportError as e:
+            raise ImportError(
+                f"{os.path.join(_HERE, '_host.so')} is missing or was built against another torch or Python ({e}): "
+                "build it with `python -m svod_amd.build`. svod_amd has no fallback implementation.") from e
 
         names = ("attention", "attention_noalloc", "attention_packed", "attention_workspace", "heads", "linear", "layer_norm",
                  "add_layer_norm", "rms_norm", "add_rms_norm", "order_rows")

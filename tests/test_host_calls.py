@@ -1,6 +1,7 @@
 """The native side of the Python calls (svod_amd/csrc/host.cpp) on operands it has to refuse itself, before the
 library sees them."""
 import ctypes
+import sys
 import weakref
 
 import pytest
@@ -87,3 +88,11 @@ def test_a_computed_option_lives_to_the_end_of_the_call():
     assert len(made) == 8 + 4 + 4
     # A later call finds the earlier ones' options gone.
     assert dead == [0, 8, 12]
+
+
+def test_a_missing_native_side_says_how_to_build_it(monkeypatch):
+    monkeypatch.setattr(svod_amd.ops, "_native", None)
+    monkeypatch.setitem(sys.modules, "svod_amd._host", None)  # what an import that cannot succeed meets
+    monkeypatch.delattr(svod_amd, "_host", raising=False)
+    with pytest.raises(ImportError, match="python -m svod_amd.build"):
+        svod_amd.rms_norm(X, W)
