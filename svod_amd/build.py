@@ -48,6 +48,7 @@ ATTENTION_PARTS = [0, 32, 48, 64, 128, 256]
 
 
 def build(verbose: bool = False) -> str:
+    """The library and ``_host.so``: what the package needs to run."""
     from concurrent.futures import ThreadPoolExecutor
 
     cc = hipcc()
@@ -65,11 +66,13 @@ def build(verbose: bool = False) -> str:
     with ThreadPoolExecutor(max_workers=workers) as pool:
         list(pool.map(lambda job: _run(job[1], verbose), jobs))
     _run([cc, *DEVICE_FLAGS, "-shared", "-fPIC", "-o", LIB, *[obj for obj, _ in jobs]], verbose)
+    build_host(verbose)
     return LIB
 
 
 def build_host(verbose: bool = False) -> str:
-    """``_host.so``: host code over torch's C++ interface, so it is compiled with g++ against the installed torch."""
+    """``_host.so``: host code over torch's C++ interface, so it is compiled with g++ against the installed torch and
+    Python, and is of use to those alone."""
     import sysconfig
 
     import torch
@@ -148,5 +151,4 @@ if __name__ == "__main__":
         print(build_code_objects(verbose=True))
     else:
         print(build(verbose=True))
-        print(build_host(verbose=True))
         print(build_code_objects(verbose=True))

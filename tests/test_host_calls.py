@@ -96,3 +96,12 @@ def test_a_missing_native_side_says_how_to_build_it(monkeypatch):
     monkeypatch.delattr(svod_amd, "_host", raising=False)
     with pytest.raises(ImportError, match="python -m svod_amd.build"):
         svod_amd.rms_norm(X, W)
+
+
+def test_the_build_is_of_everything_that_the_package_loads(monkeypatch):
+    from svod_amd import build
+
+    outputs = []
+    monkeypatch.setattr(build, "_run", lambda cmd, verbose: outputs.append(cmd[cmd.index("-o") + 1]))
+    build.build()
+    assert {build.LIB, build.HOST} <= set(outputs)
