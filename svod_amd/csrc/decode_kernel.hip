@@ -131,9 +131,11 @@ __device__ __forceinline__ f32x2 got2(const float *p) {  // 8-byte aligned
                                                      __HIP_MEMORY_SCOPE_AGENT));
 }
 
-template <bool KEEP>
+// Keys and values are read once a step, and by the next step the other layers' caches and the weights have been through
+// the chip.  Without the mark a step of 34 sequences over 570 cached keys is faster on one layer called back to back (32.2
+// -> 25.5 us with two layers' windows in turn), and slower over a model's (8 layers 30.5 -> 32.4, 16 layers 28.1 -> 30.3; 20 over
+// 440 keys 15.8 -> 17.2, 8 over 2000 24.0 -> 24.9).
 __device__ __forceinline__ u32x4 key_row(const uint16_t *p) {
-  if constexpr (KEEP) return *reinterpret_cast<const u32x4 *>(p);
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
 }
 
@@ -142,8 +144,7 @@ __device__ __forceinline__ u32x4 key_row(const uint16_t *p) {
 enum { kWhole, kPartial, kMerged };
 
 // The workgroup's program for `nw` waves, for the kernels below to inline.
-// KEEP: the keys and values may stay on the chip for the next step; else they are asked for as read once.
-template <int D, int R, bool F16, int MODE, bool KEEP>
+template <int D, int R, bool F16, int MODE>
 __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // No contraction beyond the fused multiply-adds written out below: the library's kernel (its wave count a launch
@@ -245,8 +246,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
         x.v[u] = u32x4{0, 0, 0, 0};
         x.seen[u] = there ? 1 : 0;
         if (there && pos_ok) {
-          x.k[u] = key_row<KEEP>(kb + (int64_t)key * row_elems);
-          x.v[u] = key_row<KEEP>(vb + (int64_t)key * row_elems);
+          x.k[u] = key_row(kb + (int64_t)key * row_elems);
+          x.v[u] = key_row(vb + (int64_t)key * row_elems);
         }
         if (there && mask != nullptr)
           x.seen[u] = mask_bytes == 1 ? (int)((const uint8_t *)mask)[key] : ((const int *)mask)[key];
@@ -507,7 +508,7 @@ struct Packed {
 };
 static_assert(sizeof(Packed) <= 112 && kDecodeRows <= 4, "the record's size, the group's and the tokens' two bits");
 
-template <int D, int R, bool F16, int MODE, bool KEEP>
+template <int D, int R, bool F16, int MODE>
 __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   DecodeArgs p;
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) 
   const int64_t states = (int64_t)p.splits * p.batch * p.t * p.heads;
   p.o_part = a.states, p.m_part = a.states + states * D, p.l_part = p.m_part + states;
   p.arrivals = reinterpret_cast<uint64_t *>(p.l_part + states), p.tag = a.tag;
-  decode_body<D, R, F16, MODE, KEEP>(p, decode_waves((int64_t)p.batch * p.kv_heads * p.splits));
+  decode_body<D, R, F16, MODE>(p, decode_waves((int64_t)p.batch * p.kv_heads * p.splits));
 #endif
 }
 
@@ -534,19 +535,11 @@ hipError_t launch_r(const Packed &p, bool merged, hipStream_t stream) {
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const uint32_t threads = (uint32_t)decode_waves(grid) * 64;
-  // Of 20 to 96 MB of keys and values a launch, those of the last steps are still on the chip when they are asked for again:
-  // 20 sequences over 440 keys (72 MB) 16.4 -> 15.0 us, 34 over 570 (79 MB) 34.3 -> 30.2.  More of them only push one another
-  // out: Whisper's step (123 MB) 25.9 -> 27.3, 56 sequences over 700 (321 MB) 65 -> 71; fewer are no faster kept.
-  const int64_t bytes = (int64_t)p.batch * p.tk * p.kv_heads * D * 4;
-  const bool keep = bytes >= 20000000 && bytes <= 96000000;
-  auto run = [&](auto mode, auto kept) {
-    return Launch<decode_kernel<D, R, F16, decltype(mode)::value, decltype(kept)::value>>::run(grid, threads, 0, 0, stream, p);
+  auto run = [&](auto mode) {
+    return Launch<decode_kernel<D, R, F16, decltype(mode)::value>>::run(grid, threads, 0, 0, stream, p);
   };
-  typedef std::integral_constant<int, kWhole> Whole;
-  typedef std::integral_constant<int, kMerged> Merged;
-  if (p.splits == 1) return keep ? run(Whole(), std::true_type()) : run(Whole(), std::false_type());
-  if (merged) return keep ? run(Merged(), std::true_type()) : run(Merged(), std::false_type());
-  return run(std::integral_constant<int, kPartial>(), std::false_type());
+  if (p.splits == 1) return run(std::integral_constant<int, kWhole>());
+  return merged ? run(std::integral_constant<int, kMerged>()) : run(std::integral_constant<int, kPartial>());
 }
 
 template <int D>
@@ -673,7 +666,7 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.splits = (S) && splits > 1 ? splits : 1, p.cached = cached, p.kv_head_start = kv_head_start;                    \
     p.cache_rows = cache_rows, p.app_rows = app_rows, p.scale = __builtin_bit_cast(float, scale_bits);                \
     p.arrivals = nullptr, p.tag = 0;                                                                                  \
-    svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole, false>(p, 4);                           \
+    svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole>(p, 4);                                  \
   }
 #define SVODK_DECODE_ROWS_OF(D, T, F16, S) \
   SVODK_DECODE_ENTRY(D, 1, T, F16, S) SVODK_DECODE_ENTRY(D, 2, T, F16, S) SVODK_DECODE_ENTRY(D, 4, T, F16, S)
