@@ -51,11 +51,11 @@ __device__ __forceinline__ float wave_sum(float x) {
   return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
-// What a launch marks non-temporal, by its size (launch_rows).  The sum, read again only a layer's work later, always is.
-//   kLoadsKept  the normalised rows, not the operands, which the call before wrote: marked, they took a tenth longer
-//   kKept       nothing: the rows are there for the projection that reads them
-//   kOutKept    the operands: more of them than the chip's last cache holds
-enum { kLoadsKept, kKept, kOutKept };
+// What a launch marks non-temporal, by its size (launch_rows).  The sum, read again only a layer's work later, always is;
+// the normalised rows never are: the projection reads them next.
+//   kKept     nothing else
+//   kOutKept  the operands: more of them than the chip's last cache holds
+enum { kKept, kOutKept };
 template <int CACHE>
 __device__ __forceinline__ u32x4 take(const uint16_t *p) {
   if constexpr (CACHE == kOutKept) return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
@@ -161,10 +161,7 @@ __device__ __forceinline__ void rows_body(const uint16_t *__restrict__ x, const 
         }
         packed[i] = narrow<F16>(y0, y1);
       }
-      if constexpr (CACHE != kLoadsKept)
-        *reinterpret_cast<u32x4 *>(out + base + at) = packed;
-      else
-        store_once(reinterpret_cast<u32x4 *>(out + base + at), packed);
+      *reinterpret_cast<u32x4 *>(out + base + at) = packed;
     }
   };
   // Two sets of registers take turns: one row is worked on while the next is on its way.
@@ -235,19 +232,20 @@ hipError_t launch_rows(const NormArgs &a, hipStream_t stream) {
   }
   const RowsCall c = {(const uint16_t *)a.x, (const uint16_t *)a.residual, (const uint16_t *)a.w, (const uint16_t *)a.b,
                       (uint16_t *)a.out, (uint16_t *)a.sum, a.rows, a.d, (float)(1.0 / (double)a.d), (float)a.eps, (uint32_t)blocks};
-  // Kept, the rows are there for the projection (a Qwen3 layer's prefill of 700 tokens 32.0 -> 28.8 us); from a quarter of
-  // what the L2s hold on the launch's end waits for them to be written back ([6000, 1024] RMSNorm 5.1 -> 6.0), until the
-  // launch is long enough for that to go on beside it.  Up to some 170 MB of all tensors the operands are found on the chip
-  // ([8000, 2048] add+RMSNorm, 131 MB: 20.4 us, marked 23.2); past that they push the outputs out ([16384, 2048], 268 MB:
-  // 49.8, marked 43.2, marked with the outputs 45.5).
-  const int64_t bytes = a.rows * a.d * 2;
+  // Measured in layers of which each norm reads what a projection wrote and a projection reads what it leaves (us for three
+  // layers, rows marked -> kept): Qwen3 of 1024 tokens 175 -> 165, 3072 301 -> 283, 6144 452 -> 431, 16384 1010 -> 1001; ModernBERT of
+  // 1024 100 -> 93, 5120 171 -> 163, 8192 232 -> 227; four times (projection, [3000, 2048] add+RMSNorm) 166 -> 150.  A norm
+  // by itself is no faster for it (its end waits for the rows to be written back: [12000, 1024] RMSNorm over and over 6.1 -> 8.5,
+  // over operands in turn 10.5 -> 12.0), and no program runs one by itself.
+  // The operands are what the call before left on the chip, up to some 170 MB of all tensors ([8000, 2048] add+RMSNorm, 131 MB:
+  // 19.8 us, marked 22.6; the layers the same); past that marked ones leave the room to the rows (four times
+  // (projection, norm) of [11000, 2048], 180 MB, 428 -> 423, [16384, 2048], 268 MB, 587 -> 577, [24000, 2048] 873 -> 840).
   auto run = [&](auto cache) {
     return Launch<rows_kernel<SPANS, LAYER, RESIDUAL, BIAS, F16, decltype(cache)::value>>::run(blocks, kRowsPerBlock * 64, 0, 0,
                                                                                                stream, c);
   };
-  if (bytes * (RESIDUAL ? 4 : 2) > (170 << 20)) return run(std::integral_constant<int, kOutKept>());
-  if (bytes < (6 << 20) || bytes >= (20 << 20)) return run(std::integral_constant<int, kKept>());
-  return run(std::integral_constant<int, kLoadsKept>());
+  if (a.rows * a.d * (RESIDUAL ? 8 : 4) > (170 << 20)) return run(std::integral_constant<int, kOutKept>());
+  return run(std::integral_constant<int, kKept>());
 }
 
 template <int SPANS, bool F16>
