@@ -51,24 +51,18 @@ struct Div64 {
 // 20 % slower: the many small waves keep more of HBM's channels busy than fewer long ones).
 constexpr int kItems = 1;
 
-// Every byte is touched once, but the input was written by the call before and the outputs are read by the one after.
-// What a launch of so many bytes of outputs (as many of input) marks non-temporal:
-//   kStream   loads and stores, below 16 MiB: 1400 Qwen3 rows 5.8 us, 6.7 with either kept
-//   kKeep     neither, to 70 MiB: 2800 rows 10.2 -> 9.6, 8000 rows 23.7 -> 22.0
-//   kKeepOut  loads only: at 16384 rows (134 MB) 45.0 -> 44.4 by itself, and the layer's prefill 321.5 -> 315.7, whose
-//             attention then finds the last of the outputs on the chip
-enum { kStream, kKeep, kKeepOut };
+// Every byte is touched once, but the input was written by the call before and the attention reads the outputs next: they
+// are never marked non-temporal, though the kernel by itself is faster with them marked (16384 Qwen3 rows with operands in turn
+// 44.7 us, 47.0 kept; 1400 rows 5.5 and 7.6).  Three layers of (projection, prologue, attention, projection), us, outputs
+// marked -> kept: 512 tokens the same, 1280 207 -> 203, 2048 247 -> 235, 4096 374 -> 365, 8192 608 -> 600, 16384 1152 -> 1135.
+// The input, by a launch's bytes of outputs (as many of input):
+//   kKeep     not marked, to 70 MiB: 8192 rows over and over 24.1 -> 20.6 us, the layers the same
+//   kKeepOut  marked: the room is the outputs' (the layers of 10240 tokens 811 -> 796, of 16384 1153 -> 1135)
+enum { kKeep, kKeepOut };
 template <int CACHE>
 __device__ __forceinline__ u32x4 take(const uint16_t *p) {
   if constexpr (CACHE == kKeep) return *reinterpret_cast<const u32x4 *>(p);
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
-}
-template <int CACHE>
-__device__ __forceinline__ void leave(uint16_t *p, const u32x4 &x) {
-  if constexpr (CACHE == kStream)
-    __builtin_nontemporal_store(x, reinterpret_cast<u32x4 *>(p));
-  else
-    *reinterpret_cast<u32x4 *>(p) = x;
 }
 
 // The workgroup's program, for the kernels below to inline.
@@ -174,8 +168,8 @@ __device__ __forceinline__ void heads_body(const uint16_t *__restrict__ qkv, con
       o1 = w1[u];  // untouched slots (v, or q/k with neither norm nor rope) keep their bits
       o2 = w2[u];
     }
-    leave<CACHE>(dst, o1);
-    leave<CACHE>(dst + kHalf, o2);
+    *reinterpret_cast<u32x4 *>(dst) = o1;
+    *reinterpret_cast<u32x4 *>(dst + kHalf) = o2;
   }
 }
 
@@ -219,9 +213,7 @@ hipError_t launch(const HeadsArgs &a, hipStream_t stream) {
   if (blocks * per_block < 0xffffffffLL) {
     auto rcp = [](uint32_t d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); };
     const Div32 by_slots = {(uint32_t)slots, rcp((uint32_t)slots)}, by_t = {(uint32_t)t, rcp((uint32_t)t)};
-    const int64_t bytes = items * D * 2;
-    if (bytes < (16 << 20)) return run(by_slots, by_t, std::integral_constant<int, kStream>());
-    if (bytes <= (70 << 20)) return run(by_slots, by_t, std::integral_constant<int, kKeep>());
+    if (items * D * 2 <= (70 << 20)) return run(by_slots, by_t, std::integral_constant<int, kKeep>());
     return run(by_slots, by_t, std::integral_constant<int, kKeepOut>());
   }
   return run(Div64{slots, 0}, Div64{t, 0}, std::integral_constant<int, kKeepOut>());
@@ -266,7 +258,7 @@ __device__ __forceinline__ void heads_entry(const uint16_t *qkv, const uint16_t 
   auto rcp = [](uint32_t d) { return d <= 1 ? 0xffffffffu : 0xffffffffu / d; };  // within one of floor(2^32 / d)
   const uint32_t slots = (uint32_t)(heads + 2 * kv_heads), tt = (uint32_t)(t > 0 ? t : 1);
   const Div32 by_slots = {slots, rcp(slots)}, by_t = {tt, rcp(tt)};
-  heads_body<D, Div32, F16, kStream>(qkv, q_w, k_w, cos_t, sin_t, q, k, v, (int64_t)rows * slots, by_slots, by_t, heads, kv_heads,
+  heads_body<D, Div32, F16, kKeep>(qkv, q_w, k_w, cos_t, sin_t, q, k, v, (int64_t)rows * slots, by_slots, by_t, heads, kv_heads,
                             __builtin_bit_cast(float, eps_bits), rope);
 }
 
