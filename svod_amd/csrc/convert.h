@@ -1,5 +1,5 @@
-// Widening and narrowing between the operands' 16-bit float types and f32, shared by the
-// row-wise kernels (the attention prologue and the row norms).
+// Widening and narrowing between the operands' 16-bit float types and f32, shared by the attention
+// prologue, the row norms and the projection.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -17,19 +17,12 @@
 
 #include <atomic>
 
-#include "convert.h"
 #include "kernels.h"
 #include "launch.h"
+#include "matrix.h"
 
 namespace svodk {
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-
-typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 constexpr int kWaves = 8;
 constexpr int kBk = 64;              // k-columns a wave takes at a time: a row of them is one 128-byte line
@@ -46,38 +39,6 @@ struct Tile {
   static constexpr int kWaveBytes = kChunkBytes > kPartBytes ? kChunkBytes : kPartBytes;
   static constexpr int kLds = kWaves * kWaveBytes;
 };
-
-template <bool F16>
-__device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-#else
-  return c;
-#endif
-}
-
-// Four 16-bit elements at `p` (8-byte aligned) as f32.
-template <bool F16>
-__device__ __forceinline__ f32x4 load4(const uint16_t *p) {
-  const u32x2 x = *reinterpret_cast<const u32x2 *>(p);
-  if constexpr (F16) {
-    const f32x2 lo = __builtin_convertvector(__builtin_bit_cast(f16x2, (uint32_t)x[0]), f32x2);
-    const f32x2 hi = __builtin_convertvector(__builtin_bit_cast(f16x2, (uint32_t)x[1]), f32x2);
-    return f32x4{lo[0], lo[1], hi[0], hi[1]};
-  } else {
-    return f32x4{bf16_lo(x[0]), bf16_hi(x[0]), bf16_lo(x[1]), bf16_hi(x[1])};
-  }
-}
-
-// A raw buffer descriptor over `bytes` bytes at `base`: loads past the end return zero.
-__device__ __forceinline__ i32x4 make_rsrc(const void *base, int64_t bytes) {
-  const int64_t clamped = bytes < 0 ? 0 : (bytes > 0xffffffffLL ? 0xffffffffLL : bytes);
-  const uint64_t addr = (uint64_t)(uintptr_t)base;
-  return i32x4{(int)(uint32_t)addr, (int)(uint32_t)((addr >> 32) & 0xffffu), (int)(uint32_t)clamped, 0x00020000};
-}
 
 struct FewCall {
   const uint16_t *x, *w, *bias, *cos, *sin;
@@ -127,7 +88,7 @@ __global__ __launch_bounds__(kWaves * 64) void linear_few_kernel(const FewCall c
       const int first = is_x ? 8 * j - kBn : (8 * j < kRun ? 8 * j : 8 * j - kRun);  // from the descriptor's first row
       if (is_x && row0 + first >= rows) continue;  // the rest of an x tile that is not there: never stored
       const int chunk = place ^ ((4 * (j & 1) + (frow >> 1)) & 7);
-      const int voff = half && chunk >= 4 ? (int)0xfffffff0u : (int)((first + frow) * row_bytes) + chunk * 16;
+      const int voff = half && chunk >= 4 ? (int)kPastBound : (int)((first + frow) * row_bytes) + chunk * 16;
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                    :
                    : "s"(__builtin_amdgcn_readfirstlane(lds0 + j * 1024)), "v"(voff), "s"(is_x ? rx : (8 * j < kRun ? r0 : r1))

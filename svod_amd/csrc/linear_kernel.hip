@@ -28,6 +28,7 @@
 
 #include "kernels.h"
 #include "launch.h"
+#include "matrix.h"
 
 namespace svodk {
 namespace {
@@ -36,16 +37,6 @@ namespace {
 #pragma clang diagnostic ignored "-Wunused-function"
 #pragma clang diagnostic ignored "-Wunused-const-variable"
 #endif
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 constexpr int kXcds = 8;
 constexpr int kBk = 64;                 // k-columns a stage: a row of a tile is one 128-byte line
@@ -94,52 +85,6 @@ struct Columns {
   static constexpr int kHalfBlocks = kSplit ? 2 : HD / 32;  // from a block to its partner
   __host__ __device__ static constexpr bool first_half(int cb) { return HD > 0 && at(cb) % (HD > 0 ? HD : 1) < HD / 2; }
 };
-
-template <bool F16>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  f32x2 f = {lo, hi};
-  if constexpr (F16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
-  else
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
-}
-
-// One 16-bit element of the operands' type as f32.
-template <bool F16>
-__device__ __forceinline__ float widen(uint32_t bits16) {
-  if constexpr (F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-  return __builtin_bit_cast(float, bits16 << 16);
-}
-
-template <bool F16>
-__device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// A raw buffer descriptor over `bytes` bytes at `base`: loads past the end return zero.
-__device__ __forceinline__ i32x4 make_rsrc(const void *base, int64_t bytes) {
-  const int64_t clamped = bytes < 0 ? 0 : (bytes > 0xffffffffLL ? 0xffffffffLL : bytes);
-  const uint64_t addr = (uint64_t)(uintptr_t)base;
-  i32x4 r;
-  r[0] = (int)(uint32_t)addr;
-  r[1] = (int)(uint32_t)((addr >> 32) & 0xffffu);
-  r[2] = (int)(uint32_t)clamped;
-  r[3] = 0x00020000;
-  return r;
-}
-
-// Four 16-bit elements at `p` (8-byte aligned) as f32.
-template <bool F16>
-__device__ __forceinline__ void load4(const uint16_t *p, float (&out)[4]) {
-  const u32x2 x = *reinterpret_cast<const u32x2 *>(p);
-  out[0] = widen<F16>(x[0] & 0xffffu);
-  out[1] = widen<F16>(x[0] >> 16);
-  out[2] = widen<F16>(x[1] & 0xffffu);
-  out[3] = widen<F16>(x[1] >> 16);
-}
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // HD: the head size a turning kernel is built for (64 or 128), 0: no turn.
@@ -197,7 +142,7 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
   // Fill `f` of stage `s` of the k loop into slot `slot` of its ring; past the last stage an empty descriptor (zeros
   // land in a slot nothing reads any more) keeps the count of fills in flight the same in every iteration.
   auto fill = [&](int s, int slot, int f) {
-    const int voff = (short_tail && s == nk - 1 && second_half) ? (int)0xfffffff0u : src + s * kRowBytes;
+    const int voff = (short_tail && s == nk - 1 && second_half) ? (int)kPastBound : src + s * kRowBytes;
     const int at = f < kWFills ? slot * kWBytes + f * kWaves * 1024 : kXRing + slot * kXBytes + (f - kWFills) * kWaves * 1024;
     i32x4 r = rsrc[f];
     if (s >= nk) r[2] = 0;
@@ -320,8 +265,8 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
   // set of accumulators for where its two ways meet.
 #pragma unroll
   for (int cb = 0; cb < CB; cb++) {
-    float b4[4] = {-0.0f, -0.0f, -0.0f, -0.0f};
-    if (bias != nullptr) load4<F16>(bias + min(wave_n0 + Cols::at(cb) + 4 * g, n - 4), b4);  // columns past the end are not stored
+    f32x4 b4 = {-0.0f, -0.0f, -0.0f, -0.0f};
+    if (bias != nullptr) b4 = load4<F16>(bias + min(wave_n0 + Cols::at(cb) + 4 * g, n - 4));  // columns past the end are not stored
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -359,9 +304,8 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
 #pragma unroll
       for (int rb = 0; rb < RB; rb++) {
         const int r = wave_m * 16 * RB + rb * 16 + ln;
-        float c4[4], s4[4];
-        load4<F16>(reinterpret_cast<const uint16_t *>(cos_lds + r * kPitch) + at, c4);
-        load4<F16>(reinterpret_cast<const uint16_t *>(sin_lds + r * kPitch) + at, s4);
+        const f32x4 c4 = load4<F16>(reinterpret_cast<const uint16_t *>(cos_lds + r * kPitch) + at);
+        const f32x4 s4 = load4<F16>(reinterpret_cast<const uint16_t *>(sin_lds + r * kPitch) + at);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const float y1 = acc[rb][cb][e], y2 = acc[rb][pb][e];
@@ -391,8 +335,8 @@ __device__ __forceinline__ void linear_body(uint8_t *smem, const uint16_t *__res
 #pragma unroll
       for (int cb = 0; cb < CB; cb++) {
         u32x2 out;
-        out[0] = pack2<F16>(acc[rb][cb][0], acc[rb][cb][1]);
-        out[1] = pack2<F16>(acc[rb][cb][2], acc[rb][cb][3]);
+        out[0] = narrow<F16>(acc[rb][cb][0], acc[rb][cb][1]);
+        out[1] = narrow<F16>(acc[rb][cb][2], acc[rb][cb][3]);
         *reinterpret_cast<u32x2 *>(srow + 32 * cb) = out;
       }
     }
