@@ -375,6 +375,17 @@ PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   SVODK_END
 }
 
+// (q, k, opts): the bytes of a split call's partial tensors (svodk_attention_workspace), 0 where the call would not split
+PyObject *py_attention_workspace(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  SVODK_ARGS(3, "attention_workspace")
+  SVODK_BEGIN
+  AttnCall call(args[2]);
+  svodk_tensor qd, kd;
+  describe(args[0], qd), describe(args[1], kd);
+  return PyLong_FromLongLong(abi.attention_workspace(&qd, &kd, &call.a));
+  SVODK_END
+}
+
 // (q, k, v, opts, out)
 PyObject *py_attention_noalloc(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   SVODK_ARGS(5, "attention_noalloc")
@@ -607,6 +618,7 @@ PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, nullptr},
     SVODK_FAST("attention", py_attention),
     SVODK_FAST("attention_noalloc", py_attention_noalloc),
+    SVODK_FAST("attention_workspace", py_attention_workspace),
     SVODK_FAST("attention_packed", py_attention_packed),
     SVODK_FAST("heads", py_heads),
     SVODK_FAST("linear", py_linear),

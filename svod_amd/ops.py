@@ -206,30 +206,6 @@ _ERR_KIND = {-1: "Shape", -2: "Dtype", -3: "Heads", -4: "Launch", -5: "Argument"
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2, torch.int32: 3, torch.int64: 4, torch.bool: 5}
 
 
-def _desc(t: torch.Tensor) -> _Tensor:
-    if t.dtype not in _DTYPES:
-        raise OpError("Dtype", f"unsupported element type {t.dtype}")
-    if t.dim() > 4:
-        raise OpError("Shape", f"rank {t.dim()} tensor")
-    if not t.is_contiguous():
-        raise OpError("Argument", "operands must be dense row-major (call .contiguous())")
-    d = _Tensor()
-    d.data = t.data_ptr()
-    d.dtype = _DTYPES[t.dtype]
-    d.rank = t.dim()
-    for i, s in enumerate(t.shape):
-        d.shape[i] = s
-    return d
-
-
-def _ref(keep: list, t: Optional[torch.Tensor]):
-    if t is None:
-        return ctypes.POINTER(_Tensor)()
-    d = _desc(t)
-    keep.append(d)
-    return ctypes.pointer(d)
-
-
 def _finish(op: str, status: int):
     if status == 0:
         return
@@ -301,36 +277,6 @@ class Qkv:
     eps: float = 1e-6
     rope: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
     batch_live: Optional[int] = None
-
-
-def _attn_options(opts: Attn, keep: list) -> _Attn:
-    a = _Attn()
-    a.causal = int(opts.causal)
-    a.key_kind = opts.keys.kind
-    a.keys = _ref(keep, opts.keys.tensor)
-    if opts.window is not None:
-        a.has_window, a.window_left, a.window_right = 1, opts.window[0], opts.window[1]
-    if opts.chunk is not None:
-        size, left, right = opts.chunk
-        a.has_chunk, a.chunk_size, a.chunk_right = 1, size, right
-        a.chunk_has_left, a.chunk_left = (0, 0) if left is None else (1, left)
-    a.seg_start = _ref(keep, opts.seg_start)
-    if opts.cache is not None:
-        c = _Cache()
-        c.head_start, c.kv_heads = int(opts.cache.head_start), int(opts.cache.kv_heads)
-        c.row_map = _ref(keep, opts.cache.row_map)
-        if opts.cache.appended is not None:
-            c.k_app, c.v_app = _ref(keep, opts.cache.appended[0]), _ref(keep, opts.cache.appended[1])
-        c.app_lens = _ref(keep, opts.cache.app_lens)
-        keep.append(c)
-        a.cache = ctypes.pointer(c)
-    a.bias = _ref(keep, opts.bias)
-    a.splits = opts.splits or 0
-    if opts.scale is not None:
-        a.has_scale, a.scale = 1, float(opts.scale)
-    a.batch_live = opts.batch_live or 0
-    a.row_order = _ref(keep, opts.row_order)
-    return a
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, opts: Optional[Attn] = None,

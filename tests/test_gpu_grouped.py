@@ -32,15 +32,12 @@ def test_grouped_tiles_match_repeated_kv_heads_bit_for_bit(device, name, b, t, t
     keys = KeyMask.none() if lens is None else KeyMask.lens(torch.tensor(lens, dtype=torch.int32, device=device))
     dev = lambda x: None if x is None else bf16_tensor(x, device)
     # Splits are pinned so that both calls run the same ones (unasked, the rule counts workgroups).
-    ws_q, ws_k = svod_amd.ops._desc(dev(q)), svod_amd.ops._desc(dev(k))
     opts = Attn(keys=keys, splits=splits, bias=dev(bias))
     grouped = svod_amd.attention(dev(q), dev(k), dev(v), opts)
     chosen = svod_amd.chosen()
     used = splits or (1 if "combine_splits" not in chosen else None)
     if used is None:  # the rule split it: ask how many ways, and name that count for the repeated call
-        import ctypes
-        a = svod_amd.ops._attn_options(Attn(keys=keys), [])
-        need = svod_amd.load_library().svodk_attention_workspace(ctypes.byref(ws_q), ctypes.byref(ws_k), ctypes.byref(a))
+        need = svod_amd.ops._calls().attention_workspace(dev(q), dev(k), Attn(keys=keys))
         used = need // (b * t * h * (d + 2) * 4)
         assert used > 1
     group = h // hkv
