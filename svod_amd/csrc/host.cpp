@@ -229,6 +229,8 @@ class OnDeviceOf {
  public:
   explicit OnDeviceOf(const at::Tensor &t) {
     if (!t.is_cuda()) return;
+    static const bool several = c10::hip::device_count() > 1;
+    if (!several) return;
     const c10::DeviceIndex now = c10::hip::current_device();
     if (t.device().index() == now) return;
     c10::hip::set_device(t.device().index());

@@ -162,7 +162,7 @@ int check_aliasing(const char *op, const Span *spans, int n) {
 
 // The device of the caller's stream is the current one for the length of a call: what is asked of a device (has it kernels,
 // its compute units, its scratch, a kernel's function) is then asked of the one that runs the launch.  The default streams
-// are the current device's own.
+// are the current device's own; on another stream it takes 0.1 us (a norm's call 3.9 -> 4.0).
 class OnDeviceOf {
  public:
   explicit OnDeviceOf(void *hip_stream) {
