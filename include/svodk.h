@@ -14,7 +14,8 @@
  * and the workspace (the kernels move them in 128-bit pieces) and aligned to
  * their element for integers and masks; an address off that answers
  * SVODK_ERR_ARGUMENT.  Launches are enqueued on the HIP
- * stream given and return without synchronising.
+ * stream given, on that stream's device whichever is current (a default stream
+ * is the current device's), and return without synchronising.
  */
 #ifndef SVODK_H
 #define SVODK_H
