@@ -114,7 +114,9 @@ typedef struct svodk_cache {
  * few query tiles and many keys (a decoder step) when the workspace
  * svodk_attention_workspace asks for is lent, and keeps the keys whole without it.
  * A decoder step (svodk_tune_decode) of up to 64 splits merges them itself, in the one launch, where
- * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  What the workspace
+ * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  With `splits` = 0 and
+ * twice the bytes and those words it takes the count that suits the device, up to twice the rule's (other
+ * counts round differently).  What the workspace
  * holds at first does not matter, nor does the stream, nor whether the call is captured; as with the
  * partial states, no two launches in flight may have the same workspace.
  */
@@ -218,7 +220,7 @@ int svodk_order_rows(const svodk_tensor *keys, const svodk_tensor *order, void *
  * Bytes of `workspace` svodk_attention needs for these operands and options:
  * the f32 partial tensors o_part [splits, B, T, H, D], m_part and l_part
  * [splits, B, T, H] of tk/src/ops/attention.rs:285-293, for the split count the
- * call would run with; 0 when it would not split.  Pure, no device.
+ * call would run with, given that much; 0 when it would not split.  Pure, no device.
  */
 int64_t svodk_attention_workspace(const svodk_tensor *q, const svodk_tensor *k, const svodk_attn *opts);
 

@@ -8,7 +8,10 @@
 // fills before the next; here every lane loads its 16 bytes of a key row straight into registers, several
 // rows ahead, with no LDS and no barrier in the loop, and a compute unit holds a few hundred KiB in flight.
 //
-//   a key row of D elements is shared by D/8 lanes (16 bytes each); a wave instruction covers 512/D rows
+//   a key row of D elements is shared by D/8 lanes (16 bytes each); a wave instruction takes up to four neighbouring
+//   heads' rows of a key (512 bytes in one piece) and as many keys as are left of its 64 lanes: a memory access of 512
+//   bytes streams a sixth faster than one of 128 or 256 (loads alone: 16 sequences of 8 heads of 128 over 2100 keys 29.8 ->
+//   24.9 us, of 20 heads of 64 over 1500 keys 24.7 -> 21.1; of 1 KiB, 24.8 and 23.8)
 //   score:   v_dot2_f32 over the lane's four pairs, summed over the row's lanes by DPP
 //   softmax: every lane runs the online form over the keys of its own place in the wave, in the exponent's
 //            units (scores scaled first, L365-370); probabilities stay f32 where the tile program rounds them
@@ -30,6 +33,7 @@ namespace svodk {
 namespace {
 
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
@@ -44,7 +48,23 @@ constexpr int kCountBits = 7;      // of a word of arrivals: its low bits count,
 static_assert(kMostMergedSplits < 1 << kCountBits, "the count stands at the splits when a launch ends");
 
 // Waves a workgroup: few workgroups take eight each, so that the launch still has its bytes in flight.
-__host__ __device__ constexpr int decode_waves(int64_t workgroups) { return workgroups >= 256 ? 4 : kMaxWaves; }
+// `heads_splits`: (batch, KV head, split)s of the launch.
+__host__ __device__ constexpr int decode_waves(uint32_t heads_splits) { return heads_splits >= 256 ? 4 : kMaxWaves; }
+// KV heads a workgroup takes (log2): the most (decode_most_heads) with which the workgroups fill seven eighths of the rounds
+// that they make over 256 compute units, or else what fills them best; every compute unit has one.  64 sequences of 20
+// heads of 64 over 1000 keys: 44.9 us in 320 workgroups of four heads, 40.7 in 1280 of one; 16 over 1500 keys in six splits
+// 29.2 in 1920 of one, 24.5 in 480 of four.
+__host__ __device__ constexpr int heads_together(int d, uint32_t heads_splits, uint32_t kv_heads) {
+  int best = 0, best_fill = -1;
+  for (int n = decode_most_heads(d, kv_heads); n >= 0 && best_fill < 14; n--) {
+    const uint32_t workgroups = heads_splits >> n;
+    if (n > 0 && workgroups < 256) continue;
+    // In sixteenths of the rounds' places; four rounds and more even out by themselves.
+    const int fill = workgroups >= 1024 ? 16 : (int)(workgroups * 16 / ((workgroups + 255) / 256 * 256));
+    if (fill > best_fill) best = n, best_fill = fill;
+  }
+  return best;
+}
 
 // What the kernel takes: AttnArgs without the fields a decoder step does not have.
 struct DecodeArgs {
@@ -108,110 +128,152 @@ __device__ __forceinline__ float sum_over(float x) {
 struct State {
   float m, l, acc[8];
 };
-// `a` takes in `b` (the merge of two key splits, L948-1014).
-__device__ __forceinline__ void merge(State &a, const State &b) {
-#pragma clang fp contract(off)  // the products and sums as written, wherever this is inlined
-  const float m = __builtin_fmaxf(a.m, b.m);
-  const float wa = __builtin_amdgcn_exp2f(a.m - m), wb = __builtin_amdgcn_exp2f(b.m - m);
-  a.m = m;
-  a.l = a.l * wa + b.l * wb;
-#pragma unroll
-  for (int j = 0; j < 8; j++) a.acc[j] = a.acc[j] * wa + b.acc[j] * wb;
+// `op` of x and of the lane STEP away (lane l <-> l ^ STEP); op is commutative.
+template <int STEP, typename Op>
+__device__ __forceinline__ float folded(float x, Op op) {
+  const uint32_t u = __float_as_uint(x);
+  if constexpr (STEP == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (STEP == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (STEP == 8) {
+    return op(x, moved<0x128>(x));  // row_ror:8
+  } else {
+    return op(x, __shfl_xor(x, STEP, 64));
+  }
 }
 
 // Partial states that another workgroup of the launch reads go past the L2s, each of which serves one XCD, and are read
-// the same way: stores and loads that are coherent over the device.
-__device__ __forceinline__ void put(float *p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ void put2(float *p, const f32x2 &x) {  // 8-byte aligned
-  __hip_atomic_store(reinterpret_cast<uint64_t *>(p), __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float got(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ f32x2 got2(const float *p) {  // 8-byte aligned
-  return __builtin_bit_cast(f32x2, __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT));
-}
+// the same way: stores and loads that are coherent over the device (the instructions' sc1 bit), 16 bytes a lane.
+struct Shared {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __amdgpu_buffer_rsrc_t rsrc;
+  static constexpr int kDevice = 16;
+  __device__ __forceinline__ void name(float *p, uint32_t bytes) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000);
+  }
+  __device__ __forceinline__ void put4(uint32_t at, const f32x4 &x) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rsrc, (int)at, 0, kDevice);
+  }
+  __device__ __forceinline__ void put2(uint32_t at, const f32x2 &x) const {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rsrc, (int)at, 0, kDevice);
+  }
+  __device__ __forceinline__ f32x4 got4(uint32_t at) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, 0, kDevice));
+  }
+  __device__ __forceinline__ f32x2 got2(uint32_t at) const {
+    return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)at, 0, kDevice));
+  }
+#endif
+};
 
 // Keys and values are read once a step, and by the next step the other layers' caches and the weights have been through
 // the chip.  Without the mark a step of 34 sequences over 570 cached keys is faster on one layer called back to back (32.2
 // -> 25.5 us with two layers' windows in turn), and slower over a model's (8 layers 30.5 -> 32.4, 16 layers 28.1 -> 30.3; 20 over
 // 440 keys 15.8 -> 17.2, 8 over 2000 24.0 -> 24.9).
-__device__ __forceinline__ u32x4 key_row(const uint16_t *p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+// The 16 bytes `off` past `base`, or zeros from `bytes` on.
+__device__ __forceinline__ u32x4 load16(const uint8_t *base, uint32_t bytes, uint32_t off) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int kReadOnce = 2;  // the instruction's nt bit
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base), 0, (int)bytes, 0x00020000);
+  return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, kReadOnce);
+#else
+  return u32x4{};
+#endif
+}
+
+// A value that every lane of a wave has, in a scalar register.
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// The b-th of an array of 32- or 64-bit integers, as it comes from memory.
+struct Integer {
+  int lo, hi;
+  bool wide;
+};
+__device__ __forceinline__ Integer ask(const void *p, int b, bool wide) {
+  const int *at = (const int *)p + (wide ? 2 * (int64_t)b : (int64_t)b);
+  return {at[0], at[wide ? 1 : 0], wide};
+}
+// The integer held in [0, most].
+__device__ __forceinline__ int held(const Integer &x, int most) {
+  int n = x.lo;
+  if (x.wide) n = x.hi < 0 ? 0 : (x.hi > 0 || x.lo < 0 ? 0x7fffffff : x.lo);
+  return uniform(n < 0 ? 0 : (n < most ? n : most));
 }
 
 // What a launch does with its splits: it has none; it leaves partial states for combine_kernel; the workgroup of a
 // (batch, KV head) that ends last merges them.
 enum { kWhole, kPartial, kMerged };
 
-// The workgroup's program for `nw` waves, for the kernels below to inline.
-template <int D, int R, bool F16, int MODE>
-__device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
+// The workgroup's program for `nw` waves (8 or 4) and 1 << hg_log2 heads, for the kernels below to inline.  ROOM: LDS for the
+// states of one head of eight waves, or of two.
+template <int D, int R, bool F16, int MODE, int ROOM>
+__device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, const int hg_log2) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // No contraction beyond the fused multiply-adds written out below: the library's kernel (its wave count a launch
   // argument) and a code object's (four waves, known to the compiler) are then the same arithmetic bit for bit.
 #pragma clang fp contract(off)
   constexpr int kWide = D == 48 ? 64 : D;
-  constexpr int LPK = kWide / 8;   // lanes a key row
-  constexpr int KPI = 64 / LPK;    // key rows a wave instruction
+  constexpr int LPK = kWide / 8;   // lanes a head's share of a key row
   constexpr int U = kAhead;  // the same for every R: a row's arithmetic does not depend on how many rows share the keys
-  __shared__ float merged[kMaxWaves][R][LPK][10];
+  __shared__ __attribute__((aligned(16))) float merged[ROOM * kMaxWaves * R * LPK * 10];
 
   constexpr bool SPLIT = MODE != kWhole;
-  const int wg = (int)__builtin_amdgcn_workgroup_id_x();
+  const uint32_t wg = __builtin_amdgcn_workgroup_id_x();
   const int tid = (int)__builtin_amdgcn_workitem_id_x();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int split = SPLIT ? wg % p.splits : 0;
-  const int unit = SPLIT ? wg / p.splits : wg;
-  const int b = unit / p.kv_heads;
-  const int kvh = unit - b * p.kv_heads;
-  const int pos = lane % LPK;   // which 16 bytes of a row
-  const int slot = lane / LPK;  // which row of a wave instruction
+  // A workgroup's heads lie side by side in a key row; neighbouring workgroups take neighbouring heads, then the splits.
+  const int hg = 1 << hg_log2, kpi = 64 / LPK >> hg_log2;  // heads, and key rows a wave instruction
+  const int span = LPK << hg_log2;                         // lanes a key row
+  const uint32_t groups = (uint32_t)p.kv_heads >> hg_log2;
+  const uint32_t of_heads = wg / groups;
+  const int group0 = (int)(wg - of_heads * groups);
+  const int b = SPLIT ? (int)(of_heads / (uint32_t)p.splits) : (int)of_heads;
+  const int split = SPLIT ? (int)of_heads - b * p.splits : 0;
+  const int unit = b * (int)groups + group0;
+  const int pos = lane % LPK;                       // which 16 bytes of a head
+  const int kvh = (group0 << hg_log2) + (lane / LPK & (hg - 1));
+  const int slot = lane / LPK >> hg_log2;           // which row of a wave instruction
   const bool pos_ok = 8 * pos < D;
 
-  // L533-536: len = min(key_lens[b], tk).
+  // The row's integers, asked for together: its length (L533-536: len = min(key_lens[b], tk)), where it lies in a cache
+  // (L544-550) and how many appended rows it sees.  One trip to memory for the three, so no load stands under a branch:
+  // what a call does not have is read from q and dropped.
   const int tk = p.tk;
-  int len = tk;
-  if (p.key_lens != nullptr) {
-    long long n = p.lens_i64 ? ((const long long *)p.key_lens)[b] : (long long)((const int *)p.key_lens)[b];
-    n = n < 0 ? 0 : n;
-    len = n < (long long)tk ? (int)n : tk;
-  }
-  // L609-612: a split takes an even share of the 64-key blocks below the length.
-  int k0 = 0, k1 = len;
-  if (SPLIT) {
-    const int n = (len + 63) / 64;
-    k0 = (int)((int64_t)n * split / p.splits) * 64;
-    k1 = min(len, (int)((int64_t)n * (split + 1) / p.splits) * 64);
-  }
-  // L544-550: a cache is read at the batch lane's row of it, from the launch's first head on.
-  int64_t kv_row = b;
-  int kv_col = kvh;
-  if (p.cached) {
-    if (p.row_map != nullptr) {
-      const long long x = p.row_map_i64 ? ((const long long *)p.row_map)[b] : (long long)((const int *)p.row_map)[b];
-      kv_row = x < 0 ? 0 : (x < p.cache_rows ? x : p.cache_rows - 1);
-    }
-    kv_col += p.kv_head_start;
-  }
-
+  const bool appends = p.cached && p.k_app != nullptr && (!SPLIT || split == p.splits - 1);
+  const bool has_lens = p.key_lens != nullptr, has_map = p.cached && p.row_map != nullptr;
+  const bool has_seen = appends && p.app_lens != nullptr;
+  Integer len_b = ask(has_lens ? p.key_lens : p.q, has_lens ? b : 0, p.lens_i64 != 0 && has_lens);
+  Integer row_b = ask(has_map ? p.row_map : p.q, has_map ? b : 0, p.row_map_i64 != 0 && has_map);
+  Integer seen_b = ask(has_seen ? p.app_lens : p.q, has_seen ? b : 0, p.app_lens_i64 != 0 && has_seen);
   // The rows: row r is token r % t of the group's head r / t (a grouped tile's order).
   const int rows = p.group * p.t;
+  // The output row of this lane's head's row r.
+  auto out_row = [&](int r, int kv_head) {
+    const int in_group = (r >= p.t) + (r >= 2 * p.t) + (r >= 3 * p.t);  // r / t: at most four rows
+    return ((int64_t)b * p.t + (r - in_group * p.t)) * p.heads + kv_head * p.group + in_group;
+  };
   uint32_t qf[R][4];
-  int64_t out_row[R];
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const int rr = min(r, rows - 1);
-    const int in_group = rr / p.t;
+    const int in_group = (rr >= p.t) + (rr >= 2 * p.t) + (rr >= 3 * p.t);
     const int q_row = rr - in_group * p.t;
     const int q_head = kvh * p.group + in_group;
-    out_row[r] = ((int64_t)b * p.t + q_row) * p.heads + q_head;
     const uint16_t *at = p.q + ((int64_t)b * p.t + q_row) * p.q_row_elems + (int64_t)q_head * D + 8 * pos;
     u32x4 x = {0, 0, 0, 0};
     if (pos_ok && r < rows) x = *reinterpret_cast<const u32x4 *>(at);
 #pragma unroll
     for (int i = 0; i < 4; i++) qf[r][i] = x[i];
   }
+
+  asm volatile("" : "+s"(len_b.lo), "+s"(len_b.hi), "+s"(row_b.lo), "+s"(row_b.hi), "+s"(seen_b.lo), "+s"(seen_b.hi));
+  const int len = has_lens ? held(len_b, tk) : tk;
+  const int kv_row = has_map ? held(row_b, p.cache_rows - 1) : b;
+  const int app_seen = !appends ? 0 : has_seen ? held(seen_b, p.app_rows) : p.app_rows;
 
   const float c_exp = p.scale * kLog2e;  // L619
   State st[R];
@@ -223,100 +285,146 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
     for (int j = 0; j < 8; j++) st[r].acc[j] = 0.0f;
   }
 
-  // Keys [from, to) of rows `row_elems` apart at kb / vb (this lane's 16 bytes of the first row), `mask` their
-  // visibility bytes or words (null: all visible).  A pass of the workgroup is nw * KPI rows; a lane works on U
-  // passes at a time and has the next U in flight meanwhile.  The workgroup starts `turn` such chunks into the
-  // range and wraps: the softmax does not care where it starts, and the memory does.  Rows of a cache are very
-  // often a power of two apart, and so are the batch rows; workgroups that all walk from key 0 then ask the same
-  // few memory channels for their rows at the same time (a [64, 512, 128, 64] cache read one layer's 32 heads at a
-  // time: 3.8 TB/s from key 0, 5.2 with the starts spread; rows 20 or 80 KiB apart stream the same either way).
-  auto stream = [&](const uint16_t *kb, const uint16_t *vb, int64_t row_elems, int from, int to, const void *mask,
-                    int mask_bytes, uint32_t turn) {
-    const int pass = nw * KPI;
-    struct Rows {
-      u32x4 k[U], v[U];
-      int seen[U];
-    };
-    auto load = [&](Rows &x, int key0) {
+  // What the workgroup reads: the appended rows (L739-755, L827-846), which the last split scores, the first app_lens[b] of
+  // them visible, from tensors of their own, and its chunks of the cached keys.  A pass is nw * kpi rows, a chunk U passes.
+  // The splits of a row take its chunks in turn (chunk c is split c % splits's), so that workgroups that run together
+  // read keys that lie together, and a workgroup starts some of its chunks in and wraps: the softmax does not care, and
+  // the memory does.  Rows of a cache are very often a power of two apart, and so are the batch rows; workgroups that
+  // all walk from key 0 then ask the same few memory channels for their rows at the same time.  Started by the cache row,
+  // not by who asks: a batch lane mapped to another cache row reads it as that row's own lane would.
+  static_assert(U == 2 && kMaxWaves == 8, "a chunk's rows are a power of two");
+  const int pass = nw * kpi, chunk = U * pass;
+  const int chunk_log2 = __builtin_ctz(U * 64 / LPK) + (nw == kMaxWaves ? 3 : 2) - hg_log2;
+  const uint32_t of_row = ((uint32_t)len + (uint32_t)chunk - 1) >> chunk_log2, turns = SPLIT ? (uint32_t)p.splits : 1u;
+  const int chunks = of_row > (uint32_t)split ? (int)((of_row - (uint32_t)split + turns - 1) / turns) : 0;
+  const int first = (int)__umulhi((uint32_t)kv_row * 0x9e3779b1u, (uint32_t)chunks);  // a fraction that rows differ in
+  const uint32_t in_row = (uint32_t)((lane / LPK & (hg - 1)) * (D * 2) + 16 * pos);
+  const void *mask = nullptr;  // visibility bytes or words of the cached keys
+  if (p.key_mask != nullptr) mask = (const uint8_t *)p.key_mask + (int64_t)b * tk * p.mask_bytes;
+
+  struct Rows {
+    u32x4 k[U], v[U];
+    int there[U];  // rows of a pass's wave instruction that are there: lanes past them land zeros
+    int seen[U];   // of a call with a key mask: this lane's element of it
+  };
+  // Rows of one tensor each, `row_bytes` apart, keys [0, to).
+  struct Source {
+    const uint8_t *k, *v;
+    uint32_t row_bytes, off;  // off: of this lane's 16 bytes from a wave instruction's first row
+    int to;
+  };
+  auto source = [&](const uint16_t *k, const uint16_t *v, int64_t at, uint32_t row_bytes, int to) {
+    return Source{(const uint8_t *)(k + at), (const uint8_t *)(v + at), row_bytes,
+                  pos_ok ? (uint32_t)slot * row_bytes + in_row : 0xfffffff0u, to};
+  };
+  // The rows of the chunk that starts at key `from`, asked for.  A wave instruction's rows are one descriptor, bounded at the
+  // rows that are there: no load stands under a branch, so the compiler knows how many are out and waits for the ones it
+  // needs alone.  (With a branch a load it waited for all of them, the chunk just asked for among them, before it
+  // worked on the one before: with the heads together 16 sequences of 8 KV heads of 128 over 525 to 2100 keys 29.1 -> 24.6
+  // us, over 2100 keys each 40.8 -> 28.9.)
+  auto load = [&](auto masked, Rows &x, const Source &y, int from) {
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int key = key0 + u * pass;
-        const bool there = key < to;
-        x.k[u] = u32x4{0, 0, 0, 0};
-        x.v[u] = u32x4{0, 0, 0, 0};
-        x.seen[u] = there ? 1 : 0;
-        if (there && pos_ok) {
-          x.k[u] = key_row(kb + (int64_t)key * row_elems);
-          x.v[u] = key_row(vb + (int64_t)key * row_elems);
-        }
-        if (there && mask != nullptr)
-          x.seen[u] = mask_bytes == 1 ? (int)((const uint8_t *)mask)[key] : ((const int *)mask)[key];
+    for (int u = 0; u < U; u++) {
+      const int key = from + u * pass + wave * kpi;
+      int there = max(y.to - key, 0);
+      asm("" : "+s"(there));  // on the scalar unit: the compiler makes a vector instruction of the two
+      there = min(there, kpi);
+      const uint64_t at = (uint64_t)(uint32_t)key * y.row_bytes;
+      x.there[u] = there;
+      x.k[u] = load16(y.k + at, (uint32_t)there * y.row_bytes, y.off);
+      x.v[u] = load16(y.v + at, (uint32_t)there * y.row_bytes, y.off);
+      if constexpr (decltype(masked)::value) {
+        x.seen[u] = 0;
+        if (slot < there)
+          x.seen[u] = p.mask_bytes == 1 ? (int)((const uint8_t *)mask)[key + slot] : ((const int *)mask)[key + slot];
       }
-    };
-    // The softmax and the second product of the U passes in `x`.
-    auto work = [&](Rows &x) {
-      float e[U][R];
+    }
+  };
+  // The softmax and the second product of the U passes in `x`.
+  auto work = [&](auto masked, Rows &x) {
+    float e[U][R];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const bool seen = x.seen[u] != 0;
-        if (mask != nullptr && !seen) x.v[u] = u32x4{0, 0, 0, 0};  // a hidden row weighs nothing, whatever it holds
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          float s = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 4; i++) s = dot2<F16>(x.k[u][i], qf[r][i], s);
-          s = sum_over<LPK>(s);
-          e[u][r] = seen ? s * c_exp : -__builtin_inff();
-        }
+    for (int u = 0; u < U; u++) {
+      bool seen = slot < x.there[u];
+      if constexpr (decltype(masked)::value) {
+        seen = x.seen[u] != 0;
+        if (!seen) x.v[u] = u32x4{0, 0, 0, 0};  // a hidden row weighs nothing, whatever it holds
       }
 #pragma unroll
       for (int r = 0; r < R; r++) {
-        float m = st[r].m;
+        float s = 0.0f;
 #pragma unroll
-        for (int u = 0; u < U; u++) m = __builtin_fmaxf(m, e[u][r]);
-        const float corr = __builtin_amdgcn_exp2f(st[r].m - m);
-        st[r].m = m;
-        st[r].l *= corr;
+        for (int i = 0; i < 4; i++) s = dot2<F16>(x.k[u][i], qf[r][i], s);
+        s = sum_over<LPK>(s);
+        e[u][r] = seen ? s * c_exp : -__builtin_inff();
+      }
+    }
 #pragma unroll
-        for (int j = 0; j < 8; j++) st[r].acc[j] *= corr;
-        float pr[U];
+    for (int r = 0; r < R; r++) {
+      float m = st[r].m;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-          pr[u] = __builtin_amdgcn_exp2f(e[u][r] - m);
-          st[r].l += pr[u];
-        }
+      for (int u = 0; u < U; u++) m = __builtin_fmaxf(m, e[u][r]);
+      const float corr = __builtin_amdgcn_exp2f(st[r].m - m);
+      st[r].m = m;
+      st[r].l *= corr;
 #pragma unroll
-        for (int u = 0; u < U; u += 2) {
-          const float held[2] = {pr[u], pr[u + 1]};
+      for (int j = 0; j < 8; j++) st[r].acc[j] *= corr;
+      float pr[U];
 #pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const f32x2 a = unpack2<F16>(x.v[u][i]), c = unpack2<F16>(x.v[u + 1][i]);
-            st[r].acc[2 * i] = __builtin_fmaf(held[0], a[0], st[r].acc[2 * i]);
-            st[r].acc[2 * i + 1] = __builtin_fmaf(held[0], a[1], st[r].acc[2 * i + 1]);
-            st[r].acc[2 * i] = __builtin_fmaf(held[1], c[0], st[r].acc[2 * i]);
-            st[r].acc[2 * i + 1] = __builtin_fmaf(held[1], c[1], st[r].acc[2 * i + 1]);
-          }
+      for (int u = 0; u < U; u++) {
+        pr[u] = __builtin_amdgcn_exp2f(e[u][r] - m);
+        st[r].l += pr[u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u += 2) {
+        const float held[2] = {pr[u], pr[u + 1]};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const f32x2 a = unpack2<F16>(x.v[u][i]), c = unpack2<F16>(x.v[u + 1][i]);
+          st[r].acc[2 * i] = __builtin_fmaf(held[0], a[0], st[r].acc[2 * i]);
+          st[r].acc[2 * i + 1] = __builtin_fmaf(held[0], a[1], st[r].acc[2 * i + 1]);
+          st[r].acc[2 * i] = __builtin_fmaf(held[1], c[0], st[r].acc[2 * i]);
+          st[r].acc[2 * i + 1] = __builtin_fmaf(held[1], c[1], st[r].acc[2 * i + 1]);
         }
       }
-    };
-    // Two sets of rows take turns: one is worked on while the other is on its way.
-    if (from + wave * KPI >= to) return;  // no chunk holds a row of this wave's
-    const int chunk = U * pass, chunks = (to - from + chunk - 1) / chunk;
-    const int first = (int)(turn % (uint32_t)chunks);
-    // This lane's first row of the i-th chunk the workgroup takes; past the last chunk, a row that is not there.
-    auto row_of = [&](int i) {
-      if (i >= chunks) return to;
+    }
+  };
+  // Two sets of rows take turns: one is worked on while the other is on its way.  A set past the last chunk has no rows.
+  auto stream = [&](auto masked) {
+    const int kv_col = (group0 << hg_log2) + (p.cached ? p.kv_head_start : 0);
+    const Source cache = source(p.k, p.v, (int64_t)kv_row * tk * p.kv_row_elems + (int64_t)kv_col * D,
+                                (uint32_t)p.kv_row_elems * 2, len);
+    auto chunk_of = [&](int i) {
       int c = first + i;
-      if (c >= chunks) c -= chunks;
-      return from + c * chunk + wave * KPI + slot;
+      c = c >= chunks ? c - chunks : c;
+      return i < chunks ? (split + c * (int)turns) * chunk : len;
     };
     Rows one, two;
-    load(one, row_of(0));
+    const Source app = source(p.k_app, p.v_app, ((int64_t)b * p.app_rows * p.kv_heads + (group0 << hg_log2)) * D,
+                              (uint32_t)p.kv_heads * (D * 2), app_seen);
+    int app_from = 0;
+    for (; app_from + chunk < app_seen; app_from += chunk) {
+      load(std::false_type(), two, app, app_from);
+      work(std::false_type(), two);
+    }
+    if (app_from < app_seen) {
+      load(std::false_type(), two, app, app_from);
+      load(masked, one, cache, chunk_of(0));  // under way with the last of them
+      __builtin_amdgcn_sched_barrier(0);
+      work(std::false_type(), two);
+    } else {
+      load(masked, one, cache, chunk_of(0));
+    }
     for (int i = 0; i < chunks; i += 2) {
-      load(two, row_of(i + 1));
-      work(one);
-      load(one, row_of(i + 2));
-      if (i + 1 < chunks) work(two);
+      load(masked, two, cache, chunk_of(i + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      work(masked, one);
+      if (i + 1 >= chunks) break;
+      __builtin_amdgcn_sched_barrier(0);
+      load(masked, one, cache, chunk_of(i + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      work(masked, two);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -331,94 +439,114 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
   const bool counts = MODE == kMerged && tid == 0;
   uint64_t found = 0;
   if (counts) found = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  {
-    const int64_t at = (kv_row * tk) * p.kv_row_elems + (int64_t)kv_col * D + 8 * pos;
-    const void *mask = nullptr;
-    if (p.key_mask != nullptr) mask = (const uint8_t *)p.key_mask + (int64_t)b * tk * p.mask_bytes;
-    // Turned by where the keys lie (the cache row, and the split's share of it), not by who asks: a batch lane
-    // mapped to another cache row reads it as that row's own lane would.  The heads of a row stay in step:
-    // their pieces of a key row lie side by side.
-    stream(p.k + at, p.v + at, p.kv_row_elems, k0, k1, mask, p.mask_bytes, (uint32_t)kv_row * 7u + (uint32_t)split * 3u);
-  }
+  if (mask != nullptr)
+    stream(std::true_type());
+  else
+    stream(std::false_type());
   if (counts && (found >> kCountBits != p.tag || (int)(found & ((1u << kCountBits) - 1)) >= p.splits))
     __hip_atomic_compare_exchange_strong(arrivals, &found, p.tag << kCountBits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
-  // The appended rows (L739-755, L827-846): scored by the last split after the cached keys, the first
-  // app_lens[b] of them visible, from tensors of their own.
-  if (p.cached && p.k_app != nullptr && (!SPLIT || split == p.splits - 1)) {
-    int seen = p.app_rows;
-    if (p.app_lens != nullptr) {
-      const long long n = p.app_lens_i64 ? ((const long long *)p.app_lens)[b] : (long long)((const int *)p.app_lens)[b];
-      seen = (int)(n < 0 ? 0 : (n < seen ? n : seen));
-    }
-    const int64_t at = ((int64_t)b * p.app_rows * p.kv_heads + kvh) * D + 8 * pos;
-    stream(p.k_app + at, p.v_app + at, (int64_t)p.kv_heads * D, 0, seen, nullptr, 1, 0u);
-  }
-
-  // The places of a wave that share output columns (lanes LPK apart) merge, then the waves.
+  // The places of a wave that share output columns (lanes `span` apart) merge (L948-1014): the greatest maximum, what each
+  // state weighs under it, the sums.
 #pragma unroll
   for (int r = 0; r < R; r++) {
+    auto over_places = [&](float x, auto op) {
+      if (LPK <= 4 && 4 >= span) x = folded<4>(x, op);
+      if (LPK <= 8 && 8 >= span) x = folded<8>(x, op);
+      if (LPK <= 16 && 16 >= span) x = folded<16>(x, op);
+      if (32 >= span) x = folded<32>(x, op);
+      return x;
+    };
+    const float m = over_places(st[r].m, [](float x, float y) { return __builtin_fmaxf(x, y); });
+    const float w = __builtin_amdgcn_exp2f(st[r].m - m);
+    auto sum = [](float x, float y) { return x + y; };
+    st[r].m = m;
+    st[r].l = over_places(st[r].l * w, sum);
 #pragma unroll
-    for (int step = LPK; step < 64; step <<= 1) {
-      State other;
-      other.m = __shfl_xor(st[r].m, step, 64);
-      other.l = __shfl_xor(st[r].l, step, 64);
-#pragma unroll
-      for (int j = 0; j < 8; j++) other.acc[j] = __shfl_xor(st[r].acc[j], step, 64);
-      merge(st[r], other);
-    }
-    if (slot == 0) {
-      float *at = merged[wave][r][pos];
-      at[0] = st[r].m;
-      at[1] = st[r].l;
-#pragma unroll
-      for (int j = 0; j < 8; j++) at[2 + j] = st[r].acc[j];
-    }
+    for (int j = 0; j < 8; j++) st[r].acc[j] = over_places(st[r].acc[j] * w, sum);
   }
-  __syncthreads();
-  if (wave != 0) return;
-  const bool mine = slot == 0 && pos_ok;
+  // Then the waves do, through LDS, in the same way: the first wave's lanes take a (row, lane of a key row) each and ask for
+  // all waves' states of it together.  (One state after the other, each read behind the sums of the one before: 0.17 us a
+  // state, 1.9 us more for eight waves of two rows.)
   const int64_t states = (int64_t)p.batch * p.t * p.heads;  // of a split
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    if (r >= rows || !mine) break;
-    State all = st[r];
-    for (int w = 1; w < nw; w++) {
-      State other;
-      const float *at = merged[w][r][pos];
-      other.m = at[0];
-      other.l = at[1];
-#pragma unroll
-      for (int j = 0; j < 8; j++) other.acc[j] = at[2 + j];
-      merge(all, other);
-    }
-    if (MODE == kMerged) {
-      const int64_t at = split * states + out_row[r];
-      if (pos == 0) {
-        put(p.m_part + at, all.m);
-        put(p.l_part + at, all.l);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) put2(p.o_part + at * D + 8 * pos + j, f32x2{all.acc[j], all.acc[j + 1]});
-    } else if (SPLIT) {
-      // L899-921: the accumulator as it stands, the maximum in the exponent's units, the sum.
-      const int64_t at = split * states + out_row[r];
-      if (pos == 0) {
-        p.m_part[at] = all.m;
-        p.l_part[at] = all.l;
-      }
-      f32x4 *to = reinterpret_cast<f32x4 *>(p.o_part + at * D + 8 * pos);
-      to[0] = f32x4{all.acc[0], all.acc[1], all.acc[2], all.acc[3]};
-      to[1] = f32x4{all.acc[4], all.acc[5], all.acc[6], all.acc[7]};
-    } else {
-      // L892-898: out = o / (l == 0 ? 1 : l).
-      const float inv = 1.0f / (all.l == 0.0f ? 1.0f : all.l);
-      u32x4 out;
-#pragma unroll
-      for (int i = 0; i < 4; i++) out[i] = pack2<F16>(all.acc[2 * i] * inv, all.acc[2 * i + 1] * inv);
-      *reinterpret_cast<u32x4 *>(p.o + out_row[r] * D + 8 * pos) = out;
-    }
+  // A merging launch's states lie a unit together: [unit][split][row of the unit's heads][D], then their (m, l).
+  const int unit_rows = rows << hg_log2;
+  Shared shared_o, shared_ml;
+  if (MODE == kMerged) {
+    const uint32_t of_unit = (uint32_t)(p.splits * unit_rows);
+    shared_o.name(p.o_part + (int64_t)unit * of_unit * D, of_unit * D * 4);
+    shared_ml.name(p.m_part + (int64_t)unit * of_unit * 2, of_unit * 8);
   }
+  auto merge_waves = [&](auto waves) {
+    constexpr int W = decltype(waves)::value;
+    constexpr int kRoom = ROOM * LPK * kMaxWaves / W;  // lanes of a key row that LDS holds the states of
+    const int held_log2 = min(__builtin_ctz(kRoom), __builtin_ctz(LPK) + hg_log2), held = 1 << held_log2;
+    for (int from = 0; from < span; from += held) {
+      if (from > 0) __syncthreads();
+      if (lane >= from && lane < from + held) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          f32x2 *at = reinterpret_cast<f32x2 *>(merged + (((wave * R + r) << held_log2) + lane - from) * 10);
+          at[0] = f32x2{st[r].m, st[r].l};
+#pragma unroll
+          for (int j = 0; j < 4; j++) at[1 + j] = f32x2{st[r].acc[2 * j], st[r].acc[2 * j + 1]};
+        }
+      }
+      __syncthreads();
+      if (wave != 0) continue;
+      for (int item = lane; item < R << held_log2; item += 64) {
+        const int r = item >> held_log2, of_row = from + (item & (held - 1));
+        f32x2 x[W][5];
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+          const f32x2 *at = reinterpret_cast<const f32x2 *>(merged + ((w * R << held_log2) + item) * 10);
+#pragma unroll
+          for (int j = 0; j < 5; j++) x[w][j] = at[j];
+        }
+        float m = x[0][0][0];
+#pragma unroll
+        for (int w = 1; w < W; w++) m = __builtin_fmaxf(m, x[w][0][0]);
+        float l = 0.0f, acc[8] = {};
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+          const float weight = __builtin_amdgcn_exp2f(x[w][0][0] - m);
+          l += x[w][0][1] * weight;
+#pragma unroll
+          for (int j = 0; j < 8; j++) acc[j] += x[w][1 + j / 2][j & 1] * weight;
+        }
+        const int head = of_row / LPK, at_pos = of_row % LPK;
+        if (r >= rows || 8 * at_pos >= D) continue;
+        const int64_t orow = out_row(r, (group0 << hg_log2) + head);
+        if (MODE == kMerged) {
+          const uint32_t at = (uint32_t)(split * unit_rows + head * rows + r);
+          if (at_pos == 0) shared_ml.put2(at * 8, f32x2{m, l});
+          shared_o.put4((at * D + 8 * at_pos) * 4, f32x4{acc[0], acc[1], acc[2], acc[3]});
+          shared_o.put4((at * D + 8 * at_pos + 4) * 4, f32x4{acc[4], acc[5], acc[6], acc[7]});
+        } else if (SPLIT) {
+          // L899-921: the accumulator as it stands, the maximum in the exponent's units, the sum.
+          const int64_t at = split * states + orow;
+          if (at_pos == 0) {
+            p.m_part[at] = m;
+            p.l_part[at] = l;
+          }
+          f32x4 *to = reinterpret_cast<f32x4 *>(p.o_part + at * D + 8 * at_pos);
+          to[0] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+          to[1] = f32x4{acc[4], acc[5], acc[6], acc[7]};
+        } else {
+          // L892-898: out = o / (l == 0 ? 1 : l).
+          const float inv = 1.0f / (l == 0.0f ? 1.0f : l);
+          u32x4 out;
+#pragma unroll
+          for (int i = 0; i < 4; i++) out[i] = pack2<F16>(acc[2 * i] * inv, acc[2 * i + 1] * inv);
+          *reinterpret_cast<u32x4 *>(p.o + orow * D + 8 * at_pos) = out;
+        }
+      }
+    }
+  };
+  if (nw == kMaxWaves)
+    merge_waves(std::integral_constant<int, kMaxWaves>());
+  else
+    merge_waves(std::integral_constant<int, kMaxWaves / 2>());
   if (MODE != kMerged) return;
   // ---- the merge.  This wave's states are where every workgroup sees them before it counts itself in: they were stored
   // past the L2s, and vmcnt is at zero when the memory behind those has taken them all.  The workgroup that counts itself
@@ -428,66 +556,73 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw) {
   // 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.  In a graph's replay, where
   // a launch costs no host time: one over 8000 22.3 -> 16.7, two over 4700 20.8 -> 17.7, four over 8100 36.1 -> 33.6, sixteen
   // over 1500 26.3 -> 26.6.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   const int splits = p.splits;
-  uint32_t before = 0;
-  if (lane == 0)
-    before = (uint32_t)__hip_atomic_fetch_add(arrivals, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before) & ((1u << kCountBits) - 1);
-  if ((int)before != splits - 1) return;
-  asm volatile("" ::: "memory");  // the states are read from here on
-  constexpr int kLanes = D / 4, kBatch = 8;
-  for (int c = lane; c < rows * kLanes; c += 64) {
-    const int r = c / kLanes, chunk = c - r * kLanes;
-    // out_row[r] without an index into registers: a row is (head of the group, token).
-    const int in_group = r / p.t;
-    const int64_t orow = ((int64_t)b * p.t + (r - in_group * p.t)) * p.heads + kvh * p.group + in_group;
-    struct States {
-      float m[kBatch], l[kBatch];
-      f32x2 lo[kBatch], hi[kBatch];
-    };
-    auto ask = [&](States &x, int from) {
-#pragma unroll
-      for (int i = 0; i < kBatch; i++) {
-        const int64_t at = (int64_t)min(from + i, splits - 1) * states + orow;
-        x.m[i] = got(p.m_part + at);
-        x.l[i] = got(p.l_part + at);
-        x.lo[i] = got2(p.o_part + at * D + 4 * chunk);
-        x.hi[i] = got2(p.o_part + at * D + 4 * chunk + 2);
-      }
-    };
-    States x;
-    ask(x, 0);
-    float m = x.m[0];
-#pragma unroll
-    for (int i = 1; i < kBatch; i++) m = __builtin_fmaxf(m, x.m[i]);
-    for (int from = kBatch; from < splits; from += kBatch) {
-      float y[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; i++) y[i] = got(p.m_part + (int64_t)min(from + i, splits - 1) * states + orow);
-#pragma unroll
-      for (int i = 0; i < kBatch; i++) m = __builtin_fmaxf(m, y[i]);
+  if (wave == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t before = 0;
+    if (lane == 0) {
+      before = (uint32_t)__hip_atomic_fetch_add(arrivals, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      merged[0] = __uint_as_float(before & ((1u << kCountBits) - 1));
     }
-    float l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int from = 0; from < splits; from += kBatch) {
-      if (from > 0) ask(x, from);
-#pragma unroll
-      for (int i = 0; i < kBatch; i++) {
-        if (from + i >= splits) break;
-        const float w = __builtin_amdgcn_exp2f(x.m[i] - m);
-        const float part[4] = {x.lo[i][0] * w, x.lo[i][1] * w, x.hi[i][0] * w, x.hi[i][1] * w};
-        const float lw = x.l[i] * w;
-        const bool none = from + i == 0;
-        l = none ? lw : l + lw;
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[j] = none ? part[j] : acc[j] + part[j];
-      }
-    }
-    const float ll = l == 0.0f ? 1.0f : l;
-    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-    const u32x2 out = {pack2<F16>(acc[0] / ll, acc[1] / ll), pack2<F16>(acc[2] / ll, acc[3] / ll)};
-    *reinterpret_cast<u32x2 *>(p.o + orow * D + 4 * chunk) = out;
   }
+  __syncthreads();
+  if (uniform((int)__float_as_uint(merged[0])) != splits - 1) return;
+  asm volatile("" ::: "memory");  // the states are read from here on
+  constexpr int kLanes = D / 4;
+  // States are asked for `batch` together, the first ones with the maxima of all: two trips to memory for 32 splits.
+  auto merge_splits = [&](auto batch) {
+    constexpr int kBatch = decltype(batch)::value;
+    for (int c = tid; c < hg * rows * kLanes; c += nw * 64) {
+      const int of_group = c / kLanes, chunk = c - of_group * kLanes;  // a row of one of the heads, four of its columns
+      const int in_heads = (int)((uint32_t)of_group / (uint32_t)rows);
+      const int64_t orow = out_row(of_group - in_heads * rows, (group0 << hg_log2) + in_heads);
+      f32x2 ml[kBatch];
+      f32x4 part[kBatch];
+      auto state = [&](int i) { return (uint32_t)(min(i, splits - 1) * unit_rows + of_group); };
+      auto ask_states = [&](int from) {
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) {
+          ml[i] = shared_ml.got2(state(from + i) * 8);
+          part[i] = shared_o.got4((state(from + i) * D + 4 * chunk) * 4);
+        }
+      };
+      ask_states(0);
+      float later = kNoKey;  // the greatest of the maxima past the first states
+      for (int from = kBatch; from < splits; from += kBatch) {
+        float y[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) y[i] = shared_ml.got2(state(from + i) * 8)[0];
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) later = __builtin_fmaxf(later, y[i]);
+      }
+      float m = later;
+#pragma unroll
+      for (int i = 0; i < kBatch; i++) m = __builtin_fmaxf(m, ml[i][0]);
+      float l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int from = 0; from < splits; from += kBatch) {
+        if (from > 0) ask_states(from);
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) {
+          // No branch: the loads would move into it, one trip after the other.
+          const bool none = from + i == 0, there = from + i < splits;
+          const float w = __builtin_amdgcn_exp2f(ml[i][0] - m);
+          const float lw = ml[i][1] * w;
+          l = none ? lw : (there ? l + lw : l);
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[j] = none ? part[i][j] * w : (there ? acc[j] + part[i][j] * w : acc[j]);
+        }
+      }
+      const float ll = l == 0.0f ? 1.0f : l;
+      const u32x2 out = {pack2<F16>(acc[0] / ll, acc[1] / ll), pack2<F16>(acc[2] / ll, acc[3] / ll)};
+      *reinterpret_cast<u32x2 *>(p.o + orow * D + 4 * chunk) = out;
+    }
+  };
+  if (splits <= 4)
+    merge_splits(std::integral_constant<int, 4>());
+  else if (splits <= 8)
+    merge_splits(std::integral_constant<int, 8>());
+  else
+    merge_splits(std::integral_constant<int, 16>());
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
@@ -505,7 +640,7 @@ struct Packed {
   uint64_t tag : 64 - kCountBits, app_rows : 7;
   uint64_t splits : 26, kv_row_heads : 19, kv_heads : 16, mask : 1, wide_keys : 1, packed_rows : 1;
   uint32_t batch : 26, group_less_one : 2, t_less_one : 2, row_map_i64 : 1, app_lens_i64 : 1;
-  int32_t tk, cache_rows;
+  uint32_t tk : 31, heads_lo : 1, cache_rows : 31, heads_hi : 1;  // heads: heads_together's two bits
   float scale;
 };
 static_assert(sizeof(Packed) <= 112 && kDecodeRows <= 4, "the record's size, the group's and the tokens' two bits");
@@ -527,16 +662,17 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) 
   const int64_t states = (int64_t)p.splits * p.batch * p.t * p.heads;
   p.o_part = a.states, p.m_part = a.states + states * D, p.l_part = p.m_part + states;
   p.arrivals = reinterpret_cast<uint64_t *>(p.l_part + states), p.tag = a.tag;
-  decode_body<D, R, F16, MODE>(p, decode_waves((int64_t)p.batch * p.kv_heads * p.splits));
+  const uint32_t heads_splits = (uint32_t)p.batch * (uint32_t)p.kv_heads * (uint32_t)p.splits;  // below 2^31
+  decode_body<D, R, F16, MODE, D == 48 || D <= 64 ? 2 : 1>(p, decode_waves(heads_splits), a.heads_lo | a.heads_hi << 1);
 #endif
 }
 
 template <int D, int R, bool F16>
 hipError_t launch_r(const Packed &p, bool merged, hipStream_t stream) {
-  const int64_t grid = (int64_t)p.batch * p.kv_heads * p.splits;
-  if (grid == 0) return hipSuccess;
-  if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const uint32_t threads = (uint32_t)decode_waves(grid) * 64;
+  const int64_t heads_splits = (int64_t)p.batch * p.kv_heads * p.splits;
+  if (heads_splits == 0) return hipSuccess;
+  const uint32_t threads = (uint32_t)decode_waves((uint32_t)heads_splits) * 64;
+  const int64_t grid = heads_splits >> (p.heads_lo | p.heads_hi << 1);
   auto run = [&](auto mode) {
     return Launch<decode_kernel<D, R, F16, decltype(mode)::value>>::run(grid, threads, 0, 0, stream, p);
   };
@@ -601,7 +737,7 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
   if (a.cached) {
     p.row_map = a.row_map;
     p.row_map_i64 = a.row_map_i64 != 0;
-    p.cache_rows = a.cache_rows;
+    p.cache_rows = (uint32_t)a.cache_rows;
     p.k_app = (const uint16_t *)a.k_app;
     p.v_app = (const uint16_t *)a.v_app;
     p.app_rows = (uint64_t)a.app_rows;
@@ -609,7 +745,7 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.app_lens_i64 = a.app_lens_i64 != 0;
   }
   p.states = a.o_part;
-  p.tk = a.tk;
+  p.tk = (uint32_t)a.tk;
   p.batch = (uint32_t)a.batch;
   p.kv_row_heads = (uint64_t)(kv_row / a.d);
   p.scale = a.scale;
@@ -618,6 +754,11 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
   p.group_less_one = (uint32_t)(a.heads / a.kv_heads - 1);
   p.t_less_one = (uint32_t)(a.t - 1);
   p.packed_rows = packed_rows;
+  const int64_t heads_splits = (int64_t)a.batch * a.kv_heads * splits;
+  if (heads_splits > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  const int together = heads_together(a.d, (uint32_t)heads_splits, (uint32_t)a.kv_heads);
+  p.heads_lo = (uint32_t)together & 1;
+  p.heads_hi = (uint32_t)together >> 1;
   const int rows = a.heads / a.kv_heads * a.t;
   const bool merged = splits > 1 && a.merges;
   if (merged && splits > kMostMergedSplits) return hipErrorInvalidValue;
@@ -668,7 +809,11 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
     p.splits = (S) && splits > 1 ? splits : 1, p.cached = cached, p.kv_head_start = kv_head_start;                    \
     p.cache_rows = cache_rows, p.app_rows = app_rows, p.scale = __builtin_bit_cast(float, scale_bits);                \
     p.arrivals = nullptr, p.tag = 0;                                                                                  \
-    svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole>(p, 4);                                  \
+    const uint32_t heads_splits = (uint32_t)batch * (uint32_t)kv_heads * (uint32_t)p.splits;                          \
+    const int hg_log2 = svodk::heads_together(D, heads_splits, kv_heads);                                            \
+    if (__builtin_amdgcn_workgroup_id_x() >= heads_splits >> hg_log2) return; /* launch: a (batch, KV head, split) */ \
+    svodk::decode_body<D, R, F16, (S) != 0 ? svodk::kPartial : svodk::kWhole, 1>(                                        \
+        p, 4, hg_log2);                                                                                               \
   }
 #define SVODK_DECODE_ROWS_OF(D, T, F16, S) \
   SVODK_DECODE_ENTRY(D, 1, T, F16, S) SVODK_DECODE_ENTRY(D, 2, T, F16, S) SVODK_DECODE_ENTRY(D, 4, T, F16, S)

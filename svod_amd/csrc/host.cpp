@@ -331,8 +331,11 @@ struct Workspace {
     if (lent == Py_None) {
       int64_t need = abi.attention_workspace(&q, &k, &a);
       if (need <= 0) return;
-      // The words with which a decoder step merges its own splits (svodk.h).
-      need += 128 * (a.batch_live > 0 ? a.batch_live : q.shape[0]) * (a.cache != nullptr ? a.cache->kv_heads : k.shape[2]);
+      // Twice that for a decoder step that names no count, which may take more splits then, and the words with which it merges
+      // them (svodk.h).
+      const int64_t kv_heads = a.cache != nullptr ? a.cache->kv_heads : k.shape[2];
+      if (a.splits <= 0 && q.shape[1] * q.shape[2] <= 4 * kv_heads) need *= 2;
+      need += 128 * (a.batch_live > 0 ? a.batch_live : q.shape[0]) * kv_heads;
       own = allocate(fresh, {need}, at::kByte, like);
       if (own == nullptr) throw Raised();
       lent = own;

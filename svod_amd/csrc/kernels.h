@@ -169,6 +169,13 @@ bool attention_decodes(const AttnArgs &a, int32_t limit);
 void attention_decode_rows(int32_t rows);
 int32_t attention_decode_limit();
 hipError_t launch_decode(const AttnArgs &a, hipStream_t stream);
+// The most KV heads (log2) a workgroup of the decoder step's kernel takes: as many as make 512 bytes of a key row, four at
+// most, where they divide the heads.
+constexpr int decode_most_heads(int32_t d, uint32_t kv_heads) {
+  int n = 0;
+  while ((d == 48 ? 64 : d) << (n + 1) <= 256 && n < 2 && kv_heads % (2u << n) == 0) n++;
+  return n;
+}
 // What a decoder step that merges its own splits, kMostMergedSplits at most, needs behind the partial states: a word a
 // (batch, KV head), on a line of its own (16 sequences of 8 KV heads in 4 splits: 28.9 us, 29.5 with 16 words a line).
 constexpr int kMostMergedSplits = 64;

@@ -326,6 +326,27 @@ int svodk_plan_heads(int32_t has_target, const int32_t *dtypes, int32_t n_dtypes
   return plan_heads(has_target != 0, dtypes, n_dtypes, x_dims, x_rank, head_dim);
 }
 
+// The key splits of a decoder step whose caller names none and lends room for them: as many as make one round of
+// workgroups over the part's 256 compute units, or two rounds where one would not fill them, at most twice `rule`, the
+// count that split_count answers (and svodk_attention_workspace counts with).  A round that is not full costs more than
+// its workgroups save: 16 sequences of 8 KV heads of 128 over 2100 keys take 28.3 us in 256 workgroups (4 splits), 31.6 in
+// 384, 30.3 in 512, 33 in 768; of 20 heads of 64 over 1500 keys 25.1 in 480 workgroups of two heads (3 splits), 24.2 in 480 of
+// four (6 splits), 27.5 in 640.  More than sixteen splits a merge takes a trip to memory more for: there a workgroup
+// rather takes fewer heads (one sequence over 8000 keys, 8 heads of 128: 12.8 us in 32 splits of one head, 16.4 in 64 of
+// two).  Below eight key blocks a merge costs what it saves (16 sequences over 400 keys 10.4 unsplit, 10.7 in 4 splits;
+// over 570 keys 22.8 and 20.1 in 3), and a split has at least 16 KiB of keys a head.
+static int decode_split_count(int64_t batch, int64_t kv_heads, int64_t d, int64_t tk, int rule) {
+  const int64_t blocks = (tk + 63) / 64, units = kv_heads * batch, fits = std::min<int64_t>(blocks, blocks * d / 128);
+  if (units <= 0 || blocks < 8) return 1;
+  int64_t n = 1;
+  for (int h = svodk::decode_most_heads((int32_t)d, (uint32_t)kv_heads); h >= 0; h--) {
+    const int64_t one = (256 << h) / units, two = (512 << h) / units;
+    n = one * units >= (248 << h) || two > 16 ? one : two;
+    if (n <= 16) break;
+  }
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(n, 64), std::min<int64_t>(fits, 2 * rule)));
+}
+
 // split_ranked of tk/src/ops/attention.rs:405-410 for this library's one tile shape: a named
 // count is capped at the 64-key blocks of tk; one leaves the keys unsplit.  With none named the
 // reference lets its tuner choose "among one, two, the counts around two blocks per SM and the
@@ -344,10 +365,9 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
   if (asked > 1) return (int)(asked < most ? asked : most);
   if (opts->has_window || opts->has_chunk || opts->seg_start != nullptr) return 1;
   const int64_t group = kv_heads > 0 ? heads / kv_heads : 1;
-  // A decoder step of a few rows a KV head streams its keys (svodk::attention_decodes): a workgroup a (batch, KV
-  // head, split), splits of at least four key blocks, as many as bring the launch to about a thousand workgroups
-  // (one row) or five hundred (more): enough of them resident for the bytes in flight, few enough that their
-  // streams do not thrash the memory's open pages.
+  // A decoder step of a few rows a KV head streams its keys (svodk::attention_decodes): splits of at least four key blocks,
+  // as many as bring the launch to about a thousand (batch, KV head, split)s (one row) or five hundred (more).  With more
+  // of a workspace than these need the call takes decode_split_count's.
   if (!opts->causal && opts->bias == nullptr && group * t >= 1 && group * t <= decode_limit) {
     const int64_t units = kv_heads * batch;
     if (units <= 0) return 1;
@@ -671,6 +691,14 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
   a.splits = split_count(opts, a.batch, t, heads, kv_heads, tk, decode_limit);
   void *workspace = opts->workspace;
   int64_t workspace_bytes = opts->workspace_bytes;
+  // What a decoder step rather takes than the rule's count, where there is room for it: a caller that lends what
+  // svodk_attention_workspace asks for has none for more.
+  const int64_t state_bytes = (int64_t)a.batch * t * heads * (d + 2) * 4;
+  const int better = a.decodes && opts->splits <= 0 && a.splits > 1 ? decode_split_count(a.batch, kv_heads, d, tk, a.splits) : 0;
+  if (better > 0 && (own_scratch ? better * state_bytes <= svodk::kSplitScratchBytes
+                                 : better == 1 || (workspace != nullptr &&
+                                                   better * state_bytes + svodk::decode_arrival_bytes(a) <= workspace_bytes)))
+    a.splits = better;
   if (a.splits > 1 && own_scratch) {
     // The library's own array holds the partial states.  A split count the rule chose is lowered to
     // what the array holds (down to one, as svodk_attention does without a workspace); a count the
