@@ -256,7 +256,7 @@ struct Wave {
   float m_run, l_run;
   int mask_next;
   // A key mask whose row was scanned at the start (rows of up to kScannedBlocks blocks): the
-  // blocks' 64-bit words, one copy a wave, in LDS after the ring.  Otherwise the words are read a
+  // blocks' 64-bit words, in LDS after the ring.  Otherwise the words are read a
   // lane a key, two blocks ahead of their use (mask_next).
   bool scanned;
   LDS_PTR(uint64_t) mask_words;
@@ -1008,8 +1008,10 @@ __device__ __forceinline__ void flash_fwd_body(
       w.v_src[j] = TL::source(row, pc, w.kv_row_bytes, true, j * NW * kRowsPer);
     }
   }
-  // ---- Q fragments: B operand of the score product, resident for the block.
-  {
+  // ---- Q fragments: B operand of the score product, resident for the block.  Of a head's own tile they are the wave's
+  // 32 rows behind one descriptor, bounded at the last query: no lane's address is 64 bits wide and no load stands
+  // under a branch (length known to first fill 0.90 -> 0.64 us there, 1.16 -> 0.87 at 8 rows of 2048 queries of 128).
+  if constexpr (GROUPED) {
     const uint16_t *q_ptr = q + ((int64_t)b * t + q_row) * q_row_stride + (int64_t)q_head * D + w.g * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
@@ -1017,30 +1019,43 @@ __device__ __forceinline__ void flash_fwd_body(
       if (q_ok) x = *reinterpret_cast<const u32x4 *>(q_ptr + ks * 16);
       w.qf[ks] = x;
     }
+  } else {
+    const int first_row = q_off + w.wave * kWaveRows;
+    const uint32_t q_row_bytes = (uint32_t)q_row_elems * 2;
+    const uint16_t *q_base = q + ((int64_t)b * t + first_row) * q_row_stride + (int64_t)h * D;
+    int there = max(t - first_row, 0);
+    asm("" : "+s"(there));  // on the scalar unit: the compiler makes a vector instruction of the two
+    there = min(there, kWaveRows);
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(q_base), 0, (int)((uint32_t)there * q_row_bytes), 0x00020000);
+    const int off = (int)((uint32_t)ln * q_row_bytes) + w.g * 16;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) w.qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, ks * 32, 0);
   }
-  // ---- the first eight blocks' elements of a key mask row that is scanned up front (see below) are asked for
-  // now, a lane a key, straight into this wave's stretch of LDS: behind the Q loads and ahead of the fills in
-  // the memory counter's order, so that the scan can wait for them with the fills still in flight.
-  w.mask_words = (LDS_PTR(uint64_t))(smem + TL::kLds) + w.wave * kScannedBlocks;
-  const bool scan_early = key_mask != nullptr && end <= kScannedBlocks && end > 0;
-  if (scan_early) {
+  // ---- a key mask row of up to kScannedBlocks blocks is scanned up front, its blocks dealt to the waves in turn: a wave
+  // ballots each of its blocks' 64 keys into the block's word in LDS, and every wave reads the words behind the first
+  // barrier.  (Every wave for itself, its eight early blocks one instruction each: entry to first barrier 4.2 us of a
+  // workgroup's 12.5 at 32 rows of 512 keys, 3.4 so; the launch 37.6 -> 36.7.)
+  // The elements of the first two are asked for now, a lane a key, straight into this wave's stretch of LDS: behind the
+  // Q loads and ahead of the fills in the memory counter's order, so that they can be waited for with the fills in flight.
+  w.mask_words = (LDS_PTR(uint64_t))(smem + TL::kLds);
+  w.scanned = key_mask != nullptr && end <= kScannedBlocks && end > 0;
+  LDS_PTR(int) raw = (LDS_PTR(int))(smem + TL::kLds + kScannedBlocks * 8) + w.wave * 128;
+  if (w.scanned) {
     const uint8_t *row = (const uint8_t *)key_mask + w.mask_row * mask_bytes;
     const i32x4 r = make_rsrc(row, (int64_t)w.tk * mask_bytes);  // keys past the row read as hidden
-    const int at = (int)(uintptr_t)(w.mask_words);
-    // Block i lies 64 elements further on: the instruction's own offset, which the LDS address takes as well as the
-    // memory address (block i's 256 bytes of LDS start at m0 + that offset).
-    const int voff = w.lane * mask_bytes;
+    const int at = (int)(uintptr_t)(raw);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < 2; i++) {
+      const int voff = ((w.wave + NW * i) * kBkv + w.lane) * mask_bytes;
       if (mask_bytes == 1)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ubyte %1, %2, 0 offen offset:%3 lds"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ubyte %1, %2, 0 offen lds"
                      :
-                     : "s"(at + i * 256 - i * kBkv), "v"(voff), "s"(r), "n"(i * kBkv)
+                     : "s"(at + i * 256), "v"(voff), "s"(r)
                      : "memory");
       else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen offset:%3 lds"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                      :
-                     : "s"(at + i * 256 - i * kBkv * 4), "v"(voff), "s"(r), "n"(i * kBkv * 4)
+                     : "s"(at + i * 256), "v"(voff), "s"(r)
                      : "memory");
     }
   }
@@ -1053,87 +1068,49 @@ __device__ __forceinline__ void flash_fwd_body(
   fill_k<D, NW>(w, 0, 0);
   fill_v<D, NW>(w, 0, 0);
   fill_k<D, NW>(w, 1, 1);
-  // A key mask row of up to kScannedBlocks blocks is scanned now, under the fills' flight: every
-  // wave ballots each block's 64 keys into a word of its own LDS copy.  The scan also says where
-  // the row's last visible key is (later blocks are skipped, like blocks past a length) and how
-  // many leading blocks hide nothing (those take the hot loop).  A longer row's words are read two
-  // blocks ahead of their use instead.
-  w.scanned = key_mask != nullptr && end <= kScannedBlocks;
-  int word0 = 0, lead_open = 0, seen_end = 0;
+  int word0 = 0;
   w.mask_next = 0;
   if (w.scanned) {
-    bool open = true;
-    int visible = 0, last_key = 0;  // keys the row shows, and the place after the last of them
-    // A row of up to eight blocks keeps its words in scalar registers until it is known to need them: a padding
-    // mask (the usual case) turns into a length below and never reads them.
-    const bool few = end <= 8;
-    uint64_t kept[8];
-    for (int base = 0; base < end; base += 8) {
-      // Eight blocks' elements in flight together: every lane loads (a key past the row's end, or a block
-      // past the tile's, loads the row's first element and drops it), so that no branch stands between the
-      // loads and a single wait brings them in.
+    // Everything issued before the fills is back when no more than the fills are out.
+    constexpr int kCh = W::CH;
+    if (fills_out == 3 * kCh)
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"(3 * kCh) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * kCh) : "memory");
+    auto put_word = [&](int blk, int element) {
+      const uint64_t bits = __builtin_amdgcn_ballot_w64(element != 0);
+      if (blk < end && w.lane == 0) w.mask_words[blk] = bits;
+    };
+    const int e0 = raw[w.lane], e1 = raw[64 + w.lane];
+    put_word(w.wave, e0);
+    put_word(w.wave + NW, e1);
+    for (int base = 2 * NW + w.wave; base < end; base += 8 * NW) {
+      // Eight blocks' elements in flight together: every lane loads (a key past the row's end, or a block past the tile's,
+      // loads the row's first element and drops it), so that no branch stands between the loads and a single
+      // wait brings them in.
       int words[8];
-      if (base == 0 && scan_early) {
-        // Asked for ahead of the fills: everything issued before the fills is back when no more than the fills are out.
-        constexpr int kCh = W::CH;
-        if (fills_out == 3 * kCh)
-          asm volatile("s_waitcnt vmcnt(%0)" : : "n"(3 * kCh) : "memory");
-        else if (fills_out == 2 * kCh)
-          asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * kCh) : "memory");
-        else
-          asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        LDS_PTR(const int) raw = (LDS_PTR(const int))(w.mask_words);
-#pragma unroll
-        for (int i = 0; i < 8; i++) words[i] = raw[i * 64 + w.lane];
-        // The words go where the elements lay: every element is in a register before the first word is written.
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-      } else if (w.mask_bytes == 1) {
+      auto element_at = [&](int i, bool &there) {
+        const int key = (base + NW * i) * kBkv + w.lane;
+        there = base + NW * i < end && key < w.tk;
+        return w.mask_row + (there ? key : 0);
+      };
+      if (w.mask_bytes == 1) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-          const int key = (base + i) * kBkv + w.lane;
-          const bool there = base + i < end && key < w.tk;
-          const int x = (int)((const uint8_t *)w.key_mask)[w.mask_row + (there ? key : 0)];
+          bool there;
+          const int x = (int)((const uint8_t *)w.key_mask)[element_at(i, there)];
           words[i] = there ? x : 0;
         }
       } else {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-          const int key = (base + i) * kBkv + w.lane;
-          const bool there = base + i < end && key < w.tk;
-          const int x = ((const int *)w.key_mask)[w.mask_row + (there ? key : 0)];
+          bool there;
+          const int x = ((const int *)w.key_mask)[element_at(i, there)];
           words[i] = there ? x : 0;
         }
       }
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        if (base + i >= end) break;
-        const uint64_t bits = __builtin_amdgcn_ballot_w64(words[i] != 0);
-        kept[i] = bits;
-        if (!few && w.lane == 0) w.mask_words[base + i] = bits;
-        if (bits != 0) {
-          seen_end = base + i + 1;
-          last_key = (base + i) * kBkv + 64 - __builtin_clzll(bits);
-        }
-        visible += __builtin_popcountll(bits);
-        open = open && bits == ~0ull;
-        lead_open += open ? 1 : 0;
-      }
-    }
-    end = min(end, seen_end);
-    w.end = end;
-    if (visible == last_key) {
-      // The row shows exactly its first `last_key` keys (a padding mask): that is a length, and
-      // from here on the row runs as one with a length does: no mask word per block, rows past
-      // the length never fetched.
-      len = min(len, last_key);
-      w.len = len;
-      w.key_mask = nullptr;
-      w.scanned = false;
-      w.kv_bytes = len > 0 ? (int64_t)(len - 1) * w.kv_row_bytes + D * 2 : 0;
-    } else if (few && w.lane == 0) {
-#pragma unroll
-      for (int i = 0; i < 8; i++)
-        if (i < end) w.mask_words[i] = kept[i];
+      for (int i = 0; i < 8; i++) put_word(base + NW * i, words[i]);
     }
   } else if (key_mask != nullptr) {
     word0 = mask_lane<D, NW>(w, 0);
@@ -1170,14 +1147,50 @@ __device__ __forceinline__ void flash_fwd_body(
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
 
+  // ---- what the scan found, from the blocks' words, a lane a block: where the row's last visible key is (later blocks
+  // are skipped, like blocks past a length) and how many leading blocks hide nothing (those take the hot loop).
+  int lead_open = 0;
+  if (w.scanned) {
+    int seen_end = 0;
+    for (int base = 0; base < end; base += 64) {
+      const int here = min(64, end - base);
+      uint64_t word = 0;
+      if (w.lane < here) word = w.mask_words[base + w.lane];
+      const uint64_t any = __builtin_amdgcn_ballot_w64(word != 0);
+      const uint64_t shut = __builtin_amdgcn_ballot_w64(word != ~0ull);  // lanes past the blocks too
+      if (any != 0) seen_end = base + 64 - __builtin_clzll(any);
+      if (lead_open == base) lead_open += shut == 0 ? 64 : __builtin_ctzll(shut);
+    }
+    uint64_t part = 0;  // the first block that hides a key
+    if (lead_open < end) {
+      const uint64_t x = w.mask_words[lead_open];  // the same address in every lane
+      part = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) |
+             (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)) << 32;
+    }
+    end = min(end, seen_end);
+    w.end = end;
+    if (seen_end <= lead_open + (part != 0 ? 1 : 0) && (part & (part + 1)) == 0) {
+      // The row shows exactly its first keys (a padding mask): that is a length, and from here on the row runs as one
+      // with a length does: no mask word per block, rows past the length never fetched.
+      len = min(len, lead_open * kBkv + __builtin_popcountll(part));
+      w.len = len;
+      w.key_mask = nullptr;
+      w.scanned = false;
+      w.kv_bytes = len > 0 ? (int64_t)(len - 1) * w.kv_row_bytes + D * 2 : 0;
+    }
+  }
+
   // ---- the first block's scores, masked, and their row maximum.
   // A causal wave past its last visible key has nothing to add from a block: it only keeps
-  // filling and meeting the barriers.  Blocks [0, my_end) are this wave's.
-  int my_end = end;
+  // filling and meeting the barriers.  Blocks [0, my_end) are this wave's.  So does a wave of a call's last tile whose
+  // rows are past the last query (three of four waves at 777 queries): the waves beside it on its SIMD have its issue slots
+  // (1500 queries 224.4 -> 222.3 us, 64 rows of 40 queries 9.27 -> 9.07).
+  const int tile_rows = GROUPED ? (int)geo.group * t : t;
+  int my_end = q_off + w.wave * kWaveRows < tile_rows ? end : 0;
   if (RANGED || CAUSAL) {
     // The last key the wave's last row sees; negative: the blocks lie past every row's reach.
     const int last_seen = RANGED ? w.hi_last : w.wave_first_row + kWaveRows - 1;
-    my_end = min(end, last_seen < 0 ? 0 : last_seen / kBkv + 1);
+    my_end = min(my_end, last_seen < 0 ? 0 : last_seen / kBkv + 1);
   }
 
   float sv[32], nv[32];  // S of the current and of the next block, swapping roles each hot step
