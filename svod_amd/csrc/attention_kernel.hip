@@ -643,13 +643,14 @@ __device__ __forceinline__ void hot_step(Wave<D, NW, F16, FLAGS> &w, const uint8
 
 // The general step, for the blocks at the edges: any block, a next block or none, masks, any
 // scale.  Slots are picked at run time.  `sv` holds the masked S(blk) and `bm` its row maximum;
-// on exit they hold block blk+1's (when this wave has one).
+// on exit they hold block blk+1's (when this wave has one).  This wave's blocks are [my_first, my_end): ahead of them
+// a step only scores its successor, if that is the first.
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
-__device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint8_t *smem, int blk, int my_end, float (&sv)[32],
-                                          float &bm) {
+__device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint8_t *smem, int blk, int my_first, int my_end,
+                                          float (&sv)[32], float &bm) {
   using TL = Tile<D>;
   const int par = blk & 1;
-  const bool more = blk + 1 < my_end;
+  const bool more = blk + 1 < my_end && (!w.ranged || blk + 1 >= my_first);
   const uint64_t kbits_next = uniform_bits<D, NW>(w, blk + 1, w.mask_next);
   // The next block's bias is asked for first: it has this block's P.V to arrive under.
   uint32_t bw[16];
@@ -657,17 +658,19 @@ __device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint
   fill_v<D, NW>(w, blk + 1, par ^ 1);
   if (!w.scanned && blk + 2 < w.end) w.mask_next = mask_lane<D, NW>(w, blk + 2);
   fill_k<D, NW>(w, blk + 2, par);
-  float corr;
-  const float m_exp = adopt_maximum<D, NW>(w, bm, corr);
+  if (!w.ranged || blk >= my_first) {
+    float corr;
+    const float m_exp = adopt_maximum<D, NW>(w, bm, corr);
 
-  const uint8_t *vs_ = smem + (2 + par) * TL::kBytes;
-  float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  uint32_t pk[16];
-  probabilities<F16>(sv, w.unit, m_exp, bs, pk);
-  probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
-  accumulate<D, NW>(w, vs_, 0, pk);
-  accumulate<D, NW>(w, vs_, 1, pk + 8);
-  w.l_run = w.l_run * corr + ((bs[0] + bs[1]) + (bs[2] + bs[3]));
+    const uint8_t *vs_ = smem + (2 + par) * TL::kBytes;
+    float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t pk[16];
+    probabilities<F16>(sv, w.unit, m_exp, bs, pk);
+    probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
+    accumulate<D, NW>(w, vs_, 0, pk);
+    accumulate<D, NW>(w, vs_, 1, pk + 8);
+    w.l_run = w.l_run * corr + ((bs[0] + bs[1]) + (bs[2] + bs[3]));
+  }
   if (more) {
     scores<D, NW>(w, smem, par ^ 1, sv);
     if (!w.positive) {
@@ -905,6 +908,7 @@ __device__ __forceinline__ void flash_fwd_body(
 
   // L584-608: key blocks [first, end) hold every key some query of the tile sees.
   int first = 0, end = (tk + kBkv - 1) / kBkv;
+  int row_from = 0;  // a key below which neither window nor chunks show this wave's rows any
   if (CAUSAL) end = min(end, (q_off + BQ + kBkv - 1) / kBkv);
   if (RANGED) {
     // This lane's row sees keys [lo, hi] (L659-695); rows past t stand in for row t - 1 where a
@@ -929,6 +933,7 @@ __device__ __forceinline__ void flash_fwd_body(
         first = max(first, (int)((int64_t)(max(cq0, rg.chunk_left) - rg.chunk_left) * rg.chunk_size / kBkv));
       }
     }
+    if (D <= 64) row_from = __builtin_amdgcn_readlane((int)lo, 0);
     if (rg.seg_start != nullptr) {
       auto start_of = [&](int64_t r) -> int64_t {
         const int64_t at = (int64_t)b * t + min(r, (int64_t)t - 1);
@@ -1197,7 +1202,12 @@ __device__ __forceinline__ void flash_fwd_body(
   float bm = -INFINITY;
 #pragma unroll
   for (int i = 0; i < 32; i++) sv[i] = nv[i] = 0.0f;
-  if (my_end > 0) {
+  // Blocks that end below the left edge of the wave's first row are none of its own: at a window of 64 keys a side two
+  // waves of four come past one such block (4 sequences of 4096 queries 30.4 -> 28.3 us, 16 of 300 13.05 -> 12.88, 8 of 777
+  // unchanged).  Segment starts are left out: they are the caller's, and nothing here makes them rise within a wave.  At
+  // d 128 it won nothing (2 sequences of 2000, causal, a window of 256: 20.9 -> 21.3).
+  const int my_first = RANGED && D <= 64 ? min(my_end, max(row_from - first_key, 0) / kBkv) : 0;
+  if (my_end > 0 && my_first == 0) {
     uint32_t bw[16];
     if (BIASED) load_bias<D, NW>(w, 0, q_ok, bw);
     scores<D, NW>(w, smem, 0, sv);
@@ -1231,13 +1241,13 @@ __device__ __forceinline__ void flash_fwd_body(
     // even number of them so that the hot pairs start on an even block.
     const int below = w.lo_last;
     const int lead = min(my_end, below <= 0 ? 0 : ((below + kBkv - 1) / kBkv + 1) & ~1);
-    for (; blk < lead; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm);
+    for (; blk < lead; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_first, my_end, sv, bm);
   }
   for (; blk + 2 < full; blk += 2) {
     hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
     hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
   }
-  for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm);
+  for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_first, my_end, sv, bm);
   for (; blk < end; blk++) idle_step<D, NW>(w, blk);
 
   // ---- the appended rows (L739-755, L827-846): one more block of keys, from their own tensors,
@@ -1676,7 +1686,7 @@ __global__ __launch_bounds__(NW * 64, 3) void flash_stream_kernel(
       hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
       hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
     }
-    for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm);
+    for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, 0, my_end, sv, bm);
     // Steps with nothing to compute: a causal wave past its diagonal, and the padding of an odd
     // item, which keeps the next item's blocks in the slots a first item's would be in.
     const int steps = more_items ? w.end_even : end;
