@@ -420,12 +420,19 @@ __device__ __forceinline__ bool on_edge(const Wave<D, NW, F16, FLAGS> &w, int bl
 // Scores whose bit of `mine` is clear become -inf; bit 8 (i / 4) + i % 4 (+ 32 for the second
 // half) is this lane's score i: the key that many places past the lane's first.
 __device__ __forceinline__ void hide_scores(uint64_t mine, float (&sv)[32]) {
-  const uint32_t lo = (uint32_t)mine, hi = (uint32_t)(mine >> 32);
+  const int lo = (int)(uint32_t)mine, hi = (int)(uint32_t)(mine >> 32);
+  // Two instructions a score, its bit over a whole word and a choice by bits (an and, a compare and a select were three):
+  // 32 sequences of at most 140 keys 15.1 -> 14.65 us, 4 of 4096 with a window of 64 a side 28.3 -> 27.7, 4 of at most 1030,
+  // causal, d 128, 30.7 -> 30.1.
+  auto hidden_unless = [](float x, int bit_word) {
+    const uint32_t keep = (uint32_t)bit_word, u = __float_as_uint(x);
+    return __uint_as_float((u & keep) | (0xff800000u & ~keep));
+  };
 #pragma unroll
   for (int i = 0; i < 16; i++) {
     const int rel = 8 * (i / 4) + (i % 4);  // key k0 + 32kb + 4g + rel
-    sv[i] = ((lo >> rel) & 1u) ? sv[i] : -INFINITY;
-    sv[16 + i] = ((hi >> rel) & 1u) ? sv[16 + i] : -INFINITY;
+    sv[i] = hidden_unless(sv[i], __builtin_amdgcn_sbfe(lo, rel, 1));
+    sv[16 + i] = hidden_unless(sv[16 + i], __builtin_amdgcn_sbfe(hi, rel, 1));
   }
 }
 
