@@ -240,11 +240,12 @@ struct Wave {
   // Per-row key ranges (a window, a chunk mask, segment starts: tk/src/ops/attention.rs:64-71):
   // this lane's query sees keys [row_lo, row_hi] only, a causal mask already folded into row_hi.
   // Both are non-decreasing in the row, so the wave's first and last rows bound every row's:
-  // lo_last, hi_first and hi_last are theirs.  All unused unless `ranged`.
+  // lo_last, hi_first and hi_last are theirs.  No row sees a key below lo_first, the first row's left edge by the window and
+  // the chunks alone (segment starts are the caller's).  All unused unless `ranged`.
   static constexpr bool ranged = (FLAGS & kRanged) != 0;
   static constexpr bool biased = (FLAGS & kBiased) != 0;
   int row_lo, row_hi;
-  int lo_last, hi_first, hi_last;
+  int lo_first, lo_last, hi_first, hi_last;
   // per-lane addressing
   // global byte offsets of this lane's chunk in this wave's fills of a tile (one per swizzle phase)
   static constexpr int NS = Tile<D>::sources(NW);
@@ -415,6 +416,22 @@ __device__ __forceinline__ bool on_edge(const Wave<D, NW, F16, FLAGS> &w, int bl
   // L715-731: a range's right edge for the wave's first row, its left edge for the last.
   if (w.ranged) return k0 + kBkv - 1 > w.hi_first || k0 < w.lo_last;
   return CAUSAL && (k0 + kBkv - 1 > w.wave_first_row);
+}
+
+// What the wave's rows may see of block `blk`, by halves of 32 keys: bit h when some row may see a key of half h.  An edge
+// step spends exponentials and P V on those halves only (the vector unit is what short calls wait for): 32 sequences of up to
+// 140 keys 14.65 -> 14.25 us, 64 of up to 40 8.7 -> 8.55, 12 of 200 with a window of 16 keys a side 9.8 -> 9.5; and a
+// range's wave skips the blocks below its left edge (4 of 4096 with a window of 64 a side 30.4 -> 28.3).  The scores, masks
+// and maximum stay a block's: by halves too they cost registers the kernel does not have.  At d 128 it is not worth the
+// branches (4 causal sequences of up to 1030 30.1 -> 30.6).
+template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
+__device__ __forceinline__ int halves_seen(const Wave<D, NW, F16, FLAGS> &w, int blk, uint64_t kbits) {
+  if (D > 64) return 3;
+  const int k0 = blk * kBkv;
+  const int last = w.ranged ? w.hi_last : CAUSAL ? w.wave_first_row + kWaveRows - 1 : 0x7fffffff;
+  int seen = ((uint32_t)kbits != 0 && k0 <= last ? 1 : 0) | ((uint32_t)(kbits >> 32) != 0 && k0 + 32 <= last ? 2 : 0);
+  if (w.ranged && k0 + 31 < w.lo_first) seen &= k0 + 63 < w.lo_first ? 0 : 2;
+  return seen;
 }
 
 // Scores whose bit of `mine` is clear become -inf; bit 8 (i / 4) + i % 4 (+ 32 for the second
@@ -649,15 +666,14 @@ __device__ __forceinline__ void hot_step(Wave<D, NW, F16, FLAGS> &w, const uint8
 }
 
 // The general step, for the blocks at the edges: any block, a next block or none, masks, any
-// scale.  Slots are picked at run time.  `sv` holds the masked S(blk) and `bm` its row maximum;
-// on exit they hold block blk+1's (when this wave has one).  This wave's blocks are [my_first, my_end): ahead of them
-// a step only scores its successor, if that is the first.
+// scale.  Slots are picked at run time.  `sv` holds the masked S(blk), `bm` its row maximum and `seen` its halves that
+// any row sees; on exit they hold block blk+1's (when this wave has one).
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
-__device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint8_t *smem, int blk, int my_first, int my_end,
-                                          float (&sv)[32], float &bm) {
+__device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint8_t *smem, int blk, int my_end, float (&sv)[32],
+                                          float &bm, int &seen) {
   using TL = Tile<D>;
   const int par = blk & 1;
-  const bool more = blk + 1 < my_end && (!w.ranged || blk + 1 >= my_first);
+  const bool more = blk + 1 < my_end;
   const uint64_t kbits_next = uniform_bits<D, NW>(w, blk + 1, w.mask_next);
   // The next block's bias is asked for first: it has this block's P.V to arrive under.
   uint32_t bw[16];
@@ -665,28 +681,34 @@ __device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint
   fill_v<D, NW>(w, blk + 1, par ^ 1);
   if (!w.scanned && blk + 2 < w.end) w.mask_next = mask_lane<D, NW>(w, blk + 2);
   fill_k<D, NW>(w, blk + 2, par);
-  if (!w.ranged || blk >= my_first) {
-    float corr;
-    const float m_exp = adopt_maximum<D, NW>(w, bm, corr);
+  float corr;
+  const float m_exp = adopt_maximum<D, NW>(w, bm, corr);
 
-    const uint8_t *vs_ = smem + (2 + par) * TL::kBytes;
-    float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t pk[16];
+  const uint8_t *vs_ = smem + (2 + par) * TL::kBytes;
+  float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  uint32_t pk[16];
+  if (seen & 1) {
     probabilities<F16>(sv, w.unit, m_exp, bs, pk);
-    probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
     accumulate<D, NW>(w, vs_, 0, pk);
-    accumulate<D, NW>(w, vs_, 1, pk + 8);
-    w.l_run = w.l_run * corr + ((bs[0] + bs[1]) + (bs[2] + bs[3]));
   }
+  if (seen & 2) {
+    probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
+    accumulate<D, NW>(w, vs_, 1, pk + 8);
+  }
+  w.l_run = w.l_run * corr + ((bs[0] + bs[1]) + (bs[2] + bs[3]));
   if (more) {
-    scores<D, NW>(w, smem, par ^ 1, sv);
-    if (!w.positive) {
+    seen = halves_seen<D, NW, CAUSAL>(w, blk + 1, kbits_next);
+    bm = -INFINITY;
+    if (!w.ranged || seen != 0) {
+      scores<D, NW>(w, smem, par ^ 1, sv);
+      if (!w.positive) {
 #pragma unroll
-      for (int i = 0; i < 32; i++) sv[i] *= w.c_exp;
+        for (int i = 0; i < 32; i++) sv[i] *= w.c_exp;
+      }
+      if (w.biased) add_bias<F16>(bw, sv);
+      if (on_edge<D, NW, CAUSAL>(w, blk + 1, kbits_next)) mask_scores<D, NW, CAUSAL>(w, blk + 1, kbits_next, sv);
+      bm = row_max(sv);
     }
-    if (w.biased) add_bias<F16>(bw, sv);
-    if (on_edge<D, NW, CAUSAL>(w, blk + 1, kbits_next)) mask_scores<D, NW, CAUSAL>(w, blk + 1, kbits_next, sv);
-    bm = row_max(sv);
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the fills issued this step have landed
   __syncthreads();
@@ -984,6 +1006,7 @@ __device__ __forceinline__ void flash_fwd_body(
   }
   if (RANGED) {
     w.row_lo -= first_key;
+    w.lo_first = row_from - first_key;
     w.row_hi -= first_key;
     w.lo_last = __builtin_amdgcn_readlane(w.row_lo, kWaveRows - 1);
     w.hi_first = __builtin_amdgcn_readlane(w.row_hi, 0);
@@ -1207,14 +1230,10 @@ __device__ __forceinline__ void flash_fwd_body(
 
   float sv[32], nv[32];  // S of the current and of the next block, swapping roles each hot step
   float bm = -INFINITY;
+  int seen = 0;
 #pragma unroll
   for (int i = 0; i < 32; i++) sv[i] = nv[i] = 0.0f;
-  // Blocks that end below the left edge of the wave's first row are none of its own: at a window of 64 keys a side two
-  // waves of four come past one such block (4 sequences of 4096 queries 30.4 -> 28.3 us, 16 of 300 13.05 -> 12.88, 8 of 777
-  // unchanged).  Segment starts are left out: they are the caller's, and nothing here makes them rise within a wave.  At
-  // d 128 it won nothing (2 sequences of 2000, causal, a window of 256: 20.9 -> 21.3).
-  const int my_first = RANGED && D <= 64 ? min(my_end, max(row_from - first_key, 0) / kBkv) : 0;
-  if (my_end > 0 && my_first == 0) {
+  if (my_end > 0) {
     uint32_t bw[16];
     if (BIASED) load_bias<D, NW>(w, 0, q_ok, bw);
     scores<D, NW>(w, smem, 0, sv);
@@ -1224,6 +1243,7 @@ __device__ __forceinline__ void flash_fwd_body(
     }
     if (BIASED) add_bias<F16>(bw, sv);
     const uint64_t kbits0 = uniform_bits<D, NW>(w, 0, word0);
+    seen = halves_seen<D, NW, CAUSAL>(w, 0, kbits0);
     if (on_edge<D, NW, CAUSAL>(w, 0, kbits0)) mask_scores<D, NW, CAUSAL>(w, 0, kbits0, sv);
     bm = row_max(sv);
   }
@@ -1248,13 +1268,14 @@ __device__ __forceinline__ void flash_fwd_body(
     // even number of them so that the hot pairs start on an even block.
     const int below = w.lo_last;
     const int lead = min(my_end, below <= 0 ? 0 : ((below + kBkv - 1) / kBkv + 1) & ~1);
-    for (; blk < lead; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_first, my_end, sv, bm);
+    for (; blk < lead; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   }
+  // (The blocks of these steps and the one behind them are whole: `seen` is 3 before and after.)
   for (; blk + 2 < full; blk += 2) {
     hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
     hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
   }
-  for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_first, my_end, sv, bm);
+  for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   for (; blk < end; blk++) idle_step<D, NW>(w, blk);
 
   // ---- the appended rows (L739-755, L827-846): one more block of keys, from their own tensors,
@@ -1669,6 +1690,7 @@ __global__ __launch_bounds__(NW * 64, 3) void flash_stream_kernel(
     }
     float sv[32], nv[32];
     float bm = -INFINITY;
+    int seen = 0;
     {
       scores<D, NW>(w, smem, 0, sv);
       if (!w.positive) {
@@ -1676,6 +1698,7 @@ __global__ __launch_bounds__(NW * 64, 3) void flash_stream_kernel(
         for (int i = 0; i < 32; i++) sv[i] *= w.c_exp;
       }
       const uint64_t kbits0 = uniform_bits<D, NW>(w, 0, 0);
+      seen = halves_seen<D, NW, CAUSAL>(w, 0, kbits0);
       if (on_edge<D, NW, CAUSAL>(w, 0, kbits0)) mask_scores<D, NW, CAUSAL>(w, 0, kbits0, sv);
       bm = row_max(sv);
     }
@@ -1693,7 +1716,7 @@ __global__ __launch_bounds__(NW * 64, 3) void flash_stream_kernel(
       hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
       hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
     }
-    for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, 0, my_end, sv, bm);
+    for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
     // Steps with nothing to compute: a causal wave past its diagonal, and the padding of an odd
     // item, which keeps the next item's blocks in the slots a first item's would be in.
     const int steps = more_items ? w.end_even : end;

@@ -41,3 +41,29 @@ def test_segment_starts_that_turn_within_a_wave(device, starts):
                              Attn(seg_start=torch.from_numpy(seg).to(device), window=(500, 500)))
     want = oracle.attention_direct(oracle.AttnProblem(q, k, v, seg_start=seg, window=(500, 500)))
     assert max_abs(to_np(got), want) < 2e-2
+
+
+@pytest.mark.parametrize("lens,causal", [([1, 32, 33, 64], False), ([65, 96, 97, 128], False), ([31, 95, 129, 200], True)])
+@pytest.mark.parametrize("d", [48, 64, 128])
+def test_lengths_at_the_edges_of_a_half_block(device, lens, causal, d):
+    """A block's half of 32 keys that no row sees is left out, on either side of the diagonal's and of a length's."""
+    t = 200 if causal else 70
+    g = Lcg(lens[0] + d)
+    q, k, v = g.bf16((4, t, 2, d)), g.bf16((4, 200, 2, d)), g.bf16((4, 200, 2, d))
+    keys = KeyMask.lens(torch.tensor(lens, dtype=torch.int32, device=device))
+    got = svod_amd.attention(*(bf16_tensor(x, device) for x in (q, k, v)), Attn(causal=causal, keys=keys, splits=1))
+    want = oracle.attention_direct(oracle.AttnProblem(q, k, v, causal=causal, key_lens=np.asarray(lens)))
+    assert np.isfinite(to_np(got)).all() and max_abs(to_np(got), want) < 2e-2
+
+
+def test_a_mask_that_shows_one_half_of_every_block(device):
+    """Halves shown and hidden in turn, and blocks hidden whole: what is left out is what the mask says."""
+    t, d = 40, 64
+    g = Lcg(3)
+    q, k, v = g.bf16((3, t, 2, d)), g.bf16((3, 384, 2, d)), g.bf16((3, 384, 2, d))
+    at = np.arange(384)
+    mask = np.stack([at // 32 % 2 == 0, at // 32 % 2 == 1, at // 96 % 2 == 1])
+    got = svod_amd.attention(*(bf16_tensor(x, device) for x in (q, k, v)),
+                             Attn(keys=KeyMask.bool(torch.from_numpy(mask).to(device)), splits=1))
+    want = oracle.attention_direct(oracle.AttnProblem(q, k, v, key_mask=mask))
+    assert max_abs(to_np(got), want) < 2e-2
