@@ -45,7 +45,9 @@ constexpr int kMaxWaves = 8;       // waves a workgroup
 constexpr int kAhead = 2;          // passes a lane works on at a time, with as many more in flight
 constexpr int kWordStride = kArrivalBytes / 8;  // of 64-bit words
 constexpr int kCountBits = 7;      // of a word of arrivals: its low bits count, the others are the launch's tag
-static_assert(kMostMergedSplits < 1 << kCountBits, "the count stands at the splits when a launch ends");
+constexpr uint64_t kEnded = (1 << kCountBits) - 1;  // the count of a (batch, KV head) that is merged
+static_assert(kMostMergedSplits < kEnded, "no launch under way counts that far");
+constexpr int kMostSharingRows = 64;  // a lane a row
 
 // Waves a workgroup: few workgroups take eight each, so that the launch still has its bytes in flight.
 // `heads_splits`: (batch, KV head, split)s of the launch.
@@ -200,12 +202,24 @@ __device__ __forceinline__ Integer ask(const void *p, int b, bool wide) {
 __device__ __forceinline__ int held(const Integer &x, int most) {
   int n = x.lo;
   if (x.wide) n = x.hi < 0 ? 0 : (x.hi > 0 || x.lo < 0 ? 0x7fffffff : x.lo);
-  return uniform(n < 0 ? 0 : (n < most ? n : most));
+  return n < 0 ? 0 : (n < most ? n : most);
+}
+// x summed over the lanes up to and with this one.
+__device__ __forceinline__ int prefix_sum(int x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+#endif
+  return x;
 }
 
 // What a launch does with its splits: it has none; it leaves partial states for combine_kernel; the workgroup of a
-// (batch, KV head) that ends last merges them.
-enum { kWhole, kPartial, kMerged };
+// (batch, KV head) that ends last merges them; that too, of splits that the rows share out by their lengths.
+enum { kWhole, kPartial, kMerged, kShared };
 
 // The workgroup's program for `nw` waves (8 or 4) and 1 << hg_log2 heads, for the kernels below to inline.  ROOM: LDS for the
 // states of one head of eight waves, or of two.
@@ -220,7 +234,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   constexpr int U = kAhead;  // the same for every R: a row's arithmetic does not depend on how many rows share the keys
   __shared__ __attribute__((aligned(16))) float merged[ROOM * kMaxWaves * R * LPK * 10];
 
-  constexpr bool SPLIT = MODE != kWhole;
+  constexpr bool SPLIT = MODE != kWhole, MERGES = MODE == kMerged || MODE == kShared;
   const uint32_t wg = __builtin_amdgcn_workgroup_id_x();
   const int tid = (int)__builtin_amdgcn_workitem_id_x();
   const int lane = tid & 63;
@@ -231,31 +245,66 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   const uint32_t groups = (uint32_t)p.kv_heads >> hg_log2;
   const uint32_t of_heads = wg / groups;
   const int group0 = (int)(wg - of_heads * groups);
-  const int b = SPLIT ? (int)(of_heads / (uint32_t)p.splits) : (int)of_heads;
-  const int split = SPLIT ? (int)of_heads - b * p.splits : 0;
-  const int unit = b * (int)groups + group0;
   const int pos = lane % LPK;                       // which 16 bytes of a head
   const int kvh = (group0 << hg_log2) + (lane / LPK & (hg - 1));
   const int slot = lane / LPK >> hg_log2;           // which row of a wave instruction
   const bool pos_ok = 8 * pos < D;
 
-  // The row's integers, asked for together: its length (L533-536: len = min(key_lens[b], tk)), where it lies in a cache
-  // (L544-550) and how many appended rows it sees.  One trip to memory for the three, so no load stands under a branch:
-  // what a call does not have is read from q and dropped.
-  const int tk = p.tk;
-  const bool appends = p.cached && p.k_app != nullptr && (!SPLIT || split == p.splits - 1);
-  const bool has_lens = p.key_lens != nullptr, has_map = p.cached && p.row_map != nullptr;
-  const bool has_seen = appends && p.app_lens != nullptr;
-  Integer len_b = ask(has_lens ? p.key_lens : p.q, has_lens ? b : 0, p.lens_i64 != 0 && has_lens);
-  Integer row_b = ask(has_map ? p.row_map : p.q, has_map ? b : 0, p.row_map_i64 != 0 && has_map);
-  Integer seen_b = ask(has_seen ? p.app_lens : p.q, has_seen ? b : 0, p.app_lens_i64 != 0 && has_seen);
+  const int pass = nw * kpi, chunk = U * pass;  // key rows of a pass of the waves, and of a chunk of U passes
+  static_assert(U == 2 && kMaxWaves == 8, "a chunk's rows are a power of two");
+  const int chunk_log2 = __builtin_ctz(U * 64 / LPK) + (nw == kMaxWaves ? 3 : 2) - hg_log2;
+
   // The rows: row r is token r % t of the group's head r / t (a grouped tile's order).
   const int rows = p.group * p.t;
-  // The output row of this lane's head's row r.
-  auto out_row = [&](int r, int kv_head) {
-    const int in_group = (r >= p.t) + (r >= 2 * p.t) + (r >= 3 * p.t);  // r / t: at most four rows
-    return ((int64_t)b * p.t + (r - in_group * p.t)) * p.heads + kv_head * p.group + in_group;
-  };
+  // The batch row of this workgroup, which of the row's `turns` splits it is, and the row's integers: its length
+  // (L533-536: len = min(key_lens[b], tk)), where it lies in a cache (L544-550) and how many appended rows it sees (the
+  // last split scores them).  The integers are asked for together: one trip to memory for the three, so no load stands
+  // under a branch and what a call does not have is read from q and dropped.
+  const int tk = p.tk;
+  const bool has_lens = p.key_lens != nullptr, has_map = p.cached && p.row_map != nullptr;
+  const bool has_app = p.cached && p.k_app != nullptr;
+  int b, split = 0, turns = 1, len, kv_row, app_seen;
+  Integer len_b, row_b, seen_b;
+  bool appends = has_app, has_seen = has_app && p.app_lens != nullptr;
+  uint32_t place0 = 0;  // of a launch whose rows share its splits: the first of the row's places
+  if constexpr (MODE == kShared) {
+    // A row takes one of the launch's batch * splits places and, of the others, what its keys are of all rows' keys: with
+    // the same count for each row the launch waits for its longest rows while most compute units have run out of keys.  16
+    // sequences of 8 KV heads of 128 over 210 to 2100 cached keys 22.7 -> 18.9 us, over 525 to 2100 23.0 -> 21.0, over 1260 to
+    // 2100 23.9 -> 24.2, over 2100 each 25.35 -> 25.55 (the lanes' sum); of 20 heads of 64 over 150 to 1500 20.0 -> 18.4, over
+    // 900 to 1500 22.1 -> 21.75, over 1500 each 25.15 -> 25.45.  Every workgroup finds the rows' places for itself, a lane a
+    // row, with a sum over the lanes and nothing else: a search for the shares that leave the longest split least cost
+    // 0.8 us a launch, what it won.
+    const bool there = lane < p.batch;
+    const int row = there ? lane : 0;
+    len_b = ask(p.key_lens, row, p.lens_i64 != 0);
+    row_b = ask(has_map ? p.row_map : p.key_lens, row, has_map ? p.row_map_i64 != 0 : p.lens_i64 != 0);
+    seen_b = ask(has_seen ? p.app_lens : p.key_lens, row, has_seen ? p.app_lens_i64 != 0 : p.lens_i64 != 0);
+    const int row_len = there ? held(len_b, tk) : 0;
+    const int weight = (row_len + chunk - 1) >> chunk_log2, up_to = prefix_sum(weight);
+    const int others = p.batch * (p.splits - 1);
+    const float each = (float)others * __builtin_amdgcn_rcpf((float)max(__builtin_amdgcn_readlane(up_to, 63), 1));
+    // (Rows of one length share alike: what rounding, the reciprocal's too, takes off a sum is put back.)
+    auto place = [&](int row, int keys) { return row + min((int)((float)keys * each + 0.01f), others); };
+    const int from = place(lane, up_to - weight), to = place(lane + 1, up_to);
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(there && from <= (int)of_heads && (int)of_heads < to);
+    if (mine == 0) return;  // the last places may be left to no one
+    b = __builtin_ctzll(mine);
+    place0 = (uint32_t)__builtin_amdgcn_readlane(from, b);
+    turns = min(__builtin_amdgcn_readlane(to, b) - (int)place0, kMostMergedSplits);
+    split = (int)(of_heads - place0);
+    if (split >= turns) return;
+    len = __builtin_amdgcn_readlane(row_len, b);
+    kv_row = has_map ? __builtin_amdgcn_readlane(held(row_b, p.cache_rows - 1), b) : b;
+    app_seen = !has_app || split != turns - 1 ? 0 : has_seen ? __builtin_amdgcn_readlane(held(seen_b, p.app_rows), b) : p.app_rows;
+  } else {
+    b = SPLIT ? (int)(of_heads / (uint32_t)p.splits) : (int)of_heads;
+    if (SPLIT) split = (int)of_heads - b * p.splits, turns = p.splits;
+    appends = has_app && (!SPLIT || split == turns - 1), has_seen = appends && p.app_lens != nullptr;
+    len_b = ask(has_lens ? p.key_lens : p.q, has_lens ? b : 0, p.lens_i64 != 0 && has_lens);
+    row_b = ask(has_map ? p.row_map : p.q, has_map ? b : 0, p.row_map_i64 != 0 && has_map);
+    seen_b = ask(has_seen ? p.app_lens : p.q, has_seen ? b : 0, p.app_lens_i64 != 0 && has_seen);
+  }
   uint32_t qf[R][4];
 #pragma unroll
   for (int r = 0; r < R; r++) {
@@ -269,12 +318,18 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
 #pragma unroll
     for (int i = 0; i < 4; i++) qf[r][i] = x[i];
   }
-
-  asm volatile("" : "+s"(len_b.lo), "+s"(len_b.hi), "+s"(row_b.lo), "+s"(row_b.hi), "+s"(seen_b.lo), "+s"(seen_b.hi));
-  const int len = has_lens ? held(len_b, tk) : tk;
-  const int kv_row = has_map ? held(row_b, p.cache_rows - 1) : b;
-  const int app_seen = !appends ? 0 : has_seen ? held(seen_b, p.app_rows) : p.app_rows;
-
+  if constexpr (MODE != kShared) {
+    asm volatile("" : "+s"(len_b.lo), "+s"(len_b.hi), "+s"(row_b.lo), "+s"(row_b.hi), "+s"(seen_b.lo), "+s"(seen_b.hi));
+    len = has_lens ? uniform(held(len_b, tk)) : tk;
+    kv_row = has_map ? uniform(held(row_b, p.cache_rows - 1)) : b;
+    app_seen = !appends ? 0 : has_seen ? uniform(held(seen_b, p.app_rows)) : p.app_rows;
+  }
+  const int unit = b * (int)groups + group0;
+  // The output row of this lane's head's row r.
+  auto out_row = [&](int r, int kv_head) {
+    const int in_group = (r >= p.t) + (r >= 2 * p.t) + (r >= 3 * p.t);  // r / t: at most four rows
+    return ((int64_t)b * p.t + (r - in_group * p.t)) * p.heads + kv_head * p.group + in_group;
+  };
   const float c_exp = p.scale * kLog2e;  // L619
   State st[R];
 #pragma unroll
@@ -292,11 +347,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   // the memory does.  Rows of a cache are very often a power of two apart, and so are the batch rows; workgroups that
   // all walk from key 0 then ask the same few memory channels for their rows at the same time.  Started by the cache row,
   // not by who asks: a batch lane mapped to another cache row reads it as that row's own lane would.
-  static_assert(U == 2 && kMaxWaves == 8, "a chunk's rows are a power of two");
-  const int pass = nw * kpi, chunk = U * pass;
-  const int chunk_log2 = __builtin_ctz(U * 64 / LPK) + (nw == kMaxWaves ? 3 : 2) - hg_log2;
-  const uint32_t of_row = ((uint32_t)len + (uint32_t)chunk - 1) >> chunk_log2, turns = SPLIT ? (uint32_t)p.splits : 1u;
-  const int chunks = of_row > (uint32_t)split ? (int)((of_row - (uint32_t)split + turns - 1) / turns) : 0;
+  const uint32_t of_row = ((uint32_t)len + (uint32_t)chunk - 1) >> chunk_log2;
+  const int chunks = of_row > (uint32_t)split ? (int)((of_row - (uint32_t)split + (uint32_t)turns - 1) / (uint32_t)turns) : 0;
   const int first = (int)__umulhi((uint32_t)kv_row * 0x9e3779b1u, (uint32_t)chunks);  // a fraction that rows differ in
   const uint32_t in_row = (uint32_t)((lane / LPK & (hg - 1)) * (D * 2) + 16 * pos);
   const void *mask = nullptr;  // visibility bytes or words of the cached keys
@@ -397,7 +449,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
     auto chunk_of = [&](int i) {
       int c = first + i;
       c = c >= chunks ? c - chunks : c;
-      return i < chunks ? (split + c * (int)turns) * chunk : len;
+      return i < chunks ? (split + c * turns) * chunk : len;
     };
     Rows one, two;
     const Source app = source(p.k_app, p.v_app, ((int64_t)b * p.app_rows * p.kv_heads + (group0 << hg_log2)) * D,
@@ -432,18 +484,18 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   // itself in, that the word carries this launch's tag: it becomes (tag, 0) by one compare-and-swap out of whatever was
   // there, and no other write of the launch leaves that tag again, so a late swap out of the old content fails.  Nothing
   // else ever carries the tag (57 bits, another one a launch) but the word as an earlier replay of the same captured
-  // launch left it, and that one counts `splits`, which no word of a launch under way does while a workgroup of its
-  // (batch, KV head) has yet to come.  The content is asked for ahead of the keys and the swap goes out behind them, so
+  // launch left it, and that one counts kEnded, which no word of a launch under way does: the workgroup that merges leaves
+  // it behind (`splits` would not do, a row's share of them is another with other lengths).  The content is asked for ahead of the keys and the swap goes out behind them, so
   // that neither is waited for: with the swap ahead of the keys a launch takes 1.4 us more.
   uint64_t *arrivals = p.arrivals + (int64_t)unit * kWordStride;
-  const bool counts = MODE == kMerged && tid == 0;
+  const bool counts = MERGES && tid == 0;
   uint64_t found = 0;
   if (counts) found = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (mask != nullptr)
     stream(std::true_type());
   else
     stream(std::false_type());
-  if (counts && (found >> kCountBits != p.tag || (int)(found & ((1u << kCountBits) - 1)) >= p.splits))
+  if (counts && (found >> kCountBits != p.tag || (int)(found & ((1u << kCountBits) - 1)) >= turns))
     __hip_atomic_compare_exchange_strong(arrivals, &found, p.tag << kCountBits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
   // The places of a wave that share output columns (lanes `span` apart) merge (L948-1014): the greatest maximum, what each
@@ -469,13 +521,15 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   // all waves' states of it together.  (One state after the other, each read behind the sums of the one before: 0.17 us a
   // state, 1.9 us more for eight waves of two rows.)
   const int64_t states = (int64_t)p.batch * p.t * p.heads;  // of a split
-  // A merging launch's states lie a unit together: [unit][split][row of the unit's heads][D], then their (m, l).
+  // A merging launch's states lie a unit together: [unit][split][row of the unit's heads][D], then their (m, l); the units
+  // of a launch whose rows share its splits by heads, then by their places.
   const int unit_rows = rows << hg_log2;
   Shared shared_o, shared_ml;
-  if (MODE == kMerged) {
-    const uint32_t of_unit = (uint32_t)(p.splits * unit_rows);
-    shared_o.name(p.o_part + (int64_t)unit * of_unit * D, of_unit * D * 4);
-    shared_ml.name(p.m_part + (int64_t)unit * of_unit * 2, of_unit * 8);
+  if (MERGES) {
+    const uint32_t of_unit = (uint32_t)(turns * unit_rows);
+    const int64_t before = MODE == kShared ? (int64_t)group0 * p.batch * p.splits + place0 : (int64_t)unit * turns;
+    shared_o.name(p.o_part + before * unit_rows * D, of_unit * D * 4);
+    shared_ml.name(p.m_part + before * unit_rows * 2, of_unit * 8);
   }
   auto merge_waves = [&](auto waves) {
     constexpr int W = decltype(waves)::value;
@@ -517,7 +571,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
         const int head = of_row / LPK, at_pos = of_row % LPK;
         if (r >= rows || 8 * at_pos >= D) continue;
         const int64_t orow = out_row(r, (group0 << hg_log2) + head);
-        if (MODE == kMerged) {
+        if (MERGES) {
           const uint32_t at = (uint32_t)(split * unit_rows + head * rows + r);
           if (at_pos == 0) shared_ml.put2(at * 8, f32x2{m, l});
           shared_o.put4((at * D + 8 * at_pos) * 4, f32x4{acc[0], acc[1], acc[2], acc[3]});
@@ -547,7 +601,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
     merge_waves(std::integral_constant<int, kMaxWaves>());
   else
     merge_waves(std::integral_constant<int, kMaxWaves / 2>());
-  if (MODE != kMerged) return;
+  if (!MERGES) return;
   // ---- the merge.  This wave's states are where every workgroup sees them before it counts itself in: they were stored
   // past the L2s, and vmcnt is at zero when the memory behind those has taken them all.  The workgroup that counts itself
   // in last reads them, from there as well.  No one waits for anyone.  The arithmetic is combine_kernel's, operation
@@ -556,7 +610,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   // 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.  In a graph's replay, where
   // a launch costs no host time: one over 8000 22.3 -> 16.7, two over 4700 20.8 -> 17.7, four over 8100 36.1 -> 33.6, sixteen
   // over 1500 26.3 -> 26.6.
-  const int splits = p.splits;
+  const int splits = turns;
   if (wave == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     uint32_t before = 0;
@@ -567,6 +621,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   }
   __syncthreads();
   if (uniform((int)__float_as_uint(merged[0])) != splits - 1) return;
+  if (tid == 0) __hip_atomic_store(arrivals, p.tag << kCountBits | kEnded, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   asm volatile("" ::: "memory");  // the states are read from here on
   constexpr int kLanes = D / 4;
   // States are asked for `batch` together, the first ones with the maxima of all: two trips to memory for 32 splits.
@@ -668,7 +723,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(const Packed a) 
 }
 
 template <int D, int R, bool F16>
-hipError_t launch_r(const Packed &p, bool merged, hipStream_t stream) {
+hipError_t launch_r(const Packed &p, int mode, hipStream_t stream) {
   const int64_t heads_splits = (int64_t)p.batch * p.kv_heads * p.splits;
   if (heads_splits == 0) return hipSuccess;
   const uint32_t threads = (uint32_t)decode_waves((uint32_t)heads_splits) * 64;
@@ -676,15 +731,19 @@ hipError_t launch_r(const Packed &p, bool merged, hipStream_t stream) {
   auto run = [&](auto mode) {
     return Launch<decode_kernel<D, R, F16, decltype(mode)::value>>::run(grid, threads, 0, 0, stream, p);
   };
-  if (p.splits == 1) return run(std::integral_constant<int, kWhole>());
-  return merged ? run(std::integral_constant<int, kMerged>()) : run(std::integral_constant<int, kPartial>());
+  switch (mode) {
+    case kWhole: return run(std::integral_constant<int, kWhole>());
+    case kPartial: return run(std::integral_constant<int, kPartial>());
+    case kMerged: return run(std::integral_constant<int, kMerged>());
+    default: return run(std::integral_constant<int, kShared>());
+  }
 }
 
 template <int D>
-hipError_t launch_d(const Packed &p, int rows, bool merged, bool f16, hipStream_t stream) {
-  if (rows <= 1) return f16 ? launch_r<D, 1, true>(p, merged, stream) : launch_r<D, 1, false>(p, merged, stream);
-  if (rows <= 2) return f16 ? launch_r<D, 2, true>(p, merged, stream) : launch_r<D, 2, false>(p, merged, stream);
-  return f16 ? launch_r<D, 4, true>(p, merged, stream) : launch_r<D, 4, false>(p, merged, stream);
+hipError_t launch_d(const Packed &p, int rows, int mode, bool f16, hipStream_t stream) {
+  if (rows <= 1) return f16 ? launch_r<D, 1, true>(p, mode, stream) : launch_r<D, 1, false>(p, mode, stream);
+  if (rows <= 2) return f16 ? launch_r<D, 2, true>(p, mode, stream) : launch_r<D, 2, false>(p, mode, stream);
+  return f16 ? launch_r<D, 4, true>(p, mode, stream) : launch_r<D, 4, false>(p, mode, stream);
 }
 
 // A launch's tag: no two of a process have the same, and where they start differs from process to process.
@@ -762,13 +821,21 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
   const int rows = a.heads / a.kv_heads * a.t;
   const bool merged = splits > 1 && a.merges;
   if (merged && splits > kMostMergedSplits) return hipErrorInvalidValue;
+  // Rows share the splits out by their lengths; a count that the caller named is every row's.  From four splits a row on: at
+  // two, a row that rounding leaves one short reads twice as long (32 sequences over 600 to 1000 keys 23 -> 29 us); and from
+  // 96 MiB of a cache on, which take 10 us: over less the lanes' sum gives back what even shares win (8 over 2048, 64 MiB, 210 to
+  // 2100 keys 14.95 -> 14.45 us, 1260 to 2100 15.75 -> 16.25; 3 over 1000, 7.7 -> 8.8).  The sum holds 2^31 keys.
+  const bool shared = merged && a.shares && a.key_lens != nullptr && a.key_mask == nullptr && splits >= 4 &&
+                      a.batch >= 4 && a.batch <= kMostSharingRows && (int64_t)a.batch * a.tk < 0x7fffffffLL &&
+                      (int64_t)a.batch * a.tk * a.kv_heads * a.d * 4 >= 96 << 20;
   if (merged) p.tag = next_tag();
+  const int mode = splits == 1 ? kWhole : !merged ? kPartial : shared ? kShared : kMerged;
   switch (a.d) {
-    case 32: return launch_d<32>(p, rows, merged, a.f16 != 0, stream);
-    case 48: return launch_d<48>(p, rows, merged, a.f16 != 0, stream);
-    case 64: return launch_d<64>(p, rows, merged, a.f16 != 0, stream);
-    case 128: return launch_d<128>(p, rows, merged, a.f16 != 0, stream);
-    case 256: return launch_d<256>(p, rows, merged, a.f16 != 0, stream);
+    case 32: return launch_d<32>(p, rows, mode, a.f16 != 0, stream);
+    case 48: return launch_d<48>(p, rows, mode, a.f16 != 0, stream);
+    case 64: return launch_d<64>(p, rows, mode, a.f16 != 0, stream);
+    case 128: return launch_d<128>(p, rows, mode, a.f16 != 0, stream);
+    case 256: return launch_d<256>(p, rows, mode, a.f16 != 0, stream);
   }
   return hipErrorInvalidValue;
 }

@@ -104,6 +104,7 @@ struct AttnArgs {
   int32_t decodes;   // launch_decode's call (attention_decodes): decided once, launch_attention and attention_config follow it
   // A decoder step merges its splits itself: behind l_part the workspace has decode_arrival_bytes(a) more, of any content.
   int32_t merges;
+  int32_t shares;  // and its rows may take other counts than `splits` each, batch * splits together
   // Elements from a token's row to the next in q and in k/v; 0 = dense (heads * d, kv_heads * d).
   // A fused projection read in place (tk/src/ops/attention.rs:104-122) has its own row for both.
   int64_t q_row_elems, kv_row_elems;

@@ -729,6 +729,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     // A split decoder step merges its splits itself where the workspace has room for its words.
     a.merges = a.decodes && a.splits <= svodk::kMostMergedSplits && workspace_bytes - need >= svodk::decode_arrival_bytes(a);
     if (a.merges) need += svodk::decode_arrival_bytes(a);
+    a.shares = a.merges && opts->splits <= 0;
     Span ws[2] = {{"workspace", workspace, (size_t)need, true}, {"o", out->data, (size_t)numel(out) * 2, true}};
     if (int rc = check_aliasing(op, ws, 2)) return rc;
     for (int i = 0; i < 3; i++) {
