@@ -733,8 +733,8 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, uint32_t d, uint32_t rcp)
 
 // Launch geometry the host works out once: sizes and their reciprocals for div_by.
 struct Geometry {
-  uint32_t unit_size, unit_rcp;  // workgroups of a (batch, KV head): group * nqt
-  uint32_t nqt, nqt_rcp;         // query tiles
+  uint32_t unit_size, unit_rcp;  // workgroups of a (batch, KV head): group * nqt, or of a causal one without its short tiles
+  uint32_t nqt, nqt_rcp;         // query tiles; the reciprocal is the group's in a causal launch, which divides by that
   uint32_t kv_heads, kvh_rcp;
   uint32_t group;                // heads / kv_heads
   uint32_t units;                // kv_heads * batch
@@ -832,17 +832,30 @@ __device__ __forceinline__ void flash_fwd_body(
   // tile fastest, then head, then batch, attention.rs:512,523; the order within a unit is that.)
   const uint32_t wg = __builtin_amdgcn_workgroup_id_x();
   const uint32_t local = wg / kXcds;
-  const uint32_t round = div_by(local, geo.unit_size, geo.unit_rcp);
+  uint32_t round = div_by(local, geo.unit_size, geo.unit_rcp);
   const uint32_t within = local - round * geo.unit_size;
-  uint32_t head_in_group = div_by(within, geo.nqt, geo.nqt_rcp);
-  int order = (int)(within - head_in_group * geo.nqt);
+  uint32_t head_in_group;
+  int order;
   if (CAUSAL && !GROUPED) {
     // An XCD deals its workgroups to its four shader engines strictly in turn, and one whose engine
     // is full holds back all behind it.  Head after head, every fourth tile of a causal unit (the
     // longest of each four) would go to the same engine; with the group's heads side by side for
     // each tile, neighbours cost the same and the engines fill and drain in step.
-    order = (int)(within / geo.group);
-    head_in_group = within - (uint32_t)order * geo.group;
+    uint32_t slot = div_by(within, geo.group, geo.nqt_rcp);
+    head_in_group = within - slot * geo.group;
+    order = (int)slot;
+    // The shortest quarter of every unit's tiles comes behind all units' others, the longer of them first (launch() says
+    // when): a launch that ended with a unit's longest tiles held a fifth of its time for them, half its slots empty.
+    const uint32_t rounds = (geo.units + kXcds - 1) / kXcds;
+    if (round >= rounds) {
+      const uint32_t in = local - rounds * geo.unit_size, at = div_by(in, geo.group, geo.nqt_rcp), tile = at / rounds;
+      round = at - tile * rounds;
+      head_in_group = in - at * geo.group;
+      order = (int)(div_by(geo.unit_size, geo.group, geo.nqt_rcp) + tile);
+    }
+  } else {
+    head_in_group = div_by(within, geo.nqt, geo.nqt_rcp);
+    order = (int)(within - head_in_group * geo.nqt);
   }
   // Which unit of a round an XCD takes turns with the round: with a power-of-two head count a
   // fixed deal would hand an XCD the same heads in every batch row, i.e. always the same 128-byte
@@ -1822,6 +1835,16 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
         return launch_stream<D, NW, CAUSAL, F16>(a, stream, knob, geo, q_row, kv_row);
     }
   }
+  if (CAUSAL && !GROUPED) {
+    // The short tiles come last where the launch is more than one round of the workgroups that the chip holds: 8 sequences of
+    // 2048 queries and keys, 16 heads of 128 over 8, 163 -> 157 us, of 512 to 2048 keys 136 -> 134.5, 32 of 500 63 -> 60.5, 4 of
+    // 2048, 16 heads of 64, 49.5 -> 43.8 (half of the tiles as the quarter, all of them 3 % behind it: K and V stay
+    // in an L2 while a unit's tiles run together).
+    const bool short_last = !SPLIT && !RANGED && blocks > 256 * (D <= 64 ? 3 : 2);
+    geo.unit_size -= short_last ? geo.group * (geo.nqt / 4) : 0;
+    geo.unit_rcp = rcp(geo.unit_size);
+    geo.nqt_rcp = rcp(geo.group);
+  }
   const uint32_t heads_group = (uint32_t)a.heads | geo.group << 16;
   const uint32_t tk_lens64 = (uint32_t)a.tk | (a.lens_i64 ? 0x80000000u : 0u);
   // The rows' order is worth finding where tiles are long enough for the rows to differ by and the rows few: 16 rows of
@@ -2072,7 +2095,7 @@ __device__ __forceinline__ void attention_entry(uint8_t *smem, const uint16_t *q
   rg.win_left = -1;
   rg.chunk_left = -1;
   flash_fwd_body<D, NW, CAUSAL, false, false, false, false, false, F16>(
-      smem, span, rcp_for(span), nqt, rcp_for(nqt), (uint32_t)kv_heads, rcp_for((uint32_t)kv_heads), units,
+      smem, span, rcp_for(span), nqt, rcp_for(CAUSAL ? group : nqt), (uint32_t)kv_heads, rcp_for((uint32_t)kv_heads), units,
       (uint32_t)heads | group << 16, key_lens, nullptr, t, (uint32_t)tk, q, k, v, o, key_mask, 1,
       __builtin_bit_cast(float, scale_bits), sp, heads * D, kv_heads * D, rg);
 }
@@ -2139,8 +2162,8 @@ __device__ __forceinline__ void attention_entry_full(uint8_t *smem, SVODK_FULL_P
   rg.app_lens = app_lens;
   rg.app_lens_i64 = app_lens_i64;
   flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, CACHED, GROUPED, F16>(
-      smem, span, rcp_for(span), nqt, rcp_for(nqt), (uint32_t)kv_heads, rcp_for((uint32_t)kv_heads), units,
-      (uint32_t)heads | group << 16, key_lens, nullptr, t, (uint32_t)tk | (lens_i64 ? 0x80000000u : 0u), q, k, v, o,
+      smem, span, rcp_for(span), nqt, rcp_for(CAUSAL && !GROUPED ? group : nqt), (uint32_t)kv_heads,
+      rcp_for((uint32_t)kv_heads), units, (uint32_t)heads | group << 16, key_lens, nullptr, t, (uint32_t)tk | (lens_i64 ? 0x80000000u : 0u), q, k, v, o,
       key_mask, mask_bytes, __builtin_bit_cast(float, scale_bits), sp, q_row_elems > 0 ? q_row_elems : heads * D,
       kv_row_elems > 0 ? kv_row_elems : kv_heads * D, rg);
 }
