@@ -116,7 +116,8 @@ typedef struct svodk_cache {
  * A decoder step (svodk_tune_decode) of up to 64 splits merges them itself, in the one launch, where
  * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  With `splits` = 0 and
  * twice the bytes and those words it takes the count that suits the device, up to twice the rule's (other
- * counts round differently).  What the workspace
+ * counts round differently).  Rows of a step that names no count, merges four splits a row or more and reads a cache of 96 MiB
+ * or more share the splits out by key_lens: a row's last bits then depend on the other rows' lengths.  What the workspace
  * holds at first does not matter, nor does the stream, nor whether the call is captured; as with the
  * partial states, no two launches in flight may have the same workspace.
  */

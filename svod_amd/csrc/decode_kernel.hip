@@ -606,10 +606,10 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   // past the L2s, and vmcnt is at zero when the memory behind those has taken them all.  The workgroup that counts itself
   // in last reads them, from there as well.  No one waits for anyone.  The arithmetic is combine_kernel's, operation
   // for operation: a launch that leaves the merge to that kernel gives the same bits.  It is a chain of four
-  // trips to memory, some 3 us, where a kernel of its own is a launch (2.6 us of host time) and 3.5 us: one sequence over
-  // 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.  In a graph's replay, where
-  // a launch costs no host time: one over 8000 22.3 -> 16.7, two over 4700 20.8 -> 17.7, four over 8100 36.1 -> 33.6, sixteen
-  // over 1500 26.3 -> 26.6.
+  // trips to memory, some 3 us, where a kernel of its own is a launch (2.6 us of host time) and 3.5 us: with a head a
+  // workgroup one sequence over 8000 cached keys 36.1 -> 31.8 us, two over 4700 18.4 -> 16.1, sixteen over 1500 26.1 -> 25.8.
+  // In a graph's replay, where a launch costs no host time: one over 8000 22.3 -> 16.7, two over 4700 20.8 -> 17.7, four over
+  // 8100 36.1 -> 33.6, sixteen over 1500 26.3 -> 26.6.
   const int splits = turns;
   if (wave == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
