@@ -422,8 +422,9 @@ __device__ __forceinline__ bool on_edge(const Wave<D, NW, F16, FLAGS> &w, int bl
 // step spends exponentials and P V on those halves only (the vector unit is what short calls wait for): 32 sequences of up to
 // 140 keys 14.65 -> 14.25 us, 64 of up to 40 8.7 -> 8.55, 12 of 200 with a window of 16 keys a side 9.8 -> 9.5; and a
 // range's wave skips the blocks below its left edge (4 of 4096 with a window of 64 a side 30.4 -> 28.3).  The scores, masks
-// and maximum stay a block's: by halves too they cost registers the kernel does not have.  At d 128 it is not worth the
-// branches (4 causal sequences of up to 1030 30.1 -> 30.6).
+// and maximum stay a block's: by halves too they cost registers the kernel does not have.  Above d 64 it is not worth the
+// branches: a step in pieces leaves the scheduler nothing to put beside the products (4 causal sequences of up to 1030 at d 128
+// 30.1 -> 30.6, 8 of up to 300 at d 256 19.4 -> 20.7).
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
 __device__ __forceinline__ int halves_seen(const Wave<D, NW, F16, FLAGS> &w, int blk, uint64_t kbits) {
   if (D > 64) return 3;
@@ -687,19 +688,26 @@ __device__ __forceinline__ void edge_step(Wave<D, NW, F16, FLAGS> &w, const uint
   const uint8_t *vs_ = smem + (2 + par) * TL::kBytes;
   float bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   uint32_t pk[16];
-  if (seen & 1) {
+  if constexpr (D > 64) {  // both halves always, in one piece for the scheduler
     probabilities<F16>(sv, w.unit, m_exp, bs, pk);
-    accumulate<D, NW>(w, vs_, 0, pk);
-  }
-  if (seen & 2) {
     probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
+    accumulate<D, NW>(w, vs_, 0, pk);
     accumulate<D, NW>(w, vs_, 1, pk + 8);
+  } else {
+    if (seen & 1) {
+      probabilities<F16>(sv, w.unit, m_exp, bs, pk);
+      accumulate<D, NW>(w, vs_, 0, pk);
+    }
+    if (seen & 2) {
+      probabilities<F16>(sv + 16, w.unit, m_exp, bs, pk + 8);
+      accumulate<D, NW>(w, vs_, 1, pk + 8);
+    }
   }
   w.l_run = w.l_run * corr + ((bs[0] + bs[1]) + (bs[2] + bs[3]));
   if (more) {
     seen = halves_seen<D, NW, CAUSAL>(w, blk + 1, kbits_next);
     bm = -INFINITY;
-    if (!w.ranged || seen != 0) {
+    if (D > 64 || !w.ranged || seen != 0) {
       scores<D, NW>(w, smem, par ^ 1, sv);
       if (!w.positive) {
 #pragma unroll
@@ -1059,7 +1067,9 @@ __device__ __forceinline__ void flash_fwd_body(
   // ---- Q fragments: B operand of the score product, resident for the block.  Of a head's own tile they are the wave's
   // 32 rows behind one descriptor, bounded at the last query: no lane's address is 64 bits wide and no load stands
   // under a branch (length known to first fill 0.90 -> 0.64 us there, 1.16 -> 0.87 at 8 rows of 2048 queries of 128).
-  if constexpr (GROUPED) {
+  // A head of 256 keeps a load under a branch each: loaded together its 64 registers of Q go to the accumulators' file, and
+  // the loop copies them back (4 causal rows of 1000 37.4 -> 38.3 us).
+  if constexpr (GROUPED || D > 128) {
     const uint16_t *q_ptr = q + ((int64_t)b * t + q_row) * q_row_stride + (int64_t)q_head * D + w.g * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
