@@ -747,6 +747,9 @@ struct Geometry {
   uint32_t group;                // heads / kv_heads
   uint32_t units;                // kv_heads * batch
 };
+// The instantiations whose launches may run the short tiles of all units behind the others.
+template <bool CAUSAL, bool SPLIT, bool RANGED, bool GROUPED>
+constexpr bool kShortTilesLast = CAUSAL && !GROUPED && !SPLIT && !RANGED;
 // The key splits of a launch that has them, and where their partial states go.
 struct Splits {
   uint32_t count, rcp;
@@ -844,7 +847,7 @@ __device__ __forceinline__ void flash_fwd_body(
   const uint32_t within = local - round * geo.unit_size;
   uint32_t head_in_group;
   int order;
-  if (CAUSAL && !GROUPED) {
+  if constexpr (CAUSAL && !GROUPED) {
     // An XCD deals its workgroups to its four shader engines strictly in turn, and one whose engine
     // is full holds back all behind it.  Head after head, every fourth tile of a causal unit (the
     // longest of each four) would go to the same engine; with the group's heads side by side for
@@ -852,14 +855,17 @@ __device__ __forceinline__ void flash_fwd_body(
     uint32_t slot = div_by(within, geo.group, geo.nqt_rcp);
     head_in_group = within - slot * geo.group;
     order = (int)slot;
-    // The shortest quarter of every unit's tiles comes behind all units' others, the longer of them first (launch() says
-    // when): a launch that ended with a unit's longest tiles held a fifth of its time for them, half its slots empty.
-    const uint32_t rounds = (geo.units + kXcds - 1) / kXcds;
-    if (round >= rounds) {
-      const uint32_t in = local - rounds * geo.unit_size, at = div_by(in, geo.group, geo.nqt_rcp), tile = at / rounds;
-      round = at - tile * rounds;
-      head_in_group = in - at * geo.group;
-      order = (int)(div_by(geo.unit_size, geo.group, geo.nqt_rcp) + tile);
+    if constexpr (kShortTilesLast<CAUSAL, SPLIT, RANGED, GROUPED>) {
+      // The shortest quarter of every unit's tiles comes behind all units' others, the longer of them first (launch() says
+      // when): a launch that ended with a unit's longest tiles held a fifth of its time for them, half its slots empty.
+      const uint32_t rounds = (geo.units + kXcds - 1) / kXcds;
+      if (round >= rounds) {
+        const uint32_t in = local - rounds * geo.unit_size, at = div_by(in, geo.group, geo.nqt_rcp), tile = at / rounds;
+        round = at - tile * rounds;
+        head_in_group = in - at * geo.group;
+        order = (int)(div_by(geo.unit_size, geo.group, geo.nqt_rcp) + tile);
+        if (order >= (int)geo.nqt) return;  // past the last tile: a launch of a code object in more workgroups than its tiles
+      }
     }
   } else {
     head_in_group = div_by(within, geo.nqt, geo.nqt_rcp);
@@ -1850,7 +1856,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     // 2048 queries and keys, 16 heads of 128 over 8, 163 -> 157 us, of 512 to 2048 keys 136 -> 134.5, 32 of 500 63 -> 60.5, 4 of
     // 2048, 16 heads of 64, 49.5 -> 43.8 (half of the tiles as the quarter, all of them 3 % behind it: K and V stay
     // in an L2 while a unit's tiles run together).
-    const bool short_last = !SPLIT && !RANGED && blocks > 256 * (D <= 64 ? 3 : 2);
+    const bool short_last = kShortTilesLast<CAUSAL, SPLIT, RANGED, GROUPED> && blocks > 256 * (D <= 64 ? 3 : 2);
     geo.unit_size -= short_last ? geo.group * (geo.nqt / 4) : 0;
     geo.unit_rcp = rcp(geo.unit_size);
     geo.nqt_rcp = rcp(geo.group);

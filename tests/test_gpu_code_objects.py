@@ -38,8 +38,8 @@ class Runtime:
         assert self.hip.hipModuleGetFunction(ctypes.byref(fn), self.modules[file], name.encode()) == 0, name
         return fn
 
-    def launch(self, name, values):
-        """One launch of kernel `name` with the manifest's record, workgroup count and threads."""
+    def launch(self, name, values, more=0):
+        """One launch of kernel `name` with the manifest's record, workgroup count (and `more`) and threads."""
         e = co.manifest()["kernels"][name]
         params = [tuple(p) for p in e["params"]]
         record = ctypes.create_string_buffer(co.pack(params, values, e["kernarg_size"]), e["kernarg_size"])
@@ -47,7 +47,7 @@ class Runtime:
         # HIP_LAUNCH_PARAM_BUFFER_POINTER, the record, HIP_LAUNCH_PARAM_BUFFER_SIZE, its size, HIP_LAUNCH_PARAM_END
         extra = (ctypes.c_void_p * 5)(1, ctypes.cast(record, ctypes.c_void_p), 2,
                                       ctypes.cast(ctypes.pointer(size), ctypes.c_void_p), 3)
-        groups = eval(e["workgroups"], {k: v for k, v in values.items()})
+        groups = eval(e["workgroups"], {k: v for k, v in values.items()}) + more
         assert 0 < groups < 2 ** 31
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         fn = self.function(e["file"], name)
@@ -287,6 +287,42 @@ def test_full_kernel_reads_a_fused_projection_in_place(device, runtime):
     rec["q"], rec["k"], rec["v"] = x.data_ptr(), x.data_ptr() + h * d * 2, x.data_ptr() + (h + hkv) * d * 2
     runtime.launch(co.full_name(d, "bf16", 1, 0, 0, 0, 0, 0), rec)
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("more", [1, 8, 8 * 4 * 3 + 5])
+@pytest.mark.parametrize("d,window,splits", [(64, None, 1), (128, None, 1), (64, (50, 0), 1), (128, None, 2)])
+def test_causal_workgroups_past_the_last_tile_exit(device, runtime, d, window, splits, more):
+    """A causal kernel launched in more workgroups than it has tiles writes its tiles and nothing else: the output lies in a
+    stretch of sentinels that reaches a tile and more to either side."""
+    b, t, h, hkv = 3, 300, 4, 2
+    g = Lcg(d + more)
+    q, k, v = (bf16_tensor(g.bf16(s), device) for s in ((b, t, h, d), (b, t, hkv, d), (b, t, hkv, d)))
+    lens = torch.tensor([300, 130, 0], dtype=torch.int32, device=device)
+    want = svod_amd.attention(q, k, v, Attn(causal=True, keys=KeyMask.lens(lens), window=window, splits=splits))
+    pad = 16 * 128 * h * d
+    held = torch.full((2 * pad + want.numel(),), 7.0, dtype=want.dtype, device=device)
+    got = held[pad:pad + want.numel()].view(want.shape)
+    if splits > 1:
+        rows = b * t * h
+        sizes = (splits * rows * d, splits * rows, splits * rows)
+        helds = [torch.full((2 * pad + n,), 7.0, device=device) for n in sizes]
+        parts = [x[pad:pad + n] for x, n in zip(helds, sizes)]
+        runtime.launch(co.full_name(d, "bf16", 1, 1, 0, 0, 0, 0),
+                       full_record(q, k, v, got, key_lens=lens, parts=parts, splits=splits), more)
+        for x in helds:
+            assert (x[:pad] == 7).all() and (x[-pad:] == 7).all()
+        runtime.launch(f"svodk_combine_d{d}_bf16", {"o_part": parts[0].data_ptr(), "m_part": parts[1].data_ptr(),
+                                                    "l_part": parts[2].data_ptr(), "o": got.data_ptr(), "rows": rows,
+                                                    "splits": splits})
+    elif window is None:
+        runtime.launch(f"svodk_attention_d{d}_bf16_causal",
+                       {"q": q.data_ptr(), "k": k.data_ptr(), "v": v.data_ptr(), "o": got.data_ptr(),
+                        "key_lens": lens.data_ptr(), "batch": b, "t": t, "tk": t, "heads": h, "kv_heads": hkv,
+                        "scale_bits": f32_bits(d ** -0.5)}, more)
+    else:
+        runtime.launch(co.full_name(d, "bf16", 1, 0, 1, 0, 0, 0), full_record(q, k, v, got, key_lens=lens, window=window), more)
+    assert np.array_equal(bits(got), bits(want))
+    assert (held[:pad] == 7).all() and (held[-pad:] == 7).all()
 
 
 @pytest.mark.parametrize("turn,f16,biased,shape", [(0, False, True, (3, 100, 96, 520)), (128, False, False, (2, 300, 256, 1024)),
