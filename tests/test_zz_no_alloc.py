@@ -2,6 +2,8 @@
 the partial states of a split call in the library's static device array.  Its output is held bit for
 bit to svodk_attention's with a lent workspace (the same kernels on the same operands), on two calls
 in a row, the second with a smaller input, so what the first call left in the array cannot show."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -27,6 +29,7 @@ def both(device, dev_ops, opts):
     out = torch.full_like(q, float("nan"))
     # Neither torch's allocator nor the device itself gives anything out under the call: the second
     # figure is the device's free bytes (a hipMalloc inside the library would lower it).
+    gc.collect()  # tensors that earlier tests left in reference cycles are not this call's to give back
     torch.cuda.synchronize()
     before, free_before = torch.cuda.memory_allocated(device), torch.cuda.mem_get_info(device)[0]
     got = svod_amd.attention_noalloc(q, k, v, opts, out)
