@@ -220,8 +220,9 @@ int svodk_order_rows(const svodk_tensor *keys, const svodk_tensor *order, void *
 /*
  * Bytes of `workspace` svodk_attention needs for these operands and options:
  * the f32 partial tensors o_part [splits, B, T, H, D], m_part and l_part
- * [splits, B, T, H] of tk/src/ops/attention.rs:285-293, for the split count the
- * call would run with, given that much; 0 when it would not split.  Pure, no device.
+ * [splits, B, T, H] of tk/src/ops/attention.rs:285-293, for the most splits the
+ * call would run with, given that much (a decoder step may take fewer); 0 when it
+ * would not split.  Pure, no device.
  */
 int64_t svodk_attention_workspace(const svodk_tensor *q, const svodk_tensor *k, const svodk_attn *opts);
 

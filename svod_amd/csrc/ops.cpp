@@ -840,9 +840,13 @@ int64_t svodk_attention_workspace(const svodk_tensor *q, const svodk_tensor *k, 
   if (!well_formed(q) || !well_formed(k) || opts == nullptr || q->rank != 4 || k->rank != 4) return 0;
   const int64_t batch = opts->batch_live > 0 ? opts->batch_live : q->shape[0];
   const int64_t kv_heads = opts->cache != nullptr ? opts->cache->kv_heads : k->shape[2];
-  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, k->shape[1],
-                                 svodk::attention_decode_limit());
+  const int32_t decode_limit = svodk::attention_decode_limit();
+  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, k->shape[1], decode_limit);
   if (splits <= 1) return 0;
+  // A decoder step that names no count may take fewer, down to none (attend()).
+  const int64_t rows = kv_heads > 0 && q->shape[2] % kv_heads == 0 ? q->shape[2] / kv_heads * q->shape[1] : 0;
+  const bool step = opts->splits <= 0 && !opts->causal && opts->bias == nullptr && rows >= 1 && rows <= decode_limit;
+  if (step && decode_split_count(batch, kv_heads, q->shape[3], k->shape[1], splits) == 1) return 0;
   return (int64_t)splits * batch * q->shape[1] * q->shape[2] * (q->shape[3] + 2) * 4;
 }
 

@@ -201,6 +201,17 @@ def test_with_no_count_named_few_query_tiles_over_many_keys_are_split():
         assert got == (0 if want == 1 else want * b * tq * h * (64 + 2) * 4), (b, tq, h, tk)
 
 
+@pytest.mark.parametrize("b,hkv,h,d,tk,want", [(64, 8, 8, 128, 1024, 0), (34, 16, 16, 128, 1024, 0), (60, 8, 8, 128, 1024, 2),
+                                               (25, 20, 20, 64, 600, 2)])
+def test_a_step_that_runs_whole_asks_for_no_workspace(b, hkv, h, d, tk, want):
+    """Decoder steps of which the rule makes two splits and a full round of workgroups one or two."""
+    workspace = svod_amd.ops._calls().attention_workspace
+    q, k = t([b, 1, h, d]), t([b, tk, hkv, d])
+    state = b * h * (d + 2) * 4
+    assert workspace(q, k, Attn()) == want * state
+    assert workspace(q, k, Attn(splits=2)) == 2 * state
+
+
 # ---- a cache: tk/src/ops/attention.rs:146-170
 def test_a_cache_is_validated_as_the_reference_validates_it():
     from svod_amd import Cache

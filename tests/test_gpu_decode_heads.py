@@ -87,3 +87,19 @@ def test_the_count_that_a_step_takes_unasked(device, b, h, hkv, d, tk, rule, bet
     assert np.array_equal(bits(svod_amd.attention(q, k, v, workspace=lent)), named(rule))
     out = torch.empty_like(q)
     assert np.array_equal(bits(svod_amd.attention_noalloc(q, k, v, Attn(), out)), named(better))
+
+
+@pytest.mark.parametrize("b,h,hkv,d,tk", [(64, 8, 8, 128, 1024), (34, 16, 16, 128, 1024), (60, 8, 8, 128, 1024), (25, 20, 20, 64, 600)])
+def test_a_step_splits_when_a_workspace_is_asked_for(device, b, h, hkv, d, tk):
+    """What svodk_attention_workspace answers is what the call does, given that much and in the package's own."""
+    g = torch.Generator(device=device).manual_seed(b)
+    q, k, v = (torch.randn(s, generator=g, device=device).bfloat16() for s in ((b, 1, h, d), (b, tk, hkv, d), (b, tk, hkv, d)))
+    need = svod_amd.ops._calls().attention_workspace(q, k, Attn())
+    lent = torch.empty(max(need, 16), dtype=torch.uint8, device=device)
+    for workspace in (lent, None):
+        got = svod_amd.attention(q, k, v, workspace=workspace)
+        assert ("combine_splits" in svod_amd.chosen()) == (need > 0)
+        whole = svod_amd.attention(q, k, v, Attn(splits=1))
+        assert mean_rel(to_np(got), to_np(whole)) < 2e-3
+        if need == 0:
+            assert np.array_equal(bits(got), bits(whole))
