@@ -74,6 +74,9 @@ typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 constexpr int kBkv = 64;       // keys per ring slot
 constexpr int kScannedBlocks = 256;  // key blocks (16384 keys) of a key mask row scanned up front
+// LDS behind the ring of a workgroup that scans one: the blocks' words, then the elements of each wave's first two blocks.
+constexpr int kRawElements = 128;
+constexpr int mask_lds(int waves) { return kScannedBlocks * 8 + waves * kRawElements * 4; }
 constexpr int kWaveRows = 32;  // query rows a wave owns: the N of the MFMA atom
 constexpr int kXcds = 8;       // accelerator dies of an MI355X, each with its own L2
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -812,7 +815,7 @@ struct TailOf {
 // queries of one head, for calls whose whole group fits a tile (a decoder step: heads / kv_heads
 // * T <= 128).  The group's heads then share one pass over their K and V instead of one each.
 // The workgroup's whole program, for the kernels below to inline: `smem` is the workgroup's LDS (the
-// ring, and behind it the scanned key mask words of a launch with a key mask).  Device code only:
+// ring, and behind it mask_lds() of a launch with a key mask).  Device code only:
 // the host pass needs a kernel's handle, not its instructions (and would drop the whole
 // instantiation over the LDS-fill instructions).
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1103,7 +1106,7 @@ __device__ __forceinline__ void flash_fwd_body(
   // Q loads and ahead of the fills in the memory counter's order, so that they can be waited for with the fills in flight.
   w.mask_words = (LDS_PTR(uint64_t))(smem + TL::kLds);
   w.scanned = key_mask != nullptr && end <= kScannedBlocks && end > 0;
-  LDS_PTR(int) raw = (LDS_PTR(int))(smem + TL::kLds + kScannedBlocks * 8) + w.wave * 128;
+  LDS_PTR(int) raw = (LDS_PTR(int))(smem + TL::kLds + kScannedBlocks * 8) + w.wave * kRawElements;
   if (w.scanned) {
     const uint8_t *row = (const uint8_t *)key_mask + w.mask_row * mask_bytes;
     const i32x4 r = make_rsrc(row, (int64_t)w.tk * mask_bytes);  // keys past the row read as hidden
@@ -1811,9 +1814,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   const int64_t blocks = (int64_t)nqt * a.heads * a.batch;
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7ffffff0LL) return hipErrorInvalidConfiguration;
-  // The ring, and behind it the words of a scanned key mask row (a copy a wave).
-  constexpr int kMaskLds = NW * kScannedBlocks * 8;
-  const int smem = TL::kLds + (a.key_mask != nullptr ? kMaskLds : 0);
+  const int smem = TL::kLds + (a.key_mask != nullptr ? mask_lds(NW) : 0);
   const int64_t q_row = a.q_row_elems > 0 ? a.q_row_elems : (int64_t)a.heads * a.d;
   const int64_t kv_row = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
   // A fill addresses the rows of one key block with 32-bit byte offsets from the block's 64-bit base.
@@ -1902,7 +1903,7 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     rg.app_lens = a.app_lens;
     rg.app_lens_i64 = a.app_lens_i64;
   }
-  constexpr int kMost = TL::kLds + kMaskLds;
+  constexpr int kMost = TL::kLds + mask_lds(NW);
   if constexpr (CACHED) {
     return Launch<flash_fwd_cached_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
         grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
@@ -2128,7 +2129,7 @@ __device__ __forceinline__ void attention_entry(uint8_t *smem, const uint16_t *q
 // seg_i64, bias_per_batch, kv_head_start, row_map_i64, cache_rows, app_rows, app_lens_i64.
 // A kernel reads what its flags name and ignores the rest.  Launch: ceil(batch * kv_heads, 8) * per
 // workgroups of 256 threads, per = (g ? 1 : heads / kv_heads) * (g ? 1 : ceil(t / 128)) * (s ? splits : 1).
-// LDS: the ring and the scanned mask words.  The caller keeps the op layer's checks, the caps on the
+// LDS: the ring and the scanned mask's.  The caller keeps the op layer's checks, the caps on the
 // window's and the chunks' reaches included (at most t + tk, and the chunks of t + tk).
 #define SVODK_FULL_PARAMS                                                                                             \
   const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,                     \
@@ -2188,7 +2189,7 @@ __device__ __forceinline__ void attention_entry_full(uint8_t *smem, SVODK_FULL_P
 #define SVODK_FULL_ENTRY(D, T, F16, C, S, R, B, K, G)                                                                 \
   extern "C" __global__ __launch_bounds__(256, ((D) <= 64 && !(B) && !((R) && (K))) ? 3 : ((D) <= 128 ? 2 : 1)) void  \
       svodk_attention_full_d##D##_##T##_c##C##s##S##r##R##b##B##k##K##g##G(SVODK_FULL_PARAMS) {                       \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[Tile<D>::kLds + 4 * kScannedBlocks * 8];                   \
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[Tile<D>::kLds + mask_lds(4)];                              \
     attention_entry_full<D, C, S, R, B, K, G, F16>(smem, SVODK_FULL_ARGS);                                            \
   }
 // The instantiations the library's own dispatch reaches: grouped tiles take neither a causal mask nor
@@ -2228,13 +2229,13 @@ SVODK_FULL_FAMILY(256, bf16, false) SVODK_FULL_FAMILY(256, f16, true)
     attention_entry<D, CAUSAL, F16>(smem, q, k, v, o, key_lens, nullptr, batch, t, tk, heads, kv_heads, scale_bits);  \
   }
 
-// Behind the ring, the words of the scanned key mask row: a copy a wave.
+// Behind the ring, the LDS of the scanned key mask row.
 #define SVODK_ATTENTION_MASK_ENTRY(NAME, D, CAUSAL, F16)                                                             \
   extern "C" __global__ __launch_bounds__(256, (D) <= 64 ? 3 : ((D) <= 128 ? 2 : 1)) void NAME(                       \
       const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,                 \
       uint16_t *__restrict__ o, const void *__restrict__ key_mask, int32_t batch, int32_t t, int32_t tk, int32_t heads, \
       int32_t kv_heads, int32_t scale_bits) {                                                                         \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[Tile<D>::kLds + 4 * kScannedBlocks * 8];                   \
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[Tile<D>::kLds + mask_lds(4)];                              \
     attention_entry<D, CAUSAL, F16>(smem, q, k, v, o, nullptr, key_mask, batch, t, tk, heads, kv_heads, scale_bits);  \
   }
 

@@ -58,8 +58,9 @@ def test_every_kernel_meets_the_loaders_conditions(built):
             assert kd.group_segment_fixed_size == 8 * e["rows_per_kv_head"] * (wide // 8) * 10 * 4, name
         elif e["op"] == "attention":
             # The K and V ring: two slots each of 64 keys (tk/src/kernels/attention.rs:187-190).
-            # and behind it, with a key mask, a 64-bit word a key block for each of 4 waves (256 blocks scanned).
-            mask_words = 4 * 256 * 8 if e.get("key_mask") else 0
+            # and behind it, with a key mask, a 64-bit word a key block (256 blocks scanned) and the raw elements of two blocks
+            # for each of 4 waves.
+            mask_words = 256 * 8 + 4 * 2 * 64 * 4 if e.get("key_mask") else 0
             wide = 64 if e["head_dim"] == 48 else e["head_dim"]  # a head of 48 takes the 64-wide tile
             assert kd.group_segment_fixed_size == 2 * 2 * 64 * wide * 2 + mask_words, name
         elif e["op"] == "linear":
