@@ -351,8 +351,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &p, const int nw, c
   const int chunks = of_row > (uint32_t)split ? (int)((of_row - (uint32_t)split + (uint32_t)turns - 1) / (uint32_t)turns) : 0;
   const int first = (int)__umulhi((uint32_t)kv_row * 0x9e3779b1u, (uint32_t)chunks);  // a fraction that rows differ in
   const uint32_t in_row = (uint32_t)((lane / LPK & (hg - 1)) * (D * 2) + 16 * pos);
-  const void *mask = nullptr;  // visibility bytes or words of the cached keys
-  if (p.key_mask != nullptr) mask = (const uint8_t *)p.key_mask + (int64_t)b * tk * p.mask_bytes;
+  const void *mask = nullptr;  // visibility bytes or words of the cached keys (rows share splits out by lengths, never with one)
+  if (MODE != kShared && p.key_mask != nullptr) mask = (const uint8_t *)p.key_mask + (int64_t)b * tk * p.mask_bytes;
 
   struct Rows {
     u32x4 k[U], v[U];
@@ -822,9 +822,13 @@ hipError_t launch_decode(const AttnArgs &a, hipStream_t stream) {
   const bool merged = splits > 1 && a.merges;
   if (merged && splits > kMostMergedSplits) return hipErrorInvalidValue;
   // Rows share the splits out by their lengths; a count that the caller named is every row's.  From four splits a row on: at
-  // two, a row that rounding leaves one short reads twice as long (32 sequences over 600 to 1000 keys 23 -> 29 us); and from
-  // 96 MiB of a cache on, which take 10 us: over less the lanes' sum gives back what even shares win (8 over 2048, 64 MiB, 210 to
-  // 2100 keys 14.95 -> 14.45 us, 1260 to 2100 15.75 -> 16.25; 3 over 1000, 7.7 -> 8.8).  The sum holds 2^31 keys.
+  // two, a row that rounding leaves one short reads twice as long (32 sequences over 600 to 1000 keys 23 -> 29 us).  And from
+  // 96 MiB of a cache on (8 KV heads of 128, equal splits -> shared): over less the sum over the lanes and the rounding give back
+  // what the rows whose lengths differ by less win.  At 80 MiB 4 sequences over 1280 to 5120 keys 17.5 -> 17.3 us, over 3072 to
+  // 5120 17.8 -> 18.3, 16 over 768 to 1280 17.2 -> 17.1; at 64 MiB 4 over 2457 to 4096 15.6 -> 16.4; at 112 MiB 4 over 1792 to
+  // 7168 22.1 -> 20.8, over 4300 to 7168 22.1 -> 22.3, 8 over 896 to 3584 21.0 -> 18.6, over 2150 to 3584 21.3 -> 20.8.  One
+  // length costs 0.1 to 0.2 us.  The line goes by what the cache holds at most, which is what the host knows: of 8192 keys a
+  // row, 200 each there take 8.0 us either way, 500 each 8.7 -> 8.8, 100 to 300 8.5 -> 8.0.  The sum holds 2^31 keys.
   const bool shared = merged && a.shares && a.key_lens != nullptr && a.key_mask == nullptr && splits >= 4 &&
                       a.batch >= 4 && a.batch <= kMostSharingRows && (int64_t)a.batch * a.tk < 0x7fffffffLL &&
                       (int64_t)a.batch * a.tk * a.kv_heads * a.d * 4 >= 96 << 20;
