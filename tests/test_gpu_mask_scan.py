@@ -8,7 +8,7 @@ import torch
 import oracle
 import svod_amd
 from svod_amd import Attn, KeyMask
-from util import Lcg, bf16_tensor, bits, max_abs, to_np
+from util import Lcg, bf16_tensor, bits, max_abs, tallies, tally, tally_values, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -23,11 +23,14 @@ def rows_of(tk):
     return np.stack(rows)
 
 
-@pytest.mark.parametrize("tk,causal,kind", [
+KINDS = [
     (7, False, torch.bool), (64, False, torch.int32), (129, True, torch.bool), (256, False, torch.bool), (257, False, torch.int32),
     (512, True, torch.bool), (577, False, torch.bool), (640, False, torch.int32), (2111, False, torch.bool), (2500, False, torch.int32),
     (4096, False, torch.bool), (4097, False, torch.bool), (9001, False, torch.int32), (16384, False, torch.bool),
-    (16385, False, torch.bool)])
+    (16385, False, torch.bool)]
+
+
+@pytest.mark.parametrize("tk,causal,kind", KINDS)
 def test_every_way_through_the_scan(device, tk, causal, kind):
     mask = rows_of(tk)
     if tk > 4000:
@@ -49,3 +52,33 @@ def test_every_way_through_the_scan(device, tk, causal, kind):
                                             splits=1))
     if tk <= 16384:
         assert np.array_equal(bits(got)[prefix], bits(as_lens)[prefix])
+
+
+@pytest.mark.parametrize("tk,causal,kind", KINDS)
+def test_every_key_of_every_block_counts(device, tk, causal, kind):
+    """Which keys each row saw, one a column or, of long rows, a block a column: a lost word, a swapped one or a single key shows
+    at every length."""
+    mask = rows_of(tk)
+    if tk > 4000:
+        mask = mask[::3] if tk < 16000 else mask[-7:]
+    b, d, per = len(mask), 64, 1 if tk <= 640 else 64
+    t = tk if causal else 5
+    v = tally_values(tk, d, per, device)
+    heads = v.shape[2]
+    v = v.expand(b, -1, -1, -1).contiguous()
+    k = torch.ones(b, tk, 1, d, dtype=torch.bfloat16, device=device).expand(-1, -1, heads, -1).contiguous()
+    q = torch.zeros(b, t, heads, d, dtype=torch.bfloat16, device=device)
+    shown = torch.from_numpy(mask).to(device)
+    keys = KeyMask.bool(shown if kind == torch.bool else shown.to(kind) * 3)
+    visible = np.repeat(mask[:, None], t, 1)
+    if causal:
+        visible = visible & (np.arange(tk)[None, :] <= np.arange(t)[:, None])
+    want = tally(visible, d, per)
+    got = to_np(svod_amd.attention(q, k, v, Attn(causal=causal, keys=keys, splits=1)))
+    assert tallies(got, want)
+    # What the bar is for: a row that shows keys, its last visible one hidden, and its last whole block.
+    row = int(np.argmax([m.sum() * (m != (np.arange(tk) < m.sum())).any() for m in mask]))
+    for lost in (np.flatnonzero(mask[row])[-1:], np.arange(tk) // 64 == np.flatnonzero(mask[row])[-1] // 64):
+        other = visible[row, -1].copy()
+        other[lost] = False
+        assert not tallies(tally(other, d, per), want[row, -1])

@@ -8,9 +8,29 @@ import torch
 import oracle
 import svod_amd
 from svod_amd import Attn, KeyMask
-from util import Lcg, bf16_tensor, max_abs, to_np
+from util import Lcg, bf16_tensor, max_abs, tallies, tally, tally_values, to_np
 
 pytestmark = pytest.mark.gpu
+
+
+def saw(device, visible, d, opts):
+    """The call's keys, one a column, are those of `visible` [b, t, tk] for each query."""
+    b, t, tk = visible.shape
+    v = tally_values(tk, d, 1, device)
+    heads = v.shape[2]
+    v = v.expand(b, -1, -1, -1).contiguous()
+    q = torch.zeros(b, t, heads, d, dtype=v.dtype, device=device)
+    got = to_np(svod_amd.attention(q, torch.ones_like(v), v, opts))
+    want = tally(visible, d, 1)
+    assert (np.isfinite(got)).all() and ((got != 0) == (want != 0)).all() and tallies(got, want)
+
+
+def in_window(t, tk, window, lens, causal):
+    i, j = np.arange(t)[:, None], np.arange(tk)[None, :]
+    seen = np.ones((t, tk), bool) if window is None else (j >= i - window[0]) & (j <= i + window[1])
+    if causal:
+        seen = seen & (j <= i)
+    return np.stack([seen & (j < n) for n in lens])
 
 
 @pytest.mark.parametrize("t,window,lens,splits,causal", [
@@ -27,6 +47,8 @@ def test_windows_past_the_first_blocks(device, t, window, lens, splits, causal, 
     want = oracle.attention_direct(oracle.AttnProblem(q, k, v, causal=causal, window=window,
                                                       key_lens=None if lens is None else np.asarray(lens)))
     assert np.isfinite(to_np(got)).all() and max_abs(to_np(got), want) < 2e-2
+    saw(device, in_window(t, t, window, lens or [t, t], causal), d,
+        Attn(causal=causal, keys=keys, window=window, splits=splits))
 
 
 @pytest.mark.parametrize("starts", [[0, 40, 70, 200], [0, 96, 130, 131], [0, 200, 10, 64]])
@@ -41,6 +63,7 @@ def test_segment_starts_that_turn_within_a_wave(device, starts):
                              Attn(seg_start=torch.from_numpy(seg).to(device), window=(500, 500)))
     want = oracle.attention_direct(oracle.AttnProblem(q, k, v, seg_start=seg, window=(500, 500)))
     assert max_abs(to_np(got), want) < 2e-2
+    saw(device, np.arange(256)[None, None, :] >= seg[:, :, None], d, Attn(seg_start=torch.from_numpy(seg).to(device), window=(500, 500)))
 
 
 @pytest.mark.parametrize("lens,causal", [([1, 32, 33, 64], False), ([65, 96, 97, 128], False), ([31, 95, 129, 200], True)])
@@ -54,6 +77,7 @@ def test_lengths_at_the_edges_of_a_half_block(device, lens, causal, d):
     got = svod_amd.attention(*(bf16_tensor(x, device) for x in (q, k, v)), Attn(causal=causal, keys=keys, splits=1))
     want = oracle.attention_direct(oracle.AttnProblem(q, k, v, causal=causal, key_lens=np.asarray(lens)))
     assert np.isfinite(to_np(got)).all() and max_abs(to_np(got), want) < 2e-2
+    saw(device, in_window(t, 200, None, lens, causal), d, Attn(causal=causal, keys=keys, splits=1))
 
 
 def test_a_mask_that_shows_one_half_of_every_block(device):
@@ -67,3 +91,4 @@ def test_a_mask_that_shows_one_half_of_every_block(device):
                              Attn(keys=KeyMask.bool(torch.from_numpy(mask).to(device)), splits=1))
     want = oracle.attention_direct(oracle.AttnProblem(q, k, v, key_mask=mask))
     assert max_abs(to_np(got), want) < 2e-2
+    saw(device, np.repeat(mask[:, None], t, 1), d, Attn(keys=KeyMask.bool(torch.from_numpy(mask).to(device)), splits=1))

@@ -79,3 +79,29 @@ def assert_bf16_parity(what: str, got: np.ndarray, direct64: np.ndarray, program
     mr, mr_ref = mean_rel(got, stored), mean_rel(program, stored)
     assert mr <= max(mean_rel_tol, 1.1 * mr_ref), f"{what}: mean-rel vs f64 {mr}, the reference program's own {mr_ref}"
     return worst, mr_prog, mr
+
+
+def tally_values(tk: int, d: int, per: int, device, dtype=torch.bfloat16) -> torch.Tensor:
+    """V [1, tk, heads, d] that tells which keys a softmax saw: key j is 1 in column j // per of the heads' columns and 0 in the
+    others.  Under a query of zeros every visible key weighs the same, so a column is the share of visible keys that lie in its
+    `per` keys: one key lost or gained among 64 moves it by 2^-6, four times what rounding to bf16 may."""
+    heads = -(-(-(-tk // per)) // d)
+    v = torch.zeros(1, tk, heads * d, dtype=dtype, device=device)
+    at = torch.arange(tk, device=device)
+    v[0, at, at // per] = 1
+    return v.view(1, tk, heads, d)
+
+
+def tally(visible: np.ndarray, d: int, per: int) -> np.ndarray:
+    """What those values give for visible [..., tk] keys: [..., heads, d]."""
+    tk = visible.shape[-1]
+    heads = -(-(-(-tk // per)) // d)
+    held = np.zeros((*visible.shape[:-1], heads * d * per), dtype=np.float64)
+    held[..., :tk] = visible
+    counts = held.reshape(*visible.shape[:-1], heads, d, per).sum(-1)
+    return counts / np.maximum(visible.sum(-1), 1)[..., None, None]
+
+
+def tallies(got: np.ndarray, want: np.ndarray) -> bool:
+    """Equal but for the rounding of a 16-bit result (2^-9) and of a reciprocal."""
+    return bool((np.abs(got.astype(np.float64) - want) <= 2.0 ** -8 * want).all())
