@@ -10,7 +10,10 @@ from util import bits
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(16, 16, 8, 128, 1700), (16, 20, 20, 64, 1300), (4, 16, 8, 128, 6200)]
+# (batch, heads, KV heads, head size, cached keys), and the splits that such a step takes where it names no count.
+SHAPES = [(16, 16, 8, 128, 1700), (16, 20, 20, 64, 1300), (4, 16, 8, 128, 6200),
+          (17, 8, 4, 128, 2900), (33, 4, 2, 128, 3000), (64, 4, 2, 64, 3200)]  # a lane a row: past 16 and 32 lanes, all 64
+UNASKED = [4, 6, 16, 15, 15, 4]
 
 
 def lengths(kind, b, tk):
@@ -20,9 +23,9 @@ def lengths(kind, b, tk):
             "past": torch.full((b,), 2 * tk)}[kind].long()
 
 
-def tensors(device, b, h, hkv, d, tk, app=0):
+def tensors(device, b, h, hkv, d, tk, app=0, dtype=torch.bfloat16):
     g = torch.Generator(device=device).manual_seed(b + tk)
-    rand = lambda *s: torch.randn(s, generator=g, device=device).bfloat16()
+    rand = lambda *s: torch.randn(s, generator=g, device=device).to(dtype)
     return [rand(b, 1, h, d), rand(b, tk, hkv, d), rand(b, tk, hkv, d)] + [rand(b, app, hkv, d) for _ in range(2 if app else 0)]
 
 
@@ -46,19 +49,36 @@ def exact(q, k, v, lens, rows=None, app=None, app_lens=None):
 
 
 def close(got, want):
-    # One rounding to bf16 (half of 2^-8 of the value) and f32 sums of at most 6300 terms, far below that.
-    return ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -12).all()
+    # One rounding to 16 bits (half of 2^-8 of a bf16 value, of 2^-11 of an f16 one) and f32 sums of at most 6300 terms, far
+    # below that.
+    ulp, rest = (2.0 ** -8, 2.0 ** -12) if got.dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -14)
+    return ((got.double() - want).abs() <= ulp * want.abs() + rest).all()
 
 
 @pytest.mark.parametrize("b,h,hkv,d,tk", SHAPES)
 @pytest.mark.parametrize("kind", ["even", "wide", "one", "none", "some", "short", "past"])
-def test_rows_of_any_lengths(device, b, h, hkv, d, tk, kind):
-    q, k, v = tensors(device, b, h, hkv, d, tk)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_of_any_lengths(device, b, h, hkv, d, tk, kind, dtype):
+    q, k, v = tensors(device, b, h, hkv, d, tk, dtype=dtype)
     lens = lengths(kind, b, tk)
     got = svod_amd.attention(q, k, v, Attn(keys=KeyMask.lens(lens.to(device, torch.int32))))
     assert close(got, exact(q, k, v, lens))
     wide = svod_amd.attention(q, k, v, Attn(keys=KeyMask.lens(lens.to(device))))
     assert (bits(wide) == bits(got)).all()
+
+
+@pytest.mark.parametrize("b,h,hkv,d,tk,unasked", [(*s, n) for s, n in zip(SHAPES, UNASKED)] +
+                         [(65, 4, 2, 64, 3200, 7), (16, 16, 8, 128, 1300, 4), (3, 16, 8, 128, 8500, 10)])
+def test_which_steps_share(device, b, h, hkv, d, tk, unasked):
+    """A step that shares its splits out sums rows of different lengths in other pieces than the same count for every row does,
+    which shows in some of its thousands of results; one that does not (more rows than lanes, a cache under 96 MiB, too few
+    rows) has that count's bits.  So the cases above run the kernel that they are about."""
+    q, k, v = tensors(device, b, h, hkv, d, tk, dtype=torch.float16)
+    for integers in (torch.int32, torch.int64):
+        keys = KeyMask.lens(lengths("wide", b, tk).to(device, integers))
+        got = svod_amd.attention(q, k, v, Attn(keys=keys))
+        named = svod_amd.attention(q, k, v, Attn(keys=keys, splits=unasked))
+        assert (bits(got) != bits(named)).any() == ((b, h, hkv, d, tk) in SHAPES)
 
 
 @pytest.mark.parametrize("b,h,hkv,d,tk", SHAPES)
@@ -70,8 +90,8 @@ def test_a_row_map_and_appended_rows(device, b, h, hkv, d, tk):
     assert close(got, exact(q, k, v, lens, rows, (ka, va), seen))
 
 
-def test_a_captured_step_whose_lengths_change(device):
-    b, h, hkv, d, tk = SHAPES[0]
+@pytest.mark.parametrize("b,h,hkv,d,tk", [SHAPES[0], SHAPES[5]])
+def test_a_captured_step_whose_lengths_change(device, b, h, hkv, d, tk):
     q, k, v = tensors(device, b, h, hkv, d, tk)
     lens, out = torch.empty(b, dtype=torch.int32, device=device), torch.empty_like(q)
     room = torch.empty(64 << 20, dtype=torch.uint8, device=device)
