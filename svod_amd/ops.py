@@ -227,7 +227,8 @@ class KeyMask:
 
     @staticmethod
     def lens(lens: torch.Tensor) -> "KeyMask":
-        """``[B]`` integer valid-key counts: keys at and past ``lens[b]`` are masked."""
+        """``[B]`` integer valid-key counts: keys at and past ``lens[b]`` are masked.  A row's result is its own keys', up to
+        its last bits: those may depend on the other rows' counts in a decoder step that names no ``Attn.splits``."""
         return KeyMask(1, lens)
 
     @staticmethod
@@ -250,7 +251,12 @@ class Cache:
 @dataclass
 class Attn:
     """``Attn`` of tk/src/ops/attention.rs:60-86.  ``batch_live`` stands for a bound
-    batch variable (``Batch::Var``): only the first ``batch_live`` batches run."""
+    batch variable (``Batch::Var``): only the first ``batch_live`` batches run.
+
+    ``splits`` ``None`` lets the library split the keys of a call with few queries.  In a decoder step of 4 to 64 rows with key
+    lengths over a cache of 96 MiB or more the rows then share the splits out by their lengths, so that a row's last bits
+    depend on how long the other rows are: the same sequence beside other neighbours may round differently.  A named count is
+    every row's, and 1 keeps the keys whole: a row's bits then depend on how many rows there are, not on their lengths."""
 
     causal: bool = False
     keys: KeyMask = KeyMask()
