@@ -1853,11 +1853,14 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     }
   }
   if (CAUSAL && !GROUPED) {
-    // The short tiles come last where the launch is more than one round of the workgroups that the chip holds: 8 sequences of
-    // 2048 queries and keys, 16 heads of 128 over 8, 163 -> 157 us, of 512 to 2048 keys 136 -> 134.5, 32 of 500 63 -> 60.5, 4 of
-    // 2048, 16 heads of 64, 49.5 -> 43.8 (half of the tiles as the quarter, all of them 3 % behind it: K and V stay
-    // in an L2 while a unit's tiles run together).
-    const bool short_last = kShortTilesLast<CAUSAL, SPLIT, RANGED, GROUPED> && blocks > 256 * (D <= 64 ? 3 : 2);
+    // The short tiles come last where the launch is more than one round of the workgroups that the chip holds, and a sixteenth:
+    // 8 sequences of 2048 queries and keys, 16 heads of 128 over 8, 163 -> 157 us, of 512 to 2048 keys 141.7 -> 137.5, 32 of 500 63
+    // -> 60.5, 4 of 2048, 16 heads of 64, 49.5 -> 43.8 (half of the tiles as the quarter, all of them 3 % behind it: K and V
+    // stay in an L2 while a unit's tiles run together).  Over 900 launches of four tiles and more a head, either order in turn: at
+    // 1.05 to 1.1 rounds 4 % less, at 1.1 to 1.8 5 % (single ones from a fifth less to a tenth more: which tiles share a compute unit
+    // is luck there), at 2 to 10 3 %; up to 1.05 rounds 1.5 % more at full lengths (20 of 578, 8 heads of 64, 21.3 -> 22.8).
+    constexpr int kRound = 256 * (D <= 64 ? 3 : 2);
+    const bool short_last = kShortTilesLast<CAUSAL, SPLIT, RANGED, GROUPED> && blocks > kRound + kRound / 16;
     geo.unit_size -= short_last ? geo.group * (geo.nqt / 4) : 0;
     geo.unit_rcp = rcp(geo.unit_size);
     geo.nqt_rcp = rcp(geo.group);
