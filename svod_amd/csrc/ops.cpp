@@ -331,20 +331,40 @@ int svodk_plan_heads(int32_t has_target, const int32_t *dtypes, int32_t n_dtypes
 // count that split_count answers (and svodk_attention_workspace counts with).  A round that is not full costs more than
 // its workgroups save: 16 sequences of 8 KV heads of 128 over 2100 keys take 28.3 us in 256 workgroups (4 splits), 31.6 in
 // 384, 30.3 in 512, 33 in 768; of 20 heads of 64 over 1500 keys 25.1 in 480 workgroups of two heads (3 splits), 24.2 in 480 of
-// four (6 splits), 27.5 in 640.  More than sixteen splits a merge takes a trip to memory more for: there a workgroup
-// rather takes fewer heads (one sequence over 8000 keys, 8 heads of 128: 12.8 us in 32 splits of one head, 16.4 in 64 of
-// two).  Below eight key blocks a merge costs what it saves (16 sequences over 400 keys 10.4 unsplit, 10.7 in 4 splits;
+// four (6 splits), 27.5 in 640.  Where two rounds are no seven eighths full, more are (14 sequences of 20 heads of 256 over 466
+// to 1865 keys 80.1 in one split, 280 workgroups, 64.4 in four; 25 of 16 of 128 over 442 to 1770 48.5 in two, 44.9 in five).
+// More than sixteen splits a merge takes a trip to memory more for, each sixteen of them: there a workgroup rather
+// takes fewer heads (one sequence over 8000 keys, 8 heads of 128: 12.8 us in 32 splits of one head, 16.4 in 64 of
+// two), and few (batch, KV head)s take them only where a split still has the keys for it (one head of 64 over 8000 keys: 8.1 us
+// in 16 splits, 8.9 in 32, 12.6 in 62; of 128 over 16000 12.2, 10.9, 12.8; of 256 over 32000 41.4, 25.3, 19.7).  Below eight
+// key blocks a merge costs what it saves (16 sequences over 400 keys 10.4 unsplit, 10.7 in 4 splits;
 // over 570 keys 22.8 and 20.1 in 3), and a split has at least 16 KiB of keys a head.
 static int decode_split_count(int64_t batch, int64_t kv_heads, int64_t d, int64_t tk, int rule) {
   const int64_t blocks = (tk + 63) / 64, units = kv_heads * batch, fits = std::min<int64_t>(blocks, blocks * d / 128);
   if (units <= 0 || blocks < 8) return 1;
+  const int64_t keys = tk * d, most = std::min<int64_t>(fits, 2 * rule);
+  const int64_t worth = keys < (units < 8 ? 960000 : 500000) ? 16 : keys < 3000000 ? 32 : keys < 6000000 ? 48 : 64;
   int64_t n = 1;
-  for (int h = svodk::decode_most_heads((int32_t)d, (uint32_t)kv_heads); h >= 0; h--) {
+  int h = svodk::decode_most_heads((int32_t)d, (uint32_t)kv_heads);
+  for (; h >= 0; h--) {
     const int64_t one = (256 << h) / units, two = (512 << h) / units;
     n = one * units >= (248 << h) || two > 16 ? one : two;
     if (n <= 16) break;
   }
-  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(n, 64), std::min<int64_t>(fits, 2 * rule)));
+  n = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(n, worth), most));
+  // Workgroups of the most heads over the places of the rounds that they make, in 65536ths.
+  auto fill = [&](int64_t splits) {
+    const int64_t workgroups = splits * units, round = 256 << std::max(h, 0);
+    return (workgroups << 16) / ((workgroups + round - 1) / round * round);
+  };
+  if (units * n > 256 << std::max(h, 0) && fill(n) < 7 << 13) {
+    int64_t best = fill(n);
+    for (int64_t more = n + 1; more <= std::min<int64_t>(most, 16) && best < 7 << 13; more++) {
+      const int64_t x = fill(more);
+      if (x > best) best = x, n = more;
+    }
+  }
+  return (int)n;
 }
 
 // split_ranked of tk/src/ops/attention.rs:405-410 for this library's one tile shape: a named

@@ -201,7 +201,7 @@ def test_with_no_count_named_few_query_tiles_over_many_keys_are_split():
         assert got == (0 if want == 1 else want * b * tq * h * (64 + 2) * 4), (b, tq, h, tk)
 
 
-@pytest.mark.parametrize("b,hkv,h,d,tk,want", [(64, 8, 8, 128, 1024, 0), (34, 16, 16, 128, 1024, 0), (60, 8, 8, 128, 1024, 2),
+@pytest.mark.parametrize("b,hkv,h,d,tk,want", [(64, 8, 8, 128, 1024, 0), (32, 16, 16, 128, 1024, 0), (60, 8, 8, 128, 1024, 2),
                                                (25, 20, 20, 64, 600, 2)])
 def test_a_step_that_runs_whole_asks_for_no_workspace(b, hkv, h, d, tk, want):
     """Decoder steps of which the rule makes two splits and a full round of workgroups one or two."""
