@@ -1253,8 +1253,14 @@ __device__ __forceinline__ void flash_fwd_body(
   // filling and meeting the barriers.  Blocks [0, my_end) are this wave's.  So does a wave of a call's last tile whose
   // rows are past the last query (three of four waves at 777 queries): the waves beside it on its SIMD have its issue slots
   // (1500 queries 224.4 -> 222.3 us, 64 rows of 40 queries 9.27 -> 9.07).
+  // With a bias and nothing that ends a wave's blocks ahead of the tile's, such a wave takes the loop of its own instead
+  // (`computes`), and the others' is known to end with the tile: behind a count of blocks a wave, a step with a bias was 2 to 6 %
+  // slower (2 sequences of 562, 2 heads of 64, 37.7 -> 39.9, now 37.7 us; 28 of 997, 8 of 128, 490 -> 501, now 490).  Without
+  // one it gains nothing (32 x 512 38.1 -> 36.8, 16 x 1500 209.7 -> 210.9, 64 x 40 7.16 -> 7.28).
+  constexpr bool kApart = BIASED && !RANGED && !CAUSAL;
   const int tile_rows = GROUPED ? (int)geo.group * t : t;
-  int my_end = q_off + w.wave * kWaveRows < tile_rows ? end : 0;
+  const bool has_rows = q_off + w.wave * kWaveRows < tile_rows, computes = !kApart || has_rows;
+  int my_end = kApart || has_rows ? end : 0;
   if (RANGED || CAUSAL) {
     // The last key the wave's last row sees; negative: the blocks lie past every row's reach.
     const int last_seen = RANGED ? w.hi_last : w.wave_first_row + kWaveRows - 1;
@@ -1266,7 +1272,7 @@ __device__ __forceinline__ void flash_fwd_body(
   int seen = 0;
 #pragma unroll
   for (int i = 0; i < 32; i++) sv[i] = nv[i] = 0.0f;
-  if (my_end > 0) {
+  if (computes && my_end > 0) {
     uint32_t bw[16];
     if (BIASED) load_bias<D, NW>(w, 0, q_ok, bw);
     scores<D, NW>(w, smem, 0, sv);
@@ -1304,11 +1310,13 @@ __device__ __forceinline__ void flash_fwd_body(
     for (; blk < lead; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   }
   // (The blocks of these steps and the one behind them are whole: `seen` is 3 before and after.)
-  for (; blk + 2 < full; blk += 2) {
-    hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
-    hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
+  if (computes) {
+    for (; blk + 2 < full; blk += 2) {
+      hot_step<D, NW, 0>(w, smem, blk, sv, nv, bm);
+      hot_step<D, NW, 1>(w, smem, blk + 1, nv, sv, bm);
+    }
+    for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   }
-  for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   for (; blk < end; blk++) idle_step<D, NW>(w, blk);
 
   // ---- the appended rows (L739-755, L827-846): one more block of keys, from their own tensors,

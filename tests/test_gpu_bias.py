@@ -140,3 +140,22 @@ def test_climbing_scores_rescale_the_accumulator(device, per_key, causal):
     assert svod_amd.chosen().startswith('Kernel { op: "attention"'), svod_amd.chosen()
     p = oracle.AttnProblem(q, k, v, causal=causal, bias=bias)
     assert_bf16_parity("climbing bias", to_np(got), oracle.attention_direct(p), oracle.attention_flash(p, bq=128, bkv=64))
+
+
+@pytest.mark.parametrize("t", [1, 31, 33, 65, 97, 128, 129, 193, 225])
+@pytest.mark.parametrize("d,lens,splits", [(64, None, 1), (64, [330, 0, 64], 1), (128, [330, 65, 1], 1), (64, None, 2), (32, [330, 129, 7], 1)])
+def test_waves_past_the_last_query_keep_the_ring(device, t, d, lens, splits):
+    """A tile's waves own 32 queries each: of these counts one to three of the last tile's four have none, over an odd and an even
+    count of key blocks, and of a row without keys no wave has a block.  Four heads of a KV head share a tile of up to 32
+    queries each."""
+    name = f"{t} queries of {d}, {lens}, {splits} splits"
+    for h, hkv in ((2, 2), (4, 1)):
+        got, p = run(device, 3, t, 330, h, hkv, d, 1, {}, lens, splits)
+        assert_bf16_parity(name, to_np(got), oracle.attention_direct(p), oracle.attention_flash(p, bq=128, bkv=64, splits=splits))
+    shown = np.arange(330)[None, :] % 97 != np.arange(3)[:, None]  # a hidden key in most blocks
+    q, k, v, bias = case(3, t, 330, 2, 2, d, 1)
+    up = lambda x: bf16_tensor(x, device)
+    keys = KeyMask.bool(torch.from_numpy(shown).to(device))
+    got = svod_amd.attention(up(q), up(k), up(v), Attn(keys=keys, bias=up(bias), splits=splits))
+    p = oracle.AttnProblem(q, k, v, key_mask=shown, bias=bias)
+    assert_bf16_parity(name, to_np(got), oracle.attention_direct(p), oracle.attention_flash(p, bq=128, bkv=64, splits=splits))
