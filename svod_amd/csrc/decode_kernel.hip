@@ -52,24 +52,6 @@ constexpr int kMostSharingRows = 64;  // a lane a row
 // Waves a workgroup: few workgroups take eight each, so that the launch still has its bytes in flight.
 // `heads_splits`: (batch, KV head, split)s of the launch.
 __host__ __device__ constexpr int decode_waves(uint32_t heads_splits) { return heads_splits >= 256 ? 4 : kMaxWaves; }
-// KV heads a workgroup takes (log2): the most (decode_most_heads) with which the workgroups fill seven eighths of the rounds
-// that they make over 256 compute units, or else what fills them best; every compute unit has one.  64 sequences of 20
-// heads of 64 over 1000 keys: 44.9 us in 320 workgroups of four heads, 40.7 in 1280 of one; 16 over 1500 keys in six splits
-// 29.2 in 1920 of one, 24.5 in 480 of four.  A head of 32 is 64 bytes, half a line of memory: two together whenever they may
-// (22 sequences of 16 heads over 340 to 1360 keys 20.2 us in 1056 workgroups of one, 12.2 in 704 of two).
-__host__ __device__ constexpr int heads_together(int d, uint32_t heads_splits, uint32_t kv_heads) {
-  int best = 0, best_fill = -1;
-  for (int n = decode_most_heads(d, kv_heads); n >= 0 && best_fill < 14; n--) {
-    const uint32_t workgroups = heads_splits >> n;
-    if (n > 0 && workgroups < 256) continue;
-    if (d == 32 && n == 0 && best > 0) break;
-    // In sixteenths of the rounds' places; four rounds and more even out by themselves.
-    const int fill = workgroups >= 1024 ? 16 : (int)(workgroups * 16 / ((workgroups + 255) / 256 * 256));
-    if (fill > best_fill) best = n, best_fill = fill;
-  }
-  return best;
-}
-
 // What the kernel takes: AttnArgs without the fields a decoder step does not have.
 struct DecodeArgs {
   const uint16_t *q, *k, *v;

@@ -177,6 +177,23 @@ constexpr int decode_most_heads(int32_t d, uint32_t kv_heads) {
   while ((d == 48 ? 64 : d) << (n + 1) <= 256 && n < 2 && kv_heads % (2u << n) == 0) n++;
   return n;
 }
+// KV heads a workgroup takes (log2): the most (decode_most_heads) with which the workgroups fill seven eighths of the rounds
+// that they make over 256 compute units, or else what fills them best; every compute unit has one.  64 sequences of 20
+// heads of 64 over 1000 keys: 44.9 us in 320 workgroups of four heads, 40.7 in 1280 of one; 16 over 1500 keys in six splits
+// 29.2 in 1920 of one, 24.5 in 480 of four.  A head of 32 is 64 bytes, half a line of memory: two together whenever they may
+// (22 sequences of 16 heads over 340 to 1360 keys 20.2 us in 1056 workgroups of one, 12.2 in 704 of two).
+constexpr int heads_together(int d, uint32_t heads_splits, uint32_t kv_heads) {
+  int best = 0, best_fill = -1;
+  for (int n = decode_most_heads(d, kv_heads); n >= 0 && best_fill < 14; n--) {
+    const uint32_t workgroups = heads_splits >> n;
+    if (n > 0 && workgroups < 256) continue;
+    if (d == 32 && n == 0 && best > 0) break;
+    // In sixteenths of the rounds' places; four rounds and more even out by themselves.
+    const int fill = workgroups >= 1024 ? 16 : (int)(workgroups * 16 / ((workgroups + 255) / 256 * 256));
+    if (fill > best_fill) best = n, best_fill = fill;
+  }
+  return best;
+}
 // What a decoder step that merges its own splits, kMostMergedSplits at most, needs behind the partial states: a word a
 // (batch, KV head), on a line of its own (16 sequences of 8 KV heads in 4 splits: 28.9 us, 29.5 with 16 words a line).
 constexpr int kMostMergedSplits = 64;
