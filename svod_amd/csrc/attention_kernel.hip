@@ -753,6 +753,10 @@ struct Geometry {
 // The instantiations whose launches may run the short tiles of all units behind the others.
 template <bool CAUSAL, bool SPLIT, bool RANGED, bool GROUPED>
 constexpr bool kShortTilesLast = CAUSAL && !GROUPED && !SPLIT && !RANGED;
+// The instantiations whose last round of units, where it is not full, is shared out over all XCDs.  Causal ones deal it
+// whole: their tiles differ, and an XCD's run of them would be the long or the short ones.
+template <bool CAUSAL>
+constexpr bool kSharesLastRound = !CAUSAL;
 // The key splits of a launch that has them, and where their partial states go.
 struct Splits {
   uint32_t count, rcp;
@@ -847,7 +851,28 @@ __device__ __forceinline__ void flash_fwd_body(
   const uint32_t wg = __builtin_amdgcn_workgroup_id_x();
   const uint32_t local = wg / kXcds;
   uint32_t round = div_by(local, geo.unit_size, geo.unit_rcp);
-  const uint32_t within = local - round * geo.unit_size;
+  uint32_t within = local - round * geo.unit_size;
+  // Which unit of a round an XCD takes turns with the round: with a power-of-two head count a
+  // fixed deal would hand an XCD the same heads in every batch row, i.e. always the same 128-byte
+  // residues of every K, V, Q and O row, and the XCD whose residues share a memory channel with
+  // other traffic then runs a tenth behind the rest (measured: whichever XCD read bytes 384..511
+  // of every KiB); turned, every XCD reads every residue and they finish together.
+  uint32_t unit = round * kXcds + (wg + round) % kXcds;
+  if constexpr (kSharesLastRound<CAUSAL>) {
+    // The units of a round that is not full are every XCD's: their workgroups, one unit's after the other's, in eight equal
+    // runs.  Dealt whole, the XCDs that took one of them ran that much longer: one sequence of 12 heads of 64 over 8192 keys
+    // 302 -> 233 us, 3 of 777 20.0 -> 14.8, one of 20 heads over 1500 31.0 -> 23.3, of 10 heads of 128 over 2 over 3000 (two XCDs
+    // of eight at work) 148 -> 60; with 13 sequences of 700 (20 heads: 4 units of 260) 55.6 -> 54.9, at 8 and more rounds equal.
+    // A run lies in few units, so a unit's K and V are read by 8 / (units left) L2s, not by all.
+    if (round >= geo.units / kXcds) {
+      const uint32_t first = geo.units / kXcds, left = (geo.units - first * kXcds) * geo.unit_size;
+      const uint32_t run = (left + kXcds - 1) / kXcds, in = local - first * geo.unit_size, at = wg % kXcds * run + in;
+      if (in >= run || at >= left) return;  // a code object's grid is of whole rounds
+      const uint32_t over = div_by(at, geo.unit_size, geo.unit_rcp);
+      unit = first * kXcds + over;
+      within = at - over * geo.unit_size;
+    }
+  }
   uint32_t head_in_group;
   int order;
   if constexpr (CAUSAL && !GROUPED) {
@@ -869,18 +894,13 @@ __device__ __forceinline__ void flash_fwd_body(
         round = at - tile * rounds;
         head_in_group = in - at * geo.group;
         order = (int)(div_by(geo.unit_size, geo.group, geo.nqt_rcp) + tile);
+        unit = round * kXcds + (wg + round) % kXcds;
       }
     }
   } else {
     head_in_group = div_by(within, geo.nqt, geo.nqt_rcp);
     order = (int)(within - head_in_group * geo.nqt);
   }
-  // Which unit of a round an XCD takes turns with the round: with a power-of-two head count a
-  // fixed deal would hand an XCD the same heads in every batch row, i.e. always the same 128-byte
-  // residues of every K, V, Q and O row, and the XCD whose residues share a memory channel with
-  // other traffic then runs a tenth behind the rest (measured: whichever XCD read bytes 384..511
-  // of every KiB); turned, every XCD reads every residue and they finish together.
-  const uint32_t unit = round * kXcds + (wg + round) % kXcds;
   if (unit >= geo.units) return;
   const int b_place = (int)div_by(unit, geo.kv_heads, geo.kvh_rcp);
   const int kvh = (int)(unit - (uint32_t)b_place * geo.kv_heads);  // L548: query head h reads KV head h / (heads / kv_heads)
@@ -1828,11 +1848,12 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   const int64_t kv_row = a.kv_row_elems > 0 ? a.kv_row_elems : (int64_t)a.kv_heads * a.d;
   // A fill addresses the rows of one key block with 32-bit byte offsets from the block's 64-bit base.
   if (kv_row * 2 * kBkv > 0x7fffffffLL || q_row > 0x7fffffffLL) return hipErrorInvalidValue;
-  // Units of work (batch, KV head) are dealt over the XCDs in whole rounds; the workgroups of
-  // a round's missing units exit at once.
+  // Units of work (batch, KV head) are dealt over the XCDs in whole rounds; those of a round that is not full are shared
+  // out, or (a causal launch) the workgroups of its missing units exit at once.
   const int64_t unit_size = (int64_t)(GROUPED ? 1 : a.heads / a.kv_heads) * nqt;
   const int64_t units = (int64_t)a.kv_heads * a.batch;
-  const int64_t grid = (units + kXcds - 1) / kXcds * kXcds * unit_size;
+  const int64_t dealt = kSharesLastRound<CAUSAL> ? units * unit_size : (units + kXcds - 1) / kXcds * kXcds * unit_size;
+  const int64_t grid = (dealt + kXcds - 1) / kXcds * kXcds;
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   auto rcp = [](uint32_t d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); };
   Geometry geo;
