@@ -112,7 +112,8 @@ typedef struct svodk_cache {
  * SVODK_GRAPH_CONFIG.  `splits` = 1 keeps the keys whole.  `splits` = 0 (None)
  * lets the library choose, as the reference's tuner would: it splits calls with
  * few query tiles and many keys (a decoder step) when the workspace
- * svodk_attention_workspace asks for is lent, and keeps the keys whole without it.
+ * svodk_attention_workspace asks for is lent, and keeps them in one workgroup a query tile without it; where those
+ * are no more than the compute units, a tile's key blocks go in two halves merged on the chip (by the call's sizes alone).
  * A decoder step (svodk_tune_decode) of up to 64 splits merges them itself, in the one launch, where
  * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  With `splits` = 0 and
  * twice the bytes and those words it takes the count that suits the device, up to twice the rule's (other

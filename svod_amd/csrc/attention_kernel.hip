@@ -822,8 +822,10 @@ struct TailOf {
 // ring, and behind it mask_lds() of a launch with a key mask).  Device code only:
 // the host pass needs a kernel's handle, not its instructions (and would drop the whole
 // instantiation over the LDS-fill instructions).
+// SIDES = 2: eight waves a tile instead of four.  Each side of four has a ring of its own and takes half of the tile's key
+// blocks; the sides' states merge through LDS (flash_fwd_pair_kernel).
 #if defined(__HIP_DEVICE_COMPILE__)
-template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16>
+template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16, int SIDES = 1>
 __device__ __forceinline__ void flash_fwd_body(
     uint8_t *smem, uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u,
     uint32_t kvh_rcp, uint32_t units, uint32_t heads_group, const void *__restrict__ key_lens,
@@ -960,6 +962,13 @@ __device__ __forceinline__ void flash_fwd_body(
   const int tid = __builtin_amdgcn_workitem_id_x();
   w.lane = tid & 63;
   w.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int side = 0;
+  if (SIDES == 2) {
+    static_assert(SIDES == 1 || (!SPLIT && !RANGED && !BIASED && !CACHED && !GROUPED && W::DB % 2 == 0), "plain tiles only");
+    side = w.wave / NW;
+    w.wave %= NW;
+    smem += side * TL::kLds;
+  }
   w.g = w.lane >> 5;           // half-wave: the k-chunk of MFMA operands
   const int ln = w.lane & 31;  // the query column this lane owns
 
@@ -1036,6 +1045,15 @@ __device__ __forceinline__ void flash_fwd_body(
     const int s_first = first + (int)div_by(n * (uint32_t)split, sp.count, sp.rcp);
     end = first + (int)div_by(n * (uint32_t)(split + 1), sp.count, sp.rcp);
     first = s_first;
+  }
+  // A side takes half of them, in the same way; both meet as many barriers as the first, which has no fewer.
+  int steps = 0;
+  if (SIDES == 2) {
+    steps = (end - first + 1) / 2;
+    if (side == 0)
+      end = first + steps;
+    else
+      first += steps;
   }
   const int first_key = first * kBkv;
   end -= first;
@@ -1337,7 +1355,7 @@ __device__ __forceinline__ void flash_fwd_body(
     }
     for (; blk < my_end; blk++) edge_step<D, NW, CAUSAL>(w, smem, blk, my_end, sv, bm, seen);
   }
-  for (; blk < end; blk++) idle_step<D, NW>(w, blk);
+  for (; blk < (SIDES == 2 ? steps : end); blk++) idle_step<D, NW>(w, blk);
 
   // ---- the appended rows (L739-755, L827-846): one more block of keys, from their own tensors,
   // which only the last split scores; the first `seen` of them are visible and no other mask
@@ -1391,7 +1409,42 @@ __device__ __forceinline__ void flash_fwd_body(
   }
 
   const Pair lp = both_halves(w.l_run);
-  const float l_tot = lp.a + lp.b;
+  float l_tot = lp.a + lp.b;
+  if constexpr (SIDES == 2) {
+    // ---- the sides' states as one, by the rule that merges key splits (L948-969).  A side finishes half of the columns:
+    // it hands its accumulators of the other half over in its own ring, which every wave is past the last step's reads of.
+    constexpr int HB = DB / 2;
+    f32x4 *const out = (f32x4 *)smem + w.wave * (HB * 4 + 1) * 64 + w.lane;
+    const f32x4 *const in = (const f32x4 *)(smem + (side == 0 ? TL::kLds : -TL::kLds)) + w.wave * (HB * 4 + 1) * 64 + w.lane;
+#pragma unroll
+    for (int db = 0; db < HB; db++) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const float lower = w.acc[db][i], upper = w.acc[HB + db][i];
+        w.acc[db][i] = side == 0 ? lower : upper;
+        w.acc[HB + db][i] = side == 0 ? upper : lower;
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        out[(db * 4 + c) * 64] = f32x4{w.acc[HB + db][4 * c], w.acc[HB + db][4 * c + 1], w.acc[HB + db][4 * c + 2], w.acc[HB + db][4 * c + 3]};
+    }
+    out[HB * 4 * 64] = f32x4{w.m_run, l_tot, 0.0f, 0.0f};
+    __syncthreads();
+    const f32x4 ml = in[HB * 4 * 64];
+    // A side that no key of the row lies in has m = -1e30 and l = 0: its weight is 0, or 1 beside another such.
+    const float m = __builtin_fmaxf(w.m_run, ml[0]);
+    const float mine = fast_exp2((w.m_run - m) * w.unit), other = fast_exp2((ml[0] - m) * w.unit);
+    l_tot = l_tot * mine + ml[1] * other;
+#pragma unroll
+    for (int db = 0; db < HB; db++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const f32x4 x = in[(db * 4 + c) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) w.acc[db][4 * c + e] = w.acc[db][4 * c + e] * mine + x[e] * other;
+      }
+    o += side * 32 * HB;  // this side's columns
+  }
   if (SPLIT) {
     // ---- the split's partial state (L899-921): the accumulator as it stands, the maximum in
     // the exponent's units (L848-853) and the sum.
@@ -1421,7 +1474,7 @@ __device__ __forceinline__ void flash_fwd_body(
   // at a time: the lower half the even runs of eight, the upper half the odd ones.
   uint16_t *o_ptr = o + ((int64_t)b * t + q_row) * o_row_stride + (int64_t)q_head * D + 8 * w.g;
 #pragma unroll
-  for (int db = 0; db < DB; db++) {
+  for (int db = 0; db < DB / SIDES; db++) {
 #pragma unroll
     for (int c = 0; c < 4; c += 2) {
       if (32 * db + 8 * c >= D) continue;  // the tile's columns past the head (a head of 48: its last 16)
@@ -1465,6 +1518,27 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 :
       tail.mask_bytes, tail.scale, sp, tail.q_row_elems, tail.kv_row_elems, rg);
 #endif
 }
+
+#if !defined(SVODK_CODE_OBJECT)
+// Eight waves a query tile, two a SIMD, where a launch has no more workgroups than the chip has compute units (launch() says
+// when): plain calls, with key lengths or none.  Bound by the steps of a tile in a row, as the form of four waves is
+// there; two waves of a SIMD hide each other's waits (a step of a side 1.2 times as long as alone, for half of them).
+template <int D, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED>
+constexpr bool kHasPair = (D == 64 || D == 128) && !SPLIT && !RANGED && !BIASED && !GROUPED;
+template <int D, bool CAUSAL, bool F16>
+__global__ __launch_bounds__(512, 2) void flash_fwd_pair_kernel(
+    uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u, uint32_t kvh_rcp,
+    uint32_t units, uint32_t heads_group, uint64_t key_lens, uint64_t row_order, int32_t t, uint32_t tk_lens64,
+    TailOf<false, false, false> tail) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  flash_fwd_body<D, 4, CAUSAL, false, false, false, false, false, F16, 2>(
+      smem, unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, units, heads_group, constant<void>(key_lens),
+      constant<int32_t>(row_order), t, tk_lens64, tail.q, tail.k, tail.v, tail.o, nullptr, 1, tail.scale, Splits{},
+      tail.q_row_elems, tail.kv_row_elems, Ranges{});
+#endif
+}
+#endif
 
 // Over a cache, with the addresses as arguments of their own: of a struct's the compiler cannot tell that nothing writes
 // what they name, and the appended rows' count, read behind the loop's fills, is then no scalar load.
@@ -1947,6 +2021,22 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
     const TailOf<SPLIT, RANGED, BIASED> tail = {(const uint16_t *)a.q, (const uint16_t *)a.k, (const uint16_t *)a.v,
                                                 (uint16_t *)a.o, a.mask_bytes, a.scale, (int32_t)q_row,
                                                 (int32_t)kv_row, split_args, range_args};
+    if constexpr (kHasPair<D, SPLIT, RANGED, BIASED, GROUPED>) {
+      // A compute unit with one workgroup has a wave a SIMD, and a tile's steps are a chain: two sides of four waves take half of
+      // the steps each.  Both sides together step a fifth faster than one alone, so it is worth its merge (0.5 to 1 us) from
+      // nine key blocks on (16 heads of 64: one sequence of 512 9.66 -> 9.40 us, of 768 12.7 -> 11.8, of 1500 22.0 -> 19.4, of 2048 28.6
+      // -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
+      // one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long
+      // causal launches at d 128 win by, whose tiles would otherwise end far apart (512 workgroups of 16 tiles a head 59.4 -> 51.9, 384
+      // of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Where the streaming knob is set it says what runs.
+      const bool fits = grid <= 256 || (CAUSAL && D == 128 && grid <= 512 && nqt >= 12);
+      if (a.halves && a.key_mask == nullptr && fits && a.tk > 8 * kBkv &&
+          (D != 64 || g_stream_slots.load(std::memory_order_relaxed) == 0))
+        return Launch<flash_fwd_pair_kernel<D, CAUSAL, F16>>::run(
+            grid, 512, 2 * TL::kLds, 2 * TL::kLds, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads,
+            geo.kvh_rcp, units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t,
+            tk_lens64, tail);
+    }
     return Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
         grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
         units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64,
