@@ -390,8 +390,12 @@ static int decode_split_count(int64_t batch, int64_t kv_heads, int64_t d, int64_
 // unsplit -> rule's count): 16 workgroups x 128 blocks 101.6 -> 24.2 (16 splits), 32 x 128
 // 151.5 -> 29.8 (16), 64 x 32 28.7 -> 16.8 (4), 64 x 64 82.7 -> 37.6 (8), 256 x 64 86.2 -> 67.4
 // (2), 320 x 24 32.7 -> 28.6 (2); from 640 workgroups on the rule answers one, which is fastest.
+// Those are a query or a few a tile.  What a split costs is its merge's launch, 2.5 us, and its rows' partial states, written and
+// read again at 0.65 us a MB; what it saves are steps of 0.25 + 0.0072 d us, and where tiles are full none past a workgroup
+// a compute unit.  So the count is the one with the least of both: one sequence of 16 heads of 64 over 1024 keys 18.3 us in two
+// splits, 15.1 in one, of 2048 35.4 and 27.0, two of 1024 26.7 and 16.1; of 128 over 8, causal, two of 1024 36.0 and 22.7.
 // A window, a chunk mask or segment starts leave a tile few of the keys: the rule keeps those whole.
-static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t heads, int64_t kv_heads, int64_t tk,
+static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t heads, int64_t kv_heads, int64_t d, int64_t tk,
                        int32_t decode_limit) {
   const int32_t asked = opts->splits;
   const int64_t most = tk > 0 ? (tk + 63) / 64 : 1;
@@ -416,8 +420,19 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
   if (workgroups <= 0) return 1;
   const int64_t wanted = (512 + workgroups / 2) / workgroups;  // rounded
   const int64_t fits = most / 8;
-  const int64_t n = wanted < fits ? wanted : fits;
-  return (int)(n < 1 ? 1 : (n > 64 ? 64 : n));
+  const int64_t n = std::min<int64_t>(std::min(wanted, fits), 64);
+  const int64_t tile_rows = std::min<int64_t>(grouped ? group * t : t, 128);
+  const double chain = (double)most * (0.25 + 0.0072 * (double)d);
+  const double states = (double)(batch * t * heads * (d + 2) * 4) * 0.65e-6;
+  auto cost = [&](int64_t s) {
+    // A tile of one wave's rows waits for its keys, which more workgroups hide; a fuller one for its compute unit.
+    const double rounds = tile_rows <= 32 ? 1.0 : std::max(1.0, (double)(workgroups * s) / 256);
+    return chain / (double)s * rounds + (s > 1 ? 2.5 + states * (double)s : 0.0);
+  };
+  int64_t best = 1;
+  for (int64_t s = 2; s <= n; s++)
+    if (cost(s) < cost(best)) best = s;
+  return (int)best;
 }
 
 // attend (tk/src/ops/attention.rs:126-303): attention of q, k and v, or of the `packed` operand
@@ -722,7 +737,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
   // L280-302: key splits.  The partial tensors live in the caller's workspace.
   const int32_t decode_limit = svodk::attention_decode_limit();
   a.decodes = svodk::attention_decodes(a, decode_limit);
-  a.splits = split_count(opts, a.batch, t, heads, kv_heads, tk, decode_limit);
+  a.splits = split_count(opts, a.batch, t, heads, kv_heads, d, tk, decode_limit);
   void *workspace = opts->workspace;
   int64_t workspace_bytes = opts->workspace_bytes;
   // What a decoder step rather takes than the rule's count, where there is room for it: a caller that lends what
@@ -877,7 +892,7 @@ int64_t svodk_attention_workspace(const svodk_tensor *q, const svodk_tensor *k, 
   const int64_t batch = opts->batch_live > 0 ? opts->batch_live : q->shape[0];
   const int64_t kv_heads = opts->cache != nullptr ? opts->cache->kv_heads : k->shape[2];
   const int32_t decode_limit = svodk::attention_decode_limit();
-  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, k->shape[1], decode_limit);
+  const int splits = split_count(opts, batch, q->shape[1], q->shape[2], kv_heads, q->shape[3], k->shape[1], decode_limit);
   if (splits <= 1) return 0;
   // A decoder step that names no count may take fewer, down to none (attend()).
   const int64_t rows = kv_heads > 0 && q->shape[2] % kv_heads == 0 ? q->shape[2] / kv_heads * q->shape[1] : 0;

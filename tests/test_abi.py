@@ -201,6 +201,20 @@ def test_with_no_count_named_few_query_tiles_over_many_keys_are_split():
         assert got == (0 if want == 1 else want * b * tq * h * (64 + 2) * 4), (b, tq, h, tk)
 
 
+@pytest.mark.parametrize("b,tq,h,hkv,d,tk,causal,want", [
+    (1, 1024, 16, 16, 64, 1024, False, 1), (2, 1024, 16, 8, 128, 1024, True, 1),  # full tiles that half fill the chip
+    (1, 200, 16, 16, 64, 8192, False, 8),   # no more workgroups than compute units
+    (8, 128, 20, 20, 64, 1500, False, 1),   # the states cost more than the steps
+    (1, 448, 20, 20, 64, 1500, False, 3),
+    (4, 8, 20, 20, 64, 1500, False, 3),     # a few queries each: short states
+    (2, 16, 16, 2, 128, 4096, False, 8),    # a group a tile
+])
+def test_splits_are_worth_their_partial_states(b, tq, h, hkv, d, tk, causal, want):
+    workspace = svod_amd.ops._calls().attention_workspace
+    got = workspace(t([b, tq, h, d]), t([b, tk, hkv, d]), Attn(causal=causal))
+    assert got == (0 if want == 1 else want * b * tq * h * (d + 2) * 4)
+
+
 @pytest.mark.parametrize("b,hkv,h,d,tk,want", [(64, 8, 8, 128, 1024, 0), (32, 16, 16, 128, 1024, 0), (60, 8, 8, 128, 1024, 2),
                                                (25, 20, 20, 64, 600, 2)])
 def test_a_step_that_runs_whole_asks_for_no_workspace(b, hkv, h, d, tk, want):
