@@ -1143,9 +1143,11 @@ __device__ __forceinline__ void flash_fwd_body(
   // workgroup's 12.5 at 32 rows of 512 keys, 3.4 so; the launch 37.6 -> 36.7.)
   // The elements of the first two are asked for now, a lane a key, straight into this wave's stretch of LDS: behind the
   // Q loads and ahead of the fills in the memory counter's order, so that they can be waited for with the fills in flight.
-  w.mask_words = (LDS_PTR(uint64_t))(smem + TL::kLds);
+  // (Of two sides each scans its own blocks, into a stretch of its own behind both rings.)
+  uint8_t *const mask_smem = smem + (SIDES - side) * TL::kLds + side * mask_lds(NW);
+  w.mask_words = (LDS_PTR(uint64_t))(mask_smem);
   w.scanned = key_mask != nullptr && end <= kScannedBlocks && end > 0;
-  LDS_PTR(int) raw = (LDS_PTR(int))(smem + TL::kLds + kScannedBlocks * 8) + w.wave * kRawElements;
+  LDS_PTR(int) raw = (LDS_PTR(int))(mask_smem + kScannedBlocks * 8) + w.wave * kRawElements;
   if (w.scanned) {
     const uint8_t *row = (const uint8_t *)key_mask + w.mask_row * mask_bytes;
     const i32x4 r = make_rsrc(row, (int64_t)w.tk * mask_bytes);  // keys past the row read as hidden
@@ -1521,21 +1523,21 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 :
 
 #if !defined(SVODK_CODE_OBJECT)
 // Eight waves a query tile, two a SIMD, where a launch has no more workgroups than the chip has compute units (launch() says
-// when): plain calls, with key lengths or none.  Bound by the steps of a tile in a row, as the form of four waves is
+// when): plain calls, with key lengths, a key mask or none.  Bound by the steps of a tile in a row, as the form of four waves is
 // there; two waves of a SIMD hide each other's waits (a step of a side 1.2 times as long as alone, for half of them).
 template <int D, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED>
 constexpr bool kHasPair = (D == 64 || D == 128) && !SPLIT && !RANGED && !BIASED && !GROUPED;
-template <int D, bool CAUSAL, bool F16>
+template <int D, bool CAUSAL, bool F16, bool MASKED>
 __global__ __launch_bounds__(512, 2) void flash_fwd_pair_kernel(
     uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u, uint32_t kvh_rcp,
     uint32_t units, uint32_t heads_group, uint64_t key_lens, uint64_t row_order, int32_t t, uint32_t tk_lens64,
-    TailOf<false, false, false> tail) {
+    const void *__restrict__ key_mask, TailOf<false, false, false> tail) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   flash_fwd_body<D, 4, CAUSAL, false, false, false, false, false, F16, 2>(
       smem, unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, units, heads_group, constant<void>(key_lens),
-      constant<int32_t>(row_order), t, tk_lens64, tail.q, tail.k, tail.v, tail.o, nullptr, 1, tail.scale, Splits{},
-      tail.q_row_elems, tail.kv_row_elems, Ranges{});
+      constant<int32_t>(row_order), t, tk_lens64, tail.q, tail.k, tail.v, tail.o, MASKED ? key_mask : nullptr,
+      MASKED ? tail.mask_bytes : 1, tail.scale, Splits{}, tail.q_row_elems, tail.kv_row_elems, Ranges{});
 #endif
 }
 #endif
@@ -2028,14 +2030,21 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
       // -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
       // one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long
       // causal launches at d 128 win by, whose tiles would otherwise end far apart (512 workgroups of 16 tiles a head 59.4 -> 51.9, 384
-      // of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Where the streaming knob is set it says what runs.
+      // of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Under a key mask the sides halve the blocks before
+      // the row is read: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two of 1024 15.8 -> 13.9; 4 of 513, 12
+      // heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.  Only a lone row that hides its second half leaves a side
+      // idle (1024: 10.1 -> 10.7).  Where the streaming knob is set it says what runs.
       const bool fits = grid <= 256 || (CAUSAL && D == 128 && grid <= 512 && nqt >= 12);
-      if (a.halves && a.key_mask == nullptr && fits && a.tk > 8 * kBkv &&
-          (D != 64 || g_stream_slots.load(std::memory_order_relaxed) == 0))
-        return Launch<flash_fwd_pair_kernel<D, CAUSAL, F16>>::run(
-            grid, 512, 2 * TL::kLds, 2 * TL::kLds, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads,
-            geo.kvh_rcp, units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t,
-            tk_lens64, tail);
+      if (a.halves && fits && a.tk > 8 * kBkv && (D != 64 || g_stream_slots.load(std::memory_order_relaxed) == 0)) {
+        auto pair = [&](auto launcher, int lds) {
+          return decltype(launcher)::run(grid, 512, lds, lds, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads,
+                                         geo.kvh_rcp, units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens,
+                                         (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64, a.key_mask, tail);
+        };
+        if (a.key_mask != nullptr)
+          return pair(Launch<flash_fwd_pair_kernel<D, CAUSAL, F16, true>>{}, 2 * (TL::kLds + mask_lds(NW)));
+        return pair(Launch<flash_fwd_pair_kernel<D, CAUSAL, F16, false>>{}, 2 * TL::kLds);
+      }
     }
     return Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
         grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
