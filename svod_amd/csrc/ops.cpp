@@ -390,10 +390,15 @@ static int decode_split_count(int64_t batch, int64_t kv_heads, int64_t d, int64_
 // unsplit -> rule's count): 16 workgroups x 128 blocks 101.6 -> 24.2 (16 splits), 32 x 128
 // 151.5 -> 29.8 (16), 64 x 32 28.7 -> 16.8 (4), 64 x 64 82.7 -> 37.6 (8), 256 x 64 86.2 -> 67.4
 // (2), 320 x 24 32.7 -> 28.6 (2); from 640 workgroups on the rule answers one, which is fastest.
-// Those are a query or a few a tile.  What a split costs is its merge's launch, 2.5 us, and its rows' partial states, written and
-// read again at 0.65 us a MB; what it saves are steps of 0.25 + 0.0072 d us, and where tiles are full none past a workgroup
-// a compute unit.  So the count is the one with the least of both: one sequence of 16 heads of 64 over 1024 keys 18.3 us in two
-// splits, 15.1 in one, of 2048 35.4 and 27.0, two of 1024 26.7 and 16.1; of 128 over 8, causal, two of 1024 36.0 and 22.7.
+// Those are a query or a few a tile.  At fuller ones that count is only the most: fewer are taken where they cost a sixteenth
+// less.  A count costs its merge's launch, 2.8 us, its rows' partial states, written and read again at 0.7 us a MB, and a tile's steps, of
+// 0.33 + 0.006 d us with a workgroup to a compute unit.  The unit that holds the most of them sets the pace: two step in 1.4 times one's time,
+// three in 2.1, each further one in 0.6 more; a head of 256 leaves room for one alone.  So it is whole workgroups a
+// unit that count: 5 sequences of 179, 16 heads of 64, over 10531 keys are 71.9 us in three splits and 95.3 in two (320 workgroups, two on
+// some units as with 480), one of 200 over 8192 21.3 in eight and 24.0 in sixteen, one of 1024 over 1024 15.1 whole and 18.3 in two.
+// Over 257 drawn calls 0.93 times the time of the count above, none more than 1.04 times; causal ones, whose tiles see no key past
+// their own, 0.75.  With a bias a step waits for the bias (8 of 96 over 3757: 382 us whole, 210, 117 and 90 in two, four and six
+// splits), and the count above stays.
 // A window, a chunk mask or segment starts leave a tile few of the keys: the rule keeps those whole.
 static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t heads, int64_t kv_heads, int64_t d, int64_t tk,
                        int32_t decode_limit) {
@@ -421,18 +426,22 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
   const int64_t wanted = (512 + workgroups / 2) / workgroups;  // rounded
   const int64_t fits = most / 8;
   const int64_t n = std::min<int64_t>(std::min(wanted, fits), 64);
-  const int64_t tile_rows = std::min<int64_t>(grouped ? group * t : t, 128);
-  const double chain = (double)most * (0.25 + 0.0072 * (double)d);
-  const double states = (double)(batch * t * heads * (d + 2) * 4) * 0.65e-6;
+  if (n <= 1) return 1;
+  if (opts->bias != nullptr) return (int)n;
+  // The steps of the longest tile, and a compute unit's tiles' on average: a causal unit has long ones and short ones.
+  const int64_t longest = opts->causal ? std::min(most, (t + 127) / 128 * 2) : most;
+  const double mean = opts->causal ? 0.5 * (double)longest + 1.0 : (double)longest;
+  const double step = 0.33 + 0.006 * (double)d;
+  const double states = (double)(batch * t * heads * (d + 2) * 4) * 0.7e-6;
   auto cost = [&](int64_t s) {
-    // A tile of one wave's rows waits for its keys, which more workgroups hide; a fuller one for its compute unit.
-    const double rounds = tile_rows <= 32 ? 1.0 : std::max(1.0, (double)(workgroups * s) / 256);
-    return chain / (double)s * rounds + (s > 1 ? 2.5 + states * (double)s : 0.0);
+    const int64_t a_unit = (workgroups * s + 255) / 256;
+    const double pace = d > 128 ? (double)a_unit : a_unit <= 1 ? 1.0 : a_unit == 2 ? 1.4 : 2.1 + 0.6 * (double)(a_unit - 3);
+    return std::max((double)longest, mean * pace) / (double)s * step + (s > 1 ? 2.8 + states * (double)s : 0.0);
   };
   int64_t best = 1;
   for (int64_t s = 2; s <= n; s++)
     if (cost(s) < cost(best)) best = s;
-  return (int)best;
+  return (int)(cost(best) > 0.94 * cost(n) ? n : best);
 }
 
 // attend (tk/src/ops/attention.rs:126-303): attention of q, k and v, or of the `packed` operand
