@@ -327,7 +327,8 @@ int svodk_plan_norm(int32_t has_target, const int32_t *dtypes, int32_t n_dtypes,
  * with head size 64, no key mask tensor, no window and no splits can run as "streaming"
  * workgroups that each walk a run of query tiles, the next tile's keys loading under the
  * current tile's last steps.  n > 0 = stream, n workgroups per XCD (96 fills an MI355X);
- * n <= 0 (the default) = a workgroup per tile.  Process-wide.  Results are bit-equal either way.
+ * n <= 0 (the default) = a workgroup per tile.  A call that takes a tile's keys in two halves (svodk_attn.splits) keeps
+ * that form.  Process-wide.  Results are bit-equal either way.
  *
  * A streaming launch hands out its tiles through one of SVODK_STREAMING_SETS sets of counters in
  * device memory, taken in turn at enqueue time and put back to zero by the launch's last

@@ -799,7 +799,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
   // (A call that allocates nothing answers what one that keeps its keys whole does, bit for bit.)
-  a.halves = opts->splits <= 0 && a.splits == 1 && !own_scratch;
+  a.halves = opts->splits <= 0 && a.splits == 1 && !own_scratch && svodk::attention_halves(a);
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));

@@ -308,7 +308,8 @@ def noalloc_scratch_bytes() -> int:
 def tune_streaming(workgroups_per_xcd: int) -> None:
     """n > 0 = attention calls that can (head size 64, lengths or no key mask, no window, no splits)
     run as n streaming workgroups per XCD, each walking a run of query tiles; n <= 0 (the default)
-    = a workgroup per tile.  Process-wide; results are bit-equal either way."""
+    = a workgroup per tile.  A call that takes a tile's keys in two halves (``Attn.splits``) keeps that form.
+    Process-wide; results are bit-equal either way."""
     load_library().svodk_tune_streaming(int(workgroups_per_xcd))
 
 
