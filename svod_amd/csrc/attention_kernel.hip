@@ -1524,8 +1524,8 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 :
 }
 
 #if !defined(SVODK_CODE_OBJECT)
-// Eight waves a query tile, two a SIMD, where a launch has no more workgroups than the chip has compute units (attention_halves() says
-// when): plain calls, with key lengths, a key mask or none.  Bound by the steps of a tile in a row, as the form of four waves is
+// Eight waves a query tile, two a SIMD, where a launch has no more workgroups than the chip has compute units (takes_halves() of
+// ops.cpp says when): plain calls, with key lengths, a key mask or none.  Bound by the steps of a tile in a row, as the form of four waves is
 // there; two waves of a SIMD hide each other's waits (a step of a side 1.2 times as long as alone, for half of them).
 template <int D, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED>
 constexpr bool kHasPair = (D == 64 || D == 128) && !SPLIT && !RANGED && !BIASED && !GROUPED;
@@ -2158,26 +2158,6 @@ bool attention_groups(const AttnArgs &a) {
   const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
   const int64_t group = a.kv_heads > 0 ? a.heads / a.kv_heads : 1;
   return group > 1 && !a.causal && !ranged && group * a.t <= 128;
-}
-
-// A compute unit with one workgroup has a wave a SIMD, and a tile's steps are a chain: two sides of four waves take half of
-// the steps each.  Both sides together step a fifth faster than one alone, so it is worth its merge (0.5 to 1 us) from
-// nine key blocks on (16 heads of 64: one sequence of 512 9.66 -> 9.40 us, of 768 12.7 -> 11.8, of 1500 22.0 -> 19.4, of 2048 28.6
-// -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
-// one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long
-// causal launches at d 128 win by, whose tiles would otherwise end far apart (512 workgroups of 16 tiles a head 59.4 -> 51.9, 384
-// of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Under a key mask the sides halve the blocks before
-// the row is read: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two of 1024 15.8 -> 13.9; 4 of 513, 12
-// heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.  Only a lone row that hides its second half leaves a side
-// idle (1024: 10.1 -> 10.7).
-bool attention_halves(const AttnArgs &a) {
-  const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
-  if ((a.d != 64 && a.d != 128) || a.decodes || a.cached || a.bias != nullptr || ranged || attention_groups(a)) return false;
-  // The launch's workgroups: a causal launch deals its (batch, KV head) units in whole rounds.
-  const int64_t tiles = ((int64_t)a.t + 127) / 128, units = (int64_t)a.kv_heads * a.batch;
-  const int64_t unit_size = (a.kv_heads > 0 ? a.heads / a.kv_heads : 0) * tiles;
-  const int64_t grid = a.causal ? (units + kXcds - 1) / kXcds * kXcds * unit_size : (units * unit_size + kXcds - 1) / kXcds * kXcds;
-  return (grid <= 256 || (a.causal && a.d == 128 && grid <= 512 && tiles >= 12)) && a.tk > 8 * kBkv;
 }
 
 void attention_stream_slots(int32_t slots) { g_stream_slots.store(slots, std::memory_order_relaxed); }

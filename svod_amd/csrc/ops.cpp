@@ -444,6 +444,28 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
   return (int)(cost(best) > 0.94 * cost(n) ? n : best);
 }
 
+// Whether an unsplit call that names no count of splits takes its tiles' keys in two halves (flash_fwd_pair_kernel), by its sizes alone.
+// A compute unit with one workgroup has a wave a SIMD, and a tile's steps are a chain: two sides of four waves take half of
+// the steps each.  Both sides together step a fifth faster than one alone, so it is worth its merge (0.5 to 1 us) from
+// nine key blocks on (16 heads of 64: one sequence of 512 9.66 -> 9.40 us, of 768 12.7 -> 11.8, of 1500 22.0 -> 19.4, of 2048 28.6
+// -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
+// one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long
+// causal launches at d 128 win by, whose tiles would otherwise end far apart (512 workgroups of 16 tiles a head 59.4 -> 51.9, 384
+// of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Under a key mask the sides halve the blocks before
+// the row is read: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two of 1024 15.8 -> 13.9; 4 of 513, 12
+// heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.  Only a lone row that hides its second half leaves a side
+// idle (1024: 10.1 -> 10.7).
+static bool takes_halves(const svodk::AttnArgs &a) {
+  const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
+  const int64_t group = a.kv_heads > 0 ? a.heads / a.kv_heads : 1;
+  const bool grouped = group > 1 && !a.causal && group * a.t <= 128;
+  if ((a.d != 64 && a.d != 128) || a.decodes || a.cached || a.bias != nullptr || ranged || grouped) return false;
+  // The launch's workgroups: a causal launch deals its (batch, KV head) units over the 8 XCDs in whole rounds.
+  const int64_t tiles = ((int64_t)a.t + 127) / 128, units = (int64_t)a.kv_heads * a.batch;
+  const int64_t grid = a.causal ? (units + 7) / 8 * 8 * group * tiles : (units * group * tiles + 7) / 8 * 8;
+  return (grid <= 256 || (a.causal && a.d == 128 && grid <= 512 && tiles >= 12)) && a.tk > 512;
+}
+
 // attend (tk/src/ops/attention.rs:126-303): attention of q, k and v, or of the `packed` operand
 // they are views of.
 // `own_scratch`: the partial states of a split call go to the library's static device array instead
@@ -799,7 +821,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
   // (A call that allocates nothing answers what one that keeps its keys whole does, bit for bit.)
-  a.halves = opts->splits <= 0 && a.splits == 1 && !own_scratch && svodk::attention_halves(a);
+  a.halves = opts->splits <= 0 && a.splits == 1 && !own_scratch && takes_halves(a);
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);
   if (e != hipSuccess) return fail(SVODK_ERR_LAUNCH, "%s: %s", op, hipGetErrorString(e));
