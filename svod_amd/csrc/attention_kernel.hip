@@ -2166,16 +2166,20 @@ const char *attention_config(const AttnArgs &a) {
   if (a.decodes)
     return a.splits > 1 ? "FaCfg { rows: 4, lanes_per_key: d / 8, splits: n, core: v_dot2_f32, keys streamed through registers }"
                         : "FaCfg { rows: 4, lanes_per_key: d / 8, splits: 1, core: v_dot2_f32, keys streamed through registers }";
-  static const char *const kCfg[2][2] = {
+  static const char *const kCfg[2][3] = {
       {"FaCfg { bq: 128, bkv: 64, stages: 2, splits: 1, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
+       "mfma_f32_32x32x16_bf16 }",
+       "FaCfg { bq: 128, bkv: 64, stages: 2, splits: 1, sides: 2, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
        "mfma_f32_32x32x16_bf16 }",
        "FaCfg { bq: 128, bkv: 64, stages: 2, splits: n, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
        "mfma_f32_32x32x16_bf16 }"},
       {"FaCfg { bq: 128, bkv: 64, stages: 2, splits: 1, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
        "mfma_f32_32x32x16_f16 }",
+       "FaCfg { bq: 128, bkv: 64, stages: 2, splits: 1, sides: 2, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
+       "mfma_f32_32x32x16_f16 }",
        "FaCfg { bq: 128, bkv: 64, stages: 2, splits: n, forms: { raw_max, skip_rescale }, warp_rows: 32, core: "
        "mfma_f32_32x32x16_f16 }"}};
-  return kCfg[a.f16 ? 1 : 0][a.splits > 1 ? 1 : 0];
+  return kCfg[a.f16 ? 1 : 0][a.splits > 1 ? 2 : a.halves ? 1 : 0];
 }
 
 hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {

@@ -101,7 +101,7 @@ struct AttnArgs {
   // m_part and l_part [splits, batch, t, heads], all f32; launch_combine merges them.
   int32_t splits;
   float *o_part, *m_part, *l_part;
-  int32_t halves;    // a tile's keys go in two halves: decided once, launch_attention follows it
+  int32_t halves;    // a tile's keys go in two halves: decided once, launch_attention and attention_config follow it
   int32_t decodes;   // launch_decode's call (attention_decodes): decided once, launch_attention and attention_config follow it
   // A decoder step merges its splits itself: behind l_part the workspace has decode_arrival_bytes(a) more, of any content.
   int32_t merges;
