@@ -214,6 +214,7 @@ __device__ __forceinline__ i32x4 make_rsrc(const void *base, int64_t bytes) {
 constexpr unsigned kStream = 1;  // a workgroup walks several query tiles
 constexpr unsigned kRanged = 2;  // per-row key ranges: window, chunk mask, segment starts
 constexpr unsigned kBiased = 4;  // an additive bias joins the scaled scores
+constexpr unsigned kSided = 8;   // one of a tile's two sides: every other key block is this wave's
 
 // Everything a wave carries through the key loop.
 template <int D, int NW, bool F16, unsigned FLAGS>
@@ -221,6 +222,7 @@ struct Wave {
   static constexpr int KS = D / 16;               // k-steps of the score product
   static constexpr int DB = Tile<D>::kWide / 32;  // 32-row blocks of O^T
   static constexpr int CH = Tile<D>::kInstrs / NW;  // fills per wave per tile
+  static constexpr int kStep = (FLAGS & kSided) ? 2 * kBkv : kBkv;  // keys from one of its blocks to the next
   // block constants
   const uint8_t *k_base, *v_base;
   int64_t kv_bytes;  // bytes of this (batch, kv head)'s rows below the length
@@ -284,7 +286,7 @@ __device__ __forceinline__ void fill_tile(const Wave<D, NW, F16, FLAGS> &w, cons
   constexpr int kRowsPer = 64 / Tile<D>::kCpr;  // rows a wave instruction covers
   constexpr int NS = Tile<D>::sources(NW);
   static_assert((NS * NW * kRowsPer) % 16 == 0, "the swizzle repeats over a wave's fills");
-  const int64_t off = (int64_t)blk * kBkv * row_bytes;
+  const int64_t off = (int64_t)blk * Wave<D, NW, F16, FLAGS>::kStep * row_bytes;
   const i32x4 r = make_rsrc(base + off, bytes - off);
 #pragma unroll
   for (int i = 0; i < Wave<D, NW, F16, FLAGS>::CH; i++) {
@@ -319,7 +321,7 @@ __device__ __forceinline__ void fill_v(const Wave<D, NW, F16, FLAGS> &w, int n, 
 // before that block's fills and is long back when the block's step needs it.
 template <int D, int NW, bool F16, unsigned FLAGS>
 __device__ __forceinline__ int mask_lane(const Wave<D, NW, F16, FLAGS> &w, int blk) {
-  const int key = blk * kBkv + w.lane;
+  const int key = blk * w.kStep + w.lane;
   if (w.key_mask == nullptr || key >= w.tk) return 0;
   const int64_t at = w.mask_row + key;
   return w.mask_bytes == 1 ? (int)((const uint8_t *)w.key_mask)[at] : ((const int *)w.key_mask)[at];
@@ -347,11 +349,11 @@ __device__ __forceinline__ void scores(const Wave<D, NW, F16, FLAGS> &w, const u
   }
 }
 
-// The wave-uniform part of block `blk`'s mask: bit j = key 64 blk + j is below the length and
+// The wave-uniform part of block `blk`'s mask: bit j = the block's key j is below the length and
 // kept by the key mask (`word` is this lane's key-mask element of the block).
 template <int D, int NW, bool F16, unsigned FLAGS>
 __device__ __forceinline__ uint64_t uniform_bits(const Wave<D, NW, F16, FLAGS> &w, int blk, int word) {
-  const int k0 = blk * kBkv;
+  const int k0 = blk * w.kStep;
   uint64_t kbits = ~0ull;
   if (w.key_mask != nullptr) {
     if (w.scanned) {
@@ -414,7 +416,7 @@ __device__ __forceinline__ void add_bias(const uint32_t (&bw)[16], float (&sv)[3
 // Whether a mask edge crosses block `blk` for this wave (L698-733).
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
 __device__ __forceinline__ bool on_edge(const Wave<D, NW, F16, FLAGS> &w, int blk, uint64_t kbits) {
-  const int k0 = blk * kBkv;
+  const int k0 = blk * w.kStep;
   if (kbits != ~0ull) return true;
   // L715-731: a range's right edge for the wave's first row, its left edge for the last.
   if (w.ranged) return k0 + kBkv - 1 > w.hi_first || k0 < w.lo_last;
@@ -431,7 +433,7 @@ __device__ __forceinline__ bool on_edge(const Wave<D, NW, F16, FLAGS> &w, int bl
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
 __device__ __forceinline__ int halves_seen(const Wave<D, NW, F16, FLAGS> &w, int blk, uint64_t kbits) {
   if (D > 64) return 3;
-  const int k0 = blk * kBkv;
+  const int k0 = blk * w.kStep;
   const int last = w.ranged ? w.hi_last : CAUSAL ? w.wave_first_row + kWaveRows - 1 : 0x7fffffff;
   int seen = ((uint32_t)kbits != 0 && k0 <= last ? 1 : 0) | ((uint32_t)(kbits >> 32) != 0 && k0 + 32 <= last ? 2 : 0);
   if (w.ranged && k0 + 31 < w.lo_first) seen &= k0 + 63 < w.lo_first ? 0 : 2;
@@ -461,7 +463,7 @@ __device__ __forceinline__ void hide_scores(uint64_t mine, float (&sv)[32]) {
 // scores become -inf.  `kbits` is the uniform word; causality adds a per-lane one.
 template <int D, int NW, bool CAUSAL, bool F16, unsigned FLAGS>
 __device__ __forceinline__ void mask_scores(const Wave<D, NW, F16, FLAGS> &w, int blk, uint64_t kbits, float (&sv)[32]) {
-  const int k0 = blk * kBkv;
+  const int k0 = blk * w.kStep;
   uint64_t mine = kbits;
   if (w.ranged) {
     // Keys k0 .. row_hi are seen from above and those from row_lo on from below (L659-695).
@@ -822,7 +824,7 @@ struct TailOf {
 // ring, and behind it mask_lds() of a launch with a key mask).  Device code only:
 // the host pass needs a kernel's handle, not its instructions (and would drop the whole
 // instantiation over the LDS-fill instructions).
-// SIDES = 2: eight waves a tile instead of four.  Each side of four has a ring of its own and takes half of the tile's key
+// SIDES = 2: eight waves a tile instead of four.  Each side of four has a ring of its own and takes every other of the tile's key
 // blocks; the sides' states merge through LDS (flash_fwd_pair_kernel).
 #if defined(__HIP_DEVICE_COMPILE__)
 template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16, int SIDES = 1>
@@ -840,7 +842,7 @@ __device__ __forceinline__ void flash_fwd_body(
   const int tk = (int)(tk_lens64 & 0x7fffffffu);
   const bool lens_i64 = (tk_lens64 >> 31) != 0;
   using TL = Tile<D>;
-  using W = Wave<D, NW, F16, (RANGED ? kRanged : 0u) | (BIASED ? kBiased : 0u)>;
+  using W = Wave<D, NW, F16, (RANGED ? kRanged : 0u) | (BIASED ? kBiased : 0u) | (SIDES == 2 ? kSided : 0u)>;
   constexpr int BQ = NW * kWaveRows;
   constexpr int KS = W::KS, DB = W::DB;
   static_assert(TL::kInstrs % NW == 0, "the tile fills in whole wave instructions per wave");
@@ -1048,17 +1050,18 @@ __device__ __forceinline__ void flash_fwd_body(
     end = first + (int)div_by(n * (uint32_t)(split + 1), sp.count, sp.rcp);
     first = s_first;
   }
-  // A side takes half of them, in the same way; both meet as many barriers as the first, which has no fewer.
+  int first_key = first * kBkv;
+  end -= first;
+  // A side takes every other one of them, so that what a length, a key mask or the diagonal hides is hidden from both; both meet as
+  // many barriers as the first, which has no fewer.  (Halves in a row left a side idle where a mask hid its keys: 5 rows of 1897, 3 heads
+  // of 64, that show the first 512 12.3 us in four waves, 14.1 so, 12.4 now; one of 3560, 27 % of it, 19.2, 20.6 and 17.7.  Over 32 such
+  // calls 1.06 times four waves' time so, 0.97 now, over 139 causal ones 0.987 times what halves in a row took.)
   int steps = 0;
   if (SIDES == 2) {
-    steps = (end - first + 1) / 2;
-    if (side == 0)
-      end = first + steps;
-    else
-      first += steps;
+    steps = (end + 1) / 2;
+    end = (end + 1 - side) / 2;
+    first_key += side * kBkv;
   }
-  const int first_key = first * kBkv;
-  end -= first;
   len = max(len - first_key, 0);
   w.end = end;
   w.len = len;
@@ -1156,7 +1159,7 @@ __device__ __forceinline__ void flash_fwd_body(
     const int at = (int)(uintptr_t)(raw);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int voff = ((w.wave + NW * i) * kBkv + w.lane) * mask_bytes;
+      const int voff = ((w.wave + NW * i) * W::kStep + w.lane) * mask_bytes;
       if (mask_bytes == 1)
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ubyte %1, %2, 0 offen lds"
                      :
@@ -1200,7 +1203,7 @@ __device__ __forceinline__ void flash_fwd_body(
       // wait brings them in.
       int words[8];
       auto element_at = [&](int i, bool &there) {
-        const int key = (base + NW * i) * kBkv + w.lane;
+        const int key = (base + NW * i) * W::kStep + w.lane;
         there = base + NW * i < end && key < w.tk;
         return w.mask_row + (there ? key : 0);
       };
@@ -1282,7 +1285,7 @@ __device__ __forceinline__ void flash_fwd_body(
     if (seen_end <= lead_open + (part != 0 ? 1 : 0) && (part & (part + 1)) == 0) {
       // The row shows exactly its first keys (a padding mask): that is a length, and from here on the row runs as one
       // with a length does: no mask word per block, rows past the length never fetched.
-      len = min(len, lead_open * kBkv + __builtin_popcountll(part));
+      len = min(len, lead_open * W::kStep + __builtin_popcountll(part));
       w.len = len;
       w.key_mask = nullptr;
       w.scanned = false;
@@ -1306,7 +1309,7 @@ __device__ __forceinline__ void flash_fwd_body(
   if (RANGED || CAUSAL) {
     // The last key the wave's last row sees; negative: the blocks lie past every row's reach.
     const int last_seen = RANGED ? w.hi_last : w.wave_first_row + kWaveRows - 1;
-    my_end = min(my_end, last_seen < 0 ? 0 : last_seen / kBkv + 1);
+    my_end = min(my_end, last_seen < 0 ? 0 : last_seen / W::kStep + 1);
   }
 
   float sv[32], nv[32];  // S of the current and of the next block, swapping roles each hot step
@@ -1328,20 +1331,28 @@ __device__ __forceinline__ void flash_fwd_body(
     if (on_edge<D, NW, CAUSAL>(w, 0, kbits0)) mask_scores<D, NW, CAUSAL>(w, 0, kbits0, sv);
     bm = row_max(sv);
   }
+  // Under a key mask each side tells the other how many blocks the row left it: neither goes on to steps that both would idle through.
+  if (SIDES == 2 && key_mask != nullptr && w.wave == 0) *(LDS_PTR(int))(mask_smem + kScannedBlocks * 8) = end;
   // Step 0 refills the K slot those scores were read from: every wave has read it first.
   __syncthreads();
+  if (SIDES == 2 && key_mask != nullptr) {
+    const int stretch = side == 0 ? mask_lds(NW) : -mask_lds(NW);
+    const int others = *(LDS_PTR(int))(mask_smem + stretch + kScannedBlocks * 8);
+    steps = max(end, __builtin_amdgcn_readfirstlane(others));
+  }
 
   // Blocks [0, full) are crossed by no mask edge for this wave: they lie below the length and,
   // for a causal wave, below its first row's diagonal.  A key mask puts every block on the
   // edge path.  Step j is hot when block j+1 is such a block.
   int full = 0;
   if (w.positive && (w.key_mask == nullptr || w.scanned)) {
-    full = min(my_end, len / kBkv);
+    constexpr int kOver = W::kStep - kBkv;  // keys behind a block that are not this wave's
+    full = min(my_end, (len + kOver) / W::kStep);
     if (w.scanned) full = min(full, lead_open);
     if (RANGED)
       full = min(full, w.hi_first < 0 ? 0 : (w.hi_first + 1) / kBkv);
     else if (CAUSAL)
-      full = min(full, (w.wave_first_row + 1) / kBkv);
+      full = min(full, (w.wave_first_row + 1 + kOver) / W::kStep);
   }
   int blk = 0;
   if (RANGED) {

@@ -451,10 +451,8 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
 // -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
 // one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long
 // causal launches at d 128 win by, whose tiles would otherwise end far apart (512 workgroups of 16 tiles a head 59.4 -> 51.9, 384
-// of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Under a key mask the sides halve the blocks before
-// the row is read: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two of 1024 15.8 -> 13.9; 4 of 513, 12
-// heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.  Only a lone row that hides its second half leaves a side
-// idle (1024: 10.1 -> 10.7).
+// of 12 36.8 -> 35.0, 336 of 7 23.8 -> 25.0).  Under a key mask: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two
+// of 1024 15.8 -> 13.9; 4 of 513, 12 heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.
 static bool takes_halves(const svodk::AttnArgs &a) {
   const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
   const int64_t group = a.kv_heads > 0 ? a.heads / a.kv_heads : 1;
