@@ -180,13 +180,14 @@ int svodk_attention(const svodk_tensor *q, const svodk_tensor *k, const svodk_te
  * svodk_attention for callers that cannot allocate device memory (code under HIP graph capture, a
  * serving loop with a fixed memory plan, a harness that forbids hipMalloc).  It has no counterpart
  * in the reference, whose op allocates the partial tensors of a split call itself
- * (tk/src/ops/attention.rs:285-293).  Same operands, options, checks, kernels and results as
- * svodk_attention; the one difference is where the partial states of a split call live: in a
- * static device array of the library, svodk_noalloc_scratch_bytes() (8 MiB) on each GPU the library
+ * (tk/src/ops/attention.rs:285-293).  Same operands, options and checks as svodk_attention.  The
+ * partial states of a split call live in a static device array of the library,
+ * svodk_noalloc_scratch_bytes() (8 MiB) on each GPU the library
  * runs on, held until the process ends.  `opts->workspace` is ignored.  The call and everything
  * under it allocate nothing.  With `splits` = 0 the count is chosen as if a workspace had been lent
- * and then lowered to what the array holds (down to one split: the call runs unsplit, as
- * svodk_attention runs it without a workspace).  A call whose NAMED splits need more than the array
+ * and then lowered to what the array holds, down to one.  Kernels and results are svodk_attention's
+ * for that count; a call that is not split keeps its keys whole, as with `splits` = 1, and never
+ * takes a tile's keys in two halves.  A call whose NAMED splits need more than the array
  * holds answers SVODK_ERR_ARGUMENT and launches nothing; svodk_attention_workspace says how much a
  * call needs.  Every call on a GPU shares that GPU's
  * array: calls that overlap on one GPU (two streams, two threads) race on it and must be ordered

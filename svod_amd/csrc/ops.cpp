@@ -825,7 +825,7 @@ static int attend(const svodk_tensor *q, const svodk_tensor *k, const svodk_tens
     a.m_part = a.o_part + (int64_t)a.splits * rows * d;
     a.l_part = a.m_part + (int64_t)a.splits * rows;
   }
-  // (A call that allocates nothing answers what one that keeps its keys whole does, bit for bit.)
+  // (A call that allocates nothing keeps its keys whole, as one that names a count of 1: the same bits.)
   a.halves = opts->splits <= 0 && a.splits == 1 && !own_scratch && takes_halves(a);
   ran(op, "flash_attention", svodk::attention_config(a));
   hipError_t e = svodk::launch_attention(a, (hipStream_t)hip_stream);

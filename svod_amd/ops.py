@@ -297,7 +297,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, opts: Optional[
 def attention_noalloc(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, opts: Attn, out: torch.Tensor) -> torch.Tensor:
     """``attention`` through ``svodk_attention_noalloc``: the partial states of a split call live in
     the library's static device array (``noalloc_scratch_bytes()`` per GPU), nothing is allocated
-    below this call, and the caller brings ``out``.  No counterpart in the reference."""
+    below this call, and the caller brings ``out``.  With ``splits`` ``None`` the results are ``attention``'s for the count
+    that fits the array; an unsplit call keeps its keys whole, as ``splits`` 1 does.  No counterpart in the reference."""
     return (_native or _calls()).attention_noalloc(q, k, v, opts, out)
 
 
