@@ -755,10 +755,10 @@ struct Geometry {
 // The instantiations whose launches may run the short tiles of all units behind the others.
 template <bool CAUSAL, bool SPLIT, bool RANGED, bool GROUPED>
 constexpr bool kShortTilesLast = CAUSAL && !GROUPED && !SPLIT && !RANGED;
-// The instantiations whose last round of units, where it is not full, is shared out over all XCDs.  Causal ones deal it
-// whole: their tiles differ, and an XCD's run of them would be the long or the short ones.
-template <bool CAUSAL>
-constexpr bool kSharesLastRound = !CAUSAL;
+// The kernels built both with and without the sharing of a last round that is not full (launch() says when it is); the others
+// share always.  Causal ones deal it whole: their tiles differ, and an XCD's run of them would be the long or the short ones.
+template <bool CAUSAL, bool SPLIT, bool BIASED, bool CACHED>
+constexpr bool kChoosesToShare = !CAUSAL && !SPLIT && !BIASED && !CACHED;
 // The key splits of a launch that has them, and where their partial states go.
 struct Splits {
   uint32_t count, rcp;
@@ -827,7 +827,7 @@ struct TailOf {
 // SIDES = 2: eight waves a tile instead of four.  Each side of four has a ring of its own and takes every other of the tile's key
 // blocks; the sides' states merge through LDS (flash_fwd_pair_kernel).
 #if defined(__HIP_DEVICE_COMPILE__)
-template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16, int SIDES = 1>
+template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool CACHED, bool GROUPED, bool F16, int SIDES = 1, bool SHARES = !CAUSAL>
 __device__ __forceinline__ void flash_fwd_body(
     uint8_t *smem, uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u,
     uint32_t kvh_rcp, uint32_t units, uint32_t heads_group, const void *__restrict__ key_lens,
@@ -862,14 +862,9 @@ __device__ __forceinline__ void flash_fwd_body(
   // other traffic then runs a tenth behind the rest (measured: whichever XCD read bytes 384..511
   // of every KiB); turned, every XCD reads every residue and they finish together.
   uint32_t unit = round * kXcds + (wg + round) % kXcds;
-  if constexpr (kSharesLastRound<CAUSAL>) {
+  if constexpr (SHARES) {
     // The units of a round that is not full are every XCD's: their workgroups, one unit's after the other's, in eight equal
-    // runs.  Dealt whole, the XCDs that took one of them ran that much longer: one sequence of 12 heads of 64 over 8192 keys
-    // 302 -> 233 us, 3 of 777 20.0 -> 14.8, one of 20 heads over 1500 31.0 -> 23.3, of 10 heads of 128 over 2 over 3000 (two XCDs
-    // of eight at work) 148 -> 60; with 13 sequences of 700 (20 heads: 4 units of 260) 55.6 -> 54.9, at 8 and more rounds equal.
-    // A run lies in few units, so a unit's K and V are read by 8 / (units left) L2s, not by all.
-    // The rule's instructions are 0.04 us of every launch (9 of 333, 12 heads, 9.06 -> 9.09; 7 of 333 8.90 -> 8.46); out of line, or for
-    // under 64 units alone, they are no fewer.
+    // runs.  A run lies in few units, so a unit's K and V are read by 8 / (units left) L2s, not by all.
     if (round >= geo.units / kXcds) {
       const uint32_t first = geo.units / kXcds, left = (geo.units - first * kXcds) * geo.unit_size;
       const uint32_t run = (left + kXcds - 1) / kXcds, in = local - first * geo.unit_size, at = wg % kXcds * run + in;
@@ -1509,7 +1504,7 @@ __device__ __forceinline__ void flash_fwd_body(
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED, bool F16>
+template <int D, int NW, bool CAUSAL, bool SPLIT, bool RANGED, bool BIASED, bool GROUPED, bool F16, bool SHARES>
 __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 : 1)) void flash_fwd_kernel(
     uint32_t unit_size, uint32_t unit_rcp, uint32_t nqt_u, uint32_t nqt_rcp, uint32_t kvh_u, uint32_t kvh_rcp,
     uint32_t units, uint32_t heads_group, uint64_t key_lens, uint64_t row_order, int32_t t, uint32_t tk_lens64,
@@ -1527,7 +1522,7 @@ __global__ __launch_bounds__(NW * 64, (D <= 64 && !BIASED) ? 3 : (D <= 128 ? 2 :
   // they are what the workgroup's coordinates, its batch row and its length need, so none of those
   // waits for an argument load.
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, false, GROUPED, F16>(
+  flash_fwd_body<D, NW, CAUSAL, SPLIT, RANGED, BIASED, false, GROUPED, F16, 1, SHARES>(
       smem, unit_size, unit_rcp, nqt_u, nqt_rcp, kvh_u, kvh_rcp, units, heads_group, constant<void>(key_lens),
       constant<int32_t>(row_order), t, tk_lens64, tail.q, tail.k, tail.v, tail.o, key_mask,
       tail.mask_bytes, tail.scale, sp, tail.q_row_elems, tail.kv_row_elems, rg);
@@ -1941,7 +1936,14 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
   // out, or (a causal launch) the workgroups of its missing units exit at once.
   const int64_t unit_size = (int64_t)(GROUPED ? 1 : a.heads / a.kv_heads) * nqt;
   const int64_t units = (int64_t)a.kv_heads * a.batch;
-  const int64_t dealt = kSharesLastRound<CAUSAL> ? units * unit_size : (units + kXcds - 1) / kXcds * kXcds * unit_size;
+  // Dealt whole, the XCDs that take a unit of the last round run that much longer: one sequence of 12 heads of 64 over 8192 keys 302 us,
+  // 233 shared, 3 of 777 20.0 and 14.8, one of 20 heads over 1500 31.0 and 23.3, of 10 heads of 128 over 2 over 3000 (two XCDs of eight at
+  // work) 148 and 60.  The rule's instructions are 0.04 us of every launch, so a kernel without them runs where it gives nothing (260
+  // calls in both forms, shared times whole: up to 7 units 0.98 and, past 128 workgroups, 0.58; 8 to 15 units 1.00 and 0.93, 16 to 31 1.01 and
+  // 0.96, 32 to 47 1.01 and 0.995, 48 and more 1.005 and 1.00; units a multiple of eight have no last round).
+  const bool shares = !CAUSAL && (!kChoosesToShare<CAUSAL, SPLIT, BIASED, CACHED> || a.halves ||
+                                  (units % kXcds != 0 && (units < kXcds || (units < 48 && units * unit_size > 128))));
+  const int64_t dealt = shares ? units * unit_size : (units + kXcds - 1) / kXcds * kXcds * unit_size;
   const int64_t grid = (dealt + kXcds - 1) / kXcds * kXcds;
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   auto rcp = [](uint32_t d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); };
@@ -2049,10 +2051,15 @@ hipError_t launch(const AttnArgs &a, hipStream_t stream) {
         return pair(Launch<flash_fwd_pair_kernel<D, CAUSAL, F16, false>>{}, 2 * TL::kLds);
       }
     }
-    return Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16>>::run(
-        grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads, geo.kvh_rcp,
-        units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens, (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64,
-        a.key_mask, tail);
+    auto whole = [&](auto launcher) {
+      return decltype(launcher)::run(grid, NW * 64, smem, kMost, stream, geo.unit_size, geo.unit_rcp, geo.nqt, geo.nqt_rcp, geo.kv_heads,
+                                     geo.kvh_rcp, units_order, heads_group, (uint64_t)(uintptr_t)a.key_lens,
+                                     (uint64_t)(uintptr_t)a.row_order, a.t, tk_lens64, a.key_mask, tail);
+    };
+    if constexpr (kChoosesToShare<CAUSAL, SPLIT, BIASED, CACHED>) {
+      if (!shares) return whole(Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16, false>>{});
+    }
+    return whole(Launch<flash_fwd_kernel<D, NW, CAUSAL, SPLIT, RANGED, BIASED, GROUPED, F16, !CAUSAL>>{});
   }
 }
 
