@@ -112,8 +112,12 @@ typedef struct svodk_cache {
  * SVODK_GRAPH_CONFIG.  `splits` = 1 keeps the keys whole.  `splits` = 0 (None)
  * lets the library choose, as the reference's tuner would: it splits calls with
  * few query tiles and many keys (a decoder step) when the workspace
- * svodk_attention_workspace asks for is lent, and keeps them in one workgroup a query tile without it; where those
- * are no more than the compute units, a tile's key blocks go in two halves merged on the chip (by the call's sizes alone).
+ * svodk_attention_workspace asks for is lent, and keeps them in one workgroup a query tile without it.  A call that is
+ * not split then, over more than 512 keys (causal with D 128: and as many queries), with D 64 or 128 and no window, chunk
+ * mask, segment starts, bias or cache, takes a tile's key blocks in two halves that merge on the chip where it launches at
+ * most 256 workgroups of 128 queries a head, a causal call's counted in whole rounds of eight (batch, KV head)s; up to 512 for
+ * causal calls with D 128 whose heads have tiles enough.  Sizes alone decide; svodk_last_chosen names it ("sides: 2"); a
+ * row's last bits follow from the form, so from how many rows there are.
  * A decoder step (svodk_tune_decode) of up to 64 splits merges them itself, in the one launch, where
  * the workspace has 128 bytes a (batch, KV head) more than that; the same bits.  With `splits` = 0 and
  * twice the bytes and those words it takes the count that suits the device, up to twice the rule's (other

@@ -446,16 +446,16 @@ static int split_count(const svodk_attn *opts, int64_t batch, int64_t t, int64_t
 
 // Whether an unsplit call that names no count of splits takes its tiles' keys in two halves (flash_fwd_pair_kernel), by its sizes alone.
 // A compute unit with one workgroup has a wave a SIMD, and a tile's steps are a chain: two sides of four waves take half of
-// the steps each.  Both sides together step a fifth faster than one alone, so it is worth its merge (0.5 to 1 us) from
-// nine key blocks on (16 heads of 64: one sequence of 512 9.66 -> 9.40 us, of 768 12.7 -> 11.8, of 1500 22.0 -> 19.4, of 2048 28.6
-// -> 25.6, but 4 of 333 9.1 -> 9.25; of 128, causal: 512 14.0 both, 1024 22.4 -> 20.6, 2048 39.5 -> 36.0).  A unit holds
+// the steps each.  Two steps, one a side, take 1.6 times one alone's, so it is worth its merge (0.5 to 1 us) from
+// nine key blocks on (16 heads of 64: one sequence of 768 13.9 -> 12.7 us, of 1500 22.3 -> 19.5, of 2048 27.9 -> 24.8, but 4 of 333 9.1
+// -> 9.25; of 128 over 8, causal: 512 14.0 both, 1024 22.9 -> 21.0, 2048 39.1 -> 34.0).  A unit holds
 // one such workgroup: past 256 there is a second round of them (288: 32 to 63 us become a seventh more), which only long causal
 // launches at d 128 win by, whose tiles would otherwise end far apart, the longer the fuller that round is and where the heads of a
 // group share their keys (over 350 launches of up to 512 workgroups, times four waves': 12 to 14 tiles a head 0.85 up to 352, 1.12
 // above, 1.16 past 448, in groups 0.94 and 1.05; 15 to 17 0.89 up to 384, 1.03 past 448, in groups 0.88 to 0.97; 18 to 21 0.85 to 1.06;
 // from 22 on 0.78 to 0.86).  A causal tile sees no key past its queries: at d 128 136 of them over 691 keys took 8.2 us, and 8.9 in halves
-// (up to 256 queries 1.04 times, 385 to 512 0.98; at d 64 0.94 to 0.98 from 129 on).  Under a key mask: 16 heads of 64, one of 1024 15.5 -> 13.5 us, of 1500 20.9 -> 18.4, two
-// of 1024 15.8 -> 13.9; 4 of 513, 12 heads, 11.0 -> 10.2; 16 of 128, causal, one of 2048 37.4 -> 33.2.
+// (up to 256 queries 1.04 times, 385 to 512 0.98; at d 64 0.94 to 0.98 from 129 on).  Under a key mask: 16 heads of 64, one of 1024 17.5 -> 15.6 us, of 1500 23.7 -> 21.1, two
+// of 1024 17.4 -> 15.7; 4 of 513, 12 heads, 12.5 -> 12.0; 16 of 128 over 8, causal, one of 2048 41.2 -> 35.6.
 static bool takes_halves(const svodk::AttnArgs &a) {
   const bool ranged = a.win_left >= 0 || a.chunk_size > 0 || a.seg_start != nullptr;
   const int64_t group = a.kv_heads > 0 ? a.heads / a.kv_heads : 1;

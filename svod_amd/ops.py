@@ -254,7 +254,8 @@ class Attn:
     batch variable (``Batch::Var``): only the first ``batch_live`` batches run.
 
     ``splits`` ``None`` lets the library split the keys of a call with few queries, and take a query tile's keys in two halves
-    where the launch has a workgroup a compute unit or fewer (the call's sizes alone decide either).  In a decoder step of 4 to 64 rows with key
+    in a call over more than 512 keys that launches at most 256 workgroups (head sizes 64 and 128 without a window, a chunk, segments, a bias
+    or a cache; up to 512 for causal calls of 128 with long tiles): the call's sizes alone decide either.  In a decoder step of 4 to 64 rows with key
     lengths over a cache of 96 MiB or more the rows then share the splits out by their lengths, so that a row's last bits
     depend on how long the other rows are: the same sequence beside other neighbours may round differently.  A named count is
     every row's, and 1 keeps the keys whole: a row's bits then depend on how many rows there are, not on their lengths."""
